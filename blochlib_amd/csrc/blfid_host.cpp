@@ -152,9 +152,142 @@ void crystal_tensor(double pxx, double pyy, double pzz, double a, double b, doub
     C6[3] = 0.5 * (C[1] + C[3]); C6[4] = 0.5 * (C[2] + C[6]); C6[5] = 0.5 * (C[5] + C[7]);
 }
 
+// Device memory released by plans and states, kept for the next ones: allocating and freeing
+// took most of a one-call FID (a 5-spin pulse program's 10 ms of kernels sat in a 105 ms call, and
+// every table had its own allocation).  Per device at most CACHE_BYTES are held, in blocks a
+// request may take when it fills half of one (8/9 from 64 MiB up); a block that CACHE_AGE requests have passed
+// over is freed, and everything held is freed before an allocation is reported as failed.  A block
+// enters the cache only when the device has finished all work (as hipFree waits for it), so it may
+// be handed to any thread and stream.
+constexpr size_t CACHE_BYTES = (size_t)4 << 30;
+constexpr unsigned long CACHE_AGE = 256;
+constexpr int CACHE_DEVICES = 64;
+
+class DevCache {
+    struct Blk {
+        void *p;
+        size_t bytes;
+        unsigned long stamp;
+    };
+    std::mutex mu;
+    std::vector<Blk> blks[CACHE_DEVICES];
+    size_t held_[CACHE_DEVICES] = {0};
+    unsigned long clock[CACHE_DEVICES] = {0};
+
+    // takes every block older than `age` requests out of the list (the caller frees them)
+    void expire(int dev, unsigned long age, std::vector<void *> &out) {
+        auto &v = blks[dev];
+        for (size_t i = 0; i < v.size();) {
+            if (clock[dev] - v[i].stamp >= age) {
+                out.push_back(v[i].p);
+                held_[dev] -= v[i].bytes;
+                v[i] = v.back();
+                v.pop_back();
+            } else {
+                i++;
+            }
+        }
+    }
+    static void free_all(const std::vector<void *> &v) {
+        for (void *q : v) (void)hipFree(q);
+    }
+
+  public:
+    // At least `bytes` on the current device; *cap receives the block's size, *dev the device.
+    hipError_t get(size_t bytes, void **p, size_t *cap, int *dev) {
+        *p = nullptr;
+        hipError_t e = hipGetDevice(dev);
+        if (e != hipSuccess) return e;
+        const bool kept = *dev >= 0 && *dev < CACHE_DEVICES;
+        // sizes in steps of 64 KiB, 2 MiB from 1 MiB up, so that like requests share blocks
+        const size_t step = bytes < ((size_t)1 << 20) ? (size_t)1 << 16 : (size_t)1 << 21;
+        const size_t want = (bytes + step - 1) / step * step;
+        const size_t most = want < ((size_t)64 << 20) ? 2 * want : want + want / 8;
+        if (kept) {
+            std::vector<void *> old;
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                clock[*dev]++;
+                auto &v = blks[*dev];
+                size_t best = v.size();
+                for (size_t i = 0; i < v.size(); i++)
+                    if (v[i].bytes >= bytes && v[i].bytes <= most &&
+                        (best == v.size() || v[i].bytes < v[best].bytes))
+                        best = i;
+                if (best < v.size()) {
+                    *p = v[best].p;
+                    *cap = v[best].bytes;
+                    held_[*dev] -= v[best].bytes;
+                    v[best] = v.back();
+                    v.pop_back();
+                }
+                expire(*dev, CACHE_AGE, old);
+            }
+            free_all(old);
+            if (*p) return hipSuccess;
+        }
+        *cap = want;
+        e = hipMalloc(p, want);
+        if (e == hipErrorOutOfMemory && kept) {
+            (void)hipGetLastError();
+            std::vector<void *> old;
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                expire(*dev, 0, old);
+            }
+            free_all(old);
+            *cap = bytes;
+            e = hipMalloc(p, bytes);
+        }
+        if (e != hipSuccess) *p = nullptr;
+        return e;
+    }
+    // A block no work uses any more: the device is waited for first.
+    void put(void *p, size_t cap, int dev) {
+        int cur = dev;
+        (void)hipGetDevice(&cur);
+        if (cur != dev) (void)hipSetDevice(dev);
+        const bool idle = hipDeviceSynchronize() == hipSuccess;
+        std::vector<void *> old;
+        if (idle && dev >= 0 && dev < CACHE_DEVICES && cap <= CACHE_BYTES) {
+            std::lock_guard<std::mutex> lk(mu);
+            auto &v = blks[dev];
+            v.push_back({p, cap, clock[dev]});
+            held_[dev] += cap;
+            while (held_[dev] > CACHE_BYTES) { // the longest unused block goes first
+                size_t o = 0;
+                for (size_t i = 1; i < v.size(); i++)
+                    if (v[i].stamp < v[o].stamp) o = i;
+                old.push_back(v[o].p);
+                held_[dev] -= v[o].bytes;
+                v[o] = v.back();
+                v.pop_back();
+            }
+        } else {
+            old.push_back(p);
+        }
+        free_all(old);
+        if (cur != dev) (void)hipSetDevice(cur);
+    }
+    // Bytes held for the current device: free memory as far as a memory budget is concerned.
+    size_t held() {
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= CACHE_DEVICES) return 0;
+        std::lock_guard<std::mutex> lk(mu);
+        return held_[dev];
+    }
+};
+// never destroyed: objects released while the process ends must not outlive it
+DevCache &dev_cache() {
+    static DevCache *c = new DevCache();
+    return *c;
+}
+
 template <typename T> struct DevBuf {
     T *p = nullptr;
-    size_t n = 0;
+    size_t n = 0;   // elements asked for
+    size_t cap = 0; // bytes of the block
+    int dev = 0;
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
@@ -162,19 +295,42 @@ template <typename T> struct DevBuf {
     hipError_t alloc(size_t cnt) {
         if (cnt <= n && p) return hipSuccess;
         release();
-        n = cnt;
         if (cnt == 0) return hipSuccess;
-        return hipMalloc((void **)&p, cnt * sizeof(T));
+        const hipError_t e = dev_cache().get(cnt * sizeof(T), (void **)&p, &cap, &dev);
+        if (e == hipSuccess) n = cnt;
+        return e;
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) dev_cache().put(p, cap, dev);
         p = nullptr;
         n = 0;
+        cap = 0;
     }
-    hipError_t upload(const std::vector<T> &v) {
-        hipError_t e = alloc(v.size() ? v.size() : 1);
-        if (e != hipSuccess || v.empty()) return e;
-        return hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice);
+};
+
+// A table inside a Tables block.
+template <typename T> struct DevTab {
+    T *p = nullptr;
+};
+
+// Host tables gathered into one device block with one copy; every table starts on 256 bytes.
+class Tables {
+    std::vector<char> h;
+    std::vector<std::pair<void **, size_t>> at;
+
+  public:
+    template <typename T> void add(DevTab<T> &t, const std::vector<T> &v, size_t least = 0) {
+        const size_t n = std::max<size_t>({v.size(), least, (size_t)1});
+        const size_t o = h.size();
+        h.resize(o + ((n * sizeof(T) + 255) & ~(size_t)255), 0);
+        if (!v.empty()) std::memcpy(h.data() + o, v.data(), v.size() * sizeof(T));
+        at.push_back({(void **)&t.p, o});
+    }
+    hipError_t commit(DevBuf<char> &buf) {
+        hipError_t e = buf.alloc(h.size());
+        if (e == hipSuccess) e = hipMemcpy(buf.p, h.data(), h.size(), hipMemcpyHostToDevice);
+        for (auto &q : at) *q.first = e == hipSuccess ? buf.p + q.second : nullptr;
+        return e;
     }
 };
 
@@ -200,12 +356,15 @@ struct blfid_workspace {
 // N x N complex128 matrices, column-major, plus the powder's rotations and weights.
 struct blfid_state {
     int S = 0, N = 0, K = 0;
-    DevBuf<double> d_th, d_ph, d_ga, d_w, d_RP;
+    DevBuf<char> tab, ptab, ttab; // powder, propagator and trace tables
+    DevTab<double> d_th, d_ph, d_ga, d_w;
+    DevBuf<double> d_RP;
     DevBuf<double2> rho;   // K N^2
     DevBuf<double2> rho0;  // staging of blfid_state_set / blfid_state_load
     DevBuf<char> ws;       // propagators and product slots of blfid_state_apply
-    DevBuf<int> sblk, sloc, nzi;
-    DevBuf<double> nzv, part, grp, out;
+    DevTab<int> sblk, sloc, nzi;
+    DevTab<double> nzv;
+    DevBuf<double> part, grp, out;
     double budget = 0;
 };
 
@@ -266,25 +425,27 @@ struct blfid_plan {
     int K = 0;
     bool rp_dirty = false;      // cartPowder of the new powder still to be formed (in run)
     // device
-    DevBuf<double> d_terms, d_dconst, d_ffconst, d_u3, d_RP, d_th, d_ph, d_ga, d_w;
-    DevBuf<int> d_ff_off, d_ff_term;
-    DevBuf<double> d_xd_cst, d_xd_fpr;
-    DevBuf<int> d_blk_dim, d_blk_soff, d_blk_states, d_pair_I, d_pair_J, d_pair_doff,
+    DevBuf<char> tab_plan, tab_ops, tab_powder, tab_prep; // blocks the tables below lie in
+    DevTab<double> d_terms, d_dconst, d_ffconst, d_u3, d_th, d_ph, d_ga, d_w;
+    DevBuf<double> d_RP;
+    DevTab<int> d_ff_off, d_ff_term;
+    DevTab<double> d_xd_cst, d_xd_fpr;
+    DevTab<int> d_blk_dim, d_blk_soff, d_blk_states, d_pair_I, d_pair_J, d_pair_doff,
         d_pair_roff, d_drow, d_dcol, d_rrow, d_rcol, d_er, d_es, d_erev;
-    DevBuf<long> d_blk_uoff, d_pair_eoff;
-    DevBuf<double> d_dval, d_rval;
-    std::map<int, DevBuf<int>> d_bgrp, d_pgrp, d_fgrp;
-    DevBuf<int> d_bigb, d_xd_off, d_xd_list;
-    std::map<int, DevBuf<int>> d_eig_cls;
-    DevBuf<int> d_spin_rf;
-    DevBuf<double> d_rf, d_thetak;
+    DevTab<long> d_blk_uoff, d_pair_eoff;
+    DevTab<double> d_dval, d_rval;
+    std::map<int, DevTab<int>> d_bgrp, d_pgrp, d_fgrp;
+    DevTab<int> d_bigb, d_xd_off, d_xd_list;
+    std::map<int, DevTab<int>> d_eig_cls;
+    DevTab<int> d_spin_rf;
+    DevTab<double> d_rf, d_thetak;
     // pulses applied to rho before the gamma-COMPUTE FID (blfid_plan_set_prep): a pulse plan for
     // the preparation propagator of each crystallite, its state -> (block, local index) maps, and
     // the nonzero entries (a, b, re, im) of rho, from which the prepared blocks are formed
     blfid_plan *prep = nullptr;
     double prep_rotor = 0;
-    DevBuf<int> d_prep_sblk, d_prep_sloc, d_rho_nzi;
-    DevBuf<double> d_rho_nzv;
+    DevTab<int> d_prep_sblk, d_prep_sloc, d_rho_nzi;
+    DevTab<double> d_rho_nzv;
     int rho_nnz = 0;
     // or: each crystallite's rho taken from a state (blfid_plan_set_state), not owned
     blfid_state *state = nullptr;
@@ -657,31 +818,33 @@ static blfid_status build_tables(blfid_plan *pl) {
 }
 
 static blfid_status upload_tables(blfid_plan *pl) {
-    HIPCHK(pl->d_terms.upload(pl->terms));
-    HIPCHK(pl->d_dconst.upload(pl->dconst));
-    HIPCHK(pl->d_ffconst.upload(pl->ffconst));
-    HIPCHK(pl->d_ff_off.upload(pl->ff_off));
-    HIPCHK(pl->d_ff_term.upload(pl->ff_term));
-    HIPCHK(pl->d_xd_cst.upload(pl->xd_cst));
-    HIPCHK(pl->d_xd_fpr.upload(pl->xd_fpr));
-    HIPCHK(pl->d_u3.upload(pl->u3));
-    HIPCHK(pl->d_blk_dim.upload(pl->blk_dim));
-    HIPCHK(pl->d_blk_soff.upload(pl->blk_soff));
-    HIPCHK(pl->d_blk_states.upload(pl->blk_states));
-    HIPCHK(pl->d_blk_uoff.upload(pl->blk_uoff));
-    for (auto &kv : pl->blk_groups) HIPCHK(pl->d_bgrp[kv.first].upload(kv.second));
-    for (auto &kv : pl->fuse_groups) HIPCHK(pl->d_fgrp[kv.first].upload(kv.second));
-    HIPCHK(pl->d_bigb.upload(pl->big_blocks));
-    HIPCHK(pl->d_xd_off.upload(pl->xd_off));
-    HIPCHK(pl->d_xd_list.upload(pl->xd_list));
-    for (auto &kv : pl->eig_cls) HIPCHK(pl->d_eig_cls[kv.first].upload(kv.second));
-    HIPCHK(pl->d_spin_rf.upload(pl->spin_rf));
-    HIPCHK(pl->d_rf.upload(pl->rf));
+    Tables t;
+    t.add(pl->d_terms, pl->terms);
+    t.add(pl->d_dconst, pl->dconst);
+    t.add(pl->d_ffconst, pl->ffconst);
+    t.add(pl->d_ff_off, pl->ff_off);
+    t.add(pl->d_ff_term, pl->ff_term);
+    t.add(pl->d_xd_cst, pl->xd_cst);
+    t.add(pl->d_xd_fpr, pl->xd_fpr);
+    t.add(pl->d_u3, pl->u3);
+    t.add(pl->d_blk_dim, pl->blk_dim);
+    t.add(pl->d_blk_soff, pl->blk_soff);
+    t.add(pl->d_blk_states, pl->blk_states);
+    t.add(pl->d_blk_uoff, pl->blk_uoff);
+    for (auto &kv : pl->blk_groups) t.add(pl->d_bgrp[kv.first], kv.second);
+    for (auto &kv : pl->fuse_groups) t.add(pl->d_fgrp[kv.first], kv.second);
+    t.add(pl->d_bigb, pl->big_blocks);
+    t.add(pl->d_xd_off, pl->xd_off);
+    t.add(pl->d_xd_list, pl->xd_list);
+    for (auto &kv : pl->eig_cls) t.add(pl->d_eig_cls[kv.first], kv.second);
+    t.add(pl->d_spin_rf, pl->spin_rf);
+    t.add(pl->d_rf, pl->rf);
     if (!pl->step_dt.empty()) {
         std::vector<double> th(pl->step_dt.size());
         for (size_t k = 0; k < th.size(); k++) th[k] = PI2 * pl->step_dt[k];
-        HIPCHK(pl->d_thetak.upload(th));
+        t.add(pl->d_thetak, th);
     }
+    HIPCHK(t.commit(pl->tab_plan));
     return BLFID_OK;
 }
 
@@ -1016,10 +1179,15 @@ blfid_status blfid_plan_set_prep(blfid_plan *pl, double rotor_deg, int nsteps,
                 sblk[pp->blocks[b].states[a]] = (int)b;
                 sloc[pp->blocks[b].states[a]] = (int)a;
             }
-        hipError_t e = pl->d_prep_sblk.upload(sblk);
-        if (e == hipSuccess) e = pl->d_prep_sloc.upload(sloc);
+        Tables t;
+        t.add(pl->d_prep_sblk, sblk);
+        t.add(pl->d_prep_sloc, sloc);
+        const hipError_t e = t.commit(pl->tab_prep);
         if (e != hipSuccess) {
             delete pp;
+            delete pl->prep;
+            pl->prep = nullptr;
+            pl->have_ops = false;
             return fail(BLFID_ERR_DEVICE, std::string("prep tables: ") + hipGetErrorString(e));
         }
     }
@@ -1191,6 +1359,7 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
         pl->nparts = eo > 0 ? corr_segments(pl->n, eo, corr_use_fft(pl->n) ? pl->corr_auto : 0) : 1;
     else
         pl->nparts = std::max<int>(1, (int)pl->pairs.size());
+    Tables t;
     if (pl->prep) {
         // rho's nonzero entries, from which each crystallite's prepared blocks are formed
         std::vector<int> nzi;
@@ -1204,29 +1373,31 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
                     nzv.push_back(R(i, j).imag());
                 }
         pl->rho_nnz = (int)(nzv.size() / 2);
-        HIPCHK(pl->d_rho_nzi.upload(nzi));
-        HIPCHK(pl->d_rho_nzv.upload(nzv));
+        t.add(pl->d_rho_nzi, nzi);
+        t.add(pl->d_rho_nzv, nzv);
     }
     std::vector<int> pI, pJ;
     for (auto &pp : pl->pairs) {
         pI.push_back(pp.I);
         pJ.push_back(pp.J);
     }
-    HIPCHK(pl->d_pair_I.upload(pI));
-    HIPCHK(pl->d_pair_J.upload(pJ));
-    HIPCHK(pl->d_pair_eoff.upload(pl->pair_eoff));
-    HIPCHK(pl->d_pair_doff.upload(pl->pair_doff));
-    HIPCHK(pl->d_pair_roff.upload(pl->pair_roff));
-    HIPCHK(pl->d_drow.upload(pl->d_rowptr));
-    HIPCHK(pl->d_dcol.upload(pl->d_col));
-    HIPCHK(pl->d_dval.upload(pl->d_val));
-    HIPCHK(pl->d_rrow.upload(pl->r_rowptr));
-    HIPCHK(pl->d_rcol.upload(pl->r_col));
-    HIPCHK(pl->d_rval.upload(pl->r_val));
-    HIPCHK(pl->d_er.upload(pl->elem_r));
-    HIPCHK(pl->d_es.upload(pl->elem_s));
-    HIPCHK(pl->d_erev.upload(pl->elem_rev));
-    for (auto &kv : pl->pair_groups) HIPCHK(pl->d_pgrp[kv.first].upload(kv.second));
+    t.add(pl->d_pair_I, pI);
+    t.add(pl->d_pair_J, pJ);
+    t.add(pl->d_pair_eoff, pl->pair_eoff);
+    t.add(pl->d_pair_doff, pl->pair_doff);
+    t.add(pl->d_pair_roff, pl->pair_roff);
+    t.add(pl->d_drow, pl->d_rowptr);
+    t.add(pl->d_dcol, pl->d_col);
+    t.add(pl->d_dval, pl->d_val);
+    t.add(pl->d_rrow, pl->r_rowptr);
+    t.add(pl->d_rcol, pl->r_col);
+    t.add(pl->d_rval, pl->r_val);
+    t.add(pl->d_er, pl->elem_r);
+    t.add(pl->d_es, pl->elem_s);
+    t.add(pl->d_erev, pl->elem_rev);
+    for (auto &kv : pl->pair_groups) t.add(pl->d_pgrp[kv.first], kv.second);
+    pl->have_ops = false; // until the tables are in place
+    HIPCHK(t.commit(pl->tab_ops));
     pl->have_ops = true;
     refresh_devplan(pl);
     return BLFID_OK;
@@ -1237,15 +1408,18 @@ blfid_status blfid_plan_set_powder(blfid_plan *pl, const double *theta, const do
     if (!pl || K < 0 || (K > 0 && (!theta || !phi || !gamma || !weight)))
         return fail(BLFID_ERR_INVALID, "bad powder arguments");
     pl->gen++; // a recorded graph no longer matches the plan
-    pl->K = K;
+    pl->K = 0; // until the tables are in place
     if (K == 0) return BLFID_OK;
     std::vector<double> th(theta, theta + K), ph(phi, phi + K), ga(gamma, gamma + K),
         w(weight, weight + K);
-    HIPCHK(pl->d_th.upload(th));
-    HIPCHK(pl->d_ph.upload(ph));
-    HIPCHK(pl->d_ga.upload(ga));
-    HIPCHK(pl->d_w.upload(w));
+    Tables t;
+    t.add(pl->d_th, th);
+    t.add(pl->d_ph, ph);
+    t.add(pl->d_ga, ga);
+    t.add(pl->d_w, w);
+    HIPCHK(t.commit(pl->tab_powder));
     HIPCHK(pl->d_RP.alloc((size_t)9 * K));
+    pl->K = K;
     // the rotations are formed by the next run, on its stream, so that setting a powder never
     // waits for work of other plans
     pl->rp_dirty = true;
@@ -1350,6 +1524,19 @@ static blfid_layout::Shape shape_of(const blfid_plan *pl) {
     s.Estr = pl->Estr;
     s.K = pl->K;
     s.rho_elems = (pl->prep || pl->state) ? pl->Etot : 0;
+    if (pl->K > 0) {
+        // no more scratch slots than the largest launch has tasks (a few crystallites: the
+        // slots were most of the plan's storage)
+        auto tasks = [&](const std::map<int, std::vector<int>> &g) {
+            size_t m = 1;
+            for (auto &kv : g) m = std::max(m, kv.second.size());
+            return (double)m * pl->K * pl->n;
+        };
+        s.exp_slots = (int)std::min<double>(s.exp_slots, tasks(pl->blk_groups));
+        s.qr_slots = (int)std::min<double>(s.qr_slots, tasks(pl->pair_groups));
+        if (s.eig_slots > 0)
+            s.eig_slots = (int)std::min<double>(s.eig_slots, tasks(pl->eig_cls));
+    }
     return s;
 }
 
@@ -1695,7 +1882,7 @@ static blfid_status run_upto(blfid_plan *pl, int normalize, hipStream_t st, int 
         if (avail <= 0) {
             size_t fre = 0, tot = 0;
             HIPCHK(hipMemGetInfo(&fre, &tot));
-            avail = 0.4 * (double)(fre + pl->own_ws.n);
+            avail = 0.4 * (double)(fre + pl->own_ws.n + dev_cache().held());
         }
     }
     const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
@@ -1745,10 +1932,12 @@ blfid_status blfid_state_create(int nspins, int K, const double *theta, const do
     HIPCHK(st->rho.alloc(std::max<size_t>((size_t)K * NN, 1)));
     HIPCHK(hipMemset(st->rho.p, 0, std::max<size_t>((size_t)K * NN, 1) * sizeof(double2)));
     if (K > 0) {
-        HIPCHK(st->d_th.upload(std::vector<double>(theta, theta + K)));
-        HIPCHK(st->d_ph.upload(std::vector<double>(phi, phi + K)));
-        HIPCHK(st->d_ga.upload(std::vector<double>(gamma, gamma + K)));
-        HIPCHK(st->d_w.upload(std::vector<double>(weight, weight + K)));
+        Tables t;
+        t.add(st->d_th, std::vector<double>(theta, theta + K));
+        t.add(st->d_ph, std::vector<double>(phi, phi + K));
+        t.add(st->d_ga, std::vector<double>(gamma, gamma + K));
+        t.add(st->d_w, std::vector<double>(weight, weight + K));
+        HIPCHK(t.commit(st->tab));
         HIPCHK(st->d_RP.alloc((size_t)9 * K));
         LAUNCHCHK(blfid_dev_launch_prep(K, st->d_th.p, st->d_ph.p, st->d_ga.p, st->d_RP.p, nullptr));
         HIPCHK(hipDeviceSynchronize());
@@ -1848,8 +2037,10 @@ blfid_status blfid_state_apply(blfid_state *st, const blfid_system *sys, double 
             sloc[pp->blocks[b].states[a]] = (int)a;
         }
     HIPCHK(hipStreamSynchronize(s)); // tables and working storage may still feed earlier work
-    HIPCHK(st->sblk.upload(sblk));
-    HIPCHK(st->sloc.upload(sloc));
+    Tables t;
+    t.add(st->sblk, sblk);
+    t.add(st->sloc, sloc);
+    HIPCHK(t.commit(st->ptab));
     // working storage: the pulse plan's propagator regions for Kb crystallites (its exp scratch
     // cut to 4096 workgroup slots: a propagation is a small job), then one N x N product slot
     // per crystallite of the batch (at most 4096 slots)
@@ -1864,7 +2055,7 @@ blfid_status blfid_state_apply(blfid_state *st, const blfid_system *sys, double 
     if (avail <= 0) {
         size_t fre = 0, tot = 0;
         HIPCHK(hipMemGetInfo(&fre, &tot));
-        avail = 0.4 * (double)(fre + st->ws.n);
+        avail = 0.4 * (double)(fre + st->ws.n + dev_cache().held());
     }
     if ((double)need(1) > avail)
         return fail(BLFID_ERR_NOMEM, "one crystallite's propagator does not fit the memory budget");
@@ -1927,8 +2118,10 @@ blfid_status blfid_state_trace(blfid_state *st, const double *det_d, int normali
     if (K == 0) return BLFID_OK;
     hipStream_t s = (hipStream_t)stream;
     HIPCHK(hipStreamSynchronize(s));
-    HIPCHK(st->nzi.upload(nzi));
-    HIPCHK(st->nzv.upload(nzv));
+    Tables t;
+    t.add(st->nzi, nzi);
+    t.add(st->nzv, nzv);
+    HIPCHK(t.commit(st->ttab));
     const int G = blfid_layout::CRYST_GROUP;
     const int ng = (int)blfid_layout::ngroups(K);
     HIPCHK(st->part.alloc((size_t)2 * K));
@@ -1978,7 +2171,7 @@ blfid_status blfid_plan_graph_capture(blfid_plan *pl, int normalize) {
     if (avail <= 0) {
         size_t fre = 0, tot = 0;
         HIPCHK(hipMemGetInfo(&fre, &tot));
-        avail = 0.4 * (double)(fre + pl->own_ws.n);
+        avail = 0.4 * (double)(fre + pl->own_ws.n + dev_cache().held());
     }
     const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
     if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
@@ -2048,7 +2241,7 @@ blfid_status blfid_plan_run_slice(blfid_plan *pl, int c_begin, int c_end, int no
         if (avail <= 0) {
             size_t fre = 0, tot = 0;
             HIPCHK(hipMemGetInfo(&fre, &tot));
-            avail = 0.4 * (double)(fre + pl->own_ws.n);
+            avail = 0.4 * (double)(fre + pl->own_ws.n + dev_cache().held());
         }
         const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
         if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
