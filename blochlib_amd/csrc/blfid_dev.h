@@ -89,8 +89,8 @@ inline long tuned_cap(const DevPlan *P, int fam, int M) {
 }
 
 // Correlation work split (k_corr), shared by the host planner and the kernel: a crystallite's
-// Etot elements are cut into chunks of CH elements (CH = min(CORR_SPAN / n, 256 / ceil(n / 8)))
-// and the chunks into segments of up to CORR_SEG_CHUNKS; each segment writes one FID partial sum.
+// Etot elements are cut into chunks of CH elements (corr_chunk: CORR_SPAN / L with transforms of L
+// points, min(CORR_SPAN / n, 256 / ceil(n / 8)) with the direct sum) and the chunks into segments of up to CORR_SEG_CHUNKS; each segment writes one FID partial sum.
 #define CORR_TW 256
 #define CORR_SPAN 2048
 #define CORR_VTAB 512 /* complex128 entries of the period table, within the second buffer */
@@ -99,7 +99,25 @@ inline long tuned_cap(const DevPlan *P, int fam, int M) {
 __device__ __host__ inline int corr_seg_chunks(int nchunk) {
     return nchunk < CORR_SEG_CHUNKS ? (nchunk < 1 ? 1 : nchunk) : CORR_SEG_CHUNKS;
 }
+// log2 of the transform length of the FFT variant, or 0 where the direct sum is taken.  A power of
+// two from 16 to 512 is transformed at its own length; any other n from CORR_PAD_MIN to 256 is
+// zero-padded to the power of two L >= 2 n, whose cyclic correlation holds the linear one, folded
+// back to period n (two or three transforms of at most 4 n points against 8 n^2 flops: figures at
+// k_corr).  Smaller n stay direct (the padded chunks would hold mostly zeros), larger n would need
+// transforms beyond 512 points.
+#define CORR_PAD_MIN 9
+__host__ __device__ inline int corr_fft_ln(int n) {
+    const bool p2 = (n & (n - 1)) == 0;
+    if (p2 ? (n < 16 || n > 2 * CORR_TW) : (n < CORR_PAD_MIN || n > CORR_TW)) return 0;
+    int ln = 0;
+    while ((1 << ln) < (p2 ? n : 2 * n)) ln++;
+    return ln;
+}
+__host__ __device__ inline bool corr_use_fft(int n) { return corr_fft_ln(n) > 0; }
+// elements per chunk: the FFT variant fills CORR_SPAN points
 __device__ __host__ inline int corr_chunk(int n) {
+    const int ln = corr_fft_ln(n);
+    if (ln > 0) return CORR_SPAN >> ln;
     int npg = (n + CORR_PPT - 1) / CORR_PPT;
     int a = CORR_SPAN / n, b = 256 / npg;
     int ch = a < b ? a : b;
@@ -116,7 +134,4 @@ __device__ __host__ inline int corr_segments(int n, long Etot, int auto_chunks =
     const int CH = corr_chunk(n);
     const int nchunk = (int)((Etot + CH - 1) / CH);
     return corr_range_segments(auto_chunks) + corr_range_segments(nchunk - auto_chunks);
-}
-__host__ __device__ inline bool corr_use_fft(int n) {
-    return n >= 16 && (n & (n - 1)) == 0 && n <= 2 * CORR_TW;
 }

@@ -1482,20 +1482,22 @@ static double pair_flops(const blfid_plan *pl, const std::vector<int> &g) {
 }
 
 
-// Executed flops of the correlation per element and crystallite: FFT variant (n a power of two,
-// 16..512) as T transforms of np = ceil(log2(n) / 3) passes, radix 8 (a 56-flop DFT and 7
-// twiddle products per butterfly) but the last, of radix rl without twiddles (DFT of 4, 16 or
-// 56 flops), plus the scaled product (8 per point); direct variant 8 n^2; plus twiddle staging
+// Executed flops of the correlation per element and crystallite: FFT variant (transforms of
+// L points, corr_fft_ln) as T transforms of np = ceil(log2(L) / 3) passes, radix 8 (a 56-flop DFT
+// and 7 twiddle products per butterfly) but the last, of radix rl without twiddles (DFT of 4, 16
+// or 56 flops), plus the scaled product (8 per point); direct variant 8 n^2; plus twiddle staging
 // (18 n) and the FID sums (14 per point).  T = 3 in general; the autocorrelation variant
 // (R = conj(Q)) forms two transforms, a 4-flop |q|^2 / n product and stages Q alone (9 n).
 static double corr_flops_per_elem(int n, int P, bool autoc = false) {
     double c = 8.0 * (double)n * n;
     double stage = 18.0 * n;
-    if (n >= 16 && (n & (n - 1)) == 0 && n <= 512) {
-        const int ln = __builtin_ctz((unsigned)n), np = (ln + 2) / 3, rl = 1 << (ln - 3 * (np - 1));
+    const int ln = corr_fft_ln(n);
+    if (ln > 0) {
+        const double L = (double)(1 << ln);
+        const int np = (ln + 2) / 3, rl = 1 << (ln - 3 * (np - 1));
         const double dft = rl == 2 ? 4.0 : rl == 4 ? 16.0 : 56.0;
         const double T = autoc ? 2.0 : 3.0;
-        c = T * (np - 1) * (n / 8.0) * 98.0 + T * ((double)n / rl) * dft + (autoc ? 4.0 : 8.0) * n;
+        c = T * (np - 1) * (L / 8.0) * 98.0 + T * (L / rl) * dft + (autoc ? 4.0 : 8.0) * L;
         if (autoc) stage = 9.0 * n;
     }
     return c + stage + 14.0 * P;

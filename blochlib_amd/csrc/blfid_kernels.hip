@@ -2232,11 +2232,14 @@ __device__ __forceinline__ void corr_mid_pass(typename CX<R>::T *sQ, const typen
 }
 
 // NPT FID points per thread are held over a segment (npts <= 256 NPT).  LN > 0 selects the FFT
-// variant for n = 2^LN (CorrFft<LN>), LN = 0 the direct sum for any n.  The complex64 FFT variant
+// variant with transforms of 2^LN points (CorrFft<LN>): n = 2^LN, or (PAD) any n <= 2^(LN-1), the
+// sequences zero-padded and the linear correlation folded to period n afterwards.  LN = 0 is the
+// direct sum for any n.  PAD against the direct sum (6 spins, 1154 crystallites, n = 100, 1000
+// points, complex64): CORRPAD_FIGS.  The complex64 FFT variant
 // with four points is held to three waves per SIMD (168 registers: at four it spilled, and its
 // sixteen loads per chunk then waited on the spill reloads); the others are bound by LDS or
 // registers at two.  OCC > 0 replaces that bound (a variant the launch autotuner may choose).
-template <typename R, int LN, int NPT, bool AUTO, int OCC = 0>
+template <typename R, int LN, int NPT, bool AUTO, int OCC = 0, bool PAD = false>
 __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4 && NPT == 4) ? (AUTO ? 4 : 3) : 2) k_corr(DevPlan P, int Kb,
                                               const typename CX<R>::T *__restrict__ Qt,
                                               const typename CX<R>::T *__restrict__ Rt,
@@ -2254,7 +2257,7 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
     __shared__ double sphi[NE];
     __shared__ cd sstep[NE];
     __shared__ CT s_tw[FFT ? FF::N / 2 : 1];
-    const int n = FFT ? FF::N : P.n, tid = threadIdx.x;
+    const int n = FFT && !PAD ? FF::N : P.n, tid = threadIdx.x;
     const int CH = FFT ? FF::CH : corr_chunk(n);
     // LDS slot of (step k, element el).  Direct variant: rows of CH elements, the element index
     // XOR-ed with a function of the row when CH is a power of two, so that one element read
@@ -2286,14 +2289,19 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
     // FFT variant: with J = ceil(npts / n) periods, z_e^t = z_e^p (z_e^n)^j for t = p + n j, so
     // the FID sums are sum_e G_p(e) V_j(e) with G = F z^p formed in place and the table
     // V_j(e) = z_e^(n j) (in the correlation's second buffer, free by then): no sine or cosine
-    // per point.  Used when CH J fits CORR_VTAB entries; longer FIDs go out per chunk.
+    // per point.  The table takes GE elements at a time (all CH where CH J fits CORR_VTAB
+    // entries); longer FIDs go out per chunk.
     const int J = (P.npts + n - 1) / n;
-    const bool hold = P.npts <= 256 * NPT && (!FFT || CH * J <= CORR_VTAB);
+    const bool hold = P.npts <= 256 * NPT && (!FFT || J <= CORR_VTAB);
+    const int GE = FFT ? min(CH, max(1, CORR_VTAB / J)) : CH;
     cd *sV = (cd *)sR;
     const int nth = tid < P.npts ? min(NPT, (P.npts - tid + 255) / 256) : 0;
-    int hoff[NPT];
+    int hoff[NPT], hper[PAD ? NPT : 1]; // step and period of point tid + 256 m
 #pragma unroll
-    for (int m = 0; m < NPT; m++) hoff[m] = FFT ? 0 : (tid + 256 * m) % n; // step of point tid + 256 m
+    for (int m = 0; m < NPT; m++) {
+        hoff[m] = FFT && !PAD ? 0 : (tid + 256 * m) % n;
+        if constexpr (PAD) hper[m] = (tid + 256 * m) / n;
+    }
     for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
         const int c = (int)(task / nsg), sg = (int)(task % nsg);
         const int ch_end = ch_lo + min(nchunk, (sg + 1) * spc);
@@ -2319,20 +2327,26 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                     const int rv = (!AUTO && P.rt_from_q) ? P.elem_rev[ec] : -1;
                     const double *th = thetas + (size_t)c * P.N;
                     const size_t str = (size_t)(1 << LS) * P.Estr;
-                    const CT *qb = Qt + ((size_t)c * FF::N + j) * P.Estr;
-                    const CT *rb = P.rt_from_q ? qb : Rt + ((size_t)c * FF::N + j) * P.Estr;
+                    // PAD: steps from n on are zero (all of the upper half's, so only the first
+                    // four are loaded), the load indexes clamped to the last step
+                    constexpr int NL = PAD ? 4 : 8;
+                    const CT *qb = Qt + ((size_t)c * n + (PAD ? 0 : j)) * P.Estr;
+                    const CT *rb = P.rt_from_q ? qb : Rt + ((size_t)c * n + (PAD ? 0 : j)) * P.Estr;
+                    auto row = [&](int m) {
+                        return PAD ? (size_t)min(j + (m << LS), n - 1) * P.Estr : (size_t)m * str;
+                    };
                     const long rc = P.rt_from_q ? (rv >= 0 ? (long)rv : ec) : ec;
                     const double th_r = th[er_], th_s = th[es_];
                     // AUTO (R = conj(Q): rho = (D + D^H) / 2 and no element has a reverse): the
                     // R sequence is conj of the twiddled Q sequence, so only Q is loaded
-                    CT qv[8], rw[AUTO ? 1 : 8];
+                    CT qv[NL], rw[AUTO ? 1 : NL];
 #pragma unroll
-                    for (int m = 0; m < 8; m++) qv[m] = qb[(size_t)m * str + ec];
+                    for (int m = 0; m < NL; m++) qv[m] = qb[row(m) + ec];
                     if constexpr (!AUTO) {
 #pragma unroll
-                        for (int m = 0; m < 8; m++) rw[m] = rb[(size_t)m * str + rc];
+                        for (int m = 0; m < NL; m++) rw[m] = rb[row(m) + rc];
                     }
-                    const double ph = ok ? (th_r - th_s) / (double)FF::N : 0.0;
+                    const double ph = ok ? (th_r - th_s) / (double)n : 0.0;
                     if (j == 0) {
                         sphi[el] = ph;
                         sstep[el] = cexpi(256.0 * ph);
@@ -2347,7 +2361,12 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                     cd w = w0;
 #pragma unroll
                     for (int m = 0; m < 8; m++) {
-                        x[m] = CX<R>::from(cmul(cscale(to_cd(qv[m]), okf), w));
+                        if (m >= NL) {
+                            x[m] = Arith<CT>::zero();
+                            continue;
+                        }
+                        x[m] = CX<R>::from(cmul(cscale(to_cd(qv[m % NL]), okf), w));
+                        if (PAD && j + (m << LS) >= n) x[m] = Arith<CT>::zero();
                         w = cmul(w, st);
                     }
                     RegDFT<8, -1, R>::run(x);
@@ -2361,12 +2380,17 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                         const cd sti = cconj(st);
 #pragma unroll
                         for (int m = 0; m < 8; m++) {
+                            if (m >= NL) {
+                                x[m] = Arith<CT>::zero();
+                                continue;
+                            }
                             cd rr;
                             if (P.rt_from_q) // R(s,r) = Q_(J,I)(s,r) + conj(Q_(I,J)(r,s))
-                                rr = cadd(cscale(cconj(to_cd(qv[m])), okf), cscale(to_cd(rw[m]), rvf));
+                                rr = cadd(cscale(cconj(to_cd(qv[m % NL])), okf), cscale(to_cd(rw[m % NL]), rvf));
                             else
-                                rr = cscale(to_cd(rw[m]), okf);
+                                rr = cscale(to_cd(rw[m % NL]), okf);
                             x[m] = CX<R>::from(cmul(rr, w));
+                            if (PAD && j + (m << LS) >= n) x[m] = Arith<CT>::zero();
                             w = cmul(w, sti);
                         }
                         RegDFT<8, +1, R>::run(x);
@@ -2399,7 +2423,7 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                         if (k) x[k] = cmul(x[k], FF::template twid<+1>(s_tw, j * k));
                     }
                     RegDFT<8, +1, R>::run(x);
-                    if (hold) {
+                    if (hold && !PAD) {
                         const double ph = sphi[el];
                         cd w = cexpi((double)j * ph);
                         const cd st = cexpi((double)(1 << LS) * ph);
@@ -2413,9 +2437,28 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                         for (int m = 0; m < 8; m++) sQ[base + (m << LS) * FF::ROW] = x[m];
                     }
                 }
+                if constexpr (PAD) {
+                    // F_p = lin_p + lin_{p-n} (lag p - n at slot L - n + p >= n, which no item
+                    // writes), times z^p for the held FID sums; item m of a thread is the step
+                    // j + m L/8
+                    __syncthreads();
+                    const double ph = sphi[el];
+                    cd w = cexpi((double)j * ph);
+                    const cd st = cexpi((double)(1 << LS) * ph);
+#pragma unroll
+                    for (int m = 0; m < 4; m++) {
+                        const int p = j + (m << LS);
+                        if (p < n) {
+                            CT f = sQ[FF::at(p, el)];
+                            if (p > 0) f = cadd(f, sQ[FF::at(FF::N - n + p, el)]);
+                            sQ[FF::at(p, el)] = hold ? CX<R>::from(cmul(to_cd(f), w)) : f;
+                        }
+                        w = cmul(w, st);
+                    }
+                }
                 if (hold)
-                    for (int q = tid; q < FF::CH * J; q += 256)
-                        sV[q] = cexpi((double)FF::N * (double)(q % J) * sphi[q / J]);
+                    for (int q = tid; q < GE * J; q += 256)
+                        sV[q] = cexpi((double)n * (double)(q % J) * sphi[q / J]);
                 __syncthreads();
             } else {
                 for (int el = tid; el < CH; el += 256) {
@@ -2501,12 +2544,25 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
             }
             if (FFT && hold) {
                 const int ne = (int)min((long)CH, P.Etot - e0);
-                for (int e = 0; e < ne; e++) {
+                for (int g0 = 0; g0 < ne; g0 += GE) {
+                    const int g1 = min(ne, g0 + GE);
+                    if (g0 > 0) { // the next elements' table
+                        __syncthreads();
+                        for (int q = tid; q < (g1 - g0) * J; q += 256)
+                            sV[q] = cexpi((double)n * (double)(q % J) * sphi[g0 + q / J]);
+                        __syncthreads();
+                    }
+                    for (int e = g0; e < g1; e++) {
+                        const cd *V = sV + (e - g0) * J;
 #pragma unroll
-                    for (int m = 0; m < NPT; m++) {
-                        if (m < nth) {
-                            const int t = tid + 256 * m;
-                            cfma(hacc[m], to_cd(sQ[at(t & (n - 1), e)]), sV[e * J + (t >> LN)]);
+                        for (int m = 0; m < NPT; m++) {
+                            if (m < nth) {
+                                const int t = tid + 256 * m;
+                                if constexpr (PAD)
+                                    cfma(hacc[m], to_cd(sQ[at(hoff[m], e)]), V[hper[m]]);
+                                else
+                                    cfma(hacc[m], to_cd(sQ[at(t & (n - 1), e)]), V[t >> LN]);
+                            }
                         }
                     }
                 }
@@ -3203,7 +3259,7 @@ extern "C" int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, co
 // One launch over the chunks [lo, hi) of every crystallite of the batch, its segments written as
 // partial sums seg_base...; AUTO (FFT sizes only): the autocorrelation variant, for chunks whose
 // elements have R = conj(Q) (rosym, no reverse element)
-template <typename R, int LN, int NPT, int OCC>
+template <typename R, int LN, int NPT, int OCC, bool PAD>
 static void launch_corr_t(bool autoc, const DevPlan *P, int Kb, const void *Qt, const void *Rt,
                           const double *thetas, const int *er, const int *es, double *part,
                           int lo, int hi, int seg_base, hipStream_t st) {
@@ -3213,27 +3269,38 @@ static void launch_corr_t(bool autoc, const DevPlan *P, int Kb, const void *Qt, 
     const int grid = (int)(ntask < cap ? ntask : cap);
     if (grid <= 0) return;
     if (LN > 0 && autoc)
-        k_corr<R, LN, NPT, LN != 0, OCC><<<grid, 256, 0, st>>>(*P, Kb, (const CT *)Qt, (const CT *)Rt,
+        k_corr<R, LN, NPT, LN != 0, OCC, PAD><<<grid, 256, 0, st>>>(*P, Kb, (const CT *)Qt, (const CT *)Rt,
                                                           thetas, er, es, part, lo, hi, seg_base);
     else
-        k_corr<R, LN, NPT, false, OCC><<<grid, 256, 0, st>>>(*P, Kb, (const CT *)Qt, (const CT *)Rt,
+        k_corr<R, LN, NPT, false, OCC, PAD><<<grid, 256, 0, st>>>(*P, Kb, (const CT *)Qt, (const CT *)Rt,
                                                         thetas, er, es, part, lo, hi, seg_base);
 }
-// FFT variants by log2 n (corr_use_fft(n): 16 <= n <= 512), LN = 0 the direct sum
+// FFT variants by transform length (corr_fft_ln), LN = 0 the direct sum
 template <typename R, int NPT, int OCC = 0>
 static void launch_corr(bool autoc, const DevPlan *P, int Kb, const void *Qt, const void *Rt,
                         const double *thetas, const int *er, const int *es, double *part,
                         int lo, int hi, int seg_base, hipStream_t st) {
-    const int ln = corr_use_fft(P->n) ? __builtin_ctz((unsigned)P->n) : 0;
+    const int ln = corr_fft_ln(P->n);
 #define CORR_ARGS autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, seg_base, st
+    if (ln > 0 && P->n != 1 << ln) {
+        // zero-padded; the two-wave variant (OCC) differs for the unpadded lengths only
+        switch (ln) {
+        case 5: launch_corr_t<R, 5, NPT, 0, true>(CORR_ARGS); break;
+        case 6: launch_corr_t<R, 6, NPT, 0, true>(CORR_ARGS); break;
+        case 7: launch_corr_t<R, 7, NPT, 0, true>(CORR_ARGS); break;
+        case 8: launch_corr_t<R, 8, NPT, 0, true>(CORR_ARGS); break;
+        default: launch_corr_t<R, 9, NPT, 0, true>(CORR_ARGS); break;
+        }
+        return;
+    }
     switch (ln) {
-    case 4: launch_corr_t<R, 4, NPT, OCC>(CORR_ARGS); break;
-    case 5: launch_corr_t<R, 5, NPT, OCC>(CORR_ARGS); break;
-    case 6: launch_corr_t<R, 6, NPT, OCC>(CORR_ARGS); break;
-    case 7: launch_corr_t<R, 7, NPT, OCC>(CORR_ARGS); break;
-    case 8: launch_corr_t<R, 8, NPT, OCC>(CORR_ARGS); break;
-    case 9: launch_corr_t<R, 9, NPT, OCC>(CORR_ARGS); break;
-    default: launch_corr_t<R, 0, NPT, OCC>(CORR_ARGS); break;
+    case 4: launch_corr_t<R, 4, NPT, OCC, false>(CORR_ARGS); break;
+    case 5: launch_corr_t<R, 5, NPT, OCC, false>(CORR_ARGS); break;
+    case 6: launch_corr_t<R, 6, NPT, OCC, false>(CORR_ARGS); break;
+    case 7: launch_corr_t<R, 7, NPT, OCC, false>(CORR_ARGS); break;
+    case 8: launch_corr_t<R, 8, NPT, OCC, false>(CORR_ARGS); break;
+    case 9: launch_corr_t<R, 9, NPT, OCC, false>(CORR_ARGS); break;
+    default: launch_corr_t<R, 0, NPT, OCC, false>(CORR_ARGS); break;
     }
 #undef CORR_ARGS
 }
