@@ -54,13 +54,16 @@ struct DevPlan {
     const double *rf;      // n x nrfiso x 3: amp/2, phase, offset of each step
     const double *thetak;  // n: 2 pi tau_k of steps of unequal length, or NULL (all theta)
     int rt_from_q;         // 1: R(s,r) = Q_rev + conj(Q(r,s)), R is neither formed nor stored
-    const int *elem_rev;   // Etot: element (s,r) of the reverse pair (J,I), or -1
+    // correlation elements (Ecorr <= Etot): position in a step's Q row, state-list positions of
+    // column (block I) and row (block J), position of the reverse element (s,r) of pair (J,I) or -1
+    long Ecorr;
+    const int *corr_pos, *corr_r, *corr_s, *corr_rev;
     double *expflops;      // 16: executed flops per tile variant of the propagator [0..7] and
                            // the fused propagator + Dyson chain [8..15] (profiling), or NULL
     int bf16x3;            // complex64 products as three bf16 matrix-core products (BLFID_C64_BF16X3)
     long Estr;             // Q / R row stride per step: Etot padded to a multiple of 16 elements
     int nparts;            // FID partial sums per crystallite (correlation segments or block pairs)
-    int rt_rev;            // rt_from_q and some element has a reverse element (elem_rev >= 0)
+    int rt_rev;            // rt_from_q and some element has a reverse element (corr_rev >= 0)
     const int *xd_off;     // nblocks + 1: start of each block's flip-flop positions in xd_list
     const int *xd_list;    // per block of <= DEV_LDS_BLOCK states: (r LDK + q) << 8 | (i S + j)
     const int *elem_r;     // Etot: state-list position of each pair element's column (block I)
@@ -89,15 +92,17 @@ inline long tuned_cap(const DevPlan *P, int fam, int M) {
 }
 
 // Correlation work split (k_corr), shared by the host planner and the kernel: a crystallite's
-// Etot elements are cut into chunks of CH elements (corr_chunk: CORR_SPAN / L with transforms of L
+// Ecorr elements are cut into chunks of CH elements (corr_chunk: CORR_SPAN / L with transforms of L
 // points, min(CORR_SPAN / n, 256 / ceil(n / 8)) with the direct sum) and the chunks into segments of up to CORR_SEG_CHUNKS; each segment writes one FID partial sum.
 #define CORR_TW 256
 #define CORR_SPAN 2048
-#define CORR_VTAB 512 /* complex128 entries of the period table, within the second buffer */
+#define CORR_VTAB 1024 /* complex128 entries of the period table, within the second buffer */
 #define CORR_PPT 8
 #define CORR_SEG_CHUNKS 64
+#define CORR_SEG_MIN 8
 __device__ __host__ inline int corr_seg_chunks(int nchunk) {
-    return nchunk < CORR_SEG_CHUNKS ? (nchunk < 1 ? 1 : nchunk) : CORR_SEG_CHUNKS;
+    const int c = (nchunk + CORR_SEG_MIN - 1) / CORR_SEG_MIN;
+    return c < 4 ? 4 : c > CORR_SEG_CHUNKS ? CORR_SEG_CHUNKS : c;
 }
 // log2 of the transform length of the FFT variant, or 0 where the direct sum is taken.  A power of
 // two from 16 to 512 is transformed at its own length; any other n from CORR_PAD_MIN to 256 is

@@ -56,8 +56,7 @@ int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, const int *pg
                         const void *bufB, void *scratch, size_t slot, int nslots, void *Qt,
                         void *Rt, hipStream_t st);
 int blfid_dev_launch_corr(int prec, const DevPlan *P, int Kb, const void *Qt, const void *Rt,
-                          const double *thetas, const int *er, const int *es, double *part,
-                          hipStream_t st);
+                          const double *thetas, double *part, hipStream_t st);
 int blfid_dev_launch_reduce(int Kb, int c0, int npts, int nparts, int G, const double *w,
                             double scale, const double *part, double *grp, hipStream_t st);
 int blfid_dev_launch_finish(int npts, int ngroups, const double *grp, double nre, double nim,
@@ -336,6 +335,7 @@ class Tables {
 
 struct Block {
     std::vector<int> states;
+    std::vector<int> comp; // connected component of each state within the block
 };
 
 struct Pair {
@@ -419,7 +419,8 @@ struct blfid_plan {
     bool rt_rev = false;       // rt_from_q and some element has a reverse element
     int corr_auto = 0;         // leading correlation chunks taking the autocorrelation kernel
     long corr_rev_elems = 0;   // elements with a reverse element (their R reads a second Q)
-    std::vector<int> elem_rev;  // per element (r,s) of pair (I,J): element (s,r) of (J,I) or -1
+    // correlation elements: position in a step's Q row, states, reverse element's position or -1
+    std::vector<int> corr_pos, corr_r, corr_s, corr_rev;
     std::map<int, std::vector<int>> pair_groups; // M -> pairs
     // powder
     int K = 0;
@@ -431,7 +432,7 @@ struct blfid_plan {
     DevTab<int> d_ff_off, d_ff_term;
     DevTab<double> d_xd_cst, d_xd_fpr;
     DevTab<int> d_blk_dim, d_blk_soff, d_blk_states, d_pair_I, d_pair_J, d_pair_doff,
-        d_pair_roff, d_drow, d_dcol, d_rrow, d_rcol, d_er, d_es, d_erev;
+        d_pair_roff, d_drow, d_dcol, d_rrow, d_rcol, d_er, d_es, d_cpos, d_cr, d_cs, d_crev;
     DevTab<long> d_blk_uoff, d_pair_eoff;
     DevTab<double> d_dval, d_rval;
     std::map<int, DevTab<int>> d_bgrp, d_pgrp, d_fgrp;
@@ -710,6 +711,7 @@ static blfid_status build_tables(blfid_plan *pl) {
         const auto &st = comps[ci].states;
         if (st.size() >= 16) {
             pl->blocks.push_back(comps[ci]);
+            pl->blocks.back().comp.assign(st.size(), 0);
             continue;
         }
         int placed = -1;
@@ -721,8 +723,9 @@ static blfid_status build_tables(blfid_plan *pl) {
             pl->blocks.push_back(Block());
             placed = (int)small_bins.size() - 1;
         }
-        auto &dst = pl->blocks[small_bins[placed]].states;
-        dst.insert(dst.end(), st.begin(), st.end());
+        Block &dst = pl->blocks[small_bins[placed]];
+        dst.comp.insert(dst.comp.end(), st.size(), dst.comp.empty() ? 0 : dst.comp.back() + 1);
+        dst.states.insert(dst.states.end(), st.begin(), st.end());
         binfill[placed] += (int)st.size();
     }
     pl->blk_dim.clear(); pl->blk_soff.clear(); pl->blk_uoff.clear(); pl->blk_states.clear();
@@ -860,7 +863,11 @@ static void refresh_devplan(blfid_plan *pl) {
     d.Lsum = pl->Lsum;
     d.Etot = pl->Etot;
     d.rt_from_q = pl->rt_from_q ? 1 : 0;
-    d.elem_rev = pl->d_erev.p;
+    d.Ecorr = (long)pl->corr_pos.size();
+    d.corr_pos = pl->d_cpos.p;
+    d.corr_r = pl->d_cr.p;
+    d.corr_s = pl->d_cs.p;
+    d.corr_rev = pl->d_crev.p;
     d.expflops = pl->prof ? pl->d_expflops.p : nullptr;
     d.bf16x3 = pl->bf16x3;
     d.Estr = pl->Estr;
@@ -1264,14 +1271,6 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
     for (int I = 0; I < nb; I++)
         for (int J = 0; J < nb; J++)
             if (dnz[I * nb + J] && rnz[J * nb + I]) pl->pairs.push_back({I, J});
-    if (pl->spinning && rosym) {
-        // pairs without a reverse pair (J, I) first: their elements have R = conj(Q) and form
-        // the leading correlation chunks that take the autocorrelation kernel
-        std::vector<char> has(nb * nb, 0);
-        for (auto &q : pl->pairs) has[q.I * nb + q.J] = 1;
-        std::stable_partition(pl->pairs.begin(), pl->pairs.end(),
-                              [&](const Pair &q) { return !has[q.J * nb + q.I]; });
-    }
     pl->pair_eoff.clear(); pl->pair_doff.clear(); pl->pair_roff.clear();
     pl->d_rowptr.clear(); pl->d_col.clear(); pl->d_val.clear();
     pl->r_rowptr.clear(); pl->r_col.clear(); pl->r_val.clear();
@@ -1322,41 +1321,60 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
     pl->Estr = (eo + 15) & ~15L;
     // rosym spinning case: R_(I,J) = B_J^H (det_JI + det_IJ^H) B_I, i.e. R_(I,J)(s,r) =
     // Q_(J,I)(s,r) + conj(Q_(I,J)(r,s)); the pair (J,I) exists exactly when det_JI != 0, so R
-    // needs neither its own products nor storage: k_corr forms it from Q through elem_rev
+    // needs neither its own products nor storage: k_corr forms it from Q through corr_rev
     pl->rt_from_q = pl->spinning && rosym;
-    pl->elem_rev.clear();
-    if (pl->rt_from_q) {
+    // Correlation elements: those of each pair whose components D couples.  A packed block is block
+    // diagonal in its components at every step, so A_k, the eigenvectors (the rotations skip exact
+    // zeros) and hence Q are exactly zero between components that D does not couple.  Elements
+    // without a reverse element come first (autocorrelation); both runs in row order.
+    {
         std::map<std::pair<int, int>, int> pidx;
         for (size_t p = 0; p < pl->pairs.size(); p++) pidx[{pl->pairs[p].I, pl->pairs[p].J}] = (int)p;
-        pl->elem_rev.assign(eo, -1);
+        std::vector<std::vector<char>> on(pl->pairs.size()); // per pair: component couples component
+        auto ncomp = [&](int b) { return pl->blocks[b].comp.back() + 1; };
         for (size_t p = 0; p < pl->pairs.size(); p++) {
-            int I = pl->pairs[p].I, J = pl->pairs[p].J;
-            auto it = pidx.find({J, I});
-            if (it == pidx.end()) continue;
-            const int bI = pl->blk_dim[I], bJ = pl->blk_dim[J];
-            const long ro = pl->pair_eoff[it->second];
-            for (int s2 = 0; s2 < bJ; s2++)
-                for (int r = 0; r < bI; r++)
-                    pl->elem_rev[pl->pair_eoff[p] + r + (long)s2 * bI] = (int)(ro + s2 + (long)r * bJ);
+            const Block &bi = pl->blocks[pl->pairs[p].I], &bj = pl->blocks[pl->pairs[p].J];
+            const int nj = ncomp(pl->pairs[p].J);
+            on[p].assign((size_t)ncomp(pl->pairs[p].I) * nj, 0);
+            const int *rp = &pl->d_rowptr[pl->pair_doff[p]];
+            for (size_t a = 0; a < bi.states.size(); a++)
+                for (int z = rp[a]; z < rp[a + 1]; z++)
+                    on[p][(size_t)bi.comp[a] * nj + bj.comp[pl->d_col[z]]] = 1;
         }
+        pl->corr_pos.clear(); pl->corr_r.clear(); pl->corr_s.clear(); pl->corr_rev.clear();
+        pl->corr_rev_elems = 0;
+        for (int pass = 0; pass < 2; pass++)
+            for (size_t p = 0; p < pl->pairs.size(); p++) {
+                const int I = pl->pairs[p].I, J = pl->pairs[p].J;
+                const Block &bi = pl->blocks[I], &bj = pl->blocks[J];
+                const int bI = pl->blk_dim[I], bJ = pl->blk_dim[J], nj = ncomp(J), ni = ncomp(I);
+                auto it = pidx.find({J, I});
+                for (int s2 = 0; s2 < bJ; s2++)
+                    for (int r = 0; r < bI; r++) {
+                        if (!on[p][(size_t)bi.comp[r] * nj + bj.comp[s2]]) continue;
+                        int rev = -1;
+                        if (pl->rt_from_q && it != pidx.end() &&
+                            on[it->second][(size_t)bj.comp[s2] * ni + bi.comp[r]])
+                            rev = (int)(pl->pair_eoff[it->second] + s2 + (long)r * bJ);
+                        if ((rev >= 0) != (pass == 1)) continue;
+                        pl->corr_pos.push_back((int)(pl->pair_eoff[p] + r + (long)s2 * bI));
+                        pl->corr_r.push_back(pl->blk_soff[I] + r);
+                        pl->corr_s.push_back(pl->blk_soff[J] + s2);
+                        pl->corr_rev.push_back(rev);
+                        pl->corr_rev_elems += rev >= 0;
+                    }
+            }
     }
-    pl->rt_rev = false;
-    long first_rev = eo;
-    for (long e = 0; e < (long)pl->elem_rev.size(); e++)
-        if (pl->elem_rev[e] >= 0) {
-            pl->rt_rev = true;
-            first_rev = std::min(first_rev, e);
-        }
+    const long nc = (long)pl->corr_pos.size(), first_rev = nc - pl->corr_rev_elems;
+    pl->rt_rev = pl->corr_rev_elems > 0;
     // correlation chunks before the first element with a reverse element: autocorrelation
     {
         const int CH = corr_chunk(pl->n);
-        const int nchunk = (int)((eo + CH - 1) / CH);
+        const int nchunk = (int)((nc + CH - 1) / CH);
         pl->corr_auto = !pl->rt_from_q ? 0 : !pl->rt_rev ? nchunk : (int)(first_rev / CH);
-        pl->corr_rev_elems = 0;
-        for (int v : pl->elem_rev) pl->corr_rev_elems += v >= 0;
     }
     if (pl->spinning && !pl->ptop)
-        pl->nparts = eo > 0 ? corr_segments(pl->n, eo, corr_use_fft(pl->n) ? pl->corr_auto : 0) : 1;
+        pl->nparts = nc > 0 ? corr_segments(pl->n, nc, corr_use_fft(pl->n) ? pl->corr_auto : 0) : 1;
     else
         pl->nparts = std::max<int>(1, (int)pl->pairs.size());
     Tables t;
@@ -1394,7 +1412,10 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
     t.add(pl->d_rval, pl->r_val);
     t.add(pl->d_er, pl->elem_r);
     t.add(pl->d_es, pl->elem_s);
-    t.add(pl->d_erev, pl->elem_rev);
+    t.add(pl->d_cpos, pl->corr_pos);
+    t.add(pl->d_cr, pl->corr_r);
+    t.add(pl->d_cs, pl->corr_s);
+    t.add(pl->d_crev, pl->corr_rev);
     for (auto &kv : pl->pair_groups) t.add(pl->d_pgrp[kv.first], kv.second);
     pl->have_ops = false; // until the tables are in place
     HIPCHK(t.commit(pl->tab_ops));
@@ -1590,10 +1611,10 @@ blfid_status blfid_plan_stats(const blfid_plan *pl, double *out) {
         ex += 8.0 * s3;         // B = A W
         ex += 8.0 * pairsQ;     // Q and R
         const double ea = corr_use_fft(pl->n)
-                              ? std::min<double>((double)pl->corr_auto * corr_chunk(pl->n), (double)pl->Etot)
+                              ? std::min<double>((double)pl->corr_auto * corr_chunk(pl->n), (double)pl->corr_pos.size())
                               : 0.0;
         ex += (ea * corr_flops_per_elem(pl->n, pl->npts, true) +
-               ((double)pl->Etot - ea) * corr_flops_per_elem(pl->n, pl->npts, false)) / n;
+               ((double)pl->corr_pos.size() - ea) * corr_flops_per_elem(pl->n, pl->npts, false)) / n;
     }
     out[0] = ex;
     if (pl->ptop) out[1] = 8.0 * N * N * N + 16.0 * N * N * N * P / n;
@@ -1806,17 +1827,17 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                 // Q once per element; R too unless it is formed from Q, or the reverse element's
                 // Q where there is one.  Elements of the autocorrelation chunks take that
                 // variant's flop count, the others the general one.
-                const double reads = pl->rt_from_q ? (double)pl->Etot + (double)pl->corr_rev_elems
-                                                   : 2.0 * (double)pl->Etot;
+                const double ec = (double)pl->corr_pos.size();
+                const double reads = pl->rt_from_q ? ec + (double)pl->corr_rev_elems : 2.0 * ec;
                 const double ea = corr_use_fft(pl->n)
-                                      ? std::min<double>((double)pl->corr_auto * corr_chunk(pl->n), (double)pl->Etot)
+                                      ? std::min<double>((double)pl->corr_auto * corr_chunk(pl->n), ec)
                                       : 0.0;
                 const double fl = ea * corr_flops_per_elem(pl->n, pl->npts, true) +
-                                  ((double)pl->Etot - ea) * corr_flops_per_elem(pl->n, pl->npts, false);
+                                  (ec - ea) * corr_flops_per_elem(pl->n, pl->npts, false);
                 PhaseScope ps(pl, 5 * 8, kb * fl,
                               kb * ((double)pl->n * reads * cs + (double)pl->nparts * pl->npts * 16.0), st);
                 LAUNCHCHK(blfid_dev_launch_corr(pr, P, kb, pl->bufQt, pl->bufRt, pl->thetas,
-                                                pl->d_er.p, pl->d_es.p, pl->part, st));
+                                                pl->part, st));
             }
         } else {
             for (auto &kv : pl->blk_groups)

@@ -2061,8 +2061,12 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
 // owning t when the FID is too long to hold).  No atomics: each (crystallite, segment, point) has
 // one writer, and k_reduce adds the segments in order, so the FID does not depend on scheduling.
 // CH = min(CORR_SPAN / n, 256 / ceil(n/8)) is computed identically on the host (blfid_dev.h).
-// Q rows are Estr elements apart (Etot padded to 16 elements), so every chunk row starts on a
-// 128-byte line.
+// Q rows are Estr elements apart (Etot padded to 16 elements).  The elements are those of the
+// plan's list (Ecorr of them: corr_pos in the Q row, corr_r / corr_s their states), which leaves
+// out what is zero by structure: a block of several packed components has eigenvectors of one
+// component each, and Q only couples components that D couples.  Listing them took E of 6 spins
+// from 1216 to 792 and left no element with a reverse element (4 spins: 256 to 56), k_corr at
+// n = 100 3.5 -> 1.7 ms.
 // In-register DFT of RAD = 2, 4 or 8 points, X_k = sum_m x_m e^{SG 2 pi i m k / RAD}, natural
 // order in and out (radix 8 as two radix-4 halves joined by e^{SG i pi k / 4}).
 template <int SG, typename V> __device__ __forceinline__ V mul_si(V a) { // a * (SG i)
@@ -2231,11 +2235,15 @@ __device__ __forceinline__ void corr_mid_pass(typename CX<R>::T *sQ, const typen
     }
 }
 
+// FID tiles (16 steps x 8 periods) a wave holds: up to 256 NPT points need at most 4 v tiles.
+template <int LN, int NPT, bool PAD> struct CorrTiles {
+    static constexpr int v = PAD ? NPT : LN >= 9 ? 8 : LN == 8 ? 4 : NPT / 2;
+};
 // NPT FID points per thread are held over a segment (npts <= 256 NPT).  LN > 0 selects the FFT
 // variant with transforms of 2^LN points (CorrFft<LN>): n = 2^LN, or (PAD) any n <= 2^(LN-1), the
 // sequences zero-padded and the linear correlation folded to period n afterwards.  LN = 0 is the
 // direct sum for any n.  PAD against the direct sum (6 spins, 1154 crystallites, n = 100, 1000
-// points, complex64): CORRPAD_FIGS.  The complex64 FFT variant
+// points, complex64): 10.6 -> 4.7 ms.  The complex64 FFT variant
 // with four points is held to three waves per SIMD (168 registers: at four it spilled, and its
 // sixteen loads per chunk then waited on the spill reloads); the others are bound by LDS or
 // registers at two.  OCC > 0 replaces that bound (a variant the launch autotuner may choose).
@@ -2244,8 +2252,6 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                                               const typename CX<R>::T *__restrict__ Qt,
                                               const typename CX<R>::T *__restrict__ Rt,
                                               const double *__restrict__ thetas,
-                                              const int *__restrict__ elem_r,
-                                              const int *__restrict__ elem_s,
                                               double *__restrict__ part, int ch_lo, int ch_hi,
                                               int seg_base) {
     typedef typename CX<R>::T CT;
@@ -2291,23 +2297,32 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
     // V_j(e) = z_e^(n j) (in the correlation's second buffer, free by then): no sine or cosine
     // per point.  The table takes GE elements at a time (all CH where CH J fits CORR_VTAB
     // entries); longer FIDs go out per chunk.
+    // That sum is a contraction over e on FP64 matrix cores: output tiles of 16 steps p (rows) by
+    // 8 periods j (columns 0-7 the real, 8-15 the imaginary part), k = 4 elements at a time,
+    //   [Re F | Im F] += Re G [Re V | Im V] + Im G [-Im V | Re V],
+    // the RT x CT tiles dealt round robin to the four waves and held by them over the segment.
+    // On the vector ALUs every point read G and V from LDS for every element, most of the kernel's
+    // LDS traffic (batched clusters, n = 128, 1024 points: k_corr 54.3 -> 39.4 ms).
     const int J = (P.npts + n - 1) / n;
-    const bool hold = P.npts <= 256 * NPT && (!FFT || J <= CORR_VTAB);
-    const int GE = FFT ? min(CH, max(1, CORR_VTAB / J)) : CH;
+    constexpr int TPW = CorrTiles<LN, NPT, PAD>::v;
+    const int RT = (n + 15) / 16, ntile = RT * ((J + 7) / 8);
+    const bool hold = P.npts <= 256 * NPT && (!FFT || (ntile <= 4 * TPW && 4 * J <= CORR_VTAB));
+    const int GE = FFT ? min(CH, max(4, CORR_VTAB / J & ~3)) : CH;
+    const int wv = tid >> 6, g16 = (tid >> 4) & 3, r16 = tid & 15;
     cd *sV = (cd *)sR;
     const int nth = tid < P.npts ? min(NPT, (P.npts - tid + 255) / 256) : 0;
-    int hoff[NPT], hper[PAD ? NPT : 1]; // step and period of point tid + 256 m
+    int hoff[FFT ? 1 : NPT]; // direct variant: step of point tid + 256 m
 #pragma unroll
-    for (int m = 0; m < NPT; m++) {
-        hoff[m] = FFT && !PAD ? 0 : (tid + 256 * m) % n;
-        if constexpr (PAD) hper[m] = (tid + 256 * m) / n;
-    }
+    for (int m = 0; m < (FFT ? 1 : NPT); m++) hoff[m] = FFT ? 0 : (tid + 256 * m) % n;
     for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
         const int c = (int)(task / nsg), sg = (int)(task % nsg);
         const int ch_end = ch_lo + min(nchunk, (sg + 1) * spc);
-        cd hacc[NPT];
+        cd hacc[FFT ? 1 : NPT];
+        v4d facc[FFT ? TPW : 1];
 #pragma unroll
-        for (int m = 0; m < NPT; m++) hacc[m] = cmk(0, 0);
+        for (int m = 0; m < (FFT ? 1 : NPT); m++) hacc[m] = cmk(0, 0);
+#pragma unroll
+        for (int s = 0; s < (FFT ? TPW : 1); s++) facc[s] = v4d{0, 0, 0, 0};
         for (int ch = ch_lo + sg * spc; ch < ch_end; ch++) {
             const long e0 = (long)ch * CH;
             if constexpr (FFT) {
@@ -2321,10 +2336,10 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                     // all loads are unconditional (indexes clamped in range, masked afterwards)
                     // so that the sixteen loads of Q and R issue back to back
                     const long e = e0 + el;
-                    const bool ok = e < P.Etot;
+                    const bool ok = e < P.Ecorr;
                     const long ec = ok ? e : 0;
-                    const int er_ = elem_r[ec], es_ = elem_s[ec];
-                    const int rv = (!AUTO && P.rt_from_q) ? P.elem_rev[ec] : -1;
+                    const int er_ = P.corr_r[ec], es_ = P.corr_s[ec], pos = P.corr_pos[ec];
+                    const int rv = (!AUTO && P.rt_from_q) ? P.corr_rev[ec] : -1;
                     const double *th = thetas + (size_t)c * P.N;
                     const size_t str = (size_t)(1 << LS) * P.Estr;
                     // PAD: steps from n on are zero (all of the upper half's, so only the first
@@ -2335,13 +2350,13 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                     auto row = [&](int m) {
                         return PAD ? (size_t)min(j + (m << LS), n - 1) * P.Estr : (size_t)m * str;
                     };
-                    const long rc = P.rt_from_q ? (rv >= 0 ? (long)rv : ec) : ec;
+                    const int rc = P.rt_from_q && rv >= 0 ? rv : pos;
                     const double th_r = th[er_], th_s = th[es_];
                     // AUTO (R = conj(Q): rho = (D + D^H) / 2 and no element has a reverse): the
                     // R sequence is conj of the twiddled Q sequence, so only Q is loaded
                     CT qv[NL], rw[AUTO ? 1 : NL];
 #pragma unroll
-                    for (int m = 0; m < NL; m++) qv[m] = qb[row(m) + ec];
+                    for (int m = 0; m < NL; m++) qv[m] = qb[row(m) + pos];
                     if constexpr (!AUTO) {
 #pragma unroll
                         for (int m = 0; m < NL; m++) rw[m] = rb[row(m) + rc];
@@ -2464,9 +2479,9 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                 for (int el = tid; el < CH; el += 256) {
                     long e = e0 + el;
                     double ph = 0.0;
-                    if (e < P.Etot) {
+                    if (e < P.Ecorr) {
                         const double *th = thetas + (size_t)c * P.N;
-                        ph = (th[elem_r[e]] - th[elem_s[e]]) / (double)n;
+                        ph = (th[P.corr_r[e]] - th[P.corr_s[e]]) / (double)n;
                     }
                     sphi[el] = ph;
                     sstep[el] = cexpi(256.0 * ph);
@@ -2483,14 +2498,14 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                         const cd zi = cconj(z);
                         for (int k = ka; k < kb; k++) {
                             cd q = cmk(0, 0), r = cmk(0, 0);
-                            if (e < P.Etot) {
-                                size_t o = ((size_t)c * n + k) * P.Estr + e;
+                            if (e < P.Ecorr) {
+                                const size_t ok = ((size_t)c * n + k) * P.Estr, o = ok + P.corr_pos[e];
                                 q = to_cd(Qt[o]);
                                 if (P.rt_from_q) {
                                     // R(s,r) = Q_(J,I)(s,r) + conj(Q_(I,J)(r,s))
                                     r = cconj(q);
-                                    const int rv = P.elem_rev[e];
-                                    if (rv >= 0) r = cadd(r, to_cd(Qt[((size_t)c * n + k) * P.Estr + rv]));
+                                    const int rv = P.corr_rev[e];
+                                    if (rv >= 0) r = cadd(r, to_cd(Qt[ok + rv]));
                                 } else {
                                     r = to_cd(Rt[o]);
                                 }
@@ -2543,38 +2558,41 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                 __syncthreads();
             }
             if (FFT && hold) {
-                const int ne = (int)min((long)CH, P.Etot - e0);
-                for (int g0 = 0; g0 < ne; g0 += GE) {
-                    const int g1 = min(ne, g0 + GE);
+                // every element of the chunk: those past Etot are zero in G
+                for (int g0 = 0; g0 < CH; g0 += GE) {
                     if (g0 > 0) { // the next elements' table
                         __syncthreads();
-                        for (int q = tid; q < (g1 - g0) * J; q += 256)
+                        for (int q = tid; q < min(GE, CH - g0) * J; q += 256)
                             sV[q] = cexpi((double)n * (double)(q % J) * sphi[g0 + q / J]);
                         __syncthreads();
                     }
-                    for (int e = g0; e < g1; e++) {
-                        const cd *V = sV + (e - g0) * J;
+                    const int g1 = min(GE, CH - g0);
 #pragma unroll
-                        for (int m = 0; m < NPT; m++) {
-                            if (m < nth) {
-                                const int t = tid + 256 * m;
-                                if constexpr (PAD)
-                                    cfma(hacc[m], to_cd(sQ[at(hoff[m], e)]), V[hper[m]]);
-                                else
-                                    cfma(hacc[m], to_cd(sQ[at(t & (n - 1), e)]), V[t >> LN]);
+                    for (int s = 0; s < TPW; s++) {
+                        const int tile = wv + 4 * s;
+                        if (tile < ntile) {
+                            const int rt = tile % RT, ct = tile / RT;
+                            const int p = min(16 * rt + r16, n - 1);
+                            const int j = min(8 * ct + (r16 & 7), J - 1);
+                            for (int e = 0; e < g1; e += 4) {
+                                const cd G = to_cd(sQ[at(p, g0 + e + g16)]);
+                                const cd V = sV[(e + g16) * J + j];
+                                const double b1 = r16 < 8 ? V.x : V.y, b2 = r16 < 8 ? -V.y : V.x;
+                                facc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(G.x, b1, facc[s], 0, 0, 0);
+                                facc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(G.y, b2, facc[s], 0, 0, 0);
                             }
                         }
                     }
                 }
             } else if (hold) {
-                const int ne = (int)min((long)CH, P.Etot - e0);
-                for (int e = 0; e < ne; e++) {
+                const int ne = (int)min((long)CH, P.Ecorr - e0);
+                for (int e = 0; e < ne && !FFT; e++) {
                     cd w = cexpi((double)tid * sphi[e]);
                     const cd st = sstep[e];
 #pragma unroll
-                    for (int m = 0; m < NPT; m++) {
+                    for (int m = 0; m < (FFT ? 1 : NPT); m++) {
                         if (m < nth) {
-                            cfma(hacc[m], to_cd(sQ[at(FFT ? (tid + 256 * m) & (n - 1) : hoff[m], e)]), w);
+                            cfma(hacc[m], to_cd(sQ[at(hoff[m], e)]), w);
                             w = cmul(w, st);
                         }
                     }
@@ -2588,7 +2606,7 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
 #pragma unroll
                     for (int m = 0; m < NPT; m++) acc[m] = cmk(0, 0);
                     for (int e = 0; e < CH; e++) {
-                        if (e0 + e >= P.Etot) break;
+                        if (e0 + e >= P.Ecorr) break;
                         cd w = cexpi((double)t0 * sphi[e]);
                         const cd st = sstep[e];
 #pragma unroll
@@ -2620,12 +2638,28 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
         }
         if (hold) {
             double *dst = part + 2 * (((size_t)c * P.nparts + seg_base + sg) * P.npts);
+            if constexpr (FFT) {
+                // accumulator v of a lane: step 16 rt + 4 v + g16, period 8 ct + r16 % 8
 #pragma unroll
-            for (int m = 0; m < NPT; m++) {
-                if (m < nth) {
-                    const int t = tid + 256 * m;
-                    dst[2 * t] = hacc[m].x;
-                    dst[2 * t + 1] = hacc[m].y;
+                for (int s = 0; s < TPW; s++) {
+                    const int tile = wv + 4 * s;
+                    if (tile < ntile) {
+                        const int j = 8 * (tile / RT) + (r16 & 7);
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const int p = 16 * (tile % RT) + 4 * v + g16, t = p + n * j;
+                            if (p < n && t < P.npts) dst[2 * t + (r16 >> 3)] = facc[s][v];
+                        }
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int m = 0; m < (FFT ? 1 : NPT); m++) {
+                    if (m < nth) {
+                        const int t = tid + 256 * m;
+                        dst[2 * t] = hacc[m].x;
+                        dst[2 * t + 1] = hacc[m].y;
+                    }
                 }
             }
         }
@@ -2639,27 +2673,60 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
 // w_c * scale to the group's Kahan sum (gsum, gcomp), crystallites in order.  A group split
 // across two batches carries its (sum, compensation) pair, so the result is the same bit for bit
 // whatever the batch size.  Layout of grp: [group][0: sums, 1: compensations][2 npts].
-__global__ void k_reduce(int Kb, int c0, int npts, int nparts, int G, const double *__restrict__ w,
-                         double scale, const double *__restrict__ part, double *__restrict__ grp) {
+// A workgroup takes 64 components of one group: sixteen waves add up the parts of four
+// crystallites each (their loads run side by side), then one wave adds the crystallites in order.
+// Bound by reading the parts once; a single thread per component and group, waiting for every load
+// in turn, left HBM idle (6 spins, 16 parts of 1000 points x 1154 crystallites: 0.42 -> 0.06 ms).
+#define REDUCE_W 16
+__global__ void __launch_bounds__(64 * REDUCE_W) k_reduce(int Kb, int c0, int npts, int nparts, int G,
+                                                          const double *__restrict__ w, double scale,
+                                                          const double *__restrict__ part,
+                                                          double *__restrict__ grp) {
+    __shared__ double sf[64 * 64]; // [crystallite of the chunk][component]
     const int n2 = 2 * npts;
-    const int q = blockIdx.x * blockDim.x + threadIdx.x; // re/im component index
-    const int g = c0 / G + blockIdx.y;                   // absolute group
-    if (q >= n2) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int q = blockIdx.x * 64 + lane; // re/im component index
+    const int g = c0 / G + blockIdx.y;    // absolute group
     const int ca = max(c0, g * G), cb = min(c0 + Kb, (g + 1) * G);
     if (ca >= cb) return;
+    const bool on = q < n2;
     double *gs = grp + (size_t)g * 2 * n2;
-    double s = gs[q], cmp = gs[n2 + q];
-    for (int c = ca; c < cb; c++) {
-        const double *pc = part + (size_t)(c - c0) * nparts * n2 + q;
-        double f = 0.0;
-        for (int p = 0; p < nparts; p++) f += pc[(size_t)p * n2];
-        double y = w[c] * scale * f - cmp;
-        double t = s + y;
-        cmp = (t - s) - y;
-        s = t;
+    const size_t cstr = (size_t)nparts * n2;
+    double s = 0.0, cmp = 0.0;
+    if (wv == 0 && on) {
+        s = gs[q];
+        cmp = gs[n2 + q];
     }
-    gs[q] = s;
-    gs[n2 + q] = cmp;
+    for (int c1 = ca; c1 < cb; c1 += 64) {
+        const int nc = min(64, cb - c1);
+        if (on && 4 * wv < nc) {
+            double f[4] = {0.0, 0.0, 0.0, 0.0};
+            const double *pc = part + (size_t)(c1 - c0) * cstr + q;
+            size_t o[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) o[u] = (size_t)min(4 * wv + u, nc - 1) * cstr;
+#pragma unroll 4
+            for (int p = 0; p < nparts; p++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) f[u] += pc[o[u] + (size_t)p * n2];
+#pragma unroll
+            for (int u = 0; u < 4; u++) sf[(4 * wv + u) * 64 + lane] = f[u];
+        }
+        __syncthreads();
+        if (wv == 0 && on) {
+            for (int c = 0; c < nc; c++) {
+                const double y = w[c1 + c] * scale * sf[c * 64 + lane] - cmp;
+                const double t = s + y;
+                cmp = (t - s) - y;
+                s = t;
+            }
+        }
+        __syncthreads();
+    }
+    if (wv == 0 && on) {
+        gs[q] = s;
+        gs[n2 + q] = cmp;
+    }
 }
 
 // FID point t: the groups' sums added in group order (Kahan), their compensations subtracted,
@@ -3261,8 +3328,8 @@ extern "C" int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, co
 // elements have R = conj(Q) (rosym, no reverse element)
 template <typename R, int LN, int NPT, int OCC, bool PAD>
 static void launch_corr_t(bool autoc, const DevPlan *P, int Kb, const void *Qt, const void *Rt,
-                          const double *thetas, const int *er, const int *es, double *part,
-                          int lo, int hi, int seg_base, hipStream_t st) {
+                          const double *thetas, double *part, int lo, int hi, int seg_base,
+                          hipStream_t st) {
     typedef typename CX<R>::T CT;
     const long ntask = (long)Kb * corr_range_segments(hi - lo);
     const long cap = tuned_cap(P, 5, 2);
@@ -3270,18 +3337,18 @@ static void launch_corr_t(bool autoc, const DevPlan *P, int Kb, const void *Qt, 
     if (grid <= 0) return;
     if (LN > 0 && autoc)
         k_corr<R, LN, NPT, LN != 0, OCC, PAD><<<grid, 256, 0, st>>>(*P, Kb, (const CT *)Qt, (const CT *)Rt,
-                                                          thetas, er, es, part, lo, hi, seg_base);
+                                                          thetas, part, lo, hi, seg_base);
     else
         k_corr<R, LN, NPT, false, OCC, PAD><<<grid, 256, 0, st>>>(*P, Kb, (const CT *)Qt, (const CT *)Rt,
-                                                        thetas, er, es, part, lo, hi, seg_base);
+                                                        thetas, part, lo, hi, seg_base);
 }
 // FFT variants by transform length (corr_fft_ln), LN = 0 the direct sum
 template <typename R, int NPT, int OCC = 0>
 static void launch_corr(bool autoc, const DevPlan *P, int Kb, const void *Qt, const void *Rt,
-                        const double *thetas, const int *er, const int *es, double *part,
-                        int lo, int hi, int seg_base, hipStream_t st) {
+                        const double *thetas, double *part, int lo, int hi, int seg_base,
+                        hipStream_t st) {
     const int ln = corr_fft_ln(P->n);
-#define CORR_ARGS autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, seg_base, st
+#define CORR_ARGS autoc, P, Kb, Qt, Rt, thetas, part, lo, hi, seg_base, st
     if (ln > 0 && P->n != 1 << ln) {
         // zero-padded; the two-wave variant (OCC) differs for the unpadded lengths only
         switch (ln) {
@@ -3308,10 +3375,10 @@ static void launch_corr(bool autoc, const DevPlan *P, int Kb, const void *Qt, co
 // The correlation of a batch: the leading P->corr_auto_chunks chunks with the autocorrelation
 // variant, the rest with the general one (each range segmented on its own, corr_segments).
 extern "C" int blfid_dev_launch_corr(int prec, const DevPlan *P, int Kb, const void *Qt,
-                                     const void *Rt, const double *thetas, const int *er,
-                                     const int *es, double *part, hipStream_t st) {
+                                     const void *Rt, const double *thetas, double *part,
+                                     hipStream_t st) {
     const int CH = corr_chunk(P->n);
-    const int nchunk = (int)((P->Etot + CH - 1) / CH);
+    const int nchunk = (int)((P->Ecorr + CH - 1) / CH);
     const int A = corr_use_fft(P->n) ? min(max(P->corr_auto_chunks, 0), nchunk) : 0;
     const int segA = corr_range_segments(A);
     // four points per thread up to 1024 FID points, eight above (variants 0 and 1: variant 1
@@ -3323,12 +3390,12 @@ extern "C" int blfid_dev_launch_corr(int prec, const DevPlan *P, int Kb, const v
         const int sb = pass ? segA : 0;
         if (P->npts <= 1024 && P->tn_corr != 2) {
             if (prec && P->tn_corr == 1)
-                launch_corr<float, 4, 2>(autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, sb, st);
-            else if (prec) launch_corr<float, 4>(autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, sb, st);
-            else launch_corr<double, 4>(autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, sb, st);
+                launch_corr<float, 4, 2>(autoc, P, Kb, Qt, Rt, thetas, part, lo, hi, sb, st);
+            else if (prec) launch_corr<float, 4>(autoc, P, Kb, Qt, Rt, thetas, part, lo, hi, sb, st);
+            else launch_corr<double, 4>(autoc, P, Kb, Qt, Rt, thetas, part, lo, hi, sb, st);
         } else {
-            if (prec) launch_corr<float, 8>(autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, sb, st);
-            else launch_corr<double, 8>(autoc, P, Kb, Qt, Rt, thetas, er, es, part, lo, hi, sb, st);
+            if (prec) launch_corr<float, 8>(autoc, P, Kb, Qt, Rt, thetas, part, lo, hi, sb, st);
+            else launch_corr<double, 8>(autoc, P, Kb, Qt, Rt, thetas, part, lo, hi, sb, st);
         }
     }
     return (int)hipGetLastError();
@@ -3398,8 +3465,8 @@ extern "C" int blfid_dev_launch_reduce(int Kb, int c0, int npts, int nparts, int
     if (Kb <= 0) return 0;
     const int n2 = 2 * npts;
     const int g0 = c0 / G, g1 = (c0 + Kb - 1) / G;
-    dim3 grid((n2 + 255) / 256, g1 - g0 + 1);
-    k_reduce<<<grid, 256, 0, st>>>(Kb, c0, npts, nparts, G, w, scale, part, grp);
+    dim3 grid((n2 + 63) / 64, g1 - g0 + 1);
+    k_reduce<<<grid, 64 * REDUCE_W, 0, st>>>(Kb, c0, npts, nparts, G, w, scale, part, grp);
     return (int)hipGetLastError();
 }
 
