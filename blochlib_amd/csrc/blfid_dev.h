@@ -13,6 +13,10 @@
 #ifndef LDS_PAD
 #define LDS_PAD 4
 #endif
+// The FP64 planes (k_expdyson_d): rows of 16 M + 2 doubles put the 32 eight-byte operands that
+// half a wave reads (16 rows, two columns) into distinct banks; with a padding of four, rows r and
+// r + 8 met in the same ones (41% of the kernel's cycles were bank conflicts).
+#define LDS_PAD_D 2
 
 struct DevPlan {
     int S, N;      // spins, Hilbert dimension
@@ -65,7 +69,8 @@ struct DevPlan {
     int nparts;            // FID partial sums per crystallite (correlation segments or block pairs)
     int rt_rev;            // rt_from_q and some element has a reverse element (corr_rev >= 0)
     const int *xd_off;     // nblocks + 1: start of each block's flip-flop positions in xd_list
-    const int *xd_list;    // per block of <= DEV_LDS_BLOCK states: (r LDK + q) << 8 | (i S + j)
+    const int *xd_list;    // per block of <= DEV_LDS_BLOCK states: (r LDK + q) << 8 | (i S + j),
+                           // LDK the plane rows of the plan's precision
     const int *elem_r;     // Etot: state-list position of each pair element's column (block I)
     const int *elem_s;     // Etot: state-list position of each pair element's row (block J)
     const void *rho_c;     // prepared rho per crystallite of the batch on the block pairs (storage

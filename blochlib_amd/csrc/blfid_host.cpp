@@ -42,6 +42,8 @@ int blfid_dev_launch_dyson(int prec, int M, const DevPlan *P, int Kb, const int 
                            const void *bufU, void *bufA, hipStream_t st);
 int blfid_dev_launch_expdyson(int M, const DevPlan *P, int Kb, int c0, const int *grp, int ngrp,
                               void *bufA, hipStream_t st);
+int blfid_dev_launch_expdyson_d(int M, const DevPlan *P, int Kb, int c0, const int *grp, int ngrp,
+                                double2 *bufA, hipStream_t st);
 int blfid_dev_launch_rho_prep(int prec, const DevPlan *P, const DevPlan *PP, int Kb,
                               const double2 *Aprep, const int *sblk, const int *sloc,
                               const int *nzi, const double *nzv, int nnz, void *rho_out,
@@ -400,7 +402,7 @@ struct blfid_plan {
     std::map<int, std::vector<int>> fuse_groups; // M -> blocks of <= DEV_LDS_BLOCK states
     std::vector<int> big_blocks;                 // blocks beyond DEV_LDS_BLOCK states
     // fused kernel: per block of <= DEV_LDS_BLOCK states, its flip-flop positions in the LDS plane
-    // of its tile variant M, (r LDK + q) << 8 | (i S + j), LDK = 16 M + LDS_PAD (CSR over blocks)
+    // of its tile variant M, (r LDK + q) << 8 | (i S + j), LDK = 16 M + LDS_PAD, or LDS_PAD_D for FP64 (CSR over blocks)
     std::vector<int> xd_off, xd_list;
     std::map<int, std::vector<int>> eig_cls;    // eigen-solver size class -> blocks
     int exp_slots = 0, qr_slots = 0, eig_slots = 0;
@@ -750,17 +752,23 @@ static blfid_status build_tables(blfid_plan *pl) {
         else pl->big_blocks.push_back((int)b);
     }
     pl->Lsum = uo;
-    // flip-flop positions of the fused kernel's H planes
+    // flip-flop (and rf flip) positions of the fused kernels' H planes
     pl->xd_off.assign(1, 0);
     pl->xd_list.clear();
     for (size_t b = 0; b < pl->blocks.size(); b++) {
         const auto &st = pl->blocks[b].states;
         const int d = (int)st.size();
         if (d <= DEV_LDS_BLOCK) {
-            const int LDK = 16 * ((d + 15) / 16) + LDS_PAD;
+            const int LDK = 16 * ((d + 15) / 16) + (pl->prec ? LDS_PAD : LDS_PAD_D);
             for (int r = 0; r < d; r++)
                 for (int q = 0; q < d; q++) {
                     const int x = st[r] ^ st[q];
+                    if (pl->nrfiso > 0 && __builtin_popcount((unsigned)x) == 1) {
+                        // single flip of a pulsed spin: slot S S + rf slot of the coefficients
+                        const int f = pl->spin_rf[S - 1 - __builtin_ctz((unsigned)x)];
+                        if (f >= 0) pl->xd_list.push_back(((r * LDK + q) << 8) | (S * S + f));
+                        continue;
+                    }
                     if (__builtin_popcount((unsigned)x) != 2 || (st[r] & x) == 0 || (st[r] & x) == x)
                         continue;
                     const int p1 = 31 - __builtin_clz((unsigned)x), p0 = __builtin_ctz((unsigned)x);
@@ -1538,6 +1546,7 @@ static blfid_layout::Shape shape_of(const blfid_plan *pl) {
     s.npts = pl->npts;
     s.N = pl->N;
     s.bmax = pl->bmax;
+    s.big = pl->big_blocks.empty() ? 0 : 1;
     s.rt_from_q = pl->rt_from_q ? 1 : 0;
     s.nparts = pl->nparts;
     s.exp_slots = pl->exp_slots;
@@ -1645,6 +1654,32 @@ static void carve(blfid_plan *pl, char *base, const size_t *off) {
     pl->bufRho = (pl->prep || pl->state) ? base + off[R_RHO] : nullptr;
 }
 
+// The FP64 propagators of crystallites [c0, c0 + kb) of plan pp into its bufA (launches timed on
+// plan prof when it profiles): blocks of at most 80 states by the fused chain, larger ones as step
+// propagators in bufU and their Dyson chain.
+static blfid_status enqueue_props64(blfid_plan *prof, blfid_plan *pp, const DevPlan *PP,
+                                    const blfid_layout::Shape &sh, int kb, int c0, hipStream_t st) {
+    for (auto &kv : pp->fuse_groups) {
+        PhaseScope ps(prof, 8 * 8 + kv.first, 0.0,
+                      kb * (double)PP->akeep * group_b2(pp, kv.second) * 16.0, st); // flops: device
+        LAUNCHCHK(blfid_dev_launch_expdyson_d(kv.first, PP, kb, c0, pp->d_fgrp[kv.first].p,
+                                              (int)kv.second.size(), (double2 *)pp->bufA, st));
+    }
+    if (pp->big_blocks.empty()) return BLFID_OK;
+    const std::vector<int> &big = pp->big_blocks;
+    const size_t bm2 = (size_t)pp->bmax * pp->bmax;
+    {
+        PhaseScope ps(prof, 0 * 8 + 5, 0.0, kb * (double)pp->n * group_b2(pp, big) * 16.0, st); // flops: k_exp
+        LAUNCHCHK(blfid_dev_launch_exp(0, 5, PP, kb, c0, pp->d_bigb.p, (int)big.size(), pp->scrE,
+                                       bm2, sh.exp_slots, pp->bufU, st));
+    }
+    PhaseScope ps(prof, 1 * 8 + 5, kb * (double)(pp->n - 1) * group_b3(pp, big) * 8.0,
+                  kb * (double)(pp->n + PP->akeep) * group_b2(pp, big) * 16.0, st);
+    LAUNCHCHK(blfid_dev_launch_dyson(0, 5, PP, kb, pp->d_bigb.p, (int)big.size(), pp->bufU,
+                                     pp->bufA, st));
+    return BLFID_OK;
+}
+
 // Enqueues the whole powder on `st` with the working storage at `base` (regions at off[],
 // batches of Kb crystallites) and the normalised FID written to `out` (2 npts doubles, device).
 // Every error return after the first launch leaves the launched work in the stream.
@@ -1682,18 +1717,9 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
         if (pl->ptop) {
             // U_k = exp(+i theta (H_k + H_rf,k)); A_n = U_n ... U_1; its eigenbasis gives
             // rho_m = A_n^m rho A_n^-m in closed form
-            for (auto &kv : pl->blk_groups) {
-                PhaseScope ps(pl, 0 * 8 + kv.first, 0.0,
-                              kb * (double)pl->n * group_b2(pl, kv.second) * cs, st); // flops: k_exp
-                LAUNCHCHK(blfid_dev_launch_exp(pr, kv.first, P, kb, c0, pl->d_bgrp[kv.first].p,
-                                               (int)kv.second.size(), pl->scrE, bm2, sh.exp_slots,
-                                               pl->bufU, st));
-            }
-            for (auto &kv : pl->blk_groups) {
-                PhaseScope ps(pl, 1 * 8 + kv.first, kb * (double)(pl->n - 1) * group_b3(pl, kv.second) * 8.0,
-                              kb * (double)(pl->n + 1) * group_b2(pl, kv.second) * cs, st);
-                LAUNCHCHK(blfid_dev_launch_dyson(pr, kv.first, P, kb, pl->d_bgrp[kv.first].p,
-                                                 (int)kv.second.size(), pl->bufU, pl->bufA, st));
+            {
+                const blfid_status es = enqueue_props64(pl, pl, P, sh, kb, c0, st);
+                if (es != BLFID_OK) return es;
             }
             for (auto &kv : pl->eig_cls) {
                 PhaseScope ps(pl, 2 * 8 + kv.first + 1, 0.0,
@@ -1728,21 +1754,8 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                 refresh_devplan(pp);
                 pp->dp.RP = pl->d_RP.p;
                 const DevPlan *PP = &pp->dp;
-                const size_t pbm2 = (size_t)pp->bmax * pp->bmax;
-                for (auto &kv : pp->blk_groups) {
-                    PhaseScope ps(pl, 0 * 8 + kv.first, 0.0,
-                                  kb * (double)pp->n * group_b2(pp, kv.second) * 16.0, st);
-                    LAUNCHCHK(blfid_dev_launch_exp(0, kv.first, PP, kb, c0, pp->d_bgrp[kv.first].p,
-                                                   (int)kv.second.size(), pp->scrE, pbm2,
-                                                   sh.prep->exp_slots, pp->bufU, st));
-                }
-                for (auto &kv : pp->blk_groups) {
-                    PhaseScope ps(pl, 1 * 8 + kv.first,
-                                  kb * (double)(pp->n - 1) * group_b3(pp, kv.second) * 8.0,
-                                  kb * (double)(pp->n + 1) * group_b2(pp, kv.second) * 16.0, st);
-                    LAUNCHCHK(blfid_dev_launch_dyson(0, kv.first, PP, kb, pp->d_bgrp[kv.first].p,
-                                                     (int)kv.second.size(), pp->bufU, pp->bufA, st));
-                }
+                const blfid_status es = enqueue_props64(pl, pp, PP, *sh.prep, kb, c0, st);
+                if (es != BLFID_OK) return es;
                 LAUNCHCHK(blfid_dev_launch_rho_prep(
                     pr, P, PP, kb,
                     (const double2 *)(pp->bufA + (size_t)((pp->n - 1) % 2) * pp->Lsum * 16),
@@ -1753,10 +1766,10 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                 LAUNCHCHK(blfid_dev_launch_state_gather(pr, P, kb, c0, pl->state->rho.p,
                                                         pl->bufRho, st));
             }
-            // complex64 matrix-core plans: blocks of <= 80 states take the fused propagator +
-            // Dyson chain (U_k never leaves LDS); larger blocks, the FP64 form and the BF16x3
-            // form take the propagator and the Dyson chain as two kernels; a tuning may send a
-            // tile class of the fused path to the two kernels
+            // blocks of <= 80 states take the fused propagator + Dyson chain of their precision
+            // (U_k never leaves LDS); larger blocks and the BF16x3 form take the propagator and
+            // the Dyson chain as two kernels; a tuning may send a tile class of the complex64
+            // fused path to the two kernels
             const bool fused = pr == 1 && !pl->bf16x3;
             // (tile variant, device group list, host group list) of the two-kernel path
             std::vector<std::pair<int, std::pair<const int *, const std::vector<int> *>>> two;
@@ -1772,6 +1785,9 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                                                         (int)kv.second.size(), pl->bufA, st));
                 }
                 if (!pl->big_blocks.empty()) two.push_back({5, {pl->d_bigb.p, &pl->big_blocks}});
+            } else if (pr == 0) {
+                const blfid_status es = enqueue_props64(pl, pl, P, sh, kb, c0, st);
+                if (es != BLFID_OK) return es;
             } else {
                 for (auto &kv : pl->blk_groups) two.push_back({kv.first, {pl->d_bgrp[kv.first].p, &kv.second}});
             }
@@ -2098,16 +2114,10 @@ blfid_status blfid_state_apply(blfid_state *st, const blfid_system *sys, double 
     const DevPlan *PP = &pp->dp;
     double2 *T = (double2 *)(st->ws.p + pbytes);
     const int nslots = (int)std::min<long>(Kb, 4096);
-    const size_t pbm2 = (size_t)pp->bmax * pp->bmax;
     for (int c0 = 0; c0 < K; c0 += (int)Kb) {
         const int kb = (int)std::min<long>(Kb, K - c0);
-        for (auto &kv : pp->blk_groups)
-            LAUNCHCHK(blfid_dev_launch_exp(0, kv.first, PP, kb, c0, pp->d_bgrp[kv.first].p,
-                                           (int)kv.second.size(), pp->scrE, pbm2, ps.exp_slots,
-                                           pp->bufU, s));
-        for (auto &kv : pp->blk_groups)
-            LAUNCHCHK(blfid_dev_launch_dyson(0, kv.first, PP, kb, pp->d_bgrp[kv.first].p,
-                                             (int)kv.second.size(), pp->bufU, pp->bufA, s));
+        const blfid_status es = enqueue_props64(pp.get(), pp.get(), PP, ps, kb, c0, s);
+        if (es != BLFID_OK) return es;
         LAUNCHCHK(blfid_dev_launch_state_apply(
             PP, kb, c0, (const double2 *)(pp->bufA + (size_t)((pp->n - 1) % 2) * pp->Lsum * 16),
             st->sblk.p, st->sloc.p, N, repeat, st->rho.p, T, nslots, s));

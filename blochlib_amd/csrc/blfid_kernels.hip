@@ -1319,6 +1319,643 @@ __global__ void __launch_bounds__(XdThreads<M>::v, M == 3 ? 3 : M == 2 ? 5 : 1) 
     if (P.expflops && tid == 0 && nflops > 0.0) atomicAdd(&P.expflops[8 + M], nflops);
 }
 
+// ---------------------------------------------------------------------------- k_expdyson_d
+// The fused propagator + Dyson chain in FP64 on FP64 matrix cores, for blocks of at most 80 states
+// of gamma-COMPUTE plans and of pulse (rf) propagators: one task = (crystallite c, block) walks
+// the n steps,
+//   X = theta_k H_k / 2^s, cos X and sin X as in k_exp (the same degrees, tolerance and
+//   squarings), A_k = (C + i usign S) A_{k-1},
+// and only A_k goes to global memory (every step's for gamma-COMPUTE, the last one's in slot
+// (n - 1) % akeep when only the whole propagator is wanted).
+//
+// v_mfma_f64_16x16x4f64 leaves row 4 v + g, column r of a 16 x 16 tile in register v of lane
+// 16 g + r, which is the layout of its B operand (k = g of slice v) and, for a symmetric matrix,
+// of its A operand.  So each of the M waves keeps its 16 columns (a panel of M tiles) of every
+// intermediate and of the running product in registers as the B operand of the next product, and
+// only the left operand is shared through LDS: three 16 M x 16 M planes hold X, then Y = X^2 and
+// the highest power, then C and S.  A chain Y, Y^2, Y^3 .. needs one barrier, not one per
+// product.  A block of at most 16 states is one wave with every operand in registers.
+//
+// The matrix cores reach their FP64 rate with one wave per SIMD (a dependent chain of
+// 16x16x4 products ran at 69 of 74 TFLOP/s), where the 16 M x 16 M tile products on the vector
+// ALUs waited on LDS and on their barriers: EXPD_FIGS
+//
+// With rf (RF) the step's amplitude and offset enter H and its phase is the similarity R U R^H,
+// R = diag(exp(-i sum_q phi_q M_q)): the running product is kept as R_k^H A_k, turned by
+// R_{k+1}^H R_k where the phases change and by R at the end.
+// smallest degree m in Y with rx^(2m+2)/(2m+2)! <= 1e-17 (ExpTol), 5 and 7 taken as 6 and 8
+__device__ __forceinline__ int xd_degree(double rx) {
+    return rx <= 1.2446659545e-4 ? 1 : rx <= 4.3942903513e-3 ? 2 : rx <= 2.8228647164e-2 ? 3 :
+           rx <= 9.0360016861e-2 ? 4 : rx <= 3.6912378048e-1 ? 6 : 8;
+}
+// a value every lane agrees on, in scalar registers
+__device__ __forceinline__ double to_scalar(double x) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+// LDS is complete for the workgroup; global stores under way are not waited for
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+// (-1)^j / (2j)! and (-1)^j / (2j+1)!
+__device__ __forceinline__ double xd_cos(int j) {
+    const double c[9] = {1.0, -1.0 / 2, 1.0 / 24, -1.0 / 720, 1.0 / 40320, -1.0 / 3628800,
+                         1.0 / 479001600, -1.0 / 87178291200.0, 1.0 / 20922789888000.0};
+    double v = c[0];
+#pragma unroll
+    for (int i = 1; i < 9; i++) v = j == i ? c[i] : v;
+    return v;
+}
+__device__ __forceinline__ double xd_sin(int j) {
+    const double c[9] = {1.0, -1.0 / 6, 1.0 / 120, -1.0 / 5040, 1.0 / 362880, -1.0 / 39916800,
+                         1.0 / 6227020800.0, -1.0 / 1307674368000.0, 1.0 / 355687428096000.0};
+    double v = c[0];
+#pragma unroll
+    for (int i = 1; i < 9; i++) v = j == i ? c[i] : v;
+    return v;
+}
+// phase sum_q w_q M_q(state) of one basis state, M_q = Fz of pulsed isotope q; w_q at stride 3
+__device__ __forceinline__ double xd_phase(const DevPlan &P, const double *w, int state) {
+    double phi = 0.0;
+    for (int i = 0; i < P.S; i++) {
+        const int q = P.spin_rf[i];
+        if (q >= 0) phi += w[3 * q] * (((state >> (P.S - 1 - i)) & 1) ? -0.5 : 0.5);
+    }
+    return phi;
+}
+
+__device__ __forceinline__ v4d xd_mul1(const v4d &a, const v4d &b, v4d acc, int ks) {
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        if (v < ks) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[v], b[v], acc, 0, 0, 0);
+    return acc;
+}
+
+// Blocks of at most 16 states: one wave per task.  Each lane forms its four entries of X from its
+// own rows of the quadratic-form tables (held in registers over the chain).
+template <bool RF>
+__global__ void __launch_bounds__(64) k_expdyson_d1(DevPlan P, int Kb, int c0, const int *__restrict__ grp,
+                                                    int ngrp, cd *__restrict__ bufA) {
+    const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
+    const double us = (double)P.usign;
+    const int S = P.S, n = P.n;
+    double nflops = 0.0;
+    const long ntask = (long)Kb * ngrp;
+    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int gi = (int)(task % ngrp), c = (int)(task / ngrp);
+        const int blk = __builtin_amdgcn_readfirstlane(grp[gi]);
+        const int b = __builtin_amdgcn_readfirstlane(P.blk_dim[blk]), ks = (b + 3) >> 2;
+        const int *st = P.blk_states + P.blk_soff[blk];
+        const double *RPc = P.RP + 9 * (size_t)(c0 + c);
+        cd *A0 = bufA + (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
+        // coefficients of entries (4 v + g, r); rq: rf slot of a single flip; id: the identity
+        double cf[4][7];
+        int rq[RF ? 4 : 1];
+        v4d id = v4d{0, 0, 0, 0};
+        const int sc = r < b ? st[r] : 0;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = 4 * v + g;
+            const double *src = nullptr;
+            if constexpr (RF) rq[v] = -1;
+            if (row < b && r < b) {
+                const int x = st[row] ^ sc;
+                if (row == r) {
+                    src = P.xd_cst + 7 * (size_t)sc;
+                    id[v] = 1.0;
+                } else if (__popc(x) == 2 && (sc & x) != 0 && (sc & x) != x) {
+                    const int i = S - 1 - (31 - __clz(x)), j = S - 1 - (__ffs(x) - 1);
+                    src = P.xd_fpr + 7 * (i * S + j);
+                } else if (RF && __popc(x) == 1) {
+                    rq[RF ? v : 0] = P.spin_rf[S - __ffs(x)];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 7; q++) cf[v][q] = src ? src[q] : 0.0;
+        }
+        v4d Ar = v4d{0, 0, 0, 0}, Ai = Ar;
+        for (int k = 0; k < n; k++) {
+            const double *u = P.u3 + 3 * k;
+            const double theta = RF && P.thetak ? P.thetak[k] : P.theta;
+            const double vx = RPc[0] * u[0] + RPc[3] * u[1] + RPc[6] * u[2];
+            const double vy = RPc[1] * u[0] + RPc[4] * u[1] + RPc[7] * u[2];
+            const double vz = RPc[2] * u[0] + RPc[5] * u[1] + RPc[8] * u[2];
+            const double w0 = vx * vx, w1 = vy * vy, w2 = vz * vz;
+            const double w3 = 2.0 * vx * vy, w4 = 2.0 * vx * vz, w5 = 2.0 * vy * vz;
+            v4d X;
+            double cs = 0.0;
+            const double *rfk = RF ? P.rf + (size_t)3 * P.nrfiso * k : nullptr;
+            double off = 0.0;
+            if constexpr (RF) off = r < b ? xd_phase(P, rfk + 2, sc) : 0.0;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const double *q = cf[v];
+                double x = q[0] + q[1] * w0 + q[2] * w1 + q[3] * w2 + q[4] * w3 + q[5] * w4 + q[6] * w5;
+                if constexpr (RF) {
+                    if (rq[v] >= 0) x += rfk[3 * rq[v]];
+                    x += id[v] * off;
+                }
+                X[v] = x;
+                cs += fabs(x);
+            }
+            // Y = H H (unscaled: the powers of theta / 2^s go into the coefficients), while the
+            // infinity norm is formed: column sums over the four lane groups, then their maximum
+            const v4d z = v4d{0, 0, 0, 0};
+            const v4d Y = xd_mul1(X, X, z, ks);
+            cs += __shfl_xor(cs, 16);
+            cs += __shfl_xor(cs, 32);
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) cs = fmax(cs, __shfl_xor(cs, o));
+            int sq = 0;
+            double f = theta;
+            while (cs * f > ExpTol<double>::rmax && sq < 30) {
+                f *= 0.5;
+                sq++;
+            }
+            sq = __builtin_amdgcn_readfirstlane(sq);
+            const int m = __builtin_amdgcn_readfirstlane(xd_degree(cs * f)), h = m > 4 ? m / 2 : m;
+            const double f2 = f * f;
+            v4d cur = Y;
+            v4d C = id - (0.5 * f2) * Y, Pp = id - (f2 / 6) * Y;
+            v4d Hc = z, Hs = z;
+            double fi = f2, fh = f2; // f2^i; f2^h
+            for (int i = 2; i <= h; i++) fh *= f2;
+            if (m > 4) {
+                Hc = (xd_cos(h) * fh) * id + (xd_cos(h + 1) * fh * f2) * Y;
+                Hs = (xd_sin(h) * fh) * id + (xd_sin(h + 1) * fh * f2) * Y;
+            }
+            for (int i = 2; i <= h; i++) {
+                cur = xd_mul1(Y, cur, z, ks);
+                fi *= f2;
+                if (m <= 4 || i < h) {
+                    C += (xd_cos(i) * fi) * cur;
+                    Pp += (xd_sin(i) * fi) * cur;
+                }
+                if (m > 4) {
+                    Hc += (xd_cos(h + i) * fh * fi) * cur;
+                    Hs += (xd_sin(h + i) * fh * fi) * cur;
+                }
+            }
+            if (m > 4) {
+                C = xd_mul1(cur, Hc, C, ks);
+                Pp = xd_mul1(cur, Hs, Pp, ks);
+            }
+            v4d Sn = f * xd_mul1(X, Pp, z, ks);
+            for (int it = 0; it < sq; it++) {
+                const v4d C2 = xd_mul1(-Sn, Sn, xd_mul1(C, C, z, ks), ks);
+                Sn = 2.0 * xd_mul1(C, Sn, z, ks);
+                C = C2;
+            }
+            nflops += 2.0 * b * b * b * ((m == 6 ? 6 : m == 8 ? 7 : m + 1) + 3 * sq) + (k ? 8.0 * b * b * b : 0.0);
+            if (k == 0) {
+                Ar = C;
+                Ai = us * Sn;
+            } else {
+                if constexpr (RF) {
+                    const double *rfp = rfk - 3 * P.nrfiso;
+                    bool turn = false;
+                    for (int q = 0; q < P.nrfiso; q++) turn |= rfk[3 * q + 1] != rfp[3 * q + 1];
+                    if (turn) {
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const int row = 4 * v + g;
+                            if (row < b) {
+                                const cd p = cexpi(xd_phase(P, rfk + 1, st[row]) - xd_phase(P, rfp + 1, st[row]));
+                                const cd a = cmul(p, cmk(Ar[v], Ai[v]));
+                                Ar[v] = a.x;
+                                Ai[v] = a.y;
+                            }
+                        }
+                    }
+                }
+                const v4d Su = us * Sn;
+                const v4d Nr = xd_mul1(-Su, Ai, xd_mul1(C, Ar, z, ks), ks);
+                Ai = xd_mul1(Su, Ar, xd_mul1(C, Ai, z, ks), ks);
+                Ar = Nr;
+            }
+            if (!RF || k == n - 1) {
+                cd *Ak = A0 + (size_t)(k % P.akeep) * P.Lsum;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int row = 4 * v + g;
+                    if (row < b && r < b) {
+                        cd a = cmk(Ar[v], Ai[v]);
+                        if constexpr (RF) {
+                            // A = R (R^H A R_0) R_0^H: rows by the last step's phases, columns
+                            // back by the first step's
+                            a = cmul(a, cexpi(xd_phase(P, P.rf + 1, sc) - xd_phase(P, rfk + 1, st[row])));
+                        }
+                        Ak[row + r * b] = a;
+                    }
+                }
+            }
+        }
+    }
+    if (P.expflops && lane == 0 && nflops > 0.0) atomicAdd(&P.expflops[8 + 1], nflops);
+}
+
+// The left operands of slice s + 1 are read while slice s multiplies; the scheduling barrier keeps
+// the compiler from hoisting more of them (it spilled).
+template <int M, int LD> struct XdLeft {
+    double a[M];
+    __device__ __forceinline__ void load(const double *PL, int o, int s) {
+#pragma unroll
+        for (int I = 0; I < M; I++) a[I] = PL[o + 16 * I * LD + 4 * s];
+    }
+};
+template <int M, int LD, typename F>
+__device__ __forceinline__ void xd_slices(const double *PL, int ks, F f) {
+    const int lane = threadIdx.x & 63, o = (lane & 15) * LD + (lane >> 4);
+    XdLeft<M, LD> cur, nxt;
+    cur.load(PL, o, 0);
+#pragma unroll
+    for (int s = 0; s < 4 * M; s++) {
+        if (s <= 4 * (M - 1) || s < ks) {
+            if (s + 1 < 4 * M) nxt.load(PL, o, s + 1);
+            f(s, cur.a);
+            cur = nxt;
+        }
+        if constexpr (M <= 4) { // (the largest class has no registers left for it)
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * M, 0); // the reads first,
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * M, 0); // then the products
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <int M, int LD, typename F>
+__device__ __forceinline__ void xd_slices2(const double *PL, const double *PM, int ks, F f) {
+    const int lane = threadIdx.x & 63, o = (lane & 15) * LD + (lane >> 4);
+    XdLeft<M, LD> cur, nxt, dur, nyt;
+    cur.load(PL, o, 0);
+    dur.load(PM, o, 0);
+#pragma unroll
+    for (int s = 0; s < 4 * M; s++) {
+        if (s <= 4 * (M - 1) || s < ks) {
+            if (s + 1 < 4 * M) {
+                nxt.load(PL, o, s + 1);
+                nyt.load(PM, o, s + 1);
+            }
+            f(s, cur.a, dur.a);
+            cur = nxt;
+            dur = nyt;
+        }
+        if constexpr (M <= 4) { // (the largest class has no registers left for it)
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * M, 0); // the reads first,
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * M, 0); // then the products
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <int M, int LD>
+__device__ __forceinline__ void xd_panel(const double *PL, const v4d (&B)[M], v4d (&acc)[M], int ks) {
+    xd_slices<M, LD>(PL, ks, [&](int s, const double (&a)[M]) {
+        const double bv = B[s >> 2][s & 3];
+#pragma unroll
+        for (int I = 0; I < M; I++)
+            acc[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[I], bv, acc[I], 0, 0, 0);
+    });
+}
+template <int M, int LD> __device__ __forceinline__ void xd_put(double *PL, const v4d (&T)[M]) {
+    const int lane = threadIdx.x & 63, o = (lane >> 4) * LD + 16 * (threadIdx.x >> 6) + (lane & 15);
+#pragma unroll
+    for (int I = 0; I < M; I++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) PL[o + (16 * I + 4 * v) * LD] = T[I][v];
+}
+
+// p0 d + p1 Y + p2 Y^2 + ..., one entry
+__device__ __forceinline__ double xd_poly(double d, double y1, double y2, double y3, double y4,
+                                          const double (&c)[5]) {
+    return fma(c[4], y4, fma(c[3], y3, fma(c[2], y2, fma(c[1], y1, c[0] * d))));
+}
+
+// H of a step is scattered unscaled into the X plane (its diagonal and the block's flip positions
+// xd_list, each thread keeping its share of the list in registers; s_ff holds the S x S flip-flop
+// coefficients and then amp / 2 of each pulsed isotope); the scale theta / 2^s goes into the
+// polynomial coefficients, so Y = H^2 starts before the norm is known.  Measured with the norm,
+// the scaling and their divisions ahead of the first product, half of a step's time was not spent
+// in products (64-state class, 56 states: 31.8 us a step, 14.3 of them products).
+// Blocks of 65-80 states (five waves, two on one SIMD: 256 registers each) read the running
+// product back from global memory, each lane its own entries, where the smaller classes hold it.
+#define XD_LIST 6 /* list entries per thread in registers */
+template <int M, bool RF>
+__global__ void __launch_bounds__(64 * M, M <= 3 ? 2 : 1) k_expdyson_d(DevPlan P, int Kb, int c0, const int *__restrict__ grp,
+                                                       int ngrp, cd *bufA) {
+    constexpr int NT = 64 * M, TM = 16 * M, LD = TM + LDS_PAD_D, PLANE = TM * LD;
+    constexpr bool AG = M == 5;
+    __shared__ __align__(16) double pl[3 * PLANE];
+    double *PX = pl, *PY = PX + PLANE, *PZ = PY + PLANE;
+    __shared__ double s_ff[DEV_MAX_SPINS * DEV_MAX_SPINS + (RF ? DEV_MAX_SPINS : 0)];
+    __shared__ double s_red[M];
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, r = lane & 15;
+    const int col = 16 * w + r, n = P.n, S = P.S, SS = S * S, nq = RF ? P.nrfiso : 0;
+    const double us = (double)P.usign;
+    double nflops = 0.0;
+    const long ntask = (long)Kb * ngrp;
+    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int gi = (int)(task % ngrp), c = (int)(task / ngrp);
+        const int blk = __builtin_amdgcn_readfirstlane(grp[gi]);
+        const int b = __builtin_amdgcn_readfirstlane(P.blk_dim[blk]), ks = (b + 3) >> 2;
+        const int *st = P.blk_states + P.blk_soff[blk];
+        cd *A0 = bufA + (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
+        // entries of the X plane outside H's pattern stay zero over the task
+        for (int e = tid; e < PLANE; e += NT) PX[e] = 0.0;
+        double R[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) R[i] = to_scalar(P.RP[9 * (size_t)(c0 + c) + i]);
+        const int z0 = P.xd_off[blk], z1 = P.xd_off[blk + 1];
+        int le[XD_LIST];
+#pragma unroll
+        for (int i = 0; i < XD_LIST; i++) {
+            const int z = z0 + tid + i * NT;
+            le[i] = z < z1 ? P.xd_list[z] : -1;
+        }
+        __syncthreads();
+        v4d Ar[M], Ai[M];
+#pragma unroll 1
+        for (int k = 0; k < n; k++) {
+            // lane constants made opaque in each step, or the compiler keeps every entry's
+            // identity value, address and bounds test in registers over the steps
+            int dg = col - g, rb = b - g, gc = col < b ? g + col * b : -1;
+            asm volatile("" : "+v"(dg), "+v"(rb), "+v"(gc));
+            const double theta = RF && P.thetak ? P.thetak[k] : P.theta;
+            const double *rfk = RF ? P.rf + (size_t)3 * P.nrfiso * k : nullptr;
+            {
+                const double *u = P.u3 + 3 * k;
+                const double vx = R[0] * u[0] + R[3] * u[1] + R[6] * u[2];
+                const double vy = R[1] * u[0] + R[4] * u[1] + R[7] * u[2];
+                const double vz = R[2] * u[0] + R[5] * u[1] + R[8] * u[2];
+                const double w0 = vx * vx, w1 = vy * vy, w2 = vz * vz;
+                const double w3 = 2.0 * vx * vy, w4 = 2.0 * vx * vz, w5 = 2.0 * vy * vz;
+                bool shift = false;
+                if constexpr (RF)
+                    for (int q = 0; q < nq; q++) shift |= rfk[3 * q + 2] != 0.0;
+                for (int x = tid; x < b + SS + nq; x += NT) {
+                    if (RF && x >= b + SS) {
+                        s_ff[x - b] = rfk[3 * (x - b - SS)];
+                        continue;
+                    }
+                    const double *q = x < b ? P.xd_cst + 7 * (size_t)st[x] : P.xd_fpr + 7 * (x - b);
+                    double f = q[0] + q[1] * w0 + q[2] * w1 + q[3] * w2 + q[4] * w3 + q[5] * w4 + q[6] * w5;
+                    if (RF && shift && x < b) f += xd_phase(P, rfk + 2, st[x]);
+                    if (x < b) PX[x * LD + x] = f;
+                    else s_ff[x - b] = f;
+                }
+                lds_barrier();
+#pragma unroll
+                for (int i = 0; i < XD_LIST; i++)
+                    if (le[i] >= 0) PX[le[i] >> 8] = s_ff[le[i] & 255];
+                for (int z = z0 + tid + XD_LIST * NT; z < z1; z += NT) {
+                    const int e = P.xd_list[z];
+                    PX[e >> 8] = s_ff[e & 255];
+                }
+                lds_barrier();
+            }
+            v4d C[M], Sn[M];
+            double f = theta; // theta / 2^sq
+            int sq = 0, m;
+            {
+                v4d y1[M], y2[M], y3[M], y4[M];
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) y2[I][v] = PX[(16 * I + 4 * v + g) * LD + col];
+                    y1[I] = v4d{0, 0, 0, 0};
+                }
+                xd_panel<M, LD>(PX, y2, y1, ks); // Y = H H
+                {
+                    // this wave's column sums, their maximum: the norm is the waves' maximum
+                    double cs = 0.0;
+#pragma unroll
+                    for (int I = 0; I < M; I++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) cs += fabs(y2[I][v]);
+                    cs += __shfl_xor(cs, 16);
+                    cs += __shfl_xor(cs, 32);
+#pragma unroll
+                    for (int o = 8; o > 0; o >>= 1) cs = fmax(cs, __shfl_xor(cs, o));
+                    if (lane == 0) s_red[w] = cs;
+                }
+                xd_put<M, LD>(PY, y1);
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    y2[I] = v4d{0, 0, 0, 0};
+                    y3[I] = y2[I];
+                    y4[I] = y2[I];
+                }
+                lds_barrier();
+                double hn = s_red[0];
+#pragma unroll
+                for (int i = 1; i < M; i++) hn = fmax(hn, s_red[i]);
+                while (hn * f > ExpTol<double>::rmax && sq < 30) {
+                    f *= 0.5;
+                    sq++;
+                }
+                // the same in every lane: kept in scalar registers
+                f = to_scalar(f);
+                sq = __builtin_amdgcn_readfirstlane(sq);
+                m = __builtin_amdgcn_readfirstlane(xd_degree(hn * f));
+                const int h = m > 4 ? m / 2 : m;
+                // powers of Y = (theta / 2^sq)^2 H^2: the left plane stays H^2
+                const double f2 = f * f;
+                auto scaled = [&](v4d (&y)[M]) {
+#pragma unroll
+                    for (int I = 0; I < M; I++) y[I] = f2 * y[I];
+                };
+                scaled(y1);
+                if (h >= 2) {
+                    xd_panel<M, LD>(PY, y1, y2, ks);
+                    scaled(y2);
+                }
+                if (h >= 3) {
+                    xd_panel<M, LD>(PY, y2, y3, ks);
+                    scaled(y3);
+                }
+                if (h >= 4) {
+                    xd_panel<M, LD>(PY, y3, y4, ks);
+                    scaled(y4);
+                }
+                if (m > 4) {
+                    if (h == 3) xd_put<M, LD>(PZ, y3);
+                    else xd_put<M, LD>(PZ, y4);
+                }
+                {
+                    // the four powers become four polynomials: the low parts of cos and sinc and,
+                    // where there is one, the part multiplied by Y^h (coefficients zero beyond
+                    // their degrees)
+                    double cl[5], sl[5], ch[5], sh[5];
+#pragma unroll
+                    for (int i = 0; i < 5; i++) {
+                        const bool low = m > 4 ? i < h : i <= m;
+                        cl[i] = low ? xd_cos(i) : 0.0;
+                        sl[i] = low ? xd_sin(i) : 0.0;
+                        ch[i] = i <= h ? xd_cos(h + i) : 0.0;
+                        sh[i] = i <= h ? xd_sin(h + i) : 0.0;
+                    }
+#pragma unroll
+                    for (int I = 0; I < M; I++) {
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const double d = 16 * I + 4 * v == dg && gc >= 0 ? 1.0 : 0.0;
+                            const double a1 = y1[I][v], a2 = y2[I][v], a3 = y3[I][v], a4 = y4[I][v];
+                            y1[I][v] = xd_poly(d, a1, a2, a3, a4, cl);
+                            y2[I][v] = xd_poly(d, a1, a2, a3, a4, sl);
+                            y3[I][v] = xd_poly(d, a1, a2, a3, a4, ch);
+                            y4[I][v] = xd_poly(d, a1, a2, a3, a4, sh);
+                        }
+                        // formed here, not sunk into the products below (with the powers and all
+                        // coefficients kept until then)
+                        asm volatile("" : "+v"(y1[I]), "+v"(y2[I]), "+v"(y3[I]), "+v"(y4[I]));
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (m > 4) {
+                    lds_barrier();
+                    xd_slices<M, LD>(PZ, ks, [&](int s, const double (&a)[M]) {
+                        const double qc = y3[s >> 2][s & 3], qs = y4[s >> 2][s & 3];
+#pragma unroll
+                        for (int I = 0; I < M; I++) {
+                            y1[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[I], qc, y1[I], 0, 0, 0);
+                            y2[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[I], qs, y2[I], 0, 0, 0);
+                        }
+                    });
+                }
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    C[I] = y1[I];
+                    Sn[I] = v4d{0, 0, 0, 0};
+                }
+                xd_panel<M, LD>(PX, y2, Sn, ks);
+#pragma unroll
+                for (int I = 0; I < M; I++) Sn[I] = f * Sn[I];
+            }
+            lds_barrier(); // every read of Y and of the high power done
+            xd_put<M, LD>(PY, C);
+            xd_put<M, LD>(PZ, Sn);
+            if constexpr (RF) {
+                // the turn of the running product's rows where the phases change, in the X
+                // plane's row padding (products never read it)
+                if (k > 0) {
+                    const double *rfp = rfk - 3 * P.nrfiso;
+                    for (int x = tid; x < b; x += NT) {
+                        const cd p = cexpi(xd_phase(P, rfk + 1, st[x]) - xd_phase(P, rfp + 1, st[x]));
+                        PX[x * LD + TM] = p.x;
+                        PX[x * LD + TM + 1] = p.y;
+                    }
+                }
+            }
+            lds_barrier();
+            for (int it = 0; it < sq; it++) {
+                // (C, S) <- (C^2 - S^2, 2 C S)
+                v4d c2[M], s2[M];
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    c2[I] = v4d{0, 0, 0, 0};
+                    s2[I] = c2[I];
+                }
+                xd_slices2<M, LD>(PY, PZ, ks, [&](int s, const double (&ac)[M], const double (&as)[M]) {
+                    const double bc = C[s >> 2][s & 3], bs = Sn[s >> 2][s & 3];
+#pragma unroll
+                    for (int I = 0; I < M; I++) {
+                        c2[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[I], bc, c2[I], 0, 0, 0);
+                        s2[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[I], bs, s2[I], 0, 0, 0);
+                        c2[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[I], -bs, c2[I], 0, 0, 0);
+                    }
+                });
+                lds_barrier();
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    C[I] = c2[I];
+                    Sn[I] = 2.0 * s2[I];
+                }
+                xd_put<M, LD>(PY, C);
+                xd_put<M, LD>(PZ, Sn);
+                lds_barrier();
+            }
+            nflops += 2.0 * b * b * b * ((m == 6 ? 6 : m == 8 ? 7 : m + 1) + 3 * sq) + (k ? 8.0 * b * b * b : 0.0);
+            if (k == 0) {
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    Ar[I] = C[I];
+                    Ai[I] = us * Sn[I];
+                }
+            } else {
+                if constexpr (AG) {
+                    const cd *Ap = A0 + (size_t)((k - 1) % P.akeep) * P.Lsum;
+#pragma unroll
+                    for (int I = 0; I < M; I++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const int row = 16 * I + 4 * v;
+                            const cd a = row < rb && gc >= 0 ? Ap[row + gc] : cmk(0, 0);
+                            Ar[I][v] = a.x;
+                            Ai[I][v] = a.y;
+                        }
+                }
+                if constexpr (RF) {
+                    const double *rfp = rfk - 3 * P.nrfiso;
+                    bool turn = false;
+                    for (int q = 0; q < P.nrfiso; q++) turn |= rfk[3 * q + 1] != rfp[3 * q + 1];
+                    if (turn) {
+#pragma unroll
+                        for (int I = 0; I < M; I++)
+#pragma unroll
+                            for (int v = 0; v < 4; v++) {
+                                const double *p = PX + (16 * I + 4 * v + g) * LD + TM;
+                                const cd a = cmul(cmk(p[0], p[1]), cmk(Ar[I][v], Ai[I][v]));
+                                Ar[I][v] = a.x;
+                                Ai[I][v] = a.y;
+                            }
+                    }
+                }
+                v4d nr[M], ni[M];
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    nr[I] = v4d{0, 0, 0, 0};
+                    ni[I] = nr[I];
+                }
+                xd_slices2<M, LD>(PY, PZ, ks, [&](int s, const double (&uc)[M], const double (&un)[M]) {
+                    const double br = Ar[s >> 2][s & 3], bi = Ai[s >> 2][s & 3];
+                    const double sr = us * br, si = -us * bi;
+#pragma unroll
+                    for (int I = 0; I < M; I++) {
+                        nr[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(uc[I], br, nr[I], 0, 0, 0);
+                        ni[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(uc[I], bi, ni[I], 0, 0, 0);
+                        nr[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(un[I], si, nr[I], 0, 0, 0);
+                        ni[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(un[I], sr, ni[I], 0, 0, 0);
+                    }
+                });
+#pragma unroll
+                for (int I = 0; I < M; I++) {
+                    Ar[I] = nr[I];
+                    Ai[I] = ni[I];
+                }
+            }
+            const bool last = k == n - 1;
+            if (!RF || AG || last) {
+                cd *Ak = A0 + (size_t)(k % P.akeep) * P.Lsum;
+                const double pc = RF && last && col < b ? xd_phase(P, P.rf + 1, st[col]) : 0.0;
+#pragma unroll
+                for (int I = 0; I < M; I++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const int row = 16 * I + 4 * v;
+                        if (row < rb && gc >= 0) {
+                            cd a = cmk(Ar[I][v], Ai[I][v]);
+                            if (RF && last) // A = R_n (R_n^H A R_1) R_1^H
+                                a = cmul(a, cexpi(pc - xd_phase(P, rfk + 1, st[row + g])));
+                            Ak[row + gc] = a;
+                        }
+                    }
+            }
+        }
+        __syncthreads(); // every plane read done before the next task's zeros
+    }
+    if (P.expflops && tid == 0 && nflops > 0.0) atomicAdd(&P.expflops[8 + M], nflops);
+}
+
 // ------------------------------------------------------------------------------ k_eig
 // Joint Jacobi diagonalisation of a normal matrix Mx = H1 + i H2 (H1, H2 Hermitian,
 // commuting): each 2x2 rotation is the Cardoso-Souloumiac angle for the pair (H1, H2)
@@ -3156,6 +3793,11 @@ static void launch_exp(int M, const DevPlan *P, int Kb, int c0, const int *grp, 
     R *sc = (R *)scratch;
     typename CX<R>::T *U = (typename CX<R>::T *)bufU;
     const size_t tb = sizeof(double) * DEV_TERM_STRIDE * (size_t)P->nterms; // staged terms
+    if constexpr (std::is_same<R, double>::value) {
+        // FP64 blocks of at most 80 states take the fused chain
+        k_exp<5, R><<<grid, 256, tb, st>>>(*P, Kb, c0, grp, ngrp, sc, slot, U);
+        return;
+    } else
     switch (M) {
     case 1: k_exp<1, R><<<grid, 64, tb, st>>>(*P, Kb, c0, grp, ngrp, sc, slot, U); break;
     case 2: k_exp<2, R><<<grid, 256, tb, st>>>(*P, Kb, c0, grp, ngrp, sc, slot, U); break;
@@ -3196,12 +3838,43 @@ extern "C" int blfid_dev_launch_expdyson(int M, const DevPlan *P, int Kb, int c0
     return (int)hipGetLastError();
 }
 
+// The FP64 fused chain (blocks of at most 80 states): gamma-COMPUTE plans keep every A_k, pulse
+// plans (usign > 0) the whole propagator only and take the rf form, rf or not.
+extern "C" int blfid_dev_launch_expdyson_d(int M, const DevPlan *P, int Kb, int c0, const int *grp,
+                                           int ngrp, cd *bufA, hipStream_t st) {
+    const long ntask = (long)Kb * ngrp;
+    const long cap = tuned_cap(P, 8, M);
+    const int grid = (int)(ntask < cap ? ntask : cap);
+    if (grid <= 0) return 0;
+#define XD_LAUNCH(M_)                                                                            \
+    do {                                                                                         \
+        if (P->usign < 0) k_expdyson_d<M_, false><<<grid, 64 * M_, 0, st>>>(*P, Kb, c0, grp, ngrp, bufA); \
+        else k_expdyson_d<M_, true><<<grid, 64 * M_, 0, st>>>(*P, Kb, c0, grp, ngrp, bufA);      \
+    } while (0)
+    switch (M) {
+    case 1:
+        if (P->usign < 0) k_expdyson_d1<false><<<grid, 64, 0, st>>>(*P, Kb, c0, grp, ngrp, bufA);
+        else k_expdyson_d1<true><<<grid, 64, 0, st>>>(*P, Kb, c0, grp, ngrp, bufA);
+        break;
+    case 2: XD_LAUNCH(2); break;
+    case 3: XD_LAUNCH(3); break;
+    case 4: XD_LAUNCH(4); break;
+    default: XD_LAUNCH(5); break;
+    }
+#undef XD_LAUNCH
+    return (int)hipGetLastError();
+}
+
 template <typename R>
 static void launch_dyson(int M, const DevPlan *P, int Kb, const int *grp, int ngrp, int grid,
                          const void *bufU, void *bufA, hipStream_t st) {
     typedef typename CX<R>::T CT;
     const CT *U = (const CT *)bufU;
     CT *A = (CT *)bufA;
+    if constexpr (std::is_same<R, double>::value) {
+        k_dyson<5, R, false><<<grid, 256, 0, st>>>(*P, Kb, grp, ngrp, U, A);
+        return;
+    } else
     switch (M) {
     case 1: LAUNCH_SPLIT(k_dyson, 1, R, grid, 64, st, *P, Kb, grp, ngrp, U, A); break;
     case 2: LAUNCH_SPLIT(k_dyson, 2, R, grid, 256, st, *P, Kb, grp, ngrp, U, A); break;

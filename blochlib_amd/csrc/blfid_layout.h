@@ -41,6 +41,7 @@ struct Shape {
     int npts = 1;       // FID points
     int N = 1;          // Hilbert dimension
     int bmax = 1;       // largest block
+    int big = 1;        // some block exceeds the fused chains' 80 states
     int rt_from_q = 0;  // R formed from Q (no Rt storage)
     int nparts = 1;     // FID partial sums per crystallite
     int exp_slots = 0, qr_slots = 0, eig_slots = 0;
@@ -62,15 +63,16 @@ inline void region_sizes(const Shape &s, long Kb, size_t sz[R_COUNT]) {
     const size_t cs = s.prec ? 8 : 16, rs = s.prec ? 4 : 8; // storage complex / real
     for (int i = 0; i < R_COUNT; i++) sz[i] = 0;
     if (s.kind == 2) {
-        sz[R_U] = kb * s.n * L * cs;
+        // step propagators leave LDS for blocks beyond the fused chain only
+        sz[R_U] = s.big ? kb * s.n * L * cs : 0;
         sz[R_A] = kb * 2 * L * cs;
-        sz[R_EXP] = (size_t)s.exp_slots * 9 * bm2 * rs;
+        sz[R_EXP] = s.big ? (size_t)s.exp_slots * 9 * bm2 * rs : 0;
     } else if (s.kind == 0) {
         sz[R_U] = kb * s.n * L * cs;
         sz[R_A] = kb * s.n * L * cs;
         sz[R_QT] = kb * s.n * (size_t)s.Estr * cs;
         sz[R_RT] = s.rt_from_q ? 0 : kb * s.n * (size_t)s.Estr * cs;
-        sz[R_EXP] = (size_t)s.exp_slots * 9 * bm2 * rs;
+        sz[R_EXP] = s.big || s.prec ? (size_t)s.exp_slots * 9 * bm2 * rs : 0;
         if (s.prec) sz[R_WR] = kb * L * cs;
     } else {
         sz[R_U] = kb * L * c16;
