@@ -1338,7 +1338,8 @@ __global__ void __launch_bounds__(XdThreads<M>::v, M == 3 ? 3 : M == 2 ? 5 : 1) 
 //
 // The matrix cores reach their FP64 rate with one wave per SIMD (a dependent chain of
 // 16x16x4 products ran at 69 of 74 TFLOP/s), where the 16 M x 16 M tile products on the vector
-// ALUs waited on LDS and on their barriers: EXPD_FIGS
+// ALUs waited on LDS and on their barriers (8 spins, 1154 crystallites x 128 steps: blocks of 70
+// states 79 -> 47 ms, of 56 70 -> 30 ms; 64 states under rf x 256 steps 171 -> 73 ms).
 //
 // With rf (RF) the step's amplitude and offset enter H and its phase is the similarity R U R^H,
 // R = diag(exp(-i sum_q phi_q M_q)): the running product is kept as R_k^H A_k, turned by
@@ -1393,14 +1394,71 @@ __device__ __forceinline__ v4d xd_mul1(const v4d &a, const v4d &b, v4d acc, int 
     return acc;
 }
 
-// Blocks of at most 16 states: one wave per task.  Each lane forms its four entries of X from its
-// own rows of the quadratic-form tables (held in registers over the chain).
+// C = cos X and Pp = sinc X of one 16 x 16 tile from Y = X^2 in registers, degree m
+template <int m>
+__device__ __forceinline__ void xd_series1(const v4d &Y, const v4d &id, int ks, v4d &C, v4d &Pp) {
+    constexpr double cc[9] = {1.0, -1.0 / 2, 1.0 / 24, -1.0 / 720, 1.0 / 40320, -1.0 / 3628800,
+                              1.0 / 479001600, -1.0 / 87178291200.0, 1.0 / 20922789888000.0};
+    constexpr double ss[9] = {1.0, -1.0 / 6, 1.0 / 120, -1.0 / 5040, 1.0 / 362880, -1.0 / 39916800,
+                              1.0 / 6227020800.0, -1.0 / 1307674368000.0, 1.0 / 355687428096000.0};
+    constexpr int h = m > 4 ? m / 2 : m;
+    const v4d z = v4d{0, 0, 0, 0};
+    C = id + cc[1] * Y;
+    Pp = id + ss[1] * Y;
+    v4d cur = Y, Hc = z, Hs = z;
+    if constexpr (m > 4) {
+        Hc = cc[h] * id + cc[h + 1] * Y;
+        Hs = ss[h] * id + ss[h + 1] * Y;
+    }
+#pragma unroll
+    for (int i = 2; i <= h; i++) {
+        cur = xd_mul1(Y, cur, z, ks);
+        if (m <= 4 || i < h) {
+            C += cc[i] * cur;
+            Pp += ss[i] * cur;
+        }
+        if constexpr (m > 4) {
+            Hc += cc[(h + i) % 9] * cur;
+            Hs += ss[(h + i) % 9] * cur;
+        }
+    }
+    if constexpr (m > 4) {
+        C = xd_mul1(cur, Hc, C, ks);
+        Pp = xd_mul1(cur, Hs, Pp, ks);
+    }
+}
+// Sum over the four lanes r, r + 16, r + 32, r + 48 and maximum over a row of 16 lanes, without LDS.
+__device__ __forceinline__ double xd_swap_sum(double x, bool half) {
+    const unsigned lo = __double2loint(x), hi = __double2hiint(x);
+    const auto l = half ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                        : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = half ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                        : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+template <int ROR> __device__ __forceinline__ double xd_row_max(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x120 + ROR, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x120 + ROR, 0xf, 0xf, true);
+    return fmax(x, __hiloint2double(hi, lo));
+}
+
+// Blocks of at most 16 states: one wave per task, three to a SIMD (two with rf).  The quadratic forms of a
+// step (the block's diagonal and the spin pairs) are dealt to the lanes, two each, their tables
+// in registers over the chain, and gathered through LDS into the wave's X tile.
+// Bound by the chain's latency for few crystallites (the degrees are compile-time paths and the
+// norm uses lane swaps for it) and by the FP64 matrix rate for many: proton pair, one crystallite x 64
+// steps 126 (propagators and chain as two kernels) -> 86 us, 1154 of them 473 -> 113 us.
+#define XD1_PAIRS (DEV_MAX_SPINS * (DEV_MAX_SPINS - 1) / 2)
 template <bool RF>
-__global__ void __launch_bounds__(64) k_expdyson_d1(DevPlan P, int Kb, int c0, const int *__restrict__ grp,
+__global__ void __launch_bounds__(64, RF ? 2 : 3) k_expdyson_d1(DevPlan P, int Kb, int c0, const int *__restrict__ grp,
                                                     int ngrp, cd *__restrict__ bufA) {
+    // forms of a step: block rows 0..15, then the pairs i < j; slot XD1_ZERO stays zero
+    constexpr int NF = 16 + XD1_PAIRS, XD1_ZERO = NF;
+    __shared__ double s_f[NF + 1];
     const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
     const double us = (double)P.usign;
-    const int S = P.S, n = P.n;
+    const int S = P.S, n = P.n, npair = S * (S - 1) / 2;
+    if (lane == 0) s_f[XD1_ZERO] = 0.0;
     double nflops = 0.0;
     const long ntask = (long)Kb * ngrp;
     for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
@@ -1408,99 +1466,115 @@ __global__ void __launch_bounds__(64) k_expdyson_d1(DevPlan P, int Kb, int c0, c
         const int blk = __builtin_amdgcn_readfirstlane(grp[gi]);
         const int b = __builtin_amdgcn_readfirstlane(P.blk_dim[blk]), ks = (b + 3) >> 2;
         const int *st = P.blk_states + P.blk_soff[blk];
-        const double *RPc = P.RP + 9 * (size_t)(c0 + c);
         cd *A0 = bufA + (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
-        // coefficients of entries (4 v + g, r); rq: rf slot of a single flip; id: the identity
-        double cf[4][7];
-        int rq[RF ? 4 : 1];
+        double R[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) R[i] = to_scalar(P.RP[9 * (size_t)(c0 + c) + i]);
+        // this lane's forms: x = lane and lane + 64 of [block rows (b), pairs]
+        double cf[2][7];
+        int fx[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int x = lane + 64 * i;
+            const double *src = nullptr;
+            fx[i] = -1;
+            if (x < b) {
+                src = P.xd_cst + 7 * (size_t)st[x];
+                fx[i] = x;
+            } else if (x < b + npair) {
+                int a = 0, q = x - b;
+                while (q >= S - 1 - a) q -= S - 1 - a++;
+                src = P.xd_fpr + 7 * (a * S + a + 1 + q);
+                fx[i] = 16 + x - b;
+            }
+#pragma unroll
+            for (int q = 0; q < 7; q++) cf[i][q] = src ? src[q] : 0.0;
+        }
+        // entries (4 v + g, r) of X: their form, or the rf slot of a single flip
+        int ex[4], rq[RF ? 4 : 1];
         v4d id = v4d{0, 0, 0, 0};
         const int sc = r < b ? st[r] : 0;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int row = 4 * v + g;
-            const double *src = nullptr;
+            ex[v] = XD1_ZERO;
             if constexpr (RF) rq[v] = -1;
             if (row < b && r < b) {
                 const int x = st[row] ^ sc;
                 if (row == r) {
-                    src = P.xd_cst + 7 * (size_t)sc;
+                    ex[v] = r;
                     id[v] = 1.0;
                 } else if (__popc(x) == 2 && (sc & x) != 0 && (sc & x) != x) {
                     const int i = S - 1 - (31 - __clz(x)), j = S - 1 - (__ffs(x) - 1);
-                    src = P.xd_fpr + 7 * (i * S + j);
+                    ex[v] = 16 + i * S - i * (i + 1) / 2 + j - i - 1;
                 } else if (RF && __popc(x) == 1) {
                     rq[RF ? v : 0] = P.spin_rf[S - __ffs(x)];
                 }
             }
-#pragma unroll
-            for (int q = 0; q < 7; q++) cf[v][q] = src ? src[q] : 0.0;
         }
         v4d Ar = v4d{0, 0, 0, 0}, Ai = Ar;
+        double u[3] = {P.u3[0], P.u3[1], P.u3[2]};
         for (int k = 0; k < n; k++) {
-            const double *u = P.u3 + 3 * k;
             const double theta = RF && P.thetak ? P.thetak[k] : P.theta;
-            const double vx = RPc[0] * u[0] + RPc[3] * u[1] + RPc[6] * u[2];
-            const double vy = RPc[1] * u[0] + RPc[4] * u[1] + RPc[7] * u[2];
-            const double vz = RPc[2] * u[0] + RPc[5] * u[1] + RPc[8] * u[2];
+            const double *rfk = RF ? P.rf + (size_t)3 * P.nrfiso * k : nullptr;
+            const double vx = R[0] * u[0] + R[3] * u[1] + R[6] * u[2];
+            const double vy = R[1] * u[0] + R[4] * u[1] + R[7] * u[2];
+            const double vz = R[2] * u[0] + R[5] * u[1] + R[8] * u[2];
+            {
+                const double *un = P.u3 + 3 * min(k + 1, n - 1); // the next step's, early
+#pragma unroll
+                for (int i = 0; i < 3; i++) u[i] = un[i];
+            }
             const double w0 = vx * vx, w1 = vy * vy, w2 = vz * vz;
             const double w3 = 2.0 * vx * vy, w4 = 2.0 * vx * vz, w5 = 2.0 * vy * vz;
-            v4d X;
-            double cs = 0.0;
-            const double *rfk = RF ? P.rf + (size_t)3 * P.nrfiso * k : nullptr;
-            double off = 0.0;
-            if constexpr (RF) off = r < b ? xd_phase(P, rfk + 2, sc) : 0.0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); // last step's reads first
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const double *q = cf[v];
-                double x = q[0] + q[1] * w0 + q[2] * w1 + q[3] * w2 + q[4] * w3 + q[5] * w4 + q[6] * w5;
-                if constexpr (RF) {
-                    if (rq[v] >= 0) x += rfk[3 * rq[v]];
-                    x += id[v] * off;
-                }
-                X[v] = x;
-                cs += fabs(x);
+            for (int i = 0; i < 2; i++) {
+                const double *q = cf[i];
+                const double x = q[0] + q[1] * w0 + q[2] * w1 + q[3] * w2 + q[4] * w3 + q[5] * w4 + q[6] * w5;
+                if (fx[i] >= 0) s_f[fx[i]] = x;
             }
-            // Y = H H (unscaled: the powers of theta / 2^s go into the coefficients), while the
-            // infinity norm is formed: column sums over the four lane groups, then their maximum
-            const v4d z = v4d{0, 0, 0, 0};
-            const v4d Y = xd_mul1(X, X, z, ks);
-            cs += __shfl_xor(cs, 16);
-            cs += __shfl_xor(cs, 32);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            v4d X;
 #pragma unroll
-            for (int o = 8; o > 0; o >>= 1) cs = fmax(cs, __shfl_xor(cs, o));
+            for (int v = 0; v < 4; v++) X[v] = s_f[ex[v]];
+            if constexpr (RF) {
+                bool shift = false;
+                for (int q = 0; q < P.nrfiso; q++) shift |= rfk[3 * q + 2] != 0.0;
+                const double off = shift && r < b ? xd_phase(P, rfk + 2, sc) : 0.0;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    if (rq[v] >= 0) X[v] += rfk[3 * rq[v]];
+                    X[v] += id[v] * off;
+                }
+            }
+            // Y = H H (scaled afterwards), while the infinity norm is formed: column sums over the
+            // four lane groups, then their maximum
+            const v4d z = v4d{0, 0, 0, 0};
+            v4d Y = xd_mul1(X, X, z, ks);
+            double cs = fabs(X[0]) + fabs(X[1]) + fabs(X[2]) + fabs(X[3]);
+            cs = xd_swap_sum(xd_swap_sum(cs, true), false);
+            cs = xd_row_max<8>(cs);
+            cs = xd_row_max<4>(cs);
+            cs = xd_row_max<2>(cs);
+            cs = to_scalar(xd_row_max<1>(cs));
             int sq = 0;
-            double f = theta;
+            double f = theta; // theta / 2^sq
             while (cs * f > ExpTol<double>::rmax && sq < 30) {
                 f *= 0.5;
                 sq++;
             }
+            const int m = __builtin_amdgcn_readfirstlane(xd_degree(cs * f));
             sq = __builtin_amdgcn_readfirstlane(sq);
-            const int m = __builtin_amdgcn_readfirstlane(xd_degree(cs * f)), h = m > 4 ? m / 2 : m;
-            const double f2 = f * f;
-            v4d cur = Y;
-            v4d C = id - (0.5 * f2) * Y, Pp = id - (f2 / 6) * Y;
-            v4d Hc = z, Hs = z;
-            double fi = f2, fh = f2; // f2^i; f2^h
-            for (int i = 2; i <= h; i++) fh *= f2;
-            if (m > 4) {
-                Hc = (xd_cos(h) * fh) * id + (xd_cos(h + 1) * fh * f2) * Y;
-                Hs = (xd_sin(h) * fh) * id + (xd_sin(h + 1) * fh * f2) * Y;
-            }
-            for (int i = 2; i <= h; i++) {
-                cur = xd_mul1(Y, cur, z, ks);
-                fi *= f2;
-                if (m <= 4 || i < h) {
-                    C += (xd_cos(i) * fi) * cur;
-                    Pp += (xd_sin(i) * fi) * cur;
-                }
-                if (m > 4) {
-                    Hc += (xd_cos(h + i) * fh * fi) * cur;
-                    Hs += (xd_sin(h + i) * fh * fi) * cur;
-                }
-            }
-            if (m > 4) {
-                C = xd_mul1(cur, Hc, C, ks);
-                Pp = xd_mul1(cur, Hs, Pp, ks);
+            Y = (f * f) * Y;
+            v4d C, Pp;
+            switch (m) {
+            case 1: xd_series1<1>(Y, id, ks, C, Pp); break;
+            case 2: xd_series1<2>(Y, id, ks, C, Pp); break;
+            case 3: xd_series1<3>(Y, id, ks, C, Pp); break;
+            case 4: xd_series1<4>(Y, id, ks, C, Pp); break;
+            case 6: xd_series1<6>(Y, id, ks, C, Pp); break;
+            default: xd_series1<8>(Y, id, ks, C, Pp); break;
             }
             v4d Sn = f * xd_mul1(X, Pp, z, ks);
             for (int it = 0; it < sq; it++) {
