@@ -6,6 +6,10 @@
 #define DEV_MAX_TERMS 128
 #define DEV_MAX_SPINS 12
 #define DEV_MAX_BLOCK 256 /* largest Hilbert-space block (k_eig pair tables) */
+// Scratch of one block beyond DEV_LDS_BLOCK in the eigen-solver, besides its b x b iterate: the
+// rotations of up to 16 index pairs (16 x 16 each), then its sweep flags
+#define EIGB_V 4096
+#define EIGB_EXTRA (EIGB_V + 16)
 #define DEV_LDS_BLOCK 80  /* blocks up to this size keep k_eig's matrix in LDS */
 // Row padding (floats) of the LDS-resident product planes (chain_mfma, SymTile): rows of
 // 16 M + LDS_PAD floats, a multiple of four so that every row starts on 16 bytes (8, 12 and 20
@@ -85,7 +89,7 @@ struct DevPlan {
                            // (eight above) at the default occupancy, 1 the same at two waves
                            // per SIMD (no register spill), 2 eight points per thread
     int tn_qr;             // k_qr form per complex64 tile class: bit M-1 set takes the other form
-                           // (per-step for classes 1-2, step-walking for 3-4)
+                           // (per-step for classes 1-2, step-walking for 3-4; class 1 by k_bq1)
 };
 
 // Persistent-grid cap of a kernel family: the tuned value or 4096 workgroups; single-wave

@@ -31,6 +31,7 @@
 #include "../../include/blfid.h"
 #include "blfid_dev.h"
 #include "blfid_layout.h"
+static_assert(blfid_layout::EIG_EXTRA == EIGB_EXTRA, "eigen-solver slot");
 
 typedef std::complex<double> cplx;
 
@@ -51,12 +52,14 @@ int blfid_dev_launch_rho_prep(int prec, const DevPlan *P, const DevPlan *PP, int
 int blfid_dev_launch_eig(int prec, const DevPlan *P, int Kb, const int *grp, int ngrp,
                          const void *src, size_t src_stride, int mode, double2 *bufW,
                          void *bufWr, double *outv, int cls, double2 *gscr, size_t gslot,
-                         int nslots, hipStream_t st);
+                         int nslots, int bmax, hipStream_t st);
 int blfid_dev_launch_bmul(int prec, int M, const DevPlan *P, int Kb, const int *grp, int ngrp,
                           const void *bufA, const void *bufW, void *bufB, hipStream_t st);
 int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, const int *pgrp, int ngrp,
                         const void *bufB, void *scratch, size_t slot, int nslots, void *Qt,
                         void *Rt, hipStream_t st);
+int blfid_dev_launch_bq1(int prec, const DevPlan *P, int Kb, const int *pgrp, int ngrp,
+                         const void *bufA, const void *bufW, void *Qt, void *Rt, hipStream_t st);
 int blfid_dev_launch_corr(int prec, const DevPlan *P, int Kb, const void *Qt, const void *Rt,
                           const double *thetas, double *part, hipStream_t st);
 int blfid_dev_launch_reduce(int Kb, int c0, int npts, int nparts, int G, const double *w,
@@ -424,6 +427,7 @@ struct blfid_plan {
     // correlation elements: position in a step's Q row, states, reverse element's position or -1
     std::vector<int> corr_pos, corr_r, corr_s, corr_rev;
     std::map<int, std::vector<int>> pair_groups; // M -> pairs
+    std::map<int, std::vector<int>> bm_groups;   // M -> blocks in some pair of a class above 1
     // powder
     int K = 0;
     bool rp_dirty = false;      // cartPowder of the new powder still to be formed (in run)
@@ -437,7 +441,7 @@ struct blfid_plan {
         d_pair_roff, d_drow, d_dcol, d_rrow, d_rcol, d_er, d_es, d_cpos, d_cr, d_cs, d_crev;
     DevTab<long> d_blk_uoff, d_pair_eoff;
     DevTab<double> d_dval, d_rval;
-    std::map<int, DevTab<int>> d_bgrp, d_pgrp, d_fgrp;
+    std::map<int, DevTab<int>> d_bgrp, d_pgrp, d_fgrp, d_bmgrp;
     DevTab<int> d_bigb, d_xd_off, d_xd_list;
     std::map<int, DevTab<int>> d_eig_cls;
     DevTab<int> d_spin_rf;
@@ -788,7 +792,7 @@ static blfid_status build_tables(blfid_plan *pl) {
         auto clampi = [](double v, int lo, int hi) { return (int)std::max<double>(lo, std::min<double>(hi, v)); };
         pl->exp_slots = clampi(std::floor(2.5e9 / (9.0 * bm2 * 8.0)), 64, 16384);
         pl->qr_slots = clampi(std::floor(2.5e9 / (3.0 * bm2 * 16.0)), 64, 16384);
-        pl->eig_slots = pl->eig_cls.count(5) ? clampi(std::floor(1.0e9 / (bm2 * 16.0)), 64, 2048) : 0;
+        pl->eig_slots = pl->eig_cls.count(5) ? clampi(std::floor(1.0e9 / ((bm2 + EIGB_EXTRA) * 16.0)), 64, 2048) : 0;
     }
     if (pl->bmax > DEV_MAX_BLOCK)
         return fail(BLFID_ERR_UNSUPPORTED,
@@ -1325,6 +1329,17 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
         int M = std::min(5, (std::max(bI, bJ) + 15) / 16);
         pl->pair_groups[M].push_back((int)p);
     }
+    {
+        // B = A W is stored for the blocks whose pairs read it (class 1 pairs form it themselves)
+        std::vector<char> used(nb, 0);
+        for (auto &kv : pl->pair_groups)
+            if (kv.first > 1)
+                for (int p : kv.second) used[pl->pairs[p].I] = used[pl->pairs[p].J] = 1;
+        pl->bm_groups.clear();
+        for (auto &kv : pl->blk_groups)
+            for (int b : kv.second)
+                if (used[b]) pl->bm_groups[kv.first].push_back(b);
+    }
     pl->Etot = eo;
     pl->Estr = (eo + 15) & ~15L;
     // rosym spinning case: R_(I,J) = B_J^H (det_JI + det_IJ^H) B_I, i.e. R_(I,J)(s,r) =
@@ -1425,6 +1440,7 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
     t.add(pl->d_cs, pl->corr_s);
     t.add(pl->d_crev, pl->corr_rev);
     for (auto &kv : pl->pair_groups) t.add(pl->d_pgrp[kv.first], kv.second);
+    for (auto &kv : pl->bm_groups) t.add(pl->d_bmgrp[kv.first], kv.second);
     pl->have_ops = false; // until the tables are in place
     HIPCHK(t.commit(pl->tab_ops));
     pl->have_ops = true;
@@ -1728,8 +1744,8 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                                                (int)kv.second.size(),
                                                pl->bufA + (size_t)((pl->n - 1) % 2) * pl->Lsum * cs,
                                                (size_t)2 * pl->Lsum, 0, pl->bufW, nullptr,
-                                               pl->thetas, kv.first, pl->scrEig, bm2,
-                                               sh.eig_slots, st));
+                                               pl->thetas, kv.first, pl->scrEig, bm2 + EIGB_EXTRA,
+                                               sh.eig_slots, pl->bmax, st));
             }
             if (pl->state)
                 LAUNCHCHK(blfid_dev_launch_state_gather(0, P, kb, c0, pl->state->rho.p,
@@ -1816,22 +1832,36 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                                                (int)kv.second.size(),
                                                pl->bufA + (size_t)(pl->n - 1) * pl->Lsum * cs,
                                                (size_t)pl->n * pl->Lsum, 0, pl->bufW, pl->bufWr,
-                                               pl->thetas, kv.first, pl->scrEig, bm2,
-                                               sh.eig_slots, st));
+                                               pl->thetas, kv.first, pl->scrEig, bm2 + EIGB_EXTRA,
+                                               sh.eig_slots, pl->bmax, st));
             }
-            for (auto &kv : pl->blk_groups) {
+            // pairs of class 1 form B and Q in one pass; the BF16x3 form and the tuned per-step form
+            // of class 1 read a stored B like the other classes
+            const bool one = !pl->bf16x3 && !(pr && (pl->tn[15] & 1));
+            const void *Wst = pr ? (const void *)pl->bufWr : (const void *)pl->bufW;
+            for (auto &kv : one ? pl->bm_groups : pl->blk_groups) {
                 PhaseScope ps(pl, 3 * 8 + kv.first, kb * (double)pl->n * group_b3(pl, kv.second) * 8.0,
                               kb * (2.0 * pl->n + 1.0) * group_b2(pl, kv.second) * cs, st);
-                LAUNCHCHK(blfid_dev_launch_bmul(pr, kv.first, P, kb, pl->d_bgrp[kv.first].p,
-                                                (int)kv.second.size(), pl->bufA,
-                                                pr ? (const void *)pl->bufWr : (const void *)pl->bufW,
-                                                pl->bufU, st));
+                LAUNCHCHK(blfid_dev_launch_bmul(pr, kv.first, P, kb,
+                                                (one ? pl->d_bmgrp : pl->d_bgrp)[kv.first].p,
+                                                (int)kv.second.size(), pl->bufA, Wst, pl->bufU, st));
             }
             for (auto &kv : pl->pair_groups) {
-                PhaseScope ps(pl, 4 * 8 + kv.first, kb * (double)pl->n * pair_flops(pl, kv.second),
+                double fl = pair_flops(pl, kv.second);
+                if (one && kv.first == 1)
+                    for (int p : kv.second) {
+                        const double bI = pl->blk_dim[pl->pairs[p].I], bJ = pl->blk_dim[pl->pairs[p].J];
+                        fl += 8.0 * (bI * bI * bI + (pl->pairs[p].I == pl->pairs[p].J ? 0.0 : bJ * bJ * bJ));
+                    }
+                PhaseScope ps(pl, 4 * 8 + kv.first, kb * (double)pl->n * fl,
                               kb * (double)pl->n * cs *
                                   (pair_reads(pl, kv.second) + (pl->rt_from_q ? 1.0 : 2.0) * pair_elems(pl, kv.second)),
                               st);
+                if (one && kv.first == 1) {
+                    LAUNCHCHK(blfid_dev_launch_bq1(pr, P, kb, pl->d_pgrp[1].p, (int)kv.second.size(),
+                                                   pl->bufA, Wst, pl->bufQt, pl->bufRt, st));
+                    continue;
+                }
                 size_t slot;
                 int ns;
                 group_slots(bm2, sh.qr_slots, pair_e(pl, kv.second), kv.first, &slot, &ns);
@@ -1864,7 +1894,7 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                 LAUNCHCHK(blfid_dev_launch_eig(0, P, kb, pl->d_eig_cls[kv.first].p,
                                                (int)kv.second.size(), pl->bufU, (size_t)pl->Lsum, 1,
                                                pl->bufW, nullptr, pl->thetas, kv.first,
-                                               pl->scrEig, bm2, sh.eig_slots, st));
+                                               pl->scrEig, bm2 + EIGB_EXTRA, sh.eig_slots, pl->bmax, st));
             if (pl->state)
                 LAUNCHCHK(blfid_dev_launch_state_gather(0, P, kb, c0, pl->state->rho.p,
                                                         pl->bufRho, st));
@@ -2343,7 +2373,7 @@ static void noalloc_cap(blfid_layout::Shape &sh, const blfid_plan *pl) {
     };
     sh.exp_slots = cap(sh.exp_slots, e1);
     if (sh.qr_slots > 0) sh.qr_slots = cap(sh.qr_slots, 3.0 * bm2 * 16.0);
-    if (sh.eig_slots > 0) sh.eig_slots = cap(sh.eig_slots, bm2 * 16.0);
+    if (sh.eig_slots > 0) sh.eig_slots = cap(sh.eig_slots, (bm2 + EIGB_EXTRA) * 16.0);
 }
 
 // The plan's layout (and its preparation's, in ps) with the scratch-slot counts cut so that
@@ -2590,7 +2620,9 @@ blfid_status blfid_autotune(blfid_plan **plans, int nplans, int crystallites, vo
             if (alt < keep * now) cur[M - 1] ^= 1;
         }
         for (int M = 1; M <= 4; M++) {
-            const double dflt = std::min(slot(0, 32 + M), slot(2, 32 + M)), other = slot(1, 32 + M);
+            // (class 1: the default forms B itself, the other form needs the class's B = A W too)
+            const double dflt = std::min(slot(0, 32 + M), slot(2, 32 + M));
+            const double other = slot(1, 32 + M) + (M == 1 ? slot(1, 25) - std::min(slot(0, 25), slot(2, 25)) : 0.0);
             if (dflt <= 0.0 || other <= 0.0) continue; // no pair of this class
             const bool on = (cur[15] >> (M - 1)) & 1;
             const double now = on ? other : dflt, alt = on ? dflt : other;

@@ -2039,7 +2039,7 @@ __global__ void __launch_bounds__(64 * M, M <= 3 ? 2 : 1) k_expdyson_d(DevPlan P
 // mode 1: Mx = H block (Hermitian, static path) -> out value = Re(Mx_rr)
 #define EIG_MAXB 80
 // The block lives in LDS (b <= MB), with LDS and threads sized for that class so that
-// workgroups of small blocks share a CU; larger blocks take k_eig_blk.
+// workgroups of small blocks share a CU; larger blocks take the k_eigb_ kernels.
 // The source block may be stored in FP32 (complex64 plans); the solver always runs in FP64 and
 // W stays FP64, with a storage-precision copy Wr for the B = A W products when R != double.
 template <int MB, int NT, typename R>
@@ -2047,8 +2047,7 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
                                              int ngrp, const typename CX<R>::T *__restrict__ src,
                                              size_t src_stride, int mode, cd *__restrict__ bufW,
                                              typename CX<R>::T *__restrict__ bufWr,
-                                             double *__restrict__ outv, cd *__restrict__ gscr,
-                                             size_t gslot) {
+                                             double *__restrict__ outv) {
     typedef typename CX<R>::T CT;
     // convergence: a sweep whose rotations all stay below tol_stop = sqrt(tol_rot) ends the
     // sweeps (Jacobi converges quadratically: the off-diagonal part such a sweep leaves is of
@@ -2058,7 +2057,7 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
     constexpr double tol_rot = __is_same(R, double) ? 1e-15 : 1e-10;
     constexpr double tol_stop = __is_same(R, double) ? 3.1622776601683795e-8 : 1e-5;
     constexpr double tol_off = __is_same(R, double) ? 1e-17 : 1e-12;
-    static_assert(MB > 0 && MB <= EIG_MAXB, "blocks above 80 states take k_eig_blk");
+    static_assert(MB > 0 && MB <= EIG_MAXB, "blocks above 80 states take k_eigb_*");
     constexpr int MP = (MB + 1) / 2;
     // complex64 eigenvectors of the two largest LDS classes accumulate in LDS (FP32) when only
     // the storage-precision copy is wanted (the spinning path): the rotations then never wait on
@@ -2218,7 +2217,7 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
     }
 }
 
-// ------------------------------------------------------------------------------ k_eig_blk
+// ------------------------------------------------------------------------------ k_eigb
 // Joint rotation of the index pair (p, q) of a normal-matrix iterate: the Cardoso-Souloumiac
 // angle for H1 = (M + M^H)/2, H2 = (M - M^H)/2i, as k_eig forms it.  Returns false (identity)
 // when the pair's off-diagonal part is below tol_off of its diagonal; big: |s| > tol_big.
@@ -2258,23 +2257,210 @@ __device__ __forceinline__ bool jj_rotation(cd mpp, cd mqq, cd mpq, cd mqp, doub
     return true;
 }
 
-// Blocks of more than 80 states (b <= 256): block Jacobi with the same rotations.  The b x b
-// iterate M lives in the workgroup's global scratch slot (ld = b), W in bufW.  The indices are
-// cut into column blocks of BJ_NB (the last one padded with absent indices) and the blocks
-// paired by the circle method.  In each round every pair (P, Q) of the round -- up to 16 at
-// once -- copies its 2 BJ_NB x 2 BJ_NB principal submatrix into LDS and runs one joint-Jacobi
-// sweep on it there (15 rounds of 8 rotations), accumulating its rotation V; then
-// M <- V^H M on the pair's rows (every pair), and M <- M V, W <- W V on its columns.  Sweeps
-// repeat until no rotation of a sweep exceeds sqrt(tol_rot) (as in k_eig).  A round reads and
-// writes M twice and W once, for b / BJ_NB - 1 rounds per sweep where the scalar rotations take
-// b - 1 passes over M and W.  mode as k_eig.
+// Blocks of more than 80 states (b <= 256): block Jacobi with the same rotations, every round of
+// every block of the batch as two launches over the whole device.  The b x b iterate M, the
+// rotations and the sweep flags of a task (crystallite, block) live in its scratch slot (EIGB_*),
+// W in bufW.  The indices are cut into column blocks of BJ_NB (the last one padded with absent
+// indices) and the blocks paired by the circle method, up to 16 pairs a round:
+//   k_eigb_rot   one wave per pair: its 16 x 16 principal submatrix of M in LDS, one joint-Jacobi
+//                sweep there (15 rounds of 8 rotations), accumulating the rotation V
+//   k_eigb_upd   one wave per 16 x 16 tile (pair p, pair q): M_pq <- V_p^H M_pq V_q in registers
+//                (two complex products on FP64 matrix cores: the tile is read straight into the
+//                left-operand layout, the accumulators are the next right operand and their
+//                transposes the left one), and W_.q <- W_.q V_q likewise
+// Sweeps repeat until no rotation of a sweep exceeds sqrt(tol_rot) (as in k_eig): the flag of a
+// sweep is read by the kernels of the next, which leave a finished task alone.  EIGB_SWEEPS
+// sweeps are launched (six to eight are used); k_eigb_tail then finishes a task that needs more,
+// in one workgroup, and k_eigb_fin reads off the phases.  A round moves M and W once.
+// Bound by HBM / MALL traffic and the rotations' latency.  One workgroup per block held the device to
+// as many CUs as there were blocks, each round limited by one CU's L2 path: 64 crystallites of
+// 10 spins (blocks up to 252 states) EIGB_FIGS
 #define BJ_NB 8
 #define BJ_NS (2 * BJ_NB)
 #define BJ_MAXPAIR 16 /* b <= 16 BJ_MAXPAIR */
+#define EIGB_SWEEPS 12
+__host__ __device__ inline int eigb_nbk(int b) { return 2 * ((b + BJ_NS - 1) / BJ_NS); }
+// global index of local index l of pair pi in round `round` of a block of b states, or -1
+__device__ __forceinline__ int eigb_index(int b, int round, int pi, int l) {
+    const int nbk = eigb_nbk(b);
+    const int pa = pi, pb = nbk - 1 - pi;
+    const int ia = pa == 0 ? 0 : ((pa - 1 + round) % (nbk - 1)) + 1;
+    const int ib = pb == 0 ? 0 : ((pb - 1 + round) % (nbk - 1)) + 1;
+    const int gi = l < BJ_NB ? min(ia, ib) * BJ_NB + l : max(ia, ib) * BJ_NB + (l - BJ_NB);
+    return gi < b ? gi : -1;
+}
+// sweep flags of a slot: [0, EIGB_SWEEPS) a large rotation in that sweep, then the pairs' "rotated"
+__device__ __forceinline__ int *eigb_flags(cd *slotp, size_t gslot) {
+    return (int *)(slotp + gslot - EIGB_EXTRA + EIGB_V);
+}
 template <typename R>
-__global__ void __launch_bounds__(512) k_eig_blk(DevPlan P, int Kb, const int *__restrict__ grp,
-                                                 int ngrp, const typename CX<R>::T *__restrict__ src,
-                                                 size_t src_stride, int mode, cd *__restrict__ bufW,
+__global__ void __launch_bounds__(256) k_eigb_init(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
+                                                   const typename CX<R>::T *__restrict__ src,
+                                                   size_t src_stride, cd *__restrict__ bufW,
+                                                   cd *__restrict__ gscr, size_t gslot) {
+    const int task = t0 + blockIdx.y, c = task / ngrp, blk = grp[task % ngrp], b = P.blk_dim[blk];
+    const typename CX<R>::T *S0 = src + (size_t)c * src_stride + P.blk_uoff[blk];
+    cd *W = bufW + (size_t)c * P.Lsum + P.blk_uoff[blk], *Ms = gscr + gslot * blockIdx.y;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < b * b; e += gridDim.x * 256) {
+        Ms[e] = to_cd(S0[e]);
+        W[e] = cmk(e % b == e / b ? 1.0 : 0.0, 0.0);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 2 * EIGB_SWEEPS + BJ_MAXPAIR) eigb_flags(Ms, gslot)[threadIdx.x] = 0;
+}
+template <typename R>
+__global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
+                                                 int sweep, int round, cd *__restrict__ gscr, size_t gslot) {
+    constexpr int NB = BJ_NB, NS = BJ_NS, LS = NS + 1;
+    constexpr double tol_stop = __is_same(R, double) ? 3.1622776601683795e-8 : 1e-5;
+    constexpr double tol_off = __is_same(R, double) ? 1e-17 : 1e-12;
+    __shared__ cd Sp[NS * LS], Vp[NS * LS], rs[NB];
+    __shared__ double rc[NB];
+    const int task = t0 + blockIdx.y, pi = blockIdx.x, lane = threadIdx.x;
+    const int b = P.blk_dim[grp[task % ngrp]];
+    if (pi >= eigb_nbk(b) / 2 || round >= eigb_nbk(b) - 1) return;
+    cd *Ms = gscr + gslot * blockIdx.y;
+    int *fl = eigb_flags(Ms, gslot);
+    if (sweep > 0 && !fl[sweep - 1]) return;
+    cd *V = Ms + gslot - EIGB_EXTRA + pi * NS * NS;
+    const int gl = eigb_index(b, round, pi, lane & 15);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int i = lane & 15, j = (lane >> 4) + 4 * u;
+        const int gj = eigb_index(b, round, pi, j);
+        Sp[i + j * LS] = gl >= 0 && gj >= 0 ? Ms[gl + (size_t)gj * b] : cmk(0, 0);
+        Vp[i + j * LS] = cmk(i == j ? 1.0 : 0.0, 0.0);
+    }
+    __syncthreads();
+    bool any = false, large = false;
+    for (int sr = 0; sr < NS - 1; sr++) {
+        // circle method: position 0 fixed, the others turn; rotation k pairs positions k and NS-1-k
+        auto pos = [&](int p) { return p == 0 ? 0 : ((p - 1 + sr) % (NS - 1)) + 1; };
+        if (lane < NB) {
+            const int ia = pos(lane), ib = pos(NS - 1 - lane), p = min(ia, ib), q = max(ia, ib);
+            double cth = 1.0;
+            cd sth = cmk(0, 0);
+            bool big = false;
+            if (eigb_index(b, round, pi, p) >= 0 && eigb_index(b, round, pi, q) >= 0 &&
+                jj_rotation(Sp[p + p * LS], Sp[q + q * LS], Sp[p + q * LS], Sp[q + p * LS], tol_off,
+                            tol_stop, cth, sth, big)) {
+                any = true;
+                large |= big;
+            }
+            rc[lane] = cth;
+            rs[lane] = sth;
+        }
+        __syncthreads();
+        // S <- R^H S R on the 2 x 2 block of rotations (ki, kj); V <- V R, two entries pairs a lane
+        {
+            const int ki = lane & 7, kj = lane >> 3;
+            int ia = pos(ki), ib = pos(NS - 1 - ki);
+            const int p = min(ia, ib), q = max(ia, ib);
+            ia = pos(kj);
+            ib = pos(NS - 1 - kj);
+            const int p2 = min(ia, ib), q2 = max(ia, ib);
+            const double ci = rc[ki], cj = rc[kj];
+            const cd si = rs[ki], sj = rs[kj];
+            const cd a = Sp[p + p2 * LS], bb2 = Sp[p + q2 * LS];
+            const cd c2 = Sp[q + p2 * LS], d = Sp[q + q2 * LS];
+            const cd a1 = cadd(cscale(a, ci), cmul(cconj(si), c2));
+            const cd c1 = csub(cscale(c2, ci), cmul(si, a));
+            const cd b1 = cadd(cscale(bb2, ci), cmul(cconj(si), d));
+            const cd d1 = csub(cscale(d, ci), cmul(si, bb2));
+            Sp[p + p2 * LS] = cadd(cscale(a1, cj), cmul(sj, b1));
+            Sp[p + q2 * LS] = csub(cscale(b1, cj), cmul(cconj(sj), a1));
+            Sp[q + p2 * LS] = cadd(cscale(c1, cj), cmul(sj, d1));
+            Sp[q + q2 * LS] = csub(cscale(d1, cj), cmul(cconj(sj), c1));
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int row = (lane & 7) + 8 * u;
+                const cd wp = Vp[row + p2 * LS], wq = Vp[row + q2 * LS];
+                Vp[row + p2 * LS] = cadd(cscale(wp, cj), cmul(sj, wq));
+                Vp[row + q2 * LS] = csub(cscale(wq, cj), cmul(cconj(sj), wp));
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int i = lane & 15, j = (lane >> 4) + 4 * u;
+        V[i + j * NS] = Vp[i + j * LS];
+    }
+    const bool a2 = __any(any), l2 = __any(large);
+    if (lane == 0) {
+        fl[EIGB_SWEEPS + pi] = a2;
+        if (l2) atomicOr(&fl[sweep], 1);
+    }
+}
+// grid: x: 16 x 16 tiles of M, then of W; y: task.  Tile t = p + npr q.
+__global__ void __launch_bounds__(64) k_eigb_upd(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
+                                                 int sweep, int round, cd *__restrict__ bufW,
+                                                 cd *__restrict__ gscr, size_t gslot) {
+    constexpr int NS = BJ_NS;
+    const int task = t0 + blockIdx.y, c = task / ngrp, blk = grp[task % ngrp], b = P.blk_dim[blk];
+    const int npr = eigb_nbk(b) / 2, nrt = (b + 15) / 16;
+    if (round >= 2 * npr - 1 || (int)blockIdx.x >= npr * npr + nrt * npr) return;
+    cd *Ms = gscr + gslot * blockIdx.y;
+    const int *fl = eigb_flags(Ms, gslot);
+    if (sweep > 0 && !fl[sweep - 1]) return;
+    const bool isW = (int)blockIdx.x >= npr * npr;
+    const int t = isW ? blockIdx.x - npr * npr : blockIdx.x;
+    const int p = isW ? t % nrt : t % npr, q = isW ? t / nrt : t / npr;
+    const bool rq = fl[EIGB_SWEEPS + q], rp = !isW && fl[EIGB_SWEEPS + p];
+    if (!rq && !rp) return;
+    const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
+    const cd *Vb = Ms + gslot - EIGB_EXTRA;
+    cd *X = isW ? bufW + (size_t)c * P.Lsum + P.blk_uoff[blk] : Ms;
+    // the tile as left operand (row r, column 4 v + g) and V_q as right operand (row 4 v + g,
+    // column r)
+    const int gr = isW ? (16 * p + r < b ? 16 * p + r : -1) : eigb_index(b, round, p, r);
+    v4d xr, xi, vr, vi;
+    int gc[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        gc[v] = eigb_index(b, round, q, 4 * v + g);
+        const bool on = gr >= 0 && gc[v] >= 0;
+        const cd x = X[on ? gr + (size_t)gc[v] * b : 0];
+        xr[v] = on ? x.x : 0.0;
+        xi[v] = on ? x.y : 0.0;
+        const cd y = Vb[q * NS * NS + 4 * v + g + r * NS];
+        vr[v] = y.x;
+        vi[v] = y.y;
+    }
+    v4d sr = v4d{0, 0, 0, 0}, si = sr;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        sr = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[v], vr[v], sr, 0, 0, 0);
+        si = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[v], vi[v], si, 0, 0, 0);
+        sr = __builtin_amdgcn_mfma_f64_16x16x4f64(-xi[v], vi[v], sr, 0, 0, 0);
+        si = __builtin_amdgcn_mfma_f64_16x16x4f64(xi[v], vr[v], si, 0, 0, 0);
+    }
+    if (!isW) {
+        // V_p^H as left operand: entry (r, 4 v + g) = conj V_p(4 v + g, r)
+        v4d nr = v4d{0, 0, 0, 0}, ni = nr;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const cd y = Vb[p * NS * NS + 4 * v + g + r * NS];
+            nr = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, sr[v], nr, 0, 0, 0);
+            ni = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, si[v], ni, 0, 0, 0);
+            nr = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, si[v], nr, 0, 0, 0);
+            ni = __builtin_amdgcn_mfma_f64_16x16x4f64(-y.y, sr[v], ni, 0, 0, 0);
+        }
+        sr = nr;
+        si = ni;
+    }
+    // result: row 4 v + g, column r
+    const int oc = eigb_index(b, round, q, r);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int l = 4 * v + g, orow = isW ? (16 * p + l < b ? 16 * p + l : -1) : eigb_index(b, round, p, l);
+        if (orow >= 0 && oc >= 0) X[orow + (size_t)oc * b] = cmk(sr[v], si[v]);
+    }
+}
+// Sweeps beyond EIGB_SWEEPS of the tasks whose last flag is still set, one workgroup per task (up
+// to 40 sweeps in all), then every task's phases and its storage-precision W.
+template <typename R>
+__global__ void __launch_bounds__(512) k_eigb_tail(DevPlan P, int t0, int nt, const int *__restrict__ grp,
+                                                   int ngrp, int mode, cd *__restrict__ bufW,
                                                  typename CX<R>::T *__restrict__ bufWr,
                                                  double *__restrict__ outv, cd *__restrict__ gscr,
                                                  size_t gslot) {
@@ -2292,21 +2478,16 @@ __global__ void __launch_bounds__(512) k_eig_blk(DevPlan P, int Kb, const int *_
     __shared__ int s_rot[BJ_MAXPAIR];
     __shared__ int s_any;
     const int tid = threadIdx.x;
-    cd *Ms = gscr + gslot * blockIdx.x;
-    const long ntask = (long)Kb * ngrp;
-    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
-        const int g = (int)(task % ngrp), c = (int)(task / ngrp);
+    for (int ti = blockIdx.x; ti < nt; ti += gridDim.x) {
+        const int task = t0 + ti, g = task % ngrp, c = task / ngrp;
+        cd *Ms = gscr + gslot * ti;
         const int blk = grp[g], b = P.blk_dim[blk];
-        const CT *S0 = src + (size_t)c * src_stride + P.blk_uoff[blk];
+        const bool done = !eigb_flags(Ms, gslot)[EIGB_SWEEPS - 1];
         cd *W = bufW + (size_t)c * P.Lsum + P.blk_uoff[blk];
-        for (int e = tid; e < b * b; e += NT) {
-            Ms[e] = to_cd(S0[e]);
-            W[e] = cmk(e % b == e / b ? 1.0 : 0.0, 0.0);
-        }
         const int nbk = 2 * ((b + NS - 1) / NS); // even number of column blocks
         const int npr = nbk / 2;                 // pairs per round, <= BJ_MAXPAIR
         __syncthreads();
-        for (int sweep = 0; sweep < 40 && b > 1; sweep++) {
+        for (int sweep = EIGB_SWEEPS; sweep < 40 && !done; sweep++) {
             if (tid == 0) s_any = 0;
             for (int round = 0; round < nbk - 1; round++) {
                 for (int x = tid; x < npr * NS; x += NT) {
@@ -2750,6 +2931,221 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
             Rt[eo + e] = G[s + (size_t)r * bJ];
         }
         __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------------------ k_bq1
+// B = A W and the Q (R) products of block pairs of at most 16 states in one pass, for both
+// precisions: a wave takes a run of steps of one (crystallite, pair) with everything in registers,
+//   B_I = A_I W_I,  B_J = A_J W_J,  T = D_IJ B_J,  Q = B_I^H T
+// and, when R is not formed from Q, X = rho_JI B_I and R^T = X^T conj(B_J).  An accumulator tile
+// (row kq(v, g), column r in register v of lane 16 g + r) is the next product's right operand as it
+// is, and its transpose's left operand, so no operand goes through LDS; A_k is read straight into
+// the left-operand layout (16 lanes on 16 consecutive rows), a step ahead.  Neither B nor T is
+// stored.  Bound by the matrix rate and by reading A_k; the separate kernels wrote and re-read B,
+// staged every operand in LDS and gathered T1 there (proton pair x 1154 x 64 steps, FP64: 209 ->
+// 54 us; 5 spins, general rho: 2270 -> 720 us; the class-1 pairs of 6 spins, complex64: 1.15 + 0.08 ->
+// 0.58 ms).
+template <typename R> struct MT1;
+template <> struct MT1<double> {
+    typedef v4d V;
+    static __device__ __forceinline__ int kq(int v, int g) { return 4 * v + g; }
+    static __device__ __forceinline__ V mm(double a, double b, V c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+};
+template <> struct MT1<float> {
+    typedef v4f V;
+    static __device__ __forceinline__ int kq(int v, int g) { return 4 * g + v; }
+    static __device__ __forceinline__ V mm(float a, float b, V c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+};
+// one 16 x 16 complex operand or result: slice / register v of re and im
+template <typename R> struct CT1 {
+    typename MT1<R>::V r, i;
+};
+// slices v of a product over b states that are not all padding
+template <typename R> __device__ __forceinline__ bool bq1_on(int v, int b) {
+    return std::is_same<R, double>::value ? 4 * v < b : v < b;
+}
+// P = op(L) op(Q): CL, CQ conjugate the operand
+template <typename R, bool CL, bool CQ>
+__device__ __forceinline__ CT1<R> bq1_mul(const CT1<R> &L, const CT1<R> &Q, int b) {
+    CT1<R> p;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        p.r[v] = (R)0;
+        p.i[v] = (R)0;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        if (bq1_on<R>(v, b)) {
+            const R lr = L.r[v], li = CL ? -L.i[v] : L.i[v], qr = Q.r[v], qi = CQ ? -Q.i[v] : Q.i[v];
+            p.r = MT1<R>::mm(lr, qr, p.r);
+            p.i = MT1<R>::mm(lr, qi, p.i);
+            p.r = MT1<R>::mm(-li, qi, p.r);
+            p.i = MT1<R>::mm(li, qr, p.i);
+        }
+    }
+    return p;
+}
+// P = L Q with a real left operand
+template <typename R>
+__device__ __forceinline__ CT1<R> bq1_mul_real(const CT1<R> &L, const CT1<R> &Q, int b) {
+    CT1<R> p;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        p.r[v] = (R)0;
+        p.i[v] = (R)0;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        if (bq1_on<R>(v, b)) {
+            p.r = MT1<R>::mm(L.r[v], Q.r[v], p.r);
+            p.i = MT1<R>::mm(L.r[v], Q.i[v], p.i);
+        }
+    }
+    return p;
+}
+// left operand of a column-major b x b matrix: entry (r, kq)
+template <typename R>
+__device__ __forceinline__ CT1<R> bq1_left(const typename CX<R>::T *__restrict__ A, int b, int g, int r) {
+    CT1<R> t;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int q = MT1<R>::kq(v, g);
+        const bool on = r < b && q < b;
+        const typename CX<R>::T x = A[on ? r + q * b : 0];
+        t.r[v] = on ? x.x : (R)0;
+        t.i[v] = on ? x.y : (R)0;
+    }
+    return t;
+}
+// left operand of the sparse rows rp (absolute offsets into col / val): entry (r, kq)
+template <typename R>
+__device__ __forceinline__ CT1<R> bq1_sparse(const int *__restrict__ rp, const int *__restrict__ col,
+                                             const cd *__restrict__ val, int rows, int g, int r) {
+    CT1<R> t;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        t.r[v] = (R)0;
+        t.i[v] = (R)0;
+    }
+    if (r < rows)
+        for (int z = rp[r]; z < rp[r + 1]; z++) {
+            const int q = col[z];
+            const typename CX<R>::T x = CX<R>::from(val[z]);
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (MT1<R>::kq(v, g) == q) {
+                    t.r[v] = x.x;
+                    t.i[v] = x.y;
+                }
+        }
+    return t;
+}
+
+// Steps per task: the operands fixed over the steps are loaded once for 16 of them, fewer where that
+// would leave the device's 1024 SIMDs without two waves each (one crystallite of 64 steps: 16.9 us
+// at 16 steps a task).
+static int bq1_steps(long steps) {
+    const long s = steps / 2048;
+    return s < 1 ? 1 : s > 16 ? 16 : (int)s;
+}
+template <typename R, bool GEN>
+__global__ void __launch_bounds__(64, sizeof(R) == 4 ? 4 : 2) k_bq1(DevPlan P, int Kb, const int *__restrict__ pgrp,
+                                                                    int ngrp, int spt,
+                                                                    const typename CX<R>::T *__restrict__ bufA,
+                                                                    const typename CX<R>::T *__restrict__ bufW,
+                                                                    typename CX<R>::T *__restrict__ Qt,
+                                                                    typename CX<R>::T *__restrict__ Rt) {
+    typedef typename CX<R>::T CT;
+    typedef CT1<R> T;
+    const int lane = threadIdx.x, g = lane >> 4, r = lane & 15, n = P.n;
+    const int nch = (n + spt - 1) / spt;
+    const long ntask = (long)Kb * ngrp * nch;
+    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int ch = (int)(task % nch);
+        const long cp = task / nch;
+        const int c = (int)(cp / ngrp);
+        const int pr = __builtin_amdgcn_readfirstlane(pgrp[(int)(cp % ngrp)]);
+        const int I = __builtin_amdgcn_readfirstlane(P.pair_I[pr]);
+        const int J = __builtin_amdgcn_readfirstlane(P.pair_J[pr]);
+        const int bI = __builtin_amdgcn_readfirstlane(P.blk_dim[I]);
+        const int bJ = __builtin_amdgcn_readfirstlane(P.blk_dim[J]);
+        const bool same = I == J;
+        const long uI = P.blk_uoff[I], uJ = P.blk_uoff[J], eo = P.pair_eoff[pr];
+        // right operands W: entry (kq, r)
+        auto right = [&](const CT *W, int b) {
+            T t;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int q = MT1<R>::kq(v, g);
+                const bool on = r < b && q < b;
+                const CT x = W[on ? q + r * b : 0];
+                t.r[v] = on ? x.x : (R)0;
+                t.i[v] = on ? x.y : (R)0;
+            }
+            return t;
+        };
+        const CT *Wc = bufW + (size_t)c * P.Lsum;
+        const T WI = right(Wc + uI, bI);
+        T WJ = WI;
+        if (!same) WJ = right(Wc + uJ, bJ);
+        const T D = bq1_sparse<R>(P.d_rowptr + P.pair_doff[pr], P.d_col, (const cd *)P.d_val, bI, g, r);
+        bool cplx = false;
+#pragma unroll
+        for (int v = 0; v < 4; v++) cplx |= D.i[v] != (R)0;
+        cplx = __any(cplx);
+        T RH;
+        if constexpr (GEN) {
+            if (P.rho_c) {
+                // rho_JI^H of this crystallite (b_I x b_J): left operand entry (r, kq) = rho_JI(r, kq)
+                const CT *X = (const CT *)P.rho_c + (size_t)c * P.Etot + eo;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int q = MT1<R>::kq(v, g);
+                    const bool on = r < bJ && q < bI;
+                    const CT x = X[on ? q + r * bI : 0];
+                    RH.r[v] = on ? x.x : (R)0;
+                    RH.i[v] = on ? -x.y : (R)0;
+                }
+            } else {
+                RH = bq1_sparse<R>(P.r_rowptr + P.pair_roff[pr], P.r_col, (const cd *)P.r_val, bJ, g, r);
+            }
+        }
+        const int k0 = ch * spt, k1 = min(n, k0 + spt);
+        const CT *Ac = bufA + (size_t)c * n * P.Lsum;
+        T nI = bq1_left<R>(Ac + (size_t)k0 * P.Lsum + uI, bI, g, r), nJ = nI;
+        if (!same) nJ = bq1_left<R>(Ac + (size_t)k0 * P.Lsum + uJ, bJ, g, r);
+        for (int k = k0; k < k1; k++) {
+            const T AI = nI, AJ = nJ;
+            const size_t o = (size_t)min(k + 1, k1 - 1) * P.Lsum;
+            nI = bq1_left<R>(Ac + o + uI, bI, g, r);
+            if (!same) nJ = bq1_left<R>(Ac + o + uJ, bJ, g, r);
+            const T BI = bq1_mul<R, false, false>(AI, WI, bI);
+            T BJ = BI;
+            if (!same) BJ = bq1_mul<R, false, false>(AJ, WJ, bJ);
+            const T T1 = cplx ? bq1_mul<R, false, false>(D, BJ, bJ) : bq1_mul_real<R>(D, BJ, bJ);
+            const T Q = bq1_mul<R, true, false>(BI, T1, bI);
+            CT *q = Qt + ((size_t)c * n + k) * P.Estr + eo;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = MT1<R>::kq(v, g);
+                if (row < bI && r < bJ) q[row + r * bI] = CX<R>::mk(Q.r[v], Q.i[v]);
+            }
+            if constexpr (GEN) {
+                const T X = bq1_mul<R, false, false>(RH, BI, bI);
+                const T G = bq1_mul<R, false, true>(X, BJ, bJ);
+                CT *q2 = Rt + ((size_t)c * n + k) * P.Estr + eo;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int row = MT1<R>::kq(v, g);
+                    if (row < bI && r < bJ) q2[row + r * bI] = CX<R>::mk(G.r[v], G.i[v]);
+                }
+            }
+        }
     }
 }
 
@@ -3972,34 +4368,56 @@ extern "C" int blfid_dev_launch_dyson(int prec, int M, const DevPlan *P, int Kb,
 template <typename R>
 static void launch_eig(const DevPlan *P, int Kb, const int *grp, int ngrp, int grid,
                        const void *src, size_t src_stride, int mode, cd *bufW, void *bufWr,
-                       double *outv, int cls, cd *gscr, size_t gslot, hipStream_t st) {
+                       double *outv, int cls, hipStream_t st) {
     typedef typename CX<R>::T CT;
     const CT *S0 = (const CT *)src;
     CT *Wr = (CT *)bufWr;
-#define EIG_ARGS *P, Kb, grp, ngrp, S0, src_stride, mode, bufW, Wr, outv, gscr, gslot
+#define EIG_ARGS *P, Kb, grp, ngrp, S0, src_stride, mode, bufW, Wr, outv
     switch (cls) {
     case 0: k_eig<16, 64, R><<<grid, 64, 0, st>>>(EIG_ARGS); break;
     case 1: k_eig<32, 128, R><<<grid, 128, 0, st>>>(EIG_ARGS); break;
     case 2: k_eig<48, 256, R><<<grid, 256, 0, st>>>(EIG_ARGS); break;
     case 3: k_eig<64, 1024, R><<<grid, 1024, 0, st>>>(EIG_ARGS); break;
-    case 4: k_eig<80, 1024, R><<<grid, 1024, 0, st>>>(EIG_ARGS); break;
-    default: k_eig_blk<R><<<grid, 512, 0, st>>>(EIG_ARGS); break;
+    default: k_eig<80, 1024, R><<<grid, 1024, 0, st>>>(EIG_ARGS); break;
     }
 #undef EIG_ARGS
 }
+// Blocks beyond the LDS classes, as many tasks at a time as there are scratch slots
+template <typename R>
+static void launch_eigb(const DevPlan *P, int Kb, const int *grp, int ngrp, const void *src,
+                        size_t src_stride, int mode, cd *bufW, void *bufWr, double *outv, cd *gscr,
+                        size_t gslot, int nslots, int bmax, hipStream_t st) {
+    typedef typename CX<R>::T CT;
+    const int ntask = Kb * ngrp, npr = eigb_nbk(bmax) / 2, nrt = (bmax + 15) / 16;
+    for (int t0 = 0; t0 < ntask; t0 += nslots) {
+        const int nt = ntask - t0 < nslots ? ntask - t0 : nslots;
+        k_eigb_init<R><<<dim3(16, nt), 256, 0, st>>>(*P, t0, grp, ngrp, (const CT *)src, src_stride, bufW, gscr, gslot);
+        for (int sweep = 0; sweep < EIGB_SWEEPS; sweep++)
+            for (int round = 0; round < 2 * npr - 1; round++) {
+                k_eigb_rot<R><<<dim3(npr, nt), 64, 0, st>>>(*P, t0, grp, ngrp, sweep, round, gscr, gslot);
+                k_eigb_upd<<<dim3(npr * npr + nrt * npr, nt), 64, 0, st>>>(*P, t0, grp, ngrp, sweep, round, bufW, gscr, gslot);
+            }
+        k_eigb_tail<R><<<nt, 512, 0, st>>>(*P, t0, nt, grp, ngrp, mode, bufW, (CT *)bufWr, outv, gscr, gslot);
+    }
+}
 
 // bufWr: storage-precision copy of W (complex64 plans), or NULL.  cls: block-size class
-// 0..4 (b <= 16, 32, 48, 64, 80, LDS-resident) or 5 (larger, global scratch slots).
+// 0..4 (b <= 16, 32, 48, 64, 80, LDS-resident) or 5 (up to bmax, global scratch slots).
 extern "C" int blfid_dev_launch_eig(int prec, const DevPlan *P, int Kb, const int *grp, int ngrp,
                                     const void *src, size_t src_stride, int mode, cd *bufW,
                                     void *bufWr, double *outv, int cls, cd *gscr, size_t gslot,
-                                    int nslots, hipStream_t st) {
-    long ntask = (long)Kb * ngrp;
-    long cap = cls >= 5 ? nslots : tuned_cap(P, 2, 2);
-    int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid <= 0) return 0;
-    if (prec) launch_eig<float>(P, Kb, grp, ngrp, grid, src, src_stride, mode, bufW, bufWr, outv, cls, gscr, gslot, st);
-    else launch_eig<double>(P, Kb, grp, ngrp, grid, src, src_stride, mode, bufW, bufWr, outv, cls, gscr, gslot, st);
+                                    int nslots, int bmax, hipStream_t st) {
+    const long ntask = (long)Kb * ngrp;
+    if (ntask <= 0) return 0;
+    if (cls >= 5) {
+        if (prec) launch_eigb<float>(P, Kb, grp, ngrp, src, src_stride, mode, bufW, bufWr, outv, gscr, gslot, nslots, bmax, st);
+        else launch_eigb<double>(P, Kb, grp, ngrp, src, src_stride, mode, bufW, bufWr, outv, gscr, gslot, nslots, bmax, st);
+        return (int)hipGetLastError();
+    }
+    const long cap = tuned_cap(P, 2, 2);
+    const int grid = (int)(ntask < cap ? ntask : cap);
+    if (prec) launch_eig<float>(P, Kb, grp, ngrp, grid, src, src_stride, mode, bufW, bufWr, outv, cls, st);
+    else launch_eig<double>(P, Kb, grp, ngrp, grid, src, src_stride, mode, bufW, bufWr, outv, cls, st);
     return (int)hipGetLastError();
 }
 
@@ -4050,7 +4468,9 @@ static void launch_qr(int M, const DevPlan *P, int Kb, const int *pgrp, int ngrp
         }
     }
     switch (M) {
-    case 1: LAUNCH_SPLIT(k_qr, 1, R, grid, 64, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
+    case 1: // the BF16x3 form; otherwise class 1 takes k_bq1 (or the per-step form above)
+        if constexpr (std::is_same<R, float>::value) k_qr<1, R, true><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr);
+        break;
     case 2: LAUNCH_SPLIT_TH(k_qr, QrThreads, 2, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
     case 3: LAUNCH_SPLIT_TH(k_qr, QrThreads, 3, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
     case 4: LAUNCH_SPLIT_TH(k_qr, QrThreads, 4, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
@@ -4067,6 +4487,27 @@ extern "C" int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, co
     if (grid <= 0) return 0;
     if (prec) launch_qr<float>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
     else launch_qr<double>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
+    return (int)hipGetLastError();
+}
+
+// B = A W and the Q products of the pairs of tile class 1 (bufW in the plan's precision)
+extern "C" int blfid_dev_launch_bq1(int prec, const DevPlan *P, int Kb, const int *pgrp, int ngrp,
+                                    const void *bufA, const void *bufW, void *Qt, void *Rt,
+                                    hipStream_t st) {
+    const int spt = bq1_steps((long)Kb * ngrp * P->n);
+    const long ntask = (long)Kb * ngrp * ((P->n + spt - 1) / spt);
+    const long cap = tuned_cap(P, 4, 1);
+    const int grid = (int)(ntask < cap ? ntask : cap);
+    if (grid <= 0) return 0;
+    if (prec) {
+        const cf *A = (const cf *)bufA, *W = (const cf *)bufW;
+        if (P->rt_from_q) k_bq1<float, false><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, spt, A, W, (cf *)Qt, (cf *)Rt);
+        else k_bq1<float, true><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, spt, A, W, (cf *)Qt, (cf *)Rt);
+    } else {
+        const cd *A = (const cd *)bufA, *W = (const cd *)bufW;
+        if (P->rt_from_q) k_bq1<double, false><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, spt, A, W, (cd *)Qt, (cd *)Rt);
+        else k_bq1<double, true><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, spt, A, W, (cd *)Qt, (cd *)Rt);
+    }
     return (int)hipGetLastError();
 }
 

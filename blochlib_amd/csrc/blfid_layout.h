@@ -34,6 +34,9 @@ enum Region {
 // thread per FID component, and the groups are then summed in order (k_reduce / k_finish).
 constexpr int CRYST_GROUP = 64;
 
+// complex128 entries of an eigen-solver slot beyond the block's matrix (rotations and flags)
+constexpr size_t EIG_EXTRA = 4112;
+
 struct Shape {
     int prec = 0;       // 1: complex64 storage of U, A, B, Q, R
     int kind = 0;       // 0 gamma-COMPUTE (spinning), 1 static, 2 pulse program (ptop)
@@ -82,7 +85,7 @@ inline void region_sizes(const Shape &s, long Kb, size_t sz[R_COUNT]) {
     sz[R_THETA] = kb * s.N * d8;
     sz[R_QR] = (size_t)s.qr_slots * 3 * bm2 * c16;
     sz[R_PART] = kb * (size_t)s.nparts * 2 * s.npts * d8;
-    sz[R_EIG] = (size_t)s.eig_slots * bm2 * c16;
+    sz[R_EIG] = (size_t)s.eig_slots * (bm2 + EIG_EXTRA) * c16;
     sz[R_GROUP] = ngroups(s.K) * 2 * (2 * (size_t)s.npts) * d8;
     sz[R_RHO] = kb * (size_t)s.rho_elems * cs;
     if (s.prep) {

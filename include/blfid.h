@@ -308,8 +308,9 @@ blfid_status blfid_plan_phase_bytes(blfid_plan *plan, double *bytes);
  *   [6..14] persistent-grid cap (workgroups) of the kernel families in profiling-phase order
  *           (exp, dyson, eig, bmul, qr, corr, reduce, static, expdyson); 0 the default 4096;
  *   [15]    Q-product (k_qr) form of the complex64 tile classes 1-4: bit M-1 set takes the other
- *           form (one task per step for classes 1-2, whose default walks the steps of a
- *           crystallite with the pair in LDS; the step-walking form for classes 3-4).
+ *           form (one task per step for classes 1-2, whose defaults are the one-pass B = A W and
+ *           Q products in registers and the steps of a crystallite walked with the pair in LDS;
+ *           the step-walking form for classes 3-4).
  * Every choice gives the same FID bit for bit except [0..4] and [15], which switch between two
  * complex64 forms (both within the complex64 tolerance of the FP64 form).  Each device has a process-wide
  * table (all zero at start); a plan takes the table of the current device when it is created.
