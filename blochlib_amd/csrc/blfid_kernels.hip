@@ -2276,10 +2276,10 @@ __device__ __forceinline__ bool jj_rotation(cd mpp, cd mqq, cd mpq, cd mqp, doub
 // Sweeps repeat until no rotation of a sweep exceeds sqrt(tol_rot) (as in k_eig): the flag of a
 // sweep is read by the kernels of the next, which leave a finished task alone.  EIGB_SWEEPS
 // sweeps are launched (six to eight are used); k_eigb_tail then finishes a task that needs more,
-// in one workgroup, and k_eigb_fin reads off the phases.  A round moves M and W once.
+// in one workgroup, and reads off the phases.  A round moves M and W once.
 // Bound by HBM / MALL traffic and the rotations' latency.  One workgroup per block held the device to
 // as many CUs as there were blocks, each round limited by one CU's L2 path: 64 crystallites of
-// 10 spins (blocks up to 252 states) EIGB_FIGS
+// 10 spins (blocks up to 252 states) 198 -> 82 ms.
 #define BJ_NB 8
 #define BJ_NS (2 * BJ_NB)
 #define BJ_MAXPAIR 16 /* b <= 16 BJ_MAXPAIR */
@@ -3180,15 +3180,16 @@ __global__ void __launch_bounds__(64, sizeof(R) == 4 ? 4 : 2) k_bq1(DevPlan P, i
 // from 1216 to 792 and left no element with a reverse element (4 spins: 256 to 56), k_corr at
 // n = 100 3.5 -> 1.7 ms.
 // In-register DFT of RAD = 2, 4 or 8 points, X_k = sum_m x_m e^{SG 2 pi i m k / RAD}, natural
-// order in and out (radix 8 as two radix-4 halves joined by e^{SG i pi k / 4}).
+// order in and out (radix 8 as two radix-4 halves joined by e^{SG i pi k / 4}).  COMP: the rounding
+// of 1 / sqrt(2) is made up for (CorrFft).
 template <int SG, typename V> __device__ __forceinline__ V mul_si(V a) { // a * (SG i)
     V r;
     r.x = SG > 0 ? -a.y : a.y;
     r.y = SG > 0 ? a.x : -a.x;
     return r;
 }
-template <int RAD, int SG, typename R> struct RegDFT;
-template <int SG, typename R> struct RegDFT<2, SG, R> {
+template <int RAD, int SG, typename R, bool COMP = false> struct RegDFT;
+template <int SG, typename R, bool COMP> struct RegDFT<2, SG, R, COMP> {
     typedef typename CX<R>::T V;
     static __device__ __forceinline__ void run(V (&x)[2]) {
         const V a = x[0];
@@ -3196,7 +3197,7 @@ template <int SG, typename R> struct RegDFT<2, SG, R> {
         x[1] = csub(a, x[1]);
     }
 };
-template <int SG, typename R> struct RegDFT<4, SG, R> {
+template <int SG, typename R, bool COMP> struct RegDFT<4, SG, R, COMP> {
     typedef typename CX<R>::T V;
     static __device__ __forceinline__ void run(V (&x)[4]) {
         const V a = cadd(x[0], x[2]), b = csub(x[0], x[2]);
@@ -3207,18 +3208,19 @@ template <int SG, typename R> struct RegDFT<4, SG, R> {
         x[3] = csub(b, d);
     }
 };
-template <int SG, typename R> struct RegDFT<8, SG, R> {
+template <int SG, typename R, bool COMP> struct RegDFT<8, SG, R, COMP> {
     typedef typename CX<R>::T V;
     static __device__ __forceinline__ void run(V (&x)[8]) {
         V e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
         RegDFT<4, SG, R>::run(e);
         RegDFT<4, SG, R>::run(o);
-        const R h = (R)0.70710678118654752440;
+        constexpr R h = (R)0.70710678118654752440, hl = (R)(0.70710678118654752440 - (double)h);
+        auto mh = [](R x) { return COMP ? __builtin_elementwise_fma(h, x, hl * x) : h * x; };
         V t1, t3; // o_1 (1 + SG i) h and o_3 (-1 + SG i) h
-        t1.x = h * (o[1].x - SG * o[1].y);
-        t1.y = h * (o[1].y + SG * o[1].x);
-        t3.x = h * (-o[3].x - SG * o[3].y);
-        t3.y = h * (-o[3].y + SG * o[3].x);
+        t1.x = mh(o[1].x - SG * o[1].y);
+        t1.y = mh(o[1].y + SG * o[1].x);
+        t3.x = mh(-o[3].x - SG * o[3].y);
+        t3.y = mh(-o[3].y + SG * o[3].x);
         const V t2 = mul_si<SG>(o[2]);
         x[0] = cadd(e[0], o[0]);
         x[4] = csub(e[0], o[0]);
@@ -3234,8 +3236,12 @@ template <int SG, typename R> struct RegDFT<8, SG, R> {
 // Compile-time layout of the FFT variant for n = 2^LN (16 <= n <= 512): chunks of CH = 2048 / n
 // elements, LDS slot of (step k, element el) = k (CH + 1) + el (rows padded by one element so that
 // one element read across consecutive rows, as the FID sums do, falls in distinct banks).
-// tw holds e^{-2 pi i j / n}, j < n / 2.
-template <int LN> struct CorrFft {
+// tw holds e^{-2 pi i j / n}, j < n / 2, and with COMP the rounding errors of those entries after
+// them.  COMP (padded complex64 transforms) adds them to every product: an FP32 constant's rounding
+// is the same for every element and pass and does not average out (1 / sqrt(2) is 2.4e-8 too
+// small), which took 3e-8 to 9e-8 off the size of FIDs of 35 steps where the direct sum has no
+// such bias (k_corr of 6 spins, 1154 crystallites, n = 100: 1.7 -> 1.95 ms).
+template <int LN, bool COMP = false> struct CorrFft {
     static constexpr int N = 1 << LN, CH = CORR_SPAN >> LN, LC = 11 - LN, ROW = CH + 1;
     static constexpr int NP = (LN + 2) / 3;         // passes per transform: radix 8 but the last
     static constexpr int LRL = LN - 3 * (NP - 1);   // log2 of the last pass's radix
@@ -3245,6 +3251,19 @@ template <int LN> struct CorrFft {
         if (idx & (N / 2)) { w.x = -w.x; w.y = -w.y; }
         if (SG > 0) w.y = -w.y;
         return w;
+    }
+    // x e^{SG 2 pi i idx / n}
+    template <int SG, typename CT> static __device__ __forceinline__ CT turn(CT x, const CT *tw, int idx) {
+        const CT w = twid<SG>(tw, idx);
+        if constexpr (COMP) {
+            const CT l = twid<SG>(tw + N / 2, idx);
+            CT p;
+            p.x = __builtin_elementwise_fma(x.x, w.x, __builtin_elementwise_fma(-x.y, w.y, x.x * l.x - x.y * l.y));
+            p.y = __builtin_elementwise_fma(x.x, w.y, __builtin_elementwise_fma(x.y, w.x, x.x * l.y + x.y * l.x));
+            return p;
+        } else {
+            return cmul(x, w);
+        }
     }
 };
 
@@ -3258,11 +3277,11 @@ template <int LN> struct CorrFft {
 // the opposite-sign DFT.  One work item = one butterfly of one element (2048 / RAD items).
 template <int RAD> struct Log2R { static constexpr int v = RAD == 8 ? 3 : RAD == 4 ? 2 : 1; };
 // AUTO: R~ = conj(Q~) (the autocorrelation case), only the Q transform is formed.
-template <int RAD, int LN, int LL, typename R, bool AUTO>
+template <int RAD, int LN, int LL, typename R, bool AUTO, bool COMP>
 __device__ __forceinline__ void corr_fwd_pass(typename CX<R>::T *sQ, typename CX<R>::T *sR,
                                               const typename CX<R>::T *tw) {
     typedef typename CX<R>::T CT;
-    typedef CorrFft<LN> F;
+    typedef CorrFft<LN, COMP> F;
     constexpr int LR = Log2R<RAD>::v, LS = LL - LR, TSH = LN - LL;
 #pragma unroll
     for (int it = 0; it < (CORR_SPAN >> LR) / 256; it++) {
@@ -3275,24 +3294,23 @@ __device__ __forceinline__ void corr_fwd_pass(typename CX<R>::T *sQ, typename CX
             q[m] = sQ[base + ((m << LS) * F::ROW)];
             if constexpr (!AUTO) r[m] = sR[base + ((m << LS) * F::ROW)];
         }
-        RegDFT<RAD, -1, R>::run(q);
-        if constexpr (!AUTO) RegDFT<RAD, +1, R>::run(r);
+        RegDFT<RAD, -1, R, COMP>::run(q);
+        if constexpr (!AUTO) RegDFT<RAD, +1, R, COMP>::run(r);
 #pragma unroll
         for (int k = 0; k < RAD; k++) {
             if (k) {
-                const CT w = F::template twid<-1>(tw, (j * k) << TSH);
-                q[k] = cmul(q[k], w);
-                if constexpr (!AUTO) r[k] = cmul(r[k], cconj(w));
+                q[k] = F::template turn<-1>(q[k], tw, (j * k) << TSH);
+                if constexpr (!AUTO) r[k] = F::template turn<+1>(r[k], tw, (j * k) << TSH);
             }
             sQ[base + ((k << LS) * F::ROW)] = q[k];
             if constexpr (!AUTO) sR[base + ((k << LS) * F::ROW)] = r[k];
         }
     }
 }
-template <int RAD, int LN, int LL, typename R>
+template <int RAD, int LN, int LL, typename R, bool COMP>
 __device__ __forceinline__ void corr_inv_pass(typename CX<R>::T *sQ, const typename CX<R>::T *tw) {
     typedef typename CX<R>::T CT;
-    typedef CorrFft<LN> F;
+    typedef CorrFft<LN, COMP> F;
     constexpr int LR = Log2R<RAD>::v, LS = LL - LR, TSH = LN - LL;
 #pragma unroll
     for (int it = 0; it < (CORR_SPAN >> LR) / 256; it++) {
@@ -3303,9 +3321,9 @@ __device__ __forceinline__ void corr_inv_pass(typename CX<R>::T *sQ, const typen
 #pragma unroll
         for (int k = 0; k < RAD; k++) {
             x[k] = sQ[base + ((k << LS) * F::ROW)];
-            if (k) x[k] = cmul(x[k], F::template twid<+1>(tw, (j * k) << TSH));
+            if (k) x[k] = F::template turn<+1>(x[k], tw, (j * k) << TSH);
         }
-        RegDFT<RAD, +1, R>::run(x);
+        RegDFT<RAD, +1, R, COMP>::run(x);
 #pragma unroll
         for (int m = 0; m < RAD; m++) sQ[base + ((m << LS) * F::ROW)] = x[m];
     }
@@ -3313,10 +3331,10 @@ __device__ __forceinline__ void corr_inv_pass(typename CX<R>::T *sQ, const typen
 // The last forward pass (sub-transforms of length RAD: no twiddles), the product scaled by 1/n
 // and the first inverse pass, on consecutive groups of RAD points, into sQ.  AUTO: the product
 // is |Q~|^2 / n (R~ = conj(Q~)).
-template <int LN, typename R, bool AUTO>
+template <int LN, typename R, bool AUTO, bool COMP>
 __device__ __forceinline__ void corr_mid_pass(typename CX<R>::T *sQ, const typename CX<R>::T *sR) {
     typedef typename CX<R>::T CT;
-    typedef CorrFft<LN> F;
+    typedef CorrFft<LN, COMP> F;
     constexpr int LR = F::LRL, RAD = 1 << LR;
     const R inv_n = (R)(1.0 / (double)F::N);
 #pragma unroll
@@ -3329,7 +3347,7 @@ __device__ __forceinline__ void corr_mid_pass(typename CX<R>::T *sQ, const typen
             q[m] = sQ[base + m * F::ROW];
             if constexpr (!AUTO) r[m] = sR[base + m * F::ROW];
         }
-        RegDFT<RAD, -1, R>::run(q);
+        RegDFT<RAD, -1, R, COMP>::run(q);
         if constexpr (AUTO) {
 #pragma unroll
             for (int m = 0; m < RAD; m++) {
@@ -3337,11 +3355,11 @@ __device__ __forceinline__ void corr_mid_pass(typename CX<R>::T *sQ, const typen
                 q[m].y = (R)0;
             }
         } else {
-            RegDFT<RAD, +1, R>::run(r);
+            RegDFT<RAD, +1, R, COMP>::run(r);
 #pragma unroll
             for (int m = 0; m < RAD; m++) q[m] = cscale(cmul(q[m], r[m]), inv_n);
         }
-        RegDFT<RAD, +1, R>::run(q);
+        RegDFT<RAD, +1, R, COMP>::run(q);
 #pragma unroll
         for (int m = 0; m < RAD; m++) sQ[base + m * F::ROW] = q[m];
     }
@@ -3368,13 +3386,14 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                                               int seg_base) {
     typedef typename CX<R>::T CT;
     constexpr bool FFT = LN > 0;
-    typedef CorrFft<FFT ? LN : 4> FF;
+    constexpr bool COMP = PAD && sizeof(R) == 4;
+    typedef CorrFft<FFT ? LN : 4, COMP> FF;
     constexpr int SPAN = FFT ? FF::N * FF::ROW : CORR_SPAN, NE = FFT ? FF::CH : 256;
     __shared__ CT sQ[SPAN];
     __shared__ __align__(16) CT sR[SPAN];
     __shared__ double sphi[NE];
     __shared__ cd sstep[NE];
-    __shared__ CT s_tw[FFT ? FF::N / 2 : 1];
+    __shared__ CT s_tw[FFT ? (COMP ? FF::N : FF::N / 2) : 1];
     const int n = FFT && !PAD ? FF::N : P.n, tid = threadIdx.x;
     const int CH = FFT ? FF::CH : corr_chunk(n);
     // LDS slot of (step k, element el).  Direct variant: rows of CH elements, the element index
@@ -3387,8 +3406,11 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
     };
     if constexpr (FFT) {
         // e^{-2 pi i j / n}, j < n/2
-        for (int j = tid; j < FF::N / 2; j += 256)
-            s_tw[j] = CX<R>::from(cexpi(-2.0 * 3.14159265358979323846 * (double)j / (double)FF::N));
+        for (int j = tid; j < FF::N / 2; j += 256) {
+            const cd w = cexpi(-2.0 * 3.14159265358979323846 * (double)j / (double)FF::N);
+            s_tw[j] = CX<R>::from(w);
+            if constexpr (COMP) s_tw[FF::N / 2 + j] = CX<R>::from(csub(w, to_cd(s_tw[j])));
+        }
         __syncthreads();
     }
     const int npg = (n + CORR_PPT - 1) / CORR_PPT;
@@ -3496,10 +3518,10 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                         if (PAD && j + (m << LS) >= n) x[m] = Arith<CT>::zero();
                         w = cmul(w, st);
                     }
-                    RegDFT<8, -1, R>::run(x);
+                    RegDFT<8, -1, R, COMP>::run(x);
 #pragma unroll
                     for (int k = 0; k < 8; k++) {
-                        if (k) x[k] = cmul(x[k], FF::template twid<-1>(s_tw, j * k));
+                        if (k) x[k] = FF::template turn<-1>(x[k], s_tw, j * k);
                         sQ[base + (k << LS) * FF::ROW] = x[k];
                     }
                     if constexpr (!AUTO) {
@@ -3520,23 +3542,23 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                             if (PAD && j + (m << LS) >= n) x[m] = Arith<CT>::zero();
                             w = cmul(w, sti);
                         }
-                        RegDFT<8, +1, R>::run(x);
+                        RegDFT<8, +1, R, COMP>::run(x);
 #pragma unroll
                         for (int k = 0; k < 8; k++) {
-                            if (k) x[k] = cmul(x[k], FF::template twid<+1>(s_tw, j * k));
+                            if (k) x[k] = FF::template turn<+1>(x[k], s_tw, j * k);
                             sR[base + (k << LS) * FF::ROW] = x[k];
                         }
                     }
                 }
                 __syncthreads();
                 if constexpr (FF::NP == 3) {
-                    corr_fwd_pass<8, LN, LN - 3, R, AUTO>(sQ, sR, s_tw);
+                    corr_fwd_pass<8, LN, LN - 3, R, AUTO, COMP>(sQ, sR, s_tw);
                     __syncthreads();
                 }
-                corr_mid_pass<LN, R, AUTO>(sQ, sR);
+                corr_mid_pass<LN, R, AUTO, COMP>(sQ, sR);
                 __syncthreads();
                 if constexpr (FF::NP == 3) {
-                    corr_inv_pass<8, LN, LN - 3, R>(sQ, s_tw);
+                    corr_inv_pass<8, LN, LN - 3, R, COMP>(sQ, s_tw);
                     __syncthreads();
                 }
                 // last inverse pass (radix 8, L = n) giving F_p in natural order; for the held FID
@@ -3547,9 +3569,9 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
 #pragma unroll
                     for (int k = 0; k < 8; k++) {
                         x[k] = sQ[base + (k << LS) * FF::ROW];
-                        if (k) x[k] = cmul(x[k], FF::template twid<+1>(s_tw, j * k));
+                        if (k) x[k] = FF::template turn<+1>(x[k], s_tw, j * k);
                     }
-                    RegDFT<8, +1, R>::run(x);
+                    RegDFT<8, +1, R, COMP>::run(x);
                     if (hold && !PAD) {
                         const double ph = sphi[el];
                         cd w = cexpi((double)j * ph);
