@@ -40,7 +40,7 @@ int blfid_dev_launch_exp(int prec, int M, const DevPlan *P, int Kb, int c0, cons
                          int ngrp, void *scratch, size_t slot, int nslots, void *bufU,
                          hipStream_t st);
 int blfid_dev_launch_dyson(int prec, int M, const DevPlan *P, int Kb, const int *grp, int ngrp,
-                           const void *bufU, void *bufA, hipStream_t st);
+                           int nbig, int bmax, const void *bufU, void *bufA, hipStream_t st);
 int blfid_dev_launch_expdyson(int M, const DevPlan *P, int Kb, int c0, const int *grp, int ngrp,
                               void *bufA, hipStream_t st);
 int blfid_dev_launch_expdyson_d(int M, const DevPlan *P, int Kb, int c0, const int *grp, int ngrp,
@@ -54,9 +54,9 @@ int blfid_dev_launch_eig(int prec, const DevPlan *P, int Kb, const int *grp, int
                          void *bufWr, double *outv, int cls, double2 *gscr, size_t gslot,
                          int nslots, int bmax, hipStream_t st);
 int blfid_dev_launch_bmul(int prec, int M, const DevPlan *P, int Kb, const int *grp, int ngrp,
-                          const void *bufA, const void *bufW, void *bufB, hipStream_t st);
+                          int nbig, const void *bufA, const void *bufW, void *bufB, hipStream_t st);
 int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, const int *pgrp, int ngrp,
-                        const void *bufB, void *scratch, size_t slot, int nslots, void *Qt,
+                        int nbig, const void *bufB, void *scratch, size_t slot, int nslots, void *Qt,
                         void *Rt, hipStream_t st);
 int blfid_dev_launch_bq1(int prec, const DevPlan *P, int Kb, const int *pgrp, int ngrp,
                          const void *bufA, const void *bufW, void *Qt, void *Rt, hipStream_t st);
@@ -553,6 +553,7 @@ static int eig_class(int b) {
     return 5;
 }
 
+static int pair_dim(const blfid_plan *pl, int p);
 static blfid_status build_tables(blfid_plan *pl) {
     const int S = pl->S, N = pl->N;
     pl->terms.clear();
@@ -756,6 +757,11 @@ static blfid_status build_tables(blfid_plan *pl) {
         else pl->big_blocks.push_back((int)b);
     }
     pl->Lsum = uo;
+    // largest first: the kernels of blocks beyond DEV_LDS_BLOCK take the front of a group
+    auto larger = [&](int a, int b) { return pl->blk_dim[a] > pl->blk_dim[b]; };
+    std::stable_sort(pl->big_blocks.begin(), pl->big_blocks.end(), larger);
+    if (!pl->big_blocks.empty())
+        std::stable_sort(pl->blk_groups[5].begin(), pl->blk_groups[5].end(), larger);
     // flip-flop (and rf flip) positions of the fused kernels' H planes
     pl->xd_off.assign(1, 0);
     pl->xd_list.clear();
@@ -1329,6 +1335,10 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
         int M = std::min(5, (std::max(bI, bJ) + 15) / 16);
         pl->pair_groups[M].push_back((int)p);
     }
+    if (pl->pair_groups.count(5))
+        std::stable_sort(pl->pair_groups[5].begin(), pl->pair_groups[5].end(), [&](int a, int b) {
+            return pair_dim(pl, a) > pair_dim(pl, b);
+        });
     {
         // B = A W is stored for the blocks whose pairs read it (class 1 pairs form it themselves)
         std::vector<char> used(nb, 0);
@@ -1491,6 +1501,16 @@ static size_t pair_e(const blfid_plan *pl, const std::vector<int> &g) {
     for (int p : g)
         e = std::max<size_t>(e, (size_t)pl->blk_dim[pl->pairs[p].I] * pl->blk_dim[pl->pairs[p].J]);
     return e;
+}
+// Blocks (pairs) of a group beyond DEV_LDS_BLOCK states; the groups hold them first
+static int big_count(const blfid_plan *pl, const std::vector<int> &g) {
+    return (int)std::count_if(g.begin(), g.end(), [&](int b) { return pl->blk_dim[b] > DEV_LDS_BLOCK; });
+}
+static int pair_dim(const blfid_plan *pl, int p) {
+    return std::max(pl->blk_dim[pl->pairs[p].I], pl->blk_dim[pl->pairs[p].J]);
+}
+static int big_pairs(const blfid_plan *pl, const std::vector<int> &g) {
+    return (int)std::count_if(g.begin(), g.end(), [&](int p) { return pair_dim(pl, p) > DEV_LDS_BLOCK; });
 }
 static double group_b3(const blfid_plan *pl, const std::vector<int> &g) {
     double s = 0;
@@ -1691,8 +1711,8 @@ static blfid_status enqueue_props64(blfid_plan *prof, blfid_plan *pp, const DevP
     }
     PhaseScope ps(prof, 1 * 8 + 5, kb * (double)(pp->n - 1) * group_b3(pp, big) * 8.0,
                   kb * (double)(pp->n + PP->akeep) * group_b2(pp, big) * 16.0, st);
-    LAUNCHCHK(blfid_dev_launch_dyson(0, 5, PP, kb, pp->d_bigb.p, (int)big.size(), pp->bufU,
-                                     pp->bufA, st));
+    LAUNCHCHK(blfid_dev_launch_dyson(0, 5, PP, kb, pp->d_bigb.p, (int)big.size(), (int)big.size(),
+                                     pp->bmax, pp->bufU, pp->bufA, st));
     return BLFID_OK;
 }
 
@@ -1823,7 +1843,7 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                 PhaseScope ps(pl, 1 * 8 + M, kb * (double)(pl->n - 1) * group_b3(pl, gv) * 8.0,
                               kb * 2.0 * pl->n * group_b2(pl, gv) * cs, st);
                 LAUNCHCHK(blfid_dev_launch_dyson(pr, M, P, kb, gq.second.first, (int)gv.size(),
-                                                 pl->bufU, pl->bufA, st));
+                                                 big_count(pl, gv), pl->bmax, pl->bufU, pl->bufA, st));
             }
             for (auto &kv : pl->eig_cls) {
                 PhaseScope ps(pl, 2 * 8 + kv.first + 1, 0.0,
@@ -1844,7 +1864,8 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                               kb * (2.0 * pl->n + 1.0) * group_b2(pl, kv.second) * cs, st);
                 LAUNCHCHK(blfid_dev_launch_bmul(pr, kv.first, P, kb,
                                                 (one ? pl->d_bmgrp : pl->d_bgrp)[kv.first].p,
-                                                (int)kv.second.size(), pl->bufA, Wst, pl->bufU, st));
+                                                (int)kv.second.size(), big_count(pl, kv.second),
+                                                pl->bufA, Wst, pl->bufU, st));
             }
             for (auto &kv : pl->pair_groups) {
                 double fl = pair_flops(pl, kv.second);
@@ -1866,8 +1887,9 @@ static blfid_status enqueue_range(blfid_plan *pl, const blfid_layout::Shape &sh,
                 int ns;
                 group_slots(bm2, sh.qr_slots, pair_e(pl, kv.second), kv.first, &slot, &ns);
                 LAUNCHCHK(blfid_dev_launch_qr(pr, kv.first, P, kb, pl->d_pgrp[kv.first].p,
-                                              (int)kv.second.size(), pl->bufU, pl->scrQ, slot,
-                                              ns, pl->bufQt, pl->bufRt, st));
+                                              (int)kv.second.size(), big_pairs(pl, kv.second),
+                                              pl->bufU, pl->scrQ, slot, ns, pl->bufQt, pl->bufRt,
+                                              st));
             }
             if (pl->Etot > 0) {
                 // Q once per element; R too unless it is formed from Q, or the reverse element's

@@ -448,12 +448,242 @@ template <int M, int NT, bool SPLIT> struct CGemm<M, NT, float, SPLIT> {
     }
 };
 
-// Real products of the propagator (both precisions on the VALU tile GEMM: measured faster here
-// than matrix cores, the propagator being bound by its staging and synchronisation).
+// ------------------------------------------------------------------ products by wave tiles
+// Products of blocks above 80 states on matrix cores: a wave takes up to TI x TJ tiles of 16 x 16
+// of the result in registers and reads both operands straight from global memory into the
+// matrix instruction's layout, the slice of four k after the one being multiplied, with no LDS
+// and no barrier.  A slice of 4 x 4 complex FP32 tiles is 64 products of 32 cycles against eight
+// operand reads, so the L1 / L2 path is far from its limit, and every wave runs on its own.  Edge
+// tiles clamp their row and column indexes (those results are not stored); k past the end is zero.
+// v_mfma_*_16x16x4: lane 16 g + r holds A(r, k = g), B(k = g, r); register v of the result is row
+// kq(v, g), column r.
+template <typename R> struct MT1;
+template <> struct MT1<double> {
+    typedef v4d V;
+    static __device__ __forceinline__ int kq(int v, int g) { return 4 * v + g; }
+    static __device__ __forceinline__ V mm(double a, double b, V c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+};
+template <> struct MT1<float> {
+    typedef v4f V;
+    static __device__ __forceinline__ int kq(int v, int g) { return 4 * g + v; }
+    static __device__ __forceinline__ V mm(float a, float b, V c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+};
+// tiles of 16 split evenly: `nb` of them in ceil(nb / T) parts of T or T - 1, first index of part t
+template <int T> __device__ __forceinline__ int wt_parts(int nb) { return (nb + T - 1) / T; }
+__device__ __forceinline__ int wt_first(int nb, int parts, int t) {
+    const int base = nb / parts, more = nb % parts;
+    return t * base + min(t, more);
+}
+// C(i0.., j0..) of C = op(A) B, op(A) m x kd, B kd x n, column-major; HA: op(A) = A^H
+template <typename R, int TI, int TJ, bool HA>
+__device__ __forceinline__ void wt_cmul(int m, int n, int kd, const typename CX<R>::T *__restrict__ A,
+                                        int lda, const typename CX<R>::T *B, int ldb,
+                                        typename CX<R>::T *C, int ldc, int i0, int j0) {
+    typedef typename CX<R>::T CT;
+    typedef typename MT1<R>::V V;
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    unsigned oa[TI], ob[TJ];
+#pragma unroll
+    for (int I = 0; I < TI; I++) {
+        const int row = min(i0 + 16 * I + r, m - 1);
+        oa[I] = HA ? row * lda : row;
+    }
+#pragma unroll
+    for (int J = 0; J < TJ; J++) ob[J] = min(j0 + 16 * J + r, n - 1) * ldb;
+    V cr[TI][TJ], ci[TI][TJ];
+#pragma unroll
+    for (int I = 0; I < TI; I++)
+#pragma unroll
+        for (int J = 0; J < TJ; J++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                cr[I][J][v] = (R)0;
+                ci[I][J][v] = (R)0;
+            }
+    CT a[2][TI], b[2][TJ];
+    auto load = [&](int k, CT (&x)[TI], CT (&y)[TJ]) {
+        const unsigned q = min(k + g, kd - 1), qa = HA ? q : q * lda;
+#pragma unroll
+        for (int I = 0; I < TI; I++) x[I] = A[oa[I] + qa];
+#pragma unroll
+        for (int J = 0; J < TJ; J++) y[J] = B[ob[J] + q];
+        __builtin_amdgcn_sched_barrier(0); // issued before the products that follow
+    };
+    auto mul = [&](const CT (&x)[TI], const CT (&y)[TJ]) {
+#pragma unroll
+        for (int I = 0; I < TI; I++) {
+            const R ar = x[I].x, ai = HA ? -x[I].y : x[I].y;
+#pragma unroll
+            for (int J = 0; J < TJ; J++) {
+                cr[I][J] = MT1<R>::mm(ar, y[J].x, cr[I][J]);
+                ci[I][J] = MT1<R>::mm(ar, y[J].y, ci[I][J]);
+            }
+#pragma unroll
+            for (int J = 0; J < TJ; J++) {
+                cr[I][J] = MT1<R>::mm(-ai, y[J].y, cr[I][J]);
+                ci[I][J] = MT1<R>::mm(ai, y[J].x, ci[I][J]);
+            }
+        }
+    };
+    auto last = [&](CT (&x)[TI], CT (&y)[TJ], int k) { // the slice that k ends in
+        if (k + g >= kd) {
+#pragma unroll
+            for (int I = 0; I < TI; I++) x[I] = Arith<CT>::zero();
+#pragma unroll
+            for (int J = 0; J < TJ; J++) y[J] = Arith<CT>::zero();
+        }
+        mul(x, y);
+    };
+    load(0, a[0], b[0]);
+    int k = 0;
+    for (; k + 8 <= kd; k += 8) {
+        load(k + 4, a[1], b[1]);
+        mul(a[0], b[0]);
+        load(k + 8, a[0], b[0]);
+        mul(a[1], b[1]);
+    }
+    if (k < kd) {
+        load(k + 4, a[1], b[1]);
+        last(a[0], b[0], k);
+        if (k + 4 < kd) last(a[1], b[1], k + 4);
+    }
+#pragma unroll
+    for (int J = 0; J < TJ; J++) {
+        const int col = j0 + 16 * J + r;
+#pragma unroll
+        for (int I = 0; I < TI; I++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = i0 + 16 * I + MT1<R>::kq(v, g);
+                if (row < m && col < n) C[row + (size_t)col * ldc] = CX<R>::mk(cr[I][J][v], ci[I][J][v]);
+            }
+    }
+}
+// C = A B of symmetric real b x b operands that commute (B is read by its rows)
+template <typename R, int TI, int TJ>
+__device__ __forceinline__ void wt_rmul(int b, const R *__restrict__ A, const R *__restrict__ B,
+                                        R *__restrict__ C, int i0, int j0) {
+    typedef typename MT1<R>::V V;
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    unsigned oa[TI], ob[TJ];
+#pragma unroll
+    for (int I = 0; I < TI; I++) oa[I] = min(i0 + 16 * I + r, b - 1);
+#pragma unroll
+    for (int J = 0; J < TJ; J++) ob[J] = min(j0 + 16 * J + r, b - 1);
+    V c[TI][TJ];
+#pragma unroll
+    for (int I = 0; I < TI; I++)
+#pragma unroll
+        for (int J = 0; J < TJ; J++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) c[I][J][v] = (R)0;
+    // eight k a turn, the next eight under way
+    R x[2][2][TI], y[2][2][TJ];
+    auto load = [&](int k, R (&p)[2][TI], R (&q)[2][TJ]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const unsigned o = min(k + 4 * h + g, b - 1) * b;
+#pragma unroll
+            for (int I = 0; I < TI; I++) p[h][I] = A[oa[I] + o];
+#pragma unroll
+            for (int J = 0; J < TJ; J++) q[h][J] = B[ob[J] + o];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mul = [&](const R (&p)[2][TI], const R (&q)[2][TJ]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int I = 0; I < TI; I++)
+#pragma unroll
+                for (int J = 0; J < TJ; J++) c[I][J] = MT1<R>::mm(p[h][I], q[h][J], c[I][J]);
+    };
+    auto last = [&](R (&p)[2][TI], R (&q)[2][TJ], int k) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (k + 4 * h + g >= b) {
+#pragma unroll
+                for (int I = 0; I < TI; I++) p[h][I] = (R)0;
+#pragma unroll
+                for (int J = 0; J < TJ; J++) q[h][J] = (R)0;
+            }
+        mul(p, q);
+    };
+    load(0, x[0], y[0]);
+    int k = 0;
+    for (; k + 16 <= b; k += 16) {
+        load(k + 8, x[1], y[1]);
+        mul(x[0], y[0]);
+        load(k + 16, x[0], y[0]);
+        mul(x[1], y[1]);
+    }
+    if (k < b) {
+        load(k + 8, x[1], y[1]);
+        last(x[0], y[0], k);
+        if (k + 8 < b) last(x[1], y[1], k + 8);
+    }
+#pragma unroll
+    for (int J = 0; J < TJ; J++) {
+        const int col = j0 + 16 * J + r;
+#pragma unroll
+        for (int I = 0; I < TI; I++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = i0 + 16 * I + MT1<R>::kq(v, g);
+                if (row < b && col < b) C[row + (size_t)col * b] = c[I][J][v];
+            }
+    }
+}
+// The workgroup's NW waves take the parts of C in turn; ends with a barrier.
+template <int NW, typename R, bool HA>
+__device__ __forceinline__ void wg_wt_cmul(int m, int n, int kd, const typename CX<R>::T *A, int lda,
+                                           const typename CX<R>::T *B, int ldb,
+                                           typename CX<R>::T *C, int ldc) {
+    constexpr int TI = 4, TJ = sizeof(R) == 4 ? 4 : 2;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nbm = (m + 15) >> 4, nbn = (n + 15) >> 4;
+    const int pm = wt_parts<TI>(nbm), pn = wt_parts<TJ>(nbn);
+    __syncthreads(); // operands the workgroup wrote before the call
+    for (int t = w; t < pm * pn; t += NW) {
+        const int ti = t % pm, tj = t / pm;
+        const int i0 = wt_first(nbm, pm, ti), ni = wt_first(nbm, pm, ti + 1) - i0;
+        const int j0 = wt_first(nbn, pn, tj), nj = wt_first(nbn, pn, tj + 1) - j0;
+        if (ni == TI && nj == TJ) wt_cmul<R, TI, TJ, HA>(m, n, kd, A, lda, B, ldb, C, ldc, 16 * i0, 16 * j0);
+        else if (ni == TI) wt_cmul<R, TI, TJ - 1, HA>(m, n, kd, A, lda, B, ldb, C, ldc, 16 * i0, 16 * j0);
+        else if (nj == TJ) wt_cmul<R, TI - 1, TJ, HA>(m, n, kd, A, lda, B, ldb, C, ldc, 16 * i0, 16 * j0);
+        else wt_cmul<R, TI - 1, TJ - 1, HA>(m, n, kd, A, lda, B, ldb, C, ldc, 16 * i0, 16 * j0);
+    }
+    __syncthreads();
+}
+template <int NW, typename R>
+__device__ __forceinline__ void wg_wt_rmul(int b, const R *A, const R *B, R *C) {
+    constexpr int T = 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = (b + 15) >> 4, pp = wt_parts<T>(nb);
+    __syncthreads();
+    for (int t = w; t < pp * pp; t += NW) {
+        const int i0 = wt_first(nb, pp, t % pp), ni = wt_first(nb, pp, t % pp + 1) - i0;
+        const int j0 = wt_first(nb, pp, t / pp), nj = wt_first(nb, pp, t / pp + 1) - j0;
+        if (ni == T && nj == T) wt_rmul<R, T, T>(b, A, B, C, 16 * i0, 16 * j0);
+        else if (ni == T) wt_rmul<R, T, T - 1>(b, A, B, C, 16 * i0, 16 * j0);
+        else if (nj == T) wt_rmul<R, T - 1, T>(b, A, B, C, 16 * i0, 16 * j0);
+        else wt_rmul<R, T - 1, T - 1>(b, A, B, C, 16 * i0, 16 * j0);
+    }
+    __syncthreads();
+}
+
+// Real products of the propagator: wave tiles above 64 states (64 crystallites x 64 steps, 10 spins
+// complex64 78 -> 42 ms, 9 spins FP64 22 -> 13 ms); below, the VALU tile GEMM measured faster than
+// staged matrix-core tiles (bound by staging and synchronisation).
 template <int M, int NT, typename R> struct ExpGemm {
     static constexpr int SMEM = GemmLds<M, R>::ELEMS;
     __device__ __forceinline__ static void run(int b, const R *A, const R *B, R *C, R *smem) {
-        wg_gemm<M, NT, R>(b, b, b, A, b, false, B, b, false, C, b, (R)0, smem);
+        if constexpr (M == 5) wg_wt_rmul<NT / 64, R>(b, A, B, C);
+        else wg_gemm<M, NT, R>(b, b, b, A, b, false, B, b, false, C, b, (R)0, smem);
     }
 };
 
@@ -636,7 +866,7 @@ template <> struct ExpTol<float> { static constexpr double tol = 2e-8, rmax = 2.
 // workgroups per CU: 168 registers instead of 234 with 17 spilled, still 16% faster than two
 // (k_dyson 14%, no spills; k_qr 21%, 6 spilled).
 template <int M, typename R>
-__global__ void __launch_bounds__(NThr<M>::v, (M == 1 && sizeof(R) == 4) ? 4 : (M == 4 && sizeof(R) == 8) ? 3 : 1) k_exp(DevPlan P, int Kb, int c0,
+__global__ void __launch_bounds__(NThr<M>::v, (M == 1 && sizeof(R) == 4) ? 4 : M == 5 ? 2 : 1) k_exp(DevPlan P, int Kb, int c0,
                                                     const int *__restrict__ grp, int ngrp,
                                                     R *__restrict__ scratch, size_t slot,
                                                     typename CX<R>::T *__restrict__ bufU) {
@@ -919,12 +1149,11 @@ __global__ void __launch_bounds__(NThr<M>::v, (M == 3 && sizeof(R) == 4) ? 3 : (
         const size_t abase = (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
         const CT *U0 = bufU + base;
         CT *A0 = bufA + abase;
-        // the chain holds one 16 M x 16 M tile: blocks above 80 states (M = 5) take the tiled path
-        if (CHAIN && (M < 5 || b <= 16 * M)) {
+        if (CHAIN) {
             if constexpr (CHAIN)
                 chain_mfma<M, NT, true>(b, P.n, U0, P.Lsum, nullptr, A0, P.Lsum, P.akeep,
                                         (float *)smem);
-        } else if constexpr (!CHAIN || M == 5) {
+        } else if constexpr (!CHAIN) {
             for (int e = threadIdx.x; e < b * b; e += NT) A0[e] = U0[e];
             __syncthreads();
             for (int k = 1; k < P.n; k++) {
@@ -933,6 +1162,47 @@ __global__ void __launch_bounds__(NThr<M>::v, (M == 3 && sizeof(R) == 4) ? 3 : (
                 CT *Ak = bufA + abase + (size_t)(k % P.akeep) * P.Lsum;
                 CGemm<M, NT, R, SPLIT>::run(b, b, b, Uk, b, false, Ap, b, Ak, b, smem);
             }
+        }
+    }
+}
+
+// Blocks above 80 states: the columns of the running product are independent, so a workgroup takes
+// a panel of 32 of them through the whole chain, its four waves the rows in up to four tiles of 16
+// each (wave tiles), A_{k-1} read back from global memory.  grp holds the blocks largest first;
+// consecutive slots of one XCD (workgroup index modulo 8) take the panels of one chain, which read
+// the same U_k.  One workgroup per chain left most of the chip idle with a few crystallites and
+// held every chain to one CU (64 crystallites x 64 steps: 10 spins complex64 116 -> 17 ms, 9 spins
+// FP64 15.7 -> 3.8 ms).
+#define DYB_TJ 2
+template <typename R>
+__global__ void __launch_bounds__(256, 2) k_dyson_big(DevPlan P, int Kb, const int *__restrict__ grp, int ngrp, int npan,
+                                                   const typename CX<R>::T *__restrict__ bufU,
+                                                   typename CX<R>::T *bufA) {
+    typedef typename CX<R>::T CT;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long nchain = (long)Kb * ngrp, ntask = (nchain + 7) / 8 * 8 * npan;
+    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const long slot = task / 8, ch = slot / npan * 8 + task % 8;
+        if (ch >= nchain) continue;
+        const int g = (int)(ch / Kb), c = (int)(ch % Kb);
+        const int blk = __builtin_amdgcn_readfirstlane(grp[g]);
+        const int b = __builtin_amdgcn_readfirstlane(P.blk_dim[blk]);
+        const int j0 = 16 * DYB_TJ * (int)(slot % npan);
+        if (j0 >= b) continue;
+        const int nb = (b + 15) >> 4, pp = min(4, nb), nj = min(16 * DYB_TJ, b - j0);
+        const int i0 = wt_first(nb, pp, w), ni = w < pp ? wt_first(nb, pp, w + 1) - i0 : 0;
+        const CT *U0 = bufU + (size_t)c * P.n * P.Lsum + P.blk_uoff[blk];
+        CT *A0 = bufA + (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
+        for (int e = threadIdx.x; e < b * nj; e += 256) A0[(size_t)j0 * b + e] = U0[(size_t)j0 * b + e];
+        __syncthreads();
+        for (int k = 1; k < P.n; k++) {
+            const CT *Uk = U0 + (size_t)k * P.Lsum;
+            const CT *Ap = A0 + (size_t)((k - 1) % P.akeep) * P.Lsum + (size_t)j0 * b;
+            CT *Ak = A0 + (size_t)(k % P.akeep) * P.Lsum + (size_t)j0 * b;
+            if (ni > 3) wt_cmul<R, 4, DYB_TJ, false>(b, nj, b, Uk, b, Ap, b, Ak, b, 16 * i0, 0);
+            else if (ni == 3) wt_cmul<R, 3, DYB_TJ, false>(b, nj, b, Uk, b, Ap, b, Ak, b, 16 * i0, 0);
+            else if (ni > 0) wt_cmul<R, 2, DYB_TJ, false>(b, nj, b, Uk, b, Ap, b, Ak, b, 16 * i0, 0);
+            __syncthreads();
         }
     }
 }
@@ -2652,22 +2922,14 @@ __global__ void __launch_bounds__((BmThreads<M, R, SPLIT>::v), (BmThreads<M, R, 
     constexpr int CHB = 4 * 16 * M * (16 * M + LDS_PAD) * 4, GB = CGemm<M, NT, R, SPLIT>::BYTES;
     __shared__ __align__(16) char smem[CHAIN && CHB > GB ? CHB : GB];
     if constexpr (CHAIN) {
-        // blocks above 80 states (M = 5) exceed the chain's tile: one task per step for them
         const long ntask = (long)Kb * ngrp;
         for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
             const int g = (int)(task % ngrp), c = (int)(task / ngrp);
             const int blk = grp[g], b = P.blk_dim[blk];
             const size_t base = (size_t)c * P.n * P.Lsum + P.blk_uoff[blk];
             const CT *W = bufW + (size_t)c * P.Lsum + P.blk_uoff[blk];
-            if (M < 5 || b <= 16 * M) {
-                chain_mfma<M, NT, false>(b, P.n, bufA + base, P.Lsum, W, bufB + base, P.Lsum,
-                                         P.n, (float *)smem);
-            } else if constexpr (M == 5) {
-                for (int k = 0; k < P.n; k++)
-                    CGemm<M, NT, R, SPLIT>::run(b, b, b, bufA + base + (size_t)k * P.Lsum, b,
-                                                false, W, b, bufB + base + (size_t)k * P.Lsum, b,
-                                                smem);
-            }
+            chain_mfma<M, NT, false>(b, P.n, bufA + base, P.Lsum, W, bufB + base, P.Lsum, P.n,
+                                     (float *)smem);
         }
     } else {
         const long ntask = (long)Kb * P.n * ngrp;
@@ -2680,6 +2942,60 @@ __global__ void __launch_bounds__((BmThreads<M, R, SPLIT>::v), (BmThreads<M, R, 
             const CT *W = bufW + (size_t)c * P.Lsum + P.blk_uoff[blk];
             CGemm<M, NT, R, SPLIT>::run(b, b, b, bufA + off, b, false, W, b, bufB + off, b, smem);
         }
+    }
+}
+
+// Blocks above 80 states: one task per (crystallite, step, block), wave tiles (64 crystallites x
+// 64 steps: 10 spins complex64, one workgroup per chain of steps, 86 -> 14 ms; 9 spins FP64, on the
+// vector ALUs, 9.7 -> 4.5 ms).
+template <typename R>
+__global__ void __launch_bounds__(256, 2) k_bmul_big(DevPlan P, int Kb, const int *__restrict__ grp, int ngrp,
+                                                  const typename CX<R>::T *__restrict__ bufA,
+                                                  const typename CX<R>::T *__restrict__ bufW,
+                                                  typename CX<R>::T *__restrict__ bufB) {
+    typedef typename CX<R>::T CT;
+    const long ntask = (long)Kb * P.n * ngrp;
+    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int g = (int)(task % ngrp);
+        const long ck = task / ngrp;
+        const int c = (int)(ck / P.n);
+        const int blk = __builtin_amdgcn_readfirstlane(grp[g]);
+        const int b = __builtin_amdgcn_readfirstlane(P.blk_dim[blk]);
+        const size_t off = (size_t)ck * P.Lsum + P.blk_uoff[blk];
+        wg_wt_cmul<4, R, false>(b, b, b, bufA + off, b, bufW + (size_t)c * P.Lsum + P.blk_uoff[blk], b,
+                                bufB + off, b);
+    }
+}
+
+// T[a + s rows] = sum_z val[z] B[col[z] + s ldb]: a thread takes a row's entries for SPR_U columns
+// at a time, so that a row is read once for them and their gathers are under way together (one
+// element at a time, each gather waited for the one before: k_qr_big of 10 spins 30.2 -> 23.6 ms, k_qr of
+// 65-80-state blocks in FP64 43 -> 35 ms over 1154 8-spin clusters).
+#define SPR_U 4
+template <int NT, typename R, typename V>
+__device__ __forceinline__ void sparse_rows_run(const int *rp, const int *col, const V *val, int rows,
+                                                int ncols, const typename CX<R>::T *B, int ldb,
+                                                typename CX<R>::T *T) {
+    typedef typename CX<R>::T CT;
+    const int groups = (ncols + SPR_U - 1) / SPR_U;
+    for (int x = threadIdx.x; x < rows * groups; x += NT) {
+        const int a = x % rows, s0 = x / rows * SPR_U;
+        int o[SPR_U];
+        CT acc[SPR_U];
+#pragma unroll
+        for (int u = 0; u < SPR_U; u++) {
+            o[u] = min(s0 + u, ncols - 1) * ldb;
+            acc[u] = Arith<CT>::zero();
+        }
+        for (int z = rp[a]; z < rp[a + 1]; z++) {
+            const CT v = CX<R>::from(to_cd(val[z]));
+            const int q = col[z];
+#pragma unroll
+            for (int u = 0; u < SPR_U; u++) cfma(acc[u], v, B[q + o[u]]);
+        }
+#pragma unroll
+        for (int u = 0; u < SPR_U; u++)
+            if (s0 + u < ncols) T[a + (size_t)(s0 + u) * rows] = acc[u];
     }
 }
 
@@ -2717,30 +3033,10 @@ __device__ __forceinline__ void sparse_rows_times(const int *__restrict__ rp,
         if (bl)
             for (int i = tid; i < (int)nb; i += NT) s_b[i] = B[i];
         __syncthreads();
-        if (bl) {
-            for (int e = tid; e < rows * ncols; e += NT) {
-                const int a = e % rows, s = e / rows;
-                CT acc = Arith<CT>::zero();
-                for (int z = s_rp[a]; z < s_rp[a + 1]; z++) cfma(acc, s_v[z], s_b[s_c[z] + s * ldb]);
-                T[e] = acc;
-            }
-        } else {
-            for (int e = tid; e < rows * ncols; e += NT) {
-                const int a = e % rows, s = e / rows;
-                CT acc = Arith<CT>::zero();
-                for (int z = s_rp[a]; z < s_rp[a + 1]; z++)
-                    cfma(acc, s_v[z], B[s_c[z] + (size_t)s * ldb]);
-                T[e] = acc;
-            }
-        }
+        if (bl) sparse_rows_run<NT, R>(s_rp, s_c, s_v, rows, ncols, s_b, ldb, T);
+        else sparse_rows_run<NT, R>(s_rp, s_c, s_v, rows, ncols, B, ldb, T);
     } else {
-        for (int e = tid; e < rows * ncols; e += NT) {
-            const int a = e % rows, s = e / rows;
-            CT acc = Arith<CT>::zero();
-            for (int z = rp[a]; z < rp[a + 1]; z++)
-                cfma(acc, CX<R>::from(val[z]), B[col[z] + (size_t)s * ldb]);
-            T[e] = acc;
-        }
+        sparse_rows_run<NT, R>(rp, col, val, rows, ncols, B, ldb, T);
     }
     __syncthreads();
 }
@@ -2939,6 +3235,45 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
     }
 }
 
+// Pairs with a block above 80 states: as the per-step form of k_qr, the products by wave tiles.
+// 64 crystallites x 64 steps: 10 spins complex64 38 -> 23.6 ms, 9 spins FP64 11.4 -> 5.2 ms.
+template <typename R>
+__global__ void __launch_bounds__(256, 2) k_qr_big(DevPlan P, int Kb, const int *__restrict__ pgrp, int ngrp,
+                                                const typename CX<R>::T *__restrict__ bufB,
+                                                typename CX<R>::T *scratch, size_t slot,
+                                                typename CX<R>::T *Qt, typename CX<R>::T *Rt) {
+    typedef typename CX<R>::T CT;
+    constexpr int CSR = 28 * 1024; // rows of an operator pair of 256 states and 5 values a row
+    __shared__ __align__(16) char smem[CSR];
+    CT *T1 = scratch + slot * 2 * blockIdx.x;
+    CT *G = T1 + slot;
+    const long ntask = (long)Kb * P.n * ngrp;
+    for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const long ck = task / ngrp;
+        const int c = (int)(ck / P.n);
+        const int pr = __builtin_amdgcn_readfirstlane(pgrp[(int)(task % ngrp)]);
+        const int I = __builtin_amdgcn_readfirstlane(P.pair_I[pr]), J = __builtin_amdgcn_readfirstlane(P.pair_J[pr]);
+        const int bI = __builtin_amdgcn_readfirstlane(P.blk_dim[I]), bJ = __builtin_amdgcn_readfirstlane(P.blk_dim[J]);
+        const CT *BI = bufB + (size_t)ck * P.Lsum + P.blk_uoff[I];
+        const CT *BJ = bufB + (size_t)ck * P.Lsum + P.blk_uoff[J];
+        const size_t eo = (size_t)ck * P.Estr + P.pair_eoff[pr];
+        sparse_rows_times<256, R>(P.d_rowptr + P.pair_doff[pr], P.d_col, (const cd *)P.d_val, bI, bJ,
+                                  BJ, bJ, T1, smem, CSR);
+        wg_wt_cmul<4, R, true>(bI, bJ, bI, BI, bI, T1, bI, Qt + eo, bI);
+        if (P.rt_from_q) continue;
+        if (P.rho_c) { // the prepared rho_JI^H of this crystallite
+            const CT *X = (const CT *)P.rho_c + (size_t)c * P.Etot + P.pair_eoff[pr];
+            wg_wt_cmul<4, R, true>(bJ, bI, bI, X, bI, BI, bI, T1, bJ);
+        } else {
+            sparse_rows_times<256, R>(P.r_rowptr + P.pair_roff[pr], P.r_col, (const cd *)P.r_val, bJ,
+                                      bI, BI, bI, T1, smem, CSR);
+        }
+        wg_wt_cmul<4, R, true>(bJ, bI, bJ, BJ, bJ, T1, bJ, G, bJ);
+        for (int e = threadIdx.x; e < bI * bJ; e += 256) Rt[eo + e] = G[e / bI + (size_t)(e % bI) * bJ];
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------------------------ k_bq1
 // B = A W and the Q (R) products of block pairs of at most 16 states in one pass, for both
 // precisions: a wave takes a run of steps of one (crystallite, pair) with everything in registers,
@@ -2951,21 +3286,6 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
 // staged every operand in LDS and gathered T1 there (proton pair x 1154 x 64 steps, FP64: 209 ->
 // 54 us; 5 spins, general rho: 2270 -> 720 us; the class-1 pairs of 6 spins, complex64: 1.15 + 0.08 ->
 // 0.58 ms).
-template <typename R> struct MT1;
-template <> struct MT1<double> {
-    typedef v4d V;
-    static __device__ __forceinline__ int kq(int v, int g) { return 4 * v + g; }
-    static __device__ __forceinline__ V mm(double a, double b, V c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-};
-template <> struct MT1<float> {
-    typedef v4f V;
-    static __device__ __forceinline__ int kq(int v, int g) { return 4 * g + v; }
-    static __device__ __forceinline__ V mm(float a, float b, V c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-};
 // one 16 x 16 complex operand or result: slice / register v of re and im
 template <typename R> struct CT1 {
     typename MT1<R>::V r, i;
@@ -4368,10 +4688,6 @@ static void launch_dyson(int M, const DevPlan *P, int Kb, const int *grp, int ng
     typedef typename CX<R>::T CT;
     const CT *U = (const CT *)bufU;
     CT *A = (CT *)bufA;
-    if constexpr (std::is_same<R, double>::value) {
-        k_dyson<5, R, false><<<grid, 256, 0, st>>>(*P, Kb, grp, ngrp, U, A);
-        return;
-    } else
     switch (M) {
     case 1: LAUNCH_SPLIT(k_dyson, 1, R, grid, 64, st, *P, Kb, grp, ngrp, U, A); break;
     case 2: LAUNCH_SPLIT(k_dyson, 2, R, grid, 256, st, *P, Kb, grp, ngrp, U, A); break;
@@ -4381,14 +4697,25 @@ static void launch_dyson(int M, const DevPlan *P, int Kb, const int *grp, int ng
     }
 }
 
+// The first nbig blocks of grp have more than DEV_LDS_BLOCK states (at most bmax): wave tiles, but
+// in the BF16x3 form.  FP64 chains of smaller blocks are k_expdyson_d's.
 extern "C" int blfid_dev_launch_dyson(int prec, int M, const DevPlan *P, int Kb, const int *grp,
-                                      int ngrp, const void *bufU, void *bufA, hipStream_t st) {
-    long ntask = (long)Kb * ngrp;
+                                      int ngrp, int nbig, int bmax, const void *bufU, void *bufA,
+                                      hipStream_t st) {
     const long cap = tuned_cap(P, 1, M);
-    int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid <= 0) return 0;
-    if (prec) launch_dyson<float>(M, P, Kb, grp, ngrp, grid, bufU, bufA, st);
-    else launch_dyson<double>(M, P, Kb, grp, ngrp, grid, bufU, bufA, st);
+    if (Kb <= 0 || ngrp <= 0) return 0;
+    if (!P->bf16x3 && nbig > 0) {
+        const int npan = (bmax + 16 * DYB_TJ - 1) / (16 * DYB_TJ);
+        const long ntask = ((long)Kb * nbig + 7) / 8 * 8 * npan;
+        const int grid = (int)(ntask < 8 * cap ? ntask : 8 * cap);
+        if (prec) k_dyson_big<float><<<grid, 256, 0, st>>>(*P, Kb, grp, nbig, npan, (const cf *)bufU, (cf *)bufA);
+        else k_dyson_big<double><<<grid, 256, 0, st>>>(*P, Kb, grp, nbig, npan, (const cd *)bufU, (cd *)bufA);
+        grp += nbig;
+        ngrp -= nbig;
+    }
+    const long ntask = (long)Kb * ngrp;
+    const int grid = (int)(ntask < cap ? ntask : cap);
+    if (grid > 0 && prec) launch_dyson<float>(M, P, Kb, grp, ngrp, grid, bufU, bufA, st);
     return (int)hipGetLastError();
 }
 
@@ -4465,14 +4792,24 @@ static void launch_bmul(int M, const DevPlan *P, int Kb, const int *grp, int ngr
 
 // bufW: W in the plan's storage precision
 extern "C" int blfid_dev_launch_bmul(int prec, int M, const DevPlan *P, int Kb, const int *grp,
-                                     int ngrp, const void *bufA, const void *bufW, void *bufB,
-                                     hipStream_t st) {
-    long ntask = (long)Kb * P->n * ngrp;
+                                     int ngrp, int nbig, const void *bufA, const void *bufW,
+                                     void *bufB, hipStream_t st) {
     const long cap = tuned_cap(P, 3, M);
-    int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid <= 0) return 0;
-    if (prec) launch_bmul<float>(M, P, Kb, grp, ngrp, grid, bufA, bufW, bufB, st);
-    else launch_bmul<double>(M, P, Kb, grp, ngrp, grid, bufA, bufW, bufB, st);
+    if (Kb <= 0 || ngrp <= 0) return 0;
+    if (!P->bf16x3 && nbig > 0) {
+        const long ntask = (long)Kb * P->n * nbig;
+        const int grid = (int)(ntask < cap ? ntask : cap);
+        if (prec) k_bmul_big<float><<<grid, 256, 0, st>>>(*P, Kb, grp, nbig, (const cf *)bufA, (const cf *)bufW, (cf *)bufB);
+        else k_bmul_big<double><<<grid, 256, 0, st>>>(*P, Kb, grp, nbig, (const cd *)bufA, (const cd *)bufW, (cd *)bufB);
+        grp += nbig;
+        ngrp -= nbig;
+    }
+    const long ntask = (long)Kb * P->n * ngrp;
+    const int grid = (int)(ntask < cap ? ntask : cap);
+    if (grid > 0) {
+        if (prec) launch_bmul<float>(M, P, Kb, grp, ngrp, grid, bufA, bufW, bufB, st);
+        else launch_bmul<double>(M, P, Kb, grp, ngrp, grid, bufA, bufW, bufB, st);
+    }
     return (int)hipGetLastError();
 }
 
@@ -4506,14 +4843,24 @@ static void launch_qr(int M, const DevPlan *P, int Kb, const int *pgrp, int ngrp
 }
 
 extern "C" int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, const int *pgrp,
-                                   int ngrp, const void *bufB, void *scratch, size_t slot,
+                                   int ngrp, int nbig, const void *bufB, void *scratch, size_t slot,
                                    int nslots, void *Qt, void *Rt, hipStream_t st) {
-    long ntask = (long)Kb * P->n * ngrp;
     const long cap = P->tn_cap[4] > 0 ? std::min<long>(tuned_cap(P, 4, M), nslots) : nslots;
-    int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid <= 0) return 0;
-    if (prec) launch_qr<float>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
-    else launch_qr<double>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
+    if (Kb <= 0 || ngrp <= 0) return 0;
+    if (!P->bf16x3 && nbig > 0) {
+        const long ntask = (long)Kb * P->n * nbig;
+        const int grid = (int)(ntask < cap ? ntask : cap);
+        if (prec) k_qr_big<float><<<grid, 256, 0, st>>>(*P, Kb, pgrp, nbig, (const cf *)bufB, (cf *)scratch, slot, (cf *)Qt, (cf *)Rt);
+        else k_qr_big<double><<<grid, 256, 0, st>>>(*P, Kb, pgrp, nbig, (const cd *)bufB, (cd *)scratch, slot, (cd *)Qt, (cd *)Rt);
+        pgrp += nbig;
+        ngrp -= nbig;
+    }
+    const long ntask = (long)Kb * P->n * ngrp;
+    const int grid = (int)(ntask < cap ? ntask : cap);
+    if (grid > 0) {
+        if (prec) launch_qr<float>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
+        else launch_qr<double>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
+    }
     return (int)hipGetLastError();
 }
 
