@@ -639,11 +639,10 @@ __device__ __forceinline__ void wt_rmul(int b, const R *__restrict__ A, const R 
     }
 }
 // The workgroup's NW waves take the parts of C in turn; ends with a barrier.
-template <int NW, typename R, bool HA>
+template <int NW, typename R, bool HA, int TI = 4, int TJ = (sizeof(R) == 4 ? 4 : 2)>
 __device__ __forceinline__ void wg_wt_cmul(int m, int n, int kd, const typename CX<R>::T *A, int lda,
                                            const typename CX<R>::T *B, int ldb,
                                            typename CX<R>::T *C, int ldc) {
-    constexpr int TI = 4, TJ = sizeof(R) == 4 ? 4 : 2;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nbm = (m + 15) >> 4, nbn = (n + 15) >> 4;
     const int pm = wt_parts<TI>(nbm), pn = wt_parts<TJ>(nbn);
@@ -2902,19 +2901,14 @@ __global__ void __launch_bounds__(512) k_eigb_tail(DevPlan P, int t0, int nt, co
 
 // ------------------------------------------------------------------------------ k_bmul
 // B_k = A_k W for every (crystallite, step, block) of a group; writes into bufB.
-// The complex64 chain of 65-80-state blocks runs eight waves (two per SIMD; its LDS allows one
-// workgroup per CU): at four waves it needed 432 registers and ran one wave per SIMD, and eight
-// waves took 18% off its time on 8-spin clusters (class 4 measured the same either way).
-template <int M, typename R, bool SPLIT> struct BmThreads {
-    static constexpr int v = (M == 5 && std::is_same<R, float>::value && !SPLIT) ? 512 : NThr<M>::v;
-};
+// (Wave tiles, k_bmul_wt, take the FP64 blocks above 32 states and the complex64 ones above 64.)
 template <int M, typename R, bool SPLIT = false>
-__global__ void __launch_bounds__((BmThreads<M, R, SPLIT>::v), (BmThreads<M, R, SPLIT>::v == 512) ? 1 : (M == 3 && sizeof(R) == 4) ? 3 : (M == 4 && sizeof(R) == 4) ? 2 : 1) k_bmul(DevPlan P, int Kb, const int *__restrict__ grp,
+__global__ void __launch_bounds__(NThr<M>::v, (M == 3 && sizeof(R) == 4) ? 3 : (M == 4 && sizeof(R) == 4) ? 2 : 1) k_bmul(DevPlan P, int Kb, const int *__restrict__ grp,
                                                      int ngrp,
                                                      const typename CX<R>::T *__restrict__ bufA,
                                                      const typename CX<R>::T *__restrict__ bufW,
                                                      typename CX<R>::T *__restrict__ bufB) {
-    constexpr int NT = BmThreads<M, R, SPLIT>::v;
+    constexpr int NT = NThr<M>::v;
     typedef typename CX<R>::T CT;
     // complex64: one task per (crystallite, block) walks all n steps with W resident in LDS;
     // complex128 (and the BF16x3 form): one task per (crystallite, step, block)
@@ -2945,11 +2939,11 @@ __global__ void __launch_bounds__((BmThreads<M, R, SPLIT>::v), (BmThreads<M, R, 
     }
 }
 
-// Blocks above 80 states: one task per (crystallite, step, block), wave tiles (64 crystallites x
+// B_k by wave tiles, one task per (crystallite, step, block) (blocks above 80 states, 64 crystallites x
 // 64 steps: 10 spins complex64, one workgroup per chain of steps, 86 -> 14 ms; 9 spins FP64, on the
 // vector ALUs, 9.7 -> 4.5 ms).
-template <typename R>
-__global__ void __launch_bounds__(256, 2) k_bmul_big(DevPlan P, int Kb, const int *__restrict__ grp, int ngrp,
+template <typename R, int TI, int TJ>
+__global__ void __launch_bounds__(256, TI == 4 ? 2 : sizeof(R) == 4 ? 5 : 4) k_bmul_wt(DevPlan P, int Kb, const int *__restrict__ grp, int ngrp,
                                                   const typename CX<R>::T *__restrict__ bufA,
                                                   const typename CX<R>::T *__restrict__ bufW,
                                                   typename CX<R>::T *__restrict__ bufB) {
@@ -2962,28 +2956,28 @@ __global__ void __launch_bounds__(256, 2) k_bmul_big(DevPlan P, int Kb, const in
         const int blk = __builtin_amdgcn_readfirstlane(grp[g]);
         const int b = __builtin_amdgcn_readfirstlane(P.blk_dim[blk]);
         const size_t off = (size_t)ck * P.Lsum + P.blk_uoff[blk];
-        wg_wt_cmul<4, R, false>(b, b, b, bufA + off, b, bufW + (size_t)c * P.Lsum + P.blk_uoff[blk], b,
+        wg_wt_cmul<4, R, false, TI, TJ>(b, b, b, bufA + off, b, bufW + (size_t)c * P.Lsum + P.blk_uoff[blk], b,
                                 bufB + off, b);
     }
 }
 
 // T[a + s rows] = sum_z val[z] B[col[z] + s ldb]: a thread takes a row's entries for SPR_U columns
 // at a time, so that a row is read once for them and their gathers are under way together (one
-// element at a time, each gather waited for the one before: k_qr_big of 10 spins 30.2 -> 23.6 ms, k_qr of
+// element at a time, each gather waited for the one before: k_qr_wt of 10 spins 30.2 -> 23.6 ms, k_qr of
 // 65-80-state blocks in FP64 43 -> 35 ms over 1154 8-spin clusters).
 #define SPR_U 4
-template <int NT, typename R, typename V>
+template <int NT, typename R, int U, typename V>
 __device__ __forceinline__ void sparse_rows_run(const int *rp, const int *col, const V *val, int rows,
                                                 int ncols, const typename CX<R>::T *B, int ldb,
                                                 typename CX<R>::T *T) {
     typedef typename CX<R>::T CT;
-    const int groups = (ncols + SPR_U - 1) / SPR_U;
+    const int groups = (ncols + U - 1) / U;
     for (int x = threadIdx.x; x < rows * groups; x += NT) {
-        const int a = x % rows, s0 = x / rows * SPR_U;
-        int o[SPR_U];
-        CT acc[SPR_U];
+        const int a = x % rows, s0 = x / rows * U;
+        int o[U];
+        CT acc[U];
 #pragma unroll
-        for (int u = 0; u < SPR_U; u++) {
+        for (int u = 0; u < U; u++) {
             o[u] = min(s0 + u, ncols - 1) * ldb;
             acc[u] = Arith<CT>::zero();
         }
@@ -2991,10 +2985,10 @@ __device__ __forceinline__ void sparse_rows_run(const int *rp, const int *col, c
             const CT v = CX<R>::from(to_cd(val[z]));
             const int q = col[z];
 #pragma unroll
-            for (int u = 0; u < SPR_U; u++) cfma(acc[u], v, B[q + o[u]]);
+            for (int u = 0; u < U; u++) cfma(acc[u], v, B[q + o[u]]);
         }
 #pragma unroll
-        for (int u = 0; u < SPR_U; u++)
+        for (int u = 0; u < U; u++)
             if (s0 + u < ncols) T[a + (size_t)(s0 + u) * rows] = acc[u];
     }
 }
@@ -3006,7 +3000,7 @@ __device__ __forceinline__ void sparse_rows_run(const int *rp, const int *col, c
 // gathers of B then read LDS instead of scattered global addresses.  When B does not fit it is
 // gathered from global memory; when the rows do not fit either, they are read from global
 // memory as well.  Ends with a barrier.
-template <int NT, typename R>
+template <int NT, typename R, int U = SPR_U>
 __device__ __forceinline__ void sparse_rows_times(const int *__restrict__ rp,
                                                   const int *__restrict__ col,
                                                   const cd *__restrict__ val, int rows, int ncols,
@@ -3033,10 +3027,10 @@ __device__ __forceinline__ void sparse_rows_times(const int *__restrict__ rp,
         if (bl)
             for (int i = tid; i < (int)nb; i += NT) s_b[i] = B[i];
         __syncthreads();
-        if (bl) sparse_rows_run<NT, R>(s_rp, s_c, s_v, rows, ncols, s_b, ldb, T);
-        else sparse_rows_run<NT, R>(s_rp, s_c, s_v, rows, ncols, B, ldb, T);
+        if (bl) sparse_rows_run<NT, R, U>(s_rp, s_c, s_v, rows, ncols, s_b, ldb, T);
+        else sparse_rows_run<NT, R, U>(s_rp, s_c, s_v, rows, ncols, B, ldb, T);
     } else {
-        sparse_rows_run<NT, R>(rp, col, val, rows, ncols, B, ldb, T);
+        sparse_rows_run<NT, R, U>(rp, col, val, rows, ncols, B, ldb, T);
     }
     __syncthreads();
 }
@@ -3150,25 +3144,20 @@ __device__ __forceinline__ bool qr_chain_mfma(int bI, int bJ, int n, const int *
 // Qs = Q(r,s), Rs = R(s,r).
 // FLIP (complex64, tile classes 1-4; a variant the launch autotuner may choose): the other of
 // the two forms -- the per-step form for classes 1-2, the step-walking form for 3-4.
-// The complex64 per-step products of tile classes 4-5 (blocks of 49-80 states) run eight waves,
-// two workgroups per CU (class 4: 79 registers, 19% faster than four waves; class 5: 117
-// registers, 3% faster); class 3 measured 13% slower at eight waves and keeps four, held to five
-// workgroups per CU (90 registers, no spills; 11% faster than four).
-template <int M, typename R, bool SPLIT, bool FLIP = false> struct QrThreads {
-    static constexpr int v = (M >= 4 && !FLIP && std::is_same<R, float>::value && !SPLIT) ? 512 : NThr<M>::v;
-};
-template <int M, typename R, bool SPLIT = false, bool FLIP = false>
-__global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<M, R, SPLIT, FLIP>::v == 512) ? 2 : (M == 5 && sizeof(R) == 4) ? 3 : (M == 3 && sizeof(R) == 4 && !FLIP && !SPLIT) ? 5 : (M == 4 && sizeof(R) == 8) ? 3 : 1) k_qr(DevPlan P, int Kb, const int *__restrict__ pgrp,
+// (FP64 pairs and the default form of classes 3-5 take k_qr_wt.)
+template <int M, bool SPLIT, bool FLIP = false>
+__global__ void __launch_bounds__(NThr<M>::v) k_qr(DevPlan P, int Kb, const int *__restrict__ pgrp,
                                                    int ngrp,
-                                                   const typename CX<R>::T *__restrict__ bufB,
-                                                   typename CX<R>::T *__restrict__ scratch,
-                                                   size_t slot, typename CX<R>::T *__restrict__ Qt,
-                                                   typename CX<R>::T *__restrict__ Rt) {
-    constexpr int NT = QrThreads<M, R, SPLIT, FLIP>::v;
-    typedef typename CX<R>::T CT;
+                                                   const cf *__restrict__ bufB,
+                                                   cf *__restrict__ scratch,
+                                                   size_t slot, cf *__restrict__ Qt,
+                                                   cf *__restrict__ Rt) {
+    constexpr int NT = NThr<M>::v;
+    typedef float R;
+    typedef cf CT;
     // complex64 pairs of small blocks with R formed from Q: one task per (crystallite, pair)
     // walks all steps (qr_chain_mfma); otherwise one task per (crystallite, step, pair)
-    constexpr bool CHAIN = ((M <= 2) != FLIP) && M <= 4 && std::is_same<R, float>::value && !SPLIT;
+    constexpr bool CHAIN = ((M <= 2) != FLIP) && M <= 4 && !SPLIT;
     constexpr int GB = CGemm<M, NT, R, SPLIT>::BYTES, CB = QrChainLds<M>::BYTES;
     __shared__ __align__(16) char smem[CHAIN && CB > GB ? CB : GB];
     const int tid = threadIdx.x;
@@ -3191,7 +3180,7 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
                 for (int k = 0; k < P.n; k++) { // rows too many for the LDS left: per step
                     const CT *BI = bufB + b0 + (size_t)k * P.Lsum + P.blk_uoff[I];
                     const CT *BJ = bufB + b0 + (size_t)k * P.Lsum + P.blk_uoff[J];
-                    sparse_rows_times<NT, R>(P.d_rowptr + P.pair_doff[pr], P.d_col,
+                    sparse_rows_times<NT, R, 1>(P.d_rowptr + P.pair_doff[pr], P.d_col,
                                              (const cd *)P.d_val, bI, bJ, BJ, bJ, T1, smem, GB);
                     CGemm<M, NT, R, SPLIT>::run(bI, bJ, bI, BI, bI, true, T1, bI,
                                                 Qt + e0 + (size_t)k * P.Estr, bI, smem);
@@ -3211,7 +3200,7 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
         const CT *BI = bufB + ((size_t)c * P.n + k) * P.Lsum + P.blk_uoff[I];
         const CT *BJ = bufB + ((size_t)c * P.n + k) * P.Lsum + P.blk_uoff[J];
         const size_t eo = ((size_t)c * P.n + k) * P.Estr + P.pair_eoff[pr];
-        sparse_rows_times<NT, R>(P.d_rowptr + P.pair_doff[pr], P.d_col, (const cd *)P.d_val, bI,
+        sparse_rows_times<NT, R, 1>(P.d_rowptr + P.pair_doff[pr], P.d_col, (const cd *)P.d_val, bI,
                                  bJ, BJ, bJ, T1, smem, CGemm<M, NT, R, SPLIT>::BYTES);
         CGemm<M, NT, R, SPLIT>::run(bI, bJ, bI, BI, bI, true, T1, bI, Qt + eo, bI, smem);
         if (P.rt_from_q) continue; // R is formed from Q in k_corr
@@ -3221,7 +3210,7 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
             const CT *X = (const CT *)P.rho_c + (size_t)c * P.Etot + P.pair_eoff[pr];
             CGemm<M, NT, R, SPLIT>::run(bJ, bI, bI, X, bI, true, BI, bI, T1, bJ, smem);
         } else {
-            sparse_rows_times<NT, R>(P.r_rowptr + P.pair_roff[pr], P.r_col, (const cd *)P.r_val,
+            sparse_rows_times<NT, R, 1>(P.r_rowptr + P.pair_roff[pr], P.r_col, (const cd *)P.r_val,
                                      bJ, bI, BI, bI, T1, smem, CGemm<M, NT, R, SPLIT>::BYTES);
         }
         // R^T(r,s) = sum_b T1(b,r) conj(B_J(b,s)) = (T1^T conj(B_J))(r,s): computed as
@@ -3235,15 +3224,15 @@ __global__ void __launch_bounds__((QrThreads<M, R, SPLIT, FLIP>::v), (QrThreads<
     }
 }
 
-// Pairs with a block above 80 states: as the per-step form of k_qr, the products by wave tiles.
+#define QRB_CSR (28 * 1024) // rows of an operator pair of 256 states and 5 values a row
+// As the per-step form of k_qr, the products by wave tiles.  Pairs with a block above 80 states,
 // 64 crystallites x 64 steps: 10 spins complex64 38 -> 23.6 ms, 9 spins FP64 11.4 -> 5.2 ms.
-template <typename R>
-__global__ void __launch_bounds__(256, 2) k_qr_big(DevPlan P, int Kb, const int *__restrict__ pgrp, int ngrp,
+template <typename R, int TI, int TJ, int CSR>
+__global__ void __launch_bounds__(256, TI == 4 ? 2 : sizeof(R) == 4 ? 5 : 4) k_qr_wt(DevPlan P, int Kb, const int *__restrict__ pgrp, int ngrp,
                                                 const typename CX<R>::T *__restrict__ bufB,
                                                 typename CX<R>::T *scratch, size_t slot,
                                                 typename CX<R>::T *Qt, typename CX<R>::T *Rt) {
     typedef typename CX<R>::T CT;
-    constexpr int CSR = 28 * 1024; // rows of an operator pair of 256 states and 5 values a row
     __shared__ __align__(16) char smem[CSR];
     CT *T1 = scratch + slot * 2 * blockIdx.x;
     CT *G = T1 + slot;
@@ -3259,16 +3248,16 @@ __global__ void __launch_bounds__(256, 2) k_qr_big(DevPlan P, int Kb, const int 
         const size_t eo = (size_t)ck * P.Estr + P.pair_eoff[pr];
         sparse_rows_times<256, R>(P.d_rowptr + P.pair_doff[pr], P.d_col, (const cd *)P.d_val, bI, bJ,
                                   BJ, bJ, T1, smem, CSR);
-        wg_wt_cmul<4, R, true>(bI, bJ, bI, BI, bI, T1, bI, Qt + eo, bI);
+        wg_wt_cmul<4, R, true, TI, TJ>(bI, bJ, bI, BI, bI, T1, bI, Qt + eo, bI);
         if (P.rt_from_q) continue;
         if (P.rho_c) { // the prepared rho_JI^H of this crystallite
             const CT *X = (const CT *)P.rho_c + (size_t)c * P.Etot + P.pair_eoff[pr];
-            wg_wt_cmul<4, R, true>(bJ, bI, bI, X, bI, BI, bI, T1, bJ);
+            wg_wt_cmul<4, R, true, TI, TJ>(bJ, bI, bI, X, bI, BI, bI, T1, bJ);
         } else {
             sparse_rows_times<256, R>(P.r_rowptr + P.pair_roff[pr], P.r_col, (const cd *)P.r_val, bJ,
                                       bI, BI, bI, T1, smem, CSR);
         }
-        wg_wt_cmul<4, R, true>(bJ, bI, bJ, BJ, bJ, T1, bJ, G, bJ);
+        wg_wt_cmul<4, R, true, TI, TJ>(bJ, bI, bJ, BJ, bJ, T1, bJ, G, bJ);
         for (int e = threadIdx.x; e < bI * bJ; e += 256) Rt[eo + e] = G[e / bI + (size_t)(e % bI) * bJ];
         __syncthreads();
     }
@@ -4592,15 +4581,6 @@ __global__ void __launch_bounds__(NThr<M>::v) k_static_fid(DevPlan P, int Kb, co
         else                                                                                     \
             kern<M_, R_, false><<<grid_, nt_, 0, st_>>>(__VA_ARGS__);                            \
     } while (0)
-// As LAUNCH_SPLIT, with the workgroup size of each variant from the kernel's thread traits TH.
-#define LAUNCH_SPLIT_TH(kern, TH, M_, R_, grid_, st_, ...)                                       \
-    do {                                                                                         \
-        constexpr bool SP_ = std::is_same<R_, float>::value;                                     \
-        if (SP_ && P->bf16x3)                                                                    \
-            kern<M_, R_, SP_><<<grid_, TH<M_, R_, SP_>::v, 0, st_>>>(__VA_ARGS__);               \
-        else                                                                                     \
-            kern<M_, R_, false><<<grid_, TH<M_, R_, false>::v, 0, st_>>>(__VA_ARGS__);           \
-    } while (0)
 // prec: 0 = FP64 storage (double2), 1 = complex64 storage (float2) of U, A, B, Q, R and the exp
 // scratch; the eigen-solver, phases, FIDs and reductions are FP64 in both.
 
@@ -4775,92 +4755,116 @@ extern "C" int blfid_dev_launch_eig(int prec, const DevPlan *P, int Kb, const in
     return (int)hipGetLastError();
 }
 
-template <typename R>
-static void launch_bmul(int M, const DevPlan *P, int Kb, const int *grp, int ngrp, int grid,
-                        const void *bufA, const void *bufW, void *bufB, hipStream_t st) {
+template <typename R, int TI, int TJ>
+static void launch_bmul_wt(const DevPlan *P, int Kb, const int *grp, int ngrp, const void *bufA,
+                           const void *bufW, void *bufB, hipStream_t st) {
     typedef typename CX<R>::T CT;
-    const CT *A = (const CT *)bufA, *W = (const CT *)bufW;
-    CT *B = (CT *)bufB;
-    switch (M) {
-    case 1: LAUNCH_SPLIT(k_bmul, 1, R, grid, 64, st, *P, Kb, grp, ngrp, A, W, B); break;
-    case 2: LAUNCH_SPLIT_TH(k_bmul, BmThreads, 2, R, grid, st, *P, Kb, grp, ngrp, A, W, B); break;
-    case 3: LAUNCH_SPLIT_TH(k_bmul, BmThreads, 3, R, grid, st, *P, Kb, grp, ngrp, A, W, B); break;
-    case 4: LAUNCH_SPLIT_TH(k_bmul, BmThreads, 4, R, grid, st, *P, Kb, grp, ngrp, A, W, B); break;
-    default: LAUNCH_SPLIT_TH(k_bmul, BmThreads, 5, R, grid, st, *P, Kb, grp, ngrp, A, W, B); break;
-    }
+    const long ntask = (long)Kb * P->n * ngrp, cap = tuned_cap(P, 3, 5);
+    k_bmul_wt<R, TI, TJ><<<(int)(ntask < cap ? ntask : cap), 256, 0, st>>>(*P, Kb, grp, ngrp, (const CT *)bufA, (const CT *)bufW, (CT *)bufB);
 }
 
-// bufW: W in the plan's storage precision
+// bufW: W in the plan's storage precision.  The first nbig blocks of grp have more than
+// DEV_LDS_BLOCK states: 4 x 4 (FP64 4 x 2) wave tiles; 2 x 2 ones below, where a block has fewer
+// tiles than that would take.  Wave tiles against the other forms, by tile class (8-, 7-, 6-spin
+// clusters, ms): FP64 5: 16.7 -> 11.5, 4: 15.6 -> 10.9, 3: 6.0 -> 4.6, 2: 5.2 against 5.5;
+// complex64 5: 28.0 -> 26.5, 4: 26.1 against 26.5, 3: 8.7 against 10.8 (the chain reads W once).
 extern "C" int blfid_dev_launch_bmul(int prec, int M, const DevPlan *P, int Kb, const int *grp,
                                      int ngrp, int nbig, const void *bufA, const void *bufW,
                                      void *bufB, hipStream_t st) {
-    const long cap = tuned_cap(P, 3, M);
     if (Kb <= 0 || ngrp <= 0) return 0;
     if (!P->bf16x3 && nbig > 0) {
-        const long ntask = (long)Kb * P->n * nbig;
-        const int grid = (int)(ntask < cap ? ntask : cap);
-        if (prec) k_bmul_big<float><<<grid, 256, 0, st>>>(*P, Kb, grp, nbig, (const cf *)bufA, (const cf *)bufW, (cf *)bufB);
-        else k_bmul_big<double><<<grid, 256, 0, st>>>(*P, Kb, grp, nbig, (const cd *)bufA, (const cd *)bufW, (cd *)bufB);
+        if (prec) launch_bmul_wt<float, 4, 4>(P, Kb, grp, nbig, bufA, bufW, bufB, st);
+        else launch_bmul_wt<double, 4, 2>(P, Kb, grp, nbig, bufA, bufW, bufB, st);
         grp += nbig;
         ngrp -= nbig;
     }
-    const long ntask = (long)Kb * P->n * ngrp;
-    const int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid > 0) {
-        if (prec) launch_bmul<float>(M, P, Kb, grp, ngrp, grid, bufA, bufW, bufB, st);
-        else launch_bmul<double>(M, P, Kb, grp, ngrp, grid, bufA, bufW, bufB, st);
+    if (ngrp <= 0) return (int)hipGetLastError();
+    if (!P->bf16x3 && M >= (prec ? 5 : 3)) {
+        if (prec) launch_bmul_wt<float, 2, 2>(P, Kb, grp, ngrp, bufA, bufW, bufB, st);
+        else launch_bmul_wt<double, 2, 2>(P, Kb, grp, ngrp, bufA, bufW, bufB, st);
+        return (int)hipGetLastError();
     }
+    const long ntask = (long)Kb * P->n * ngrp, cap = tuned_cap(P, 3, M);
+    const int grid = (int)(ntask < cap ? ntask : cap);
+#define BMUL_ARGS(CT) *P, Kb, grp, ngrp, (const CT *)bufA, (const CT *)bufW, (CT *)bufB
+    if (!prec) {
+        if (M == 1) k_bmul<1, double><<<grid, 64, 0, st>>>(BMUL_ARGS(cd));
+        else k_bmul<2, double><<<grid, 256, 0, st>>>(BMUL_ARGS(cd));
+    } else {
+        switch (M) {
+        case 1: LAUNCH_SPLIT(k_bmul, 1, float, grid, 64, st, BMUL_ARGS(cf)); break;
+        case 2: LAUNCH_SPLIT(k_bmul, 2, float, grid, 256, st, BMUL_ARGS(cf)); break;
+        case 3: LAUNCH_SPLIT(k_bmul, 3, float, grid, 256, st, BMUL_ARGS(cf)); break;
+        case 4: LAUNCH_SPLIT(k_bmul, 4, float, grid, 256, st, BMUL_ARGS(cf)); break;
+        default: k_bmul<5, float, true><<<grid, 256, 0, st>>>(BMUL_ARGS(cf)); break;
+        }
+    }
+#undef BMUL_ARGS
     return (int)hipGetLastError();
 }
 
-template <typename R>
-static void launch_qr(int M, const DevPlan *P, int Kb, const int *pgrp, int ngrp, int grid,
-                      const void *bufB, void *scratch, size_t slot, void *Qt, void *Rt,
-                      hipStream_t st) {
+template <typename R, int TI, int TJ, int CSR>
+static void launch_qr_wt(const DevPlan *P, int Kb, const int *pgrp, int ngrp, long cap,
+                         const void *bufB, void *scratch, size_t slot, void *Qt, void *Rt,
+                         hipStream_t st) {
     typedef typename CX<R>::T CT;
-    const CT *B = (const CT *)bufB;
-    CT *sc = (CT *)scratch, *Q = (CT *)Qt, *Rr = (CT *)Rt;
-    if constexpr (std::is_same<R, float>::value) {
-        if (!P->bf16x3 && M <= 4 && ((P->tn_qr >> (M - 1)) & 1)) {
-            switch (M) {
-            case 1: k_qr<1, R, false, true><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-            case 2: k_qr<2, R, false, true><<<grid, 256, 0, st>>>(*P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-            case 3: k_qr<3, R, false, true><<<grid, 256, 0, st>>>(*P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-            default: k_qr<4, R, false, true><<<grid, 256, 0, st>>>(*P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-            }
-            return;
-        }
-    }
-    switch (M) {
-    case 1: // the BF16x3 form; otherwise class 1 takes k_bq1 (or the per-step form above)
-        if constexpr (std::is_same<R, float>::value) k_qr<1, R, true><<<grid, 64, 0, st>>>(*P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr);
-        break;
-    case 2: LAUNCH_SPLIT_TH(k_qr, QrThreads, 2, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-    case 3: LAUNCH_SPLIT_TH(k_qr, QrThreads, 3, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-    case 4: LAUNCH_SPLIT_TH(k_qr, QrThreads, 4, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-    default: LAUNCH_SPLIT_TH(k_qr, QrThreads, 5, R, grid, st, *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr); break;
-    }
+    const long ntask = (long)Kb * P->n * ngrp;
+    k_qr_wt<R, TI, TJ, CSR><<<(int)(ntask < cap ? ntask : cap), 256, 0, st>>>(*P, Kb, pgrp, ngrp, (const CT *)bufB, (CT *)scratch, slot, (CT *)Qt, (CT *)Rt);
 }
 
+// Q (and R) by wave tiles: the first nbig pairs of pgrp (a block above DEV_LDS_BLOCK states) with
+// 4 x 4 (FP64 4 x 2) tiles, the FP64 pairs of every class above 1 and the complex64 ones of
+// classes 3 to 5 with 2 x 2.  By class, against the tile products they replace (8-, 7-, 6-spin
+// clusters, ms): FP64 5: 35.4 -> 26.4, 4: 15.7 -> 10.0, 3: 11.1 -> 8.6, 2: 9.4 -> 8.3; complex64
+// 5: 65.3 -> 57.6, 4: 29.1 -> 22.5, 3: 21.7 -> 17.8; 2: 17.9 walking the steps, 17.4 by wave tiles
+// (left as it was).  Tuned plans may choose the step-walking form (classes 3, 4) or the per-step one
+// (classes 1, 2); the BF16x3 form has its own products.
 extern "C" int blfid_dev_launch_qr(int prec, int M, const DevPlan *P, int Kb, const int *pgrp,
                                    int ngrp, int nbig, const void *bufB, void *scratch, size_t slot,
                                    int nslots, void *Qt, void *Rt, hipStream_t st) {
     const long cap = P->tn_cap[4] > 0 ? std::min<long>(tuned_cap(P, 4, M), nslots) : nslots;
-    if (Kb <= 0 || ngrp <= 0) return 0;
+    if (Kb <= 0 || ngrp <= 0 || cap <= 0) return 0;
     if (!P->bf16x3 && nbig > 0) {
-        const long ntask = (long)Kb * P->n * nbig;
-        const int grid = (int)(ntask < cap ? ntask : cap);
-        if (prec) k_qr_big<float><<<grid, 256, 0, st>>>(*P, Kb, pgrp, nbig, (const cf *)bufB, (cf *)scratch, slot, (cf *)Qt, (cf *)Rt);
-        else k_qr_big<double><<<grid, 256, 0, st>>>(*P, Kb, pgrp, nbig, (const cd *)bufB, (cd *)scratch, slot, (cd *)Qt, (cd *)Rt);
+        if (prec) launch_qr_wt<float, 4, 4, QRB_CSR>(P, Kb, pgrp, nbig, cap, bufB, scratch, slot, Qt, Rt, st);
+        else launch_qr_wt<double, 4, 2, QRB_CSR>(P, Kb, pgrp, nbig, cap, bufB, scratch, slot, Qt, Rt, st);
         pgrp += nbig;
         ngrp -= nbig;
     }
+    if (ngrp <= 0) return (int)hipGetLastError();
+    if (!prec) {
+        launch_qr_wt<double, 2, 2, 12288>(P, Kb, pgrp, ngrp, cap, bufB, scratch, slot, Qt, Rt, st);
+        return (int)hipGetLastError();
+    }
+    const bool flip = !P->bf16x3 && M <= 4 && ((P->tn_qr >> (M - 1)) & 1);
+    if (!P->bf16x3 && !flip && M >= 3) {
+        launch_qr_wt<float, 2, 2, 8192>(P, Kb, pgrp, ngrp, cap, bufB, scratch, slot, Qt, Rt, st);
+        return (int)hipGetLastError();
+    }
     const long ntask = (long)Kb * P->n * ngrp;
     const int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid > 0) {
-        if (prec) launch_qr<float>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
-        else launch_qr<double>(M, P, Kb, pgrp, ngrp, grid, bufB, scratch, slot, Qt, Rt, st);
+    const cf *B = (const cf *)bufB;
+    cf *sc = (cf *)scratch, *Q = (cf *)Qt, *Rr = (cf *)Rt;
+#define QR_ARGS *P, Kb, pgrp, ngrp, B, sc, slot, Q, Rr
+    if (P->bf16x3) {
+        switch (M) {
+        case 1: k_qr<1, true><<<grid, 64, 0, st>>>(QR_ARGS); break;
+        case 2: k_qr<2, true><<<grid, 256, 0, st>>>(QR_ARGS); break;
+        case 3: k_qr<3, true><<<grid, 256, 0, st>>>(QR_ARGS); break;
+        case 4: k_qr<4, true><<<grid, 256, 0, st>>>(QR_ARGS); break;
+        default: k_qr<5, true><<<grid, 256, 0, st>>>(QR_ARGS); break;
+        }
+    } else {
+        switch (M) {
+        case 1: k_qr<1, false, true><<<grid, 64, 0, st>>>(QR_ARGS); break;
+        case 2:
+            if (flip) k_qr<2, false, true><<<grid, 256, 0, st>>>(QR_ARGS);
+            else k_qr<2, false><<<grid, 256, 0, st>>>(QR_ARGS);
+            break;
+        case 3: k_qr<3, false, true><<<grid, 256, 0, st>>>(QR_ARGS); break;
+        default: k_qr<4, false, true><<<grid, 256, 0, st>>>(QR_ARGS); break;
+        }
     }
+#undef QR_ARGS
     return (int)hipGetLastError();
 }
 
