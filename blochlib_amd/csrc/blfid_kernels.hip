@@ -2304,6 +2304,58 @@ __global__ void __launch_bounds__(64 * M, M <= 3 ? 2 : 1) k_expdyson_d(DevPlan P
     if (P.expflops && tid == 0 && nflops > 0.0) atomicAdd(&P.expflops[8 + M], nflops);
 }
 
+// Joint rotation of the index pair (p, q) of a normal-matrix iterate: the Cardoso-Souloumiac
+// angle for H1 = (M + M^H)/2, H2 = (M - M^H)/2i.  Returns false (identity) when the pair's
+// off-diagonal part is below tol_off of its diagonal; big: |s| > tol_big.  With c^2 = (1 + ux / r) / 2
+// and s = (uy, -uz) / (2 r c), r = |u|, the angle takes three reciprocal square roots; square
+// roots and divisions were most of a round's latency, on which every other thread waits (8-spin
+// clusters complex64: the 64- and 80-state classes 35.2 -> 27.0 and 29.0 -> 23.5 ms; 6 spins static x
+// 1154: 32 and 16 347 -> 260 and 339 -> 239 us, with each thread's items taken out of the rounds).
+__device__ __forceinline__ bool jj_rotation(cd mpp, cd mqq, cd mpq, cd mqp, double tol_off,
+                                            double tol_big, double &cth, cd &sth, bool &big) {
+    cth = 1.0;
+    sth = cmk(0, 0);
+    big = false;
+    const cd h1pq = cscale(cadd(mpq, cconj(mqp)), 0.5);
+    const cd d2 = csub(mpq, cconj(mqp));
+    const cd h2pq = cmk(0.5 * d2.y, -0.5 * d2.x);
+    const double off = fabs(h1pq.x) + fabs(h1pq.y) + fabs(h2pq.x) + fabs(h2pq.y);
+    const double scale = fabs(mpp.x) + fabs(mpp.y) + fabs(mqq.x) + fabs(mqq.y) + 1e-300;
+    if (!(off > tol_off * scale)) return false;
+    const double h1[3] = {mpp.x - mqq.x, 2.0 * h1pq.x, 2.0 * h1pq.y};
+    const double h2[3] = {mpp.y - mqq.y, 2.0 * h2pq.x, 2.0 * h2pq.y};
+    const double ka = h1[0] * h1[0] + h1[1] * h1[1] + h1[2] * h1[2];
+    const double kd = h2[0] * h2[0] + h2[1] * h2[1] + h2[2] * h2[2];
+    const double kb = h1[0] * h2[0] + h1[1] * h2[1] + h1[2] * h2[2];
+    const double hm = 0.5 * (ka + kd);
+    const double disc = 0.25 * (ka - kd) * (ka - kd) + kb * kb;
+    const double lam = hm + (disc > 1e-280 ? disc * rsqrt(disc) : 0.0);
+    const double a1 = lam - kd, b1 = kb, a2 = kb, b2 = lam - ka;
+    double al, be;
+    if (a1 * a1 + b1 * b1 >= a2 * a2 + b2 * b2) { al = a1; be = b1; }
+    else { al = a2; be = b2; }
+    if (al == 0.0 && be == 0.0) { al = 1.0; be = 0.0; }
+    double ux = al * h1[0] + be * h2[0];
+    double uy = al * h1[1] + be * h2[1];
+    double uz = al * h1[2] + be * h2[2];
+    if (ux < 0) { ux = -ux; uy = -uy; uz = -uz; }
+    const double n2 = ux * ux + uy * uy + uz * uz;
+    double sc; // |s| / |(uy, uz)|
+    if (n2 > 1e-280) {
+        const double ri = rsqrt(n2), c2 = fma(0.5 * ux, ri, 0.5), c = rsqrt(c2);
+        cth = c2 * c;
+        sc = 0.5 * ri * c;
+    } else {
+        const double r = sqrt(n2);
+        if (!(r > 0.0)) return false;
+        cth = sqrt((ux + r) / (2.0 * r));
+        sc = 1.0 / sqrt(2.0 * r * (ux + r));
+    }
+    sth = cmk(uy * sc, -uz * sc);
+    big = fabs(sth.x) + fabs(sth.y) > tol_big;
+    return true;
+}
+
 // ------------------------------------------------------------------------------ k_eig
 // Joint Jacobi diagonalisation of a normal matrix Mx = H1 + i H2 (H1, H2 Hermitian,
 // commuting): each 2x2 rotation is the Cardoso-Souloumiac angle for the pair (H1, H2)
@@ -2313,11 +2365,13 @@ __global__ void __launch_bounds__(64 * M, M <= 3 ? 2 : 1) k_expdyson_d(DevPlan P
 // mode 1: Mx = H block (Hermitian, static path) -> out value = Re(Mx_rr)
 #define EIG_MAXB 80
 // The block lives in LDS (b <= MB), with LDS and threads sized for that class so that
-// workgroups of small blocks share a CU; larger blocks take the k_eigb_ kernels.
+// workgroups of small blocks share a CU (held to four waves per SIMD up to 48 states, five up to
+// 16: unbounded, the FP64 48-state class took 3.36 instead of 2.25 ms); larger blocks take the
+// k_eigb_ kernels.
 // The source block may be stored in FP32 (complex64 plans); the solver always runs in FP64 and
 // W stays FP64, with a storage-precision copy Wr for the B = A W products when R != double.
 template <int MB, int NT, typename R>
-__global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__restrict__ grp,
+__global__ void __launch_bounds__(NT, MB == 16 ? 5 : MB <= 48 ? 4 : 1) k_eig(DevPlan P, int Kb, const int *__restrict__ grp,
                                              int ngrp, const typename CX<R>::T *__restrict__ src,
                                              size_t src_stride, int mode, cd *__restrict__ bufW,
                                              typename CX<R>::T *__restrict__ bufWr,
@@ -2328,7 +2382,7 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
     // order tol_rot, which the confirming sweep of a rotations-below-tol_rot test would only
     // square); pairs below tol_off are skipped.  A complex64 period propagator carries ~1e-7
     // relative error, so its solve stops earlier.
-    constexpr double tol_rot = __is_same(R, double) ? 1e-15 : 1e-10;
+    // tol_rot: 1e-15 (FP64), 1e-10 (complex64)
     constexpr double tol_stop = __is_same(R, double) ? 3.1622776601683795e-8 : 1e-5;
     constexpr double tol_off = __is_same(R, double) ? 1e-17 : 1e-12;
     static_assert(MB > 0 && MB <= EIG_MAXB, "blocks above 80 states take k_eigb_*");
@@ -2367,6 +2421,20 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
         __syncthreads();
         const int bb = (b + 1) & ~1; // even count, index b is a dummy when b is odd
         const int npair = bb / 2;
+        // this thread's 2 x 2 blocks of M (pair of rows, pair of columns) and its entries of W (row,
+        // pair of columns), the same in every round
+        constexpr int NM = (MP * MP + NT - 1) / NT, NWI = (MP * MB + NT - 1) / NT;
+        int mi[NM], wi[NWI];
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            const int e = tid + i * NT;
+            mi[i] = e < npair * npair ? e % npair | e / npair << 8 : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < NWI; i++) {
+            const int e = tid + i * NT;
+            wi[i] = e < npair * b ? e % b | e / b << 8 : -1;
+        }
         for (int sweep = 0; sweep < 40 && b > 1; sweep++) {
             if (tid == 0) s_any = 0;
             __syncthreads();
@@ -2374,46 +2442,17 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
                 for (int pi = tid; pi < npair; pi += NT) {
                     // circle method: position 0 fixed, positions 1..bb-1 rotate
                     int pa = pi, pb = bb - 1 - pi;
-                    int ia = (pa == 0) ? 0 : ((pa - 1 + round) % (bb - 1)) + 1;
-                    int ib = (pb == 0) ? 0 : ((pb - 1 + round) % (bb - 1)) + 1;
+                    int ia = pa + round, ib = pb + round; // 1 .. bb - 1, turned by round
+                    if (ia >= bb) ia -= bb - 1;
+                    if (ib >= bb) ib -= bb - 1;
+                    if (pa == 0) ia = 0;
                     int p = min(ia, ib), q = max(ia, ib);
                     double cth = 1.0;
                     cd sth = cmk(0, 0);
-                    if (q < b) {
-                        cd mpp = Ms[p + p * ld], mqq = Ms[q + q * ld];
-                        cd mpq = Ms[p + q * ld], mqp = Ms[q + p * ld];
-                        // H1 = (M + M^H)/2, H2 = (M - M^H)/(2i)
-                        cd h1pq = cscale(cadd(mpq, cconj(mqp)), 0.5);
-                        cd d2 = csub(mpq, cconj(mqp));           // = 2i H2pq
-                        cd h2pq = cmk(0.5 * d2.y, -0.5 * d2.x); // d2 / (2i)
-                        double off = fabs(h1pq.x) + fabs(h1pq.y) + fabs(h2pq.x) + fabs(h2pq.y);
-                        double scale = fabs(mpp.x) + fabs(mpp.y) + fabs(mqq.x) + fabs(mqq.y) + 1e-300;
-                        if (off > tol_off * scale) {
-                            double h1[3] = {mpp.x - mqq.x, 2.0 * h1pq.x, 2.0 * h1pq.y};
-                            double h2[3] = {mpp.y - mqq.y, 2.0 * h2pq.x, 2.0 * h2pq.y};
-                            double ka = h1[0] * h1[0] + h1[1] * h1[1] + h1[2] * h1[2];
-                            double kd = h2[0] * h2[0] + h2[1] * h2[1] + h2[2] * h2[2];
-                            double kb = h1[0] * h2[0] + h1[1] * h2[1] + h1[2] * h2[2];
-                            double hm = 0.5 * (ka + kd);
-                            double lam = hm + sqrt(0.25 * (ka - kd) * (ka - kd) + kb * kb);
-                            double a1 = lam - kd, b1 = kb, a2 = kb, b2 = lam - ka;
-                            double al, be;
-                            if (a1 * a1 + b1 * b1 >= a2 * a2 + b2 * b2) { al = a1; be = b1; }
-                            else { al = a2; be = b2; }
-                            if (al == 0.0 && be == 0.0) { al = 1.0; be = 0.0; }
-                            double ux = al * h1[0] + be * h2[0];
-                            double uy = al * h1[1] + be * h2[1];
-                            double uz = al * h1[2] + be * h2[2];
-                            if (ux < 0) { ux = -ux; uy = -uy; uz = -uz; }
-                            double r = sqrt(ux * ux + uy * uy + uz * uz);
-                            if (r > 0.0) {
-                                cth = sqrt((ux + r) / (2.0 * r));
-                                double den = sqrt(2.0 * r * (ux + r));
-                                sth = cmk(uy / den, -uz / den);
-                                if (fabs(sth.x) + fabs(sth.y) > tol_stop) s_any = 1;
-                            }
-                        }
-                    }
+                    bool big = false;
+                    if (q < b && jj_rotation(Ms[p + p * ld], Ms[q + q * ld], Ms[p + q * ld], Ms[q + p * ld],
+                                             tol_off, tol_stop, cth, sth, big) && big)
+                        s_any = 1;
                     rc[pi] = cth;
                     rs[pi] = sth;
                     rp[pi] = p;
@@ -2423,8 +2462,10 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
                 // M <- R^H M R and W <- W R in one pass, R = [[c, -conj(s)], [s, c]] on each
                 // pair (p, q): every 2 x 2 block (rows of pair i, columns of pair j) is rotated
                 // by both of its pairs' rotations; a dummy index (odd b) rotates by identity.
-                for (int e = tid; e < npair * npair; e += NT) {
-                    const int pi = e % npair, pj = e / npair;
+#pragma unroll
+                for (int i = 0; i < NM; i++) {
+                    if (mi[i] < 0) continue;
+                    const int pi = mi[i] & 255, pj = mi[i] >> 8;
                     const int p = rp[pi], q = rq[pi], p2 = rp[pj], q2 = rq[pj];
                     const bool vq = q < b, vq2 = q2 < b;
                     const double ci = rc[pi], cj = rc[pj];
@@ -2446,9 +2487,11 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
                 }
                 // W <- W R: consecutive threads take consecutive rows of one column pair, so
                 // the global accesses of a wave are contiguous
-                for (int e = tid; e < npair * b; e += NT) {
-                    int row = e % b, pi = e / b;
-                    int p = rp[pi], q = rq[pi];
+#pragma unroll
+                for (int i = 0; i < NWI; i++) {
+                    if (wi[i] < 0) continue;
+                    const int row = wi[i] & 255, pi = wi[i] >> 8;
+                    const int p = rp[pi], q = rq[pi];
                     if (q >= b) continue;
                     double cth = rc[pi];
                     cd sth = rs[pi];
@@ -2492,45 +2535,6 @@ __global__ void __launch_bounds__(NT) k_eig(DevPlan P, int Kb, const int *__rest
 }
 
 // ------------------------------------------------------------------------------ k_eigb
-// Joint rotation of the index pair (p, q) of a normal-matrix iterate: the Cardoso-Souloumiac
-// angle for H1 = (M + M^H)/2, H2 = (M - M^H)/2i, as k_eig forms it.  Returns false (identity)
-// when the pair's off-diagonal part is below tol_off of its diagonal; big: |s| > tol_big.
-__device__ __forceinline__ bool jj_rotation(cd mpp, cd mqq, cd mpq, cd mqp, double tol_off,
-                                            double tol_big, double &cth, cd &sth, bool &big) {
-    cth = 1.0;
-    sth = cmk(0, 0);
-    big = false;
-    const cd h1pq = cscale(cadd(mpq, cconj(mqp)), 0.5);
-    const cd d2 = csub(mpq, cconj(mqp));
-    const cd h2pq = cmk(0.5 * d2.y, -0.5 * d2.x);
-    const double off = fabs(h1pq.x) + fabs(h1pq.y) + fabs(h2pq.x) + fabs(h2pq.y);
-    const double scale = fabs(mpp.x) + fabs(mpp.y) + fabs(mqq.x) + fabs(mqq.y) + 1e-300;
-    if (!(off > tol_off * scale)) return false;
-    const double h1[3] = {mpp.x - mqq.x, 2.0 * h1pq.x, 2.0 * h1pq.y};
-    const double h2[3] = {mpp.y - mqq.y, 2.0 * h2pq.x, 2.0 * h2pq.y};
-    const double ka = h1[0] * h1[0] + h1[1] * h1[1] + h1[2] * h1[2];
-    const double kd = h2[0] * h2[0] + h2[1] * h2[1] + h2[2] * h2[2];
-    const double kb = h1[0] * h2[0] + h1[1] * h2[1] + h1[2] * h2[2];
-    const double hm = 0.5 * (ka + kd);
-    const double lam = hm + sqrt(0.25 * (ka - kd) * (ka - kd) + kb * kb);
-    const double a1 = lam - kd, b1 = kb, a2 = kb, b2 = lam - ka;
-    double al, be;
-    if (a1 * a1 + b1 * b1 >= a2 * a2 + b2 * b2) { al = a1; be = b1; }
-    else { al = a2; be = b2; }
-    if (al == 0.0 && be == 0.0) { al = 1.0; be = 0.0; }
-    double ux = al * h1[0] + be * h2[0];
-    double uy = al * h1[1] + be * h2[1];
-    double uz = al * h1[2] + be * h2[2];
-    if (ux < 0) { ux = -ux; uy = -uy; uz = -uz; }
-    const double r = sqrt(ux * ux + uy * uy + uz * uz);
-    if (!(r > 0.0)) return false;
-    cth = sqrt((ux + r) / (2.0 * r));
-    const double den = sqrt(2.0 * r * (ux + r));
-    sth = cmk(uy / den, -uz / den);
-    big = fabs(sth.x) + fabs(sth.y) > tol_big;
-    return true;
-}
-
 // Blocks of more than 80 states (b <= 256): block Jacobi with the same rotations, every round of
 // every block of the batch as two launches over the whole device.  The b x b iterate M, the
 // rotations and the sweep flags of a task (crystallite, block) live in its scratch slot (EIGB_*),
