@@ -199,6 +199,26 @@ class DevCache {
     }
 
   public:
+    // hipMalloc on device dev; before memory is reported as exhausted, everything held there is
+    // freed and the allocation tried once more.
+    hipError_t raw(size_t bytes, void **p, int dev) {
+        hipError_t e = hipMalloc(p, bytes);
+        if (e == hipErrorOutOfMemory && dev >= 0 && dev < CACHE_DEVICES) {
+            (void)hipGetLastError();
+            std::vector<void *> old;
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                expire(dev, 0, old);
+            }
+            free_all(old);
+            e = hipMalloc(p, bytes);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError(); // returned here, not reported again by the next launch
+            *p = nullptr;
+        }
+        return e;
+    }
     // At least `bytes` on the current device; *cap receives the block's size, *dev the device.
     hipError_t get(size_t bytes, void **p, size_t *cap, int *dev) {
         *p = nullptr;
@@ -233,19 +253,11 @@ class DevCache {
             if (*p) return hipSuccess;
         }
         *cap = want;
-        e = hipMalloc(p, want);
-        if (e == hipErrorOutOfMemory && kept) {
-            (void)hipGetLastError();
-            std::vector<void *> old;
-            {
-                std::lock_guard<std::mutex> lk(mu);
-                expire(*dev, 0, old);
-            }
-            free_all(old);
+        e = raw(want, p, *dev);
+        if (e == hipErrorOutOfMemory && want > bytes) {
             *cap = bytes;
-            e = hipMalloc(p, bytes);
+            e = raw(bytes, p, *dev);
         }
-        if (e != hipSuccess) *p = nullptr;
         return e;
     }
     // A block no work uses any more: the device is waited for first.
@@ -555,7 +567,11 @@ static int eig_class(int b) {
     return 5;
 }
 
-static int pair_dim(const blfid_plan *pl, int p);
+// States of the larger block of a pair
+static int pair_dim(const blfid_plan *pl, int p) {
+    return std::max(pl->blk_dim[pl->pairs[p].I], pl->blk_dim[pl->pairs[p].J]);
+}
+
 static blfid_status build_tables(blfid_plan *pl) {
     const int S = pl->S, N = pl->N;
     pl->terms.clear();
@@ -1508,9 +1524,6 @@ static size_t pair_e(const blfid_plan *pl, const std::vector<int> &g) {
 static int big_count(const blfid_plan *pl, const std::vector<int> &g) {
     return (int)std::count_if(g.begin(), g.end(), [&](int b) { return pl->blk_dim[b] > DEV_LDS_BLOCK; });
 }
-static int pair_dim(const blfid_plan *pl, int p) {
-    return std::max(pl->blk_dim[pl->pairs[p].I], pl->blk_dim[pl->pairs[p].J]);
-}
 static int big_pairs(const blfid_plan *pl, const std::vector<int> &g) {
     return (int)std::count_if(g.begin(), g.end(), [&](int p) { return pair_dim(pl, p) > DEV_LDS_BLOCK; });
 }
@@ -2444,7 +2457,9 @@ blfid_status blfid_workspace_create(double bytes, blfid_workspace **out) {
     *out = nullptr;
     blfid_workspace *w = new blfid_workspace();
     w->bytes = (size_t)bytes;
-    hipError_t e = hipMalloc((void **)&w->base, w->bytes);
+    int dev = -1;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = dev_cache().raw(w->bytes, (void **)&w->base, dev);
     if (e != hipSuccess) {
         delete w;
         return fail(e == hipErrorOutOfMemory ? BLFID_ERR_NOMEM : BLFID_ERR_DEVICE,

@@ -1,0 +1,83 @@
+// CPU check of the device memory that the host code takes, keeps and gives back, on a runtime
+// without a device (fake_hip.h).  Usage: memory_check <check>; prints OK or what failed.
+#include "fake_hip.h"
+
+#include "../../blochlib_amd/csrc/blfid_host.cpp"
+
+#include <functional>
+
+static int fails = 0;
+#define REQUIRE(c)                                                                               \
+    do {                                                                                         \
+        if (!(c)) {                                                                              \
+            std::printf("FAIL line %d: %s (%s)\n", __LINE__, #c, blfid_last_error());            \
+            fails++;                                                                             \
+        }                                                                                        \
+    } while (0)
+
+constexpr size_t GB = (size_t)1 << 30, MB = (size_t)1 << 20;
+
+// S protons with every dipole coupling and a shielding each
+struct Sys {
+    std::vector<int> iso;
+    std::vector<double> csa, dip;
+    blfid_system s;
+    explicit Sys(int S) : iso(S, 1) {
+        for (int i = 0; i < S; i++) {
+            const double c[7] = {100.0 * i, 3000.0, 0.3, (double)i, 10.0 * i, 20.0, 30.0};
+            csa.insert(csa.end(), c, c + 7);
+            for (int j = i + 1; j < S; j++) {
+                const double d[6] = {-9000.0, (double)i, (double)j, 0.0, 15.0 * j, 25.0};
+                dip.insert(dip.end(), d, d + 6);
+            }
+        }
+        s = {S, iso.data(), S, csa.data(), (int)(dip.size() / 6), dip.data(), 0, nullptr};
+    }
+};
+// I+ of every spin, and with general set a second operator that is no (D + D^H) / 2
+static std::vector<double> op(int S, bool plus, bool general = false) {
+    const size_t N = (size_t)1 << S;
+    std::vector<double> m(2 * N * N, 0.0);
+    for (int i = 0; i < S; i++)
+        for (size_t a = 0; a < N; a++)
+            if (a >> i & 1) {
+                const size_t b = a ^ ((size_t)1 << i);
+                m[2 * (b + a * N)] = plus ? 1.0 : 0.5;
+                if (!plus) m[2 * (a + b * N)] = general ? 0.25 * (i + 1) : 0.5;
+            }
+    return m;
+}
+static blfid_plan *plan(int S, int n, int npts, blfid_precision prec, int K, bool general = false) {
+    Sys sy(S);
+    blfid_plan *p = nullptr;
+    REQUIRE(blfid_plan_create(&sy.s, 10000.0, 54.7356, 10000.0 * n, npts, 0.0, prec, &p) == BLFID_OK);
+    const auto rho = op(S, false, general), det = op(S, true);
+    REQUIRE(blfid_plan_set_operators(p, rho.data(), det.data()) == BLFID_OK);
+    std::vector<double> a(K, 0.3), w(K, 1.0);
+    REQUIRE(blfid_plan_set_powder(p, a.data(), a.data(), a.data(), w.data(), K) == BLFID_OK);
+    return p;
+}
+
+// A workspace that fits the device once the memory kept from destroyed plans is given up.
+static void workspace() {
+    fake::limit = 4 * GB;
+    blfid_plan *p = plan(6, 64, 512, BLFID_FP64, 400);
+    REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+    blfid_plan_destroy(p);
+    REQUIRE(fake::used > 256 * MB); // kept
+    blfid_workspace *w = nullptr;
+    REQUIRE(blfid_workspace_create((double)(fake::limit - 64 * MB), &w) == BLFID_OK);
+    blfid_workspace_destroy(w);
+    // one beyond the device is still refused, with no error left for the next launch to report
+    w = nullptr;
+    REQUIRE(blfid_workspace_create((double)(fake::limit + GB), &w) == BLFID_ERR_NOMEM && !w);
+    REQUIRE(hipGetLastError() == hipSuccess);
+}
+
+int main(int argc, char **argv) {
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}};
+    if (argc != 2 || !checks.count(argv[1])) return 2;
+    checks.at(argv[1])();
+    if (!fails) std::printf("OK\n");
+    return fails ? 1 : 0;
+}
