@@ -162,10 +162,8 @@ void crystal_tensor(double pxx, double pyy, double pzz, double a, double b, doub
 // request may take when it fills half of one (8/9 from 64 MiB up); a block that CACHE_AGE requests have passed
 // over is freed, and everything held is freed before an allocation is reported as failed.  A block
 // enters the cache only when the device has finished all work (as hipFree waits for it), so it may
-// be handed to any thread and stream.  16 GiB (an 18th of the card) hold the storage of one gamma-
-// COMPUTE call of 6 spins x 1154, 100 steps with a general rho in FP64, which 4 GiB did not: a
-// pulse program and that FID 31.0 -> 30.1 ms, where allocating is quick.
-constexpr size_t CACHE_BYTES = (size_t)16 << 30;
+// be handed to any thread and stream.
+constexpr size_t CACHE_BYTES = (size_t)4 << 30;
 constexpr unsigned long CACHE_AGE = 256;
 constexpr int CACHE_DEVICES = 64;
 
