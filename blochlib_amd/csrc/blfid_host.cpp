@@ -285,6 +285,19 @@ class DevCache {
         free_all(old);
         if (cur != dev) (void)hipSetDevice(cur);
     }
+    // Frees everything held for the current device.
+    hipError_t release() {
+        int dev = -1;
+        const hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess || dev < 0 || dev >= CACHE_DEVICES) return e;
+        std::vector<void *> old;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            expire(dev, 0, old);
+        }
+        free_all(old);
+        return hipSuccess;
+    }
     // Bytes held for the current device: free memory as far as a memory budget is concerned.
     size_t held() {
         int dev = -1;
@@ -1244,7 +1257,7 @@ void blfid_plan_destroy(blfid_plan *pl) {
     if (!pl) return;
     if (pl->last_stream) (void)hipStreamSynchronize(pl->last_stream);
     else (void)hipDeviceSynchronize();
-    delete pl; // DevBuf destructors free the device memory
+    delete pl; // DevBuf destructors hand the device memory to the block cache
 }
 
 double blfid_plan_sw(const blfid_plan *pl) { return pl ? pl->sw_adj : 0.0; }
@@ -2470,6 +2483,17 @@ blfid_status blfid_workspace_create(double bytes, blfid_workspace **out) {
         return fail(BLFID_ERR_DEVICE, "workspace event");
     }
     *out = w;
+    return BLFID_OK;
+}
+
+blfid_status blfid_memory_kept(double *bytes) {
+    if (!bytes) return fail(BLFID_ERR_INVALID, "bytes is NULL");
+    *bytes = (double)dev_cache().held();
+    return BLFID_OK;
+}
+
+blfid_status blfid_memory_release(void) {
+    HIPCHK(dev_cache().release());
     return BLFID_OK;
 }
 

@@ -101,6 +101,7 @@ def lib():
         L.blfid_workspace_destroy.argtypes = [vp]
         L.blfid_workspace_destroy.restype = None
         L.blfid_plan_set_workspace.argtypes = [vp, vp]
+        L.blfid_memory_kept.argtypes = [_d]
         L.blfid_plan_set_profiling.argtypes = [vp, ctypes.c_int]
         L.blfid_plan_phase_times.argtypes = [vp, _d, _i, _d]
         L.blfid_plan_phase_bytes.argtypes = [vp, _d]
@@ -148,6 +149,19 @@ def _cm(M, N):
     if M.shape != (N, N):
         raise BlochLibError(f"operator must be {N}x{N}, got {M.shape}")
     return np.ascontiguousarray(M.ravel(order="F").view(np.float64))
+
+
+def memory_kept() -> float:
+    """Bytes of device memory kept from closed plans and states for the next ones (current device;
+    see blfid_memory_kept)."""
+    v = np.zeros(1)
+    _check(lib().blfid_memory_kept(_p(v)))
+    return float(v[0])
+
+
+def release_memory():
+    """Give the kept memory back to the device, for other allocators and processes."""
+    _check(lib().blfid_memory_release())
 
 
 class Workspace:

@@ -121,6 +121,8 @@ class FIDServer:
             raise ValueError("policy is 'srpt' (least remaining work first) or 'fifo'")
         self.hip = _hip()
         if budget_bytes is None:
+            # memory kept from closed plans is free as far as the budget is concerned
+            engine.release_memory()
             free, tot = ctypes.c_size_t(), ctypes.c_size_t()
             self.hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(tot))
             budget_bytes = 0.6 * free.value

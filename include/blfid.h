@@ -273,6 +273,16 @@ blfid_status blfid_workspace_create(double bytes, blfid_workspace **out);
 void blfid_workspace_destroy(blfid_workspace *ws);
 blfid_status blfid_plan_set_workspace(blfid_plan *plan, blfid_workspace *ws);
 
+/* Device memory kept between plans.  The blocks that destroyed plans and states give up stay with
+ * the library for the next ones, at most 4 GiB per device: allocating and freeing took most of a
+ * one-call FID.  A kept block is freed when 256 later requests have passed it over, and all of them
+ * before an allocation of this library is reported as BLFID_ERR_NOMEM.  Other allocators of the
+ * process and other processes on the device cannot make it give them back: a program that is done
+ * with its plans, or is about to measure or take the device's free memory, calls
+ * blfid_memory_release.  Both calls concern the current device and may be made from any thread. */
+blfid_status blfid_memory_kept(double *bytes);
+blfid_status blfid_memory_release(void);
+
 /* Per-kernel timing with HIP events recorded on the run's stream around every launch
  * (enable before blfid_plan_run; costs a few microseconds per launch).  Phases:
  *   0 exp (H build + propagator)   1 dyson   2 period eig   3 B = A W   4 Q/R similarity

@@ -74,8 +74,30 @@ static void workspace() {
     REQUIRE(hipGetLastError() == hipSuccess);
 }
 
+// Memory kept from destroyed plans and states is bounded, counted, and given back on request.
+static void release() {
+    fake::limit = 64 * GB;
+    double kept = -1;
+    REQUIRE(blfid_memory_kept(&kept) == BLFID_OK && kept == 0);
+    std::vector<blfid_plan *> ps;
+    for (int i = 0; i < 4; i++) {
+        ps.push_back(plan(6, 64, 512, BLFID_FP64, 400));
+        REQUIRE(blfid_plan_set_memory_budget(ps.back(), 3.0 * GB) == BLFID_OK);
+        REQUIRE(blfid_plan_run(ps.back(), 1, nullptr) == BLFID_OK);
+    }
+    for (auto *p : ps) blfid_plan_destroy(p);
+    REQUIRE(blfid_memory_kept(&kept) == BLFID_OK && kept > 0 && kept <= 4.0 * GB);
+    REQUIRE((double)fake::used == kept); // nothing else is left of the plans
+    REQUIRE(blfid_memory_release() == BLFID_OK);
+    REQUIRE(blfid_memory_kept(&kept) == BLFID_OK && kept == 0 && fake::used == 0);
+    blfid_plan *p = plan(3, 16, 64, BLFID_FP64, 10);
+    REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+    blfid_plan_destroy(p);
+    REQUIRE(blfid_memory_kept(nullptr) == BLFID_ERR_INVALID);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}};
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
     if (!fails) std::printf("OK\n");

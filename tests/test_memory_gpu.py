@@ -1,0 +1,46 @@
+"""Device memory kept from closed plans: counted, given back on request, and free as far as a
+server's default budget is concerned."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from blochlib_amd import engine, workloads
+from blochlib_amd.powder import zcw
+from blochlib_amd.serve import FIDServer
+
+pytestmark = pytest.mark.gpu
+
+
+def free_bytes():
+    L = ctypes.CDLL("libamdhip64.so")
+    f, t = ctypes.c_size_t(), ctypes.c_size_t()
+    assert L.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+    return f.value
+
+
+def one_call():
+    sy = workloads.small_cluster(5, 45)
+    f, _ = engine.powder_fid(sy, 12000.0, workloads.MAGIC_DEG, 32 * 12000.0, 130, zcw(1154),
+                             sy.op("Ix"), sy.op("Ip"))
+    return f
+
+
+def test_release_and_server_budget():
+    ref = one_call()
+    kept = engine.memory_kept()
+    assert kept > 64 << 20
+    s = FIDServer()
+    try:
+        assert engine.memory_kept() == 0
+        # the budget is 0.6 of what is free with nothing kept; 2 MiB for allocations since
+        assert s.budget >= 0.6 * (free_bytes() - (2 << 20))
+    finally:
+        s.close()
+    assert np.array_equal(one_call(), ref)
+    before, kept = free_bytes(), engine.memory_kept()
+    assert kept > 64 << 20
+    engine.release_memory()
+    assert engine.memory_kept() == 0
+    assert free_bytes() >= before + kept - (2 << 20)
+    assert np.array_equal(one_call(), ref)
