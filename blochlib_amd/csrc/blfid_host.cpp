@@ -167,33 +167,59 @@ constexpr size_t CACHE_BYTES = (size_t)4 << 30;
 constexpr unsigned long CACHE_AGE = 256;
 constexpr int CACHE_DEVICES = 64;
 
+// One device allocation.  `id` is the runtime's own number of it, unique in the process: a block
+// whose address no longer has that number went with a hipDeviceReset, and the address may be
+// another allocator's by now, so it is neither handed out nor freed (0: the runtime gave none).
+struct DevBlock {
+    void *p = nullptr;
+    size_t bytes = 0;
+    int dev = 0;
+    unsigned long long id = 0;
+    unsigned long stamp = 0;
+
+    static unsigned long long id_of(void *q) {
+        unsigned long long v = 0;
+        if (hipPointerGetAttribute(&v, HIP_POINTER_ATTRIBUTE_BUFFER_ID, (hipDeviceptr_t)q) == hipSuccess) return v;
+        (void)hipGetLastError();
+        return 0;
+    }
+    bool alive() const { return id != 0 && id_of(p) == id; }
+};
+
 class DevCache {
-    struct Blk {
-        void *p;
-        size_t bytes;
-        unsigned long stamp;
-    };
     std::mutex mu;
-    std::vector<Blk> blks[CACHE_DEVICES];
+    std::vector<DevBlock> blks[CACHE_DEVICES];
     size_t held_[CACHE_DEVICES] = {0};
     unsigned long clock[CACHE_DEVICES] = {0};
 
-    // takes every block older than `age` requests out of the list (the caller frees them)
-    void expire(int dev, unsigned long age, std::vector<void *> &out) {
+    static bool in_range(int dev) { return dev >= 0 && dev < CACHE_DEVICES; }
+    // takes block i out of the list
+    DevBlock take(int dev, size_t i) {
         auto &v = blks[dev];
-        for (size_t i = 0; i < v.size();) {
-            if (clock[dev] - v[i].stamp >= age) {
-                out.push_back(v[i].p);
-                held_[dev] -= v[i].bytes;
-                v[i] = v.back();
-                v.pop_back();
-            } else {
-                i++;
-            }
+        const DevBlock b = v[i];
+        held_[dev] -= b.bytes;
+        v[i] = v.back();
+        v.pop_back();
+        return b;
+    }
+    // takes every block older than `age` requests out of the list (the caller frees them)
+    void expire(int dev, unsigned long age, std::vector<DevBlock> &out) {
+        for (size_t i = 0; i < blks[dev].size();) {
+            if (clock[dev] - blks[dev][i].stamp >= age) out.push_back(take(dev, i));
+            else i++;
         }
     }
-    static void free_all(const std::vector<void *> &v) {
-        for (void *q : v) (void)hipFree(q);
+    static void free_all(const std::vector<DevBlock> &v) {
+        for (const DevBlock &b : v)
+            if (b.id == 0 || b.alive()) (void)hipFree(b.p);
+    }
+    void free_held(int dev) {
+        std::vector<DevBlock> old;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            expire(dev, 0, old);
+        }
+        free_all(old);
     }
 
   public:
@@ -201,14 +227,9 @@ class DevCache {
     // freed and the allocation tried once more.
     hipError_t raw(size_t bytes, void **p, int dev) {
         hipError_t e = hipMalloc(p, bytes);
-        if (e == hipErrorOutOfMemory && dev >= 0 && dev < CACHE_DEVICES) {
+        if (e == hipErrorOutOfMemory && in_range(dev)) {
             (void)hipGetLastError();
-            std::vector<void *> old;
-            {
-                std::lock_guard<std::mutex> lk(mu);
-                expire(dev, 0, old);
-            }
-            free_all(old);
+            free_held(dev);
             e = hipMalloc(p, bytes);
         }
         if (e != hipSuccess) {
@@ -217,70 +238,69 @@ class DevCache {
         }
         return e;
     }
-    // At least `bytes` on the current device; *cap receives the block's size, *dev the device.
-    hipError_t get(size_t bytes, void **p, size_t *cap, int *dev) {
-        *p = nullptr;
-        hipError_t e = hipGetDevice(dev);
+    // A block of at least `bytes` on the current device.
+    hipError_t get(size_t bytes, DevBlock &out) {
+        out = DevBlock();
+        hipError_t e = hipGetDevice(&out.dev);
         if (e != hipSuccess) return e;
-        const bool kept = *dev >= 0 && *dev < CACHE_DEVICES;
+        const int dev = out.dev;
         // sizes in steps of 64 KiB, 2 MiB from 1 MiB up, so that like requests share blocks
         const size_t step = bytes < ((size_t)1 << 20) ? (size_t)1 << 16 : (size_t)1 << 21;
         const size_t want = (bytes + step - 1) / step * step;
         const size_t most = want < ((size_t)64 << 20) ? 2 * want : want + want / 8;
-        if (kept) {
-            std::vector<void *> old;
-            {
+        if (in_range(dev)) {
+            std::vector<DevBlock> old;
+            DevBlock hit;
+            do {
                 std::lock_guard<std::mutex> lk(mu);
-                clock[*dev]++;
-                auto &v = blks[*dev];
+                if (!hit.p) clock[dev]++;
+                hit = DevBlock();
+                auto &v = blks[dev];
                 size_t best = v.size();
                 for (size_t i = 0; i < v.size(); i++)
                     if (v[i].bytes >= bytes && v[i].bytes <= most &&
                         (best == v.size() || v[i].bytes < v[best].bytes))
                         best = i;
-                if (best < v.size()) {
-                    *p = v[best].p;
-                    *cap = v[best].bytes;
-                    held_[*dev] -= v[best].bytes;
-                    v[best] = v.back();
-                    v.pop_back();
-                }
-                expire(*dev, CACHE_AGE, old);
-            }
+                if (best < v.size()) hit = take(dev, best);
+                expire(dev, CACHE_AGE, old);
+            } while (hit.p && !hit.alive());
             free_all(old);
-            if (*p) return hipSuccess;
+            if (hit.p) {
+                out = hit;
+                return hipSuccess;
+            }
         }
-        *cap = want;
-        e = raw(want, p, *dev);
+        out.bytes = want;
+        e = raw(want, &out.p, dev);
         if (e == hipErrorOutOfMemory && want > bytes) {
-            *cap = bytes;
-            e = raw(bytes, p, *dev);
+            out.bytes = bytes;
+            e = raw(bytes, &out.p, dev);
         }
+        if (e == hipSuccess) out.id = DevBlock::id_of(out.p);
         return e;
     }
     // A block no work uses any more: the device is waited for first.
-    void put(void *p, size_t cap, int dev) {
+    void put(DevBlock b) {
+        const int dev = b.dev;
         int cur = dev;
         (void)hipGetDevice(&cur);
         if (cur != dev) (void)hipSetDevice(dev);
         const bool idle = hipDeviceSynchronize() == hipSuccess;
-        std::vector<void *> old;
-        if (idle && dev >= 0 && dev < CACHE_DEVICES && cap <= CACHE_BYTES) {
+        std::vector<DevBlock> old;
+        if (idle && in_range(dev) && b.bytes <= CACHE_BYTES && b.id != 0) {
             std::lock_guard<std::mutex> lk(mu);
             auto &v = blks[dev];
-            v.push_back({p, cap, clock[dev]});
-            held_[dev] += cap;
+            b.stamp = clock[dev];
+            v.push_back(b);
+            held_[dev] += b.bytes;
             while (held_[dev] > CACHE_BYTES) { // the longest unused block goes first
                 size_t o = 0;
                 for (size_t i = 1; i < v.size(); i++)
                     if (v[i].stamp < v[o].stamp) o = i;
-                old.push_back(v[o].p);
-                held_[dev] -= v[o].bytes;
-                v[o] = v.back();
-                v.pop_back();
+                old.push_back(take(dev, o));
             }
         } else {
-            old.push_back(p);
+            old.push_back(b);
         }
         free_all(old);
         if (cur != dev) (void)hipSetDevice(cur);
@@ -289,19 +309,13 @@ class DevCache {
     hipError_t release() {
         int dev = -1;
         const hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess || dev < 0 || dev >= CACHE_DEVICES) return e;
-        std::vector<void *> old;
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            expire(dev, 0, old);
-        }
-        free_all(old);
-        return hipSuccess;
+        if (e == hipSuccess && in_range(dev)) free_held(dev);
+        return e;
     }
     // Bytes held for the current device: free memory as far as a memory budget is concerned.
     size_t held() {
         int dev = -1;
-        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= CACHE_DEVICES) return 0;
+        if (hipGetDevice(&dev) != hipSuccess || !in_range(dev)) return 0;
         std::lock_guard<std::mutex> lk(mu);
         return held_[dev];
     }
@@ -314,9 +328,8 @@ DevCache &dev_cache() {
 
 template <typename T> struct DevBuf {
     T *p = nullptr;
-    size_t n = 0;   // elements asked for
-    size_t cap = 0; // bytes of the block
-    int dev = 0;
+    size_t n = 0; // elements asked for
+    DevBlock blk;
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
@@ -325,15 +338,17 @@ template <typename T> struct DevBuf {
         if (cnt <= n && p) return hipSuccess;
         release();
         if (cnt == 0) return hipSuccess;
-        const hipError_t e = dev_cache().get(cnt * sizeof(T), (void **)&p, &cap, &dev);
-        if (e == hipSuccess) n = cnt;
+        const hipError_t e = dev_cache().get(cnt * sizeof(T), blk);
+        if (e == hipSuccess) {
+            p = (T *)blk.p;
+            n = cnt;
+        }
         return e;
     }
     void release() {
-        if (p) dev_cache().put(p, cap, dev);
+        if (p) dev_cache().put(blk);
         p = nullptr;
         n = 0;
-        cap = 0;
     }
 };
 

@@ -96,8 +96,30 @@ static void release() {
     REQUIRE(blfid_memory_kept(nullptr) == BLFID_ERR_INVALID);
 }
 
+// Kept blocks that went with a hipDeviceReset are neither handed out nor freed: their addresses
+// belong to whoever allocated since.
+static void reset() {
+    blfid_plan_destroy(plan(4, 32, 128, BLFID_FP64, 50));
+    REQUIRE(fake::used > 0);
+    std::map<size_t, size_t> was;
+    for (auto &kv : fake::mem) was[kv.first] = kv.second.bytes;
+    fake::reset();
+    // another allocator takes the same addresses in the same sizes
+    std::vector<void *> other(was.size());
+    size_t i = 0;
+    for (auto &kv : was) REQUIRE(hipMalloc(&other[i++], kv.second) == hipSuccess);
+    const auto theirs = fake::mem;
+    blfid_plan *p = plan(4, 32, 128, BLFID_FP64, 50);
+    REQUIRE(fake::mem.size() > theirs.size()); // blocks of its own
+    blfid_plan_destroy(p);
+    REQUIRE(blfid_memory_release() == BLFID_OK);
+    REQUIRE(fake::mem.size() == theirs.size());
+    for (auto &kv : theirs) REQUIRE(fake::mem.count(kv.first) && fake::mem[kv.first].id == kv.second.id);
+    REQUIRE(hipGetLastError() == hipSuccess);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}};
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
     if (!fails) std::printf("OK\n");
