@@ -238,16 +238,16 @@ class DevCache {
         }
         return e;
     }
-    // A block of at least `bytes` on the current device.
-    hipError_t get(size_t bytes, DevBlock &out) {
+    // A block of at least `bytes` on the current device, and of at most `limit` (a memory budget).
+    hipError_t get(size_t bytes, size_t limit, DevBlock &out) {
         out = DevBlock();
         hipError_t e = hipGetDevice(&out.dev);
         if (e != hipSuccess) return e;
         const int dev = out.dev;
         // sizes in steps of 64 KiB, 2 MiB from 1 MiB up, so that like requests share blocks
         const size_t step = bytes < ((size_t)1 << 20) ? (size_t)1 << 16 : (size_t)1 << 21;
-        const size_t want = (bytes + step - 1) / step * step;
-        const size_t most = want < ((size_t)64 << 20) ? 2 * want : want + want / 8;
+        const size_t want = std::max(bytes, std::min(limit, (bytes + step - 1) / step * step));
+        const size_t most = std::min(limit, want < ((size_t)64 << 20) ? 2 * want : want + want / 8);
         if (in_range(dev)) {
             std::vector<DevBlock> old;
             DevBlock hit;
@@ -334,11 +334,11 @@ template <typename T> struct DevBuf {
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { release(); }
-    hipError_t alloc(size_t cnt) {
+    hipError_t alloc(size_t cnt, size_t limit = SIZE_MAX) {
         if (cnt <= n && p) return hipSuccess;
         release();
         if (cnt == 0) return hipSuccess;
-        const hipError_t e = dev_cache().get(cnt * sizeof(T), blk);
+        const hipError_t e = dev_cache().get(cnt * sizeof(T), limit, blk);
         if (e == hipSuccess) {
             p = (T *)blk.p;
             n = cnt;
@@ -2028,7 +2028,7 @@ static blfid_status run_upto(blfid_plan *pl, int normalize, hipStream_t st, int 
         base = pl->ws->base;
         if (pl->ws->used && pl->ws->last != st) HIPCHK(hipStreamWaitEvent(st, pl->ws->ev, 0));
     } else {
-        HIPCHK(pl->own_ws.alloc(need));
+        HIPCHK(pl->own_ws.alloc(need, (size_t)avail));
         base = pl->own_ws.p;
     }
     HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
@@ -2198,7 +2198,7 @@ blfid_status blfid_state_apply(blfid_state *st, const blfid_system *sys, double 
         else hi = mid - 1;
     }
     const long Kb = lo;
-    HIPCHK(st->ws.alloc(need(Kb)));
+    HIPCHK(st->ws.alloc(need(Kb), (size_t)avail));
     size_t poff[blfid_layout::R_COUNT];
     const size_t pbytes = blfid_layout::align256(blfid_layout::layout_bytes(ps, Kb, poff));
     carve(pp.get(), st->ws.p, poff);
@@ -2303,7 +2303,7 @@ blfid_status blfid_plan_graph_capture(blfid_plan *pl, int normalize) {
     if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
     size_t off[blfid_layout::R_COUNT];
     const size_t need = blfid_layout::layout_bytes(sh, Kb, off);
-    HIPCHK(pl->own_ws.alloc(need));
+    HIPCHK(pl->own_ws.alloc(need, (size_t)avail));
     HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
     if (pl->gexec) (void)hipGraphExecDestroy(pl->gexec);
     if (pl->graph) (void)hipGraphDestroy(pl->graph);
@@ -2371,7 +2371,7 @@ blfid_status blfid_plan_run_slice(blfid_plan *pl, int c_begin, int c_end, int no
         }
         const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
         if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
-        HIPCHK(pl->own_ws.alloc(blfid_layout::layout_bytes(sh, Kb)));
+        HIPCHK(pl->own_ws.alloc(blfid_layout::layout_bytes(sh, Kb), (size_t)avail));
         HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
         pl->sl_Kb = Kb;
         pl->sl_gen = pl->gen;

@@ -118,8 +118,44 @@ static void reset() {
     REQUIRE(hipGetLastError() == hipSuccess);
 }
 
+// A plan's and a state's working storage stay within their memory budgets, whichever block they
+// come from: a kept one that is larger, or a new one whose size would be rounded up.
+static void budget() {
+    blfid_plan *p = plan(5, 64, 256, BLFID_FP64, 300);
+    REQUIRE(blfid_plan_set_memory_budget(p, 400.0 * MB) == BLFID_OK);
+    REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+    blfid_plan_destroy(p); // keeps about 400 MB
+    p = plan(5, 64, 256, BLFID_FP64, 300);
+    for (double b : {390.0 * MB, 380.0 * MB + 4097, 300.0 * MB + 12345}) {
+        p->own_ws.release();
+        REQUIRE(blfid_plan_set_memory_budget(p, b) == BLFID_OK);
+        REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+        REQUIRE((double)p->own_ws.blk.bytes <= b);
+        REQUIRE(fake::mem.at((size_t)p->own_ws.p).bytes <= b);
+        p->own_ws.release();
+        REQUIRE(blfid_plan_run_slice(p, 0, 300, 1, nullptr) == BLFID_OK);
+        REQUIRE((double)p->own_ws.blk.bytes <= b);
+        p->own_ws.release();
+        REQUIRE(blfid_plan_graph_capture(p, 1) == BLFID_OK);
+        REQUIRE((double)p->own_ws.blk.bytes <= b);
+    }
+    blfid_plan_destroy(p);
+    Sys sy(5);
+    std::vector<double> a(300, 0.3), dt(4, 1e-6);
+    blfid_state *st = nullptr;
+    REQUIRE(blfid_state_create(5, 300, a.data(), a.data(), a.data(), a.data(), &st) == BLFID_OK);
+    for (double b : {3.0 * MB, 1.0 * MB + 300}) {
+        st->ws.release();
+        REQUIRE(blfid_state_set_memory_budget(st, b) == BLFID_OK);
+        REQUIRE(blfid_state_apply(st, &sy.s, 10000.0, 54.7, 4, nullptr, dt.data(), 0, nullptr, 1, nullptr) == BLFID_OK);
+        REQUIRE(fake::mem.at((size_t)st->ws.p).bytes <= b);
+    }
+    blfid_state_destroy(st);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}};
+    std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
     if (!fails) std::printf("OK\n");
