@@ -160,7 +160,7 @@ void crystal_tensor(double pxx, double pyy, double pzz, double a, double b, doub
 // took most of a one-call FID (a 5-spin pulse program's 10 ms of kernels sat in a 105 ms call, and
 // every table had its own allocation).  Per device at most CACHE_BYTES are held, in blocks a
 // request may take when it fills half of one (8/9 from 64 MiB up); a block that CACHE_AGE requests have passed
-// over is freed, and everything held is freed before an allocation is reported as failed.  A block
+// over is freed by the next release, and everything held is freed before an allocation is reported as failed.  A block
 // enters the cache only when the device has finished all work (as hipFree waits for it), so it may
 // be handed to any thread and stream.
 constexpr size_t CACHE_BYTES = (size_t)4 << 30;
@@ -249,7 +249,6 @@ class DevCache {
         const size_t want = std::max(bytes, std::min(limit, (bytes + step - 1) / step * step));
         const size_t most = std::min(limit, want < ((size_t)64 << 20) ? 2 * want : want + want / 8);
         if (in_range(dev)) {
-            std::vector<DevBlock> old;
             DevBlock hit;
             do {
                 std::lock_guard<std::mutex> lk(mu);
@@ -262,9 +261,7 @@ class DevCache {
                         (best == v.size() || v[i].bytes < v[best].bytes))
                         best = i;
                 if (best < v.size()) hit = take(dev, best);
-                expire(dev, CACHE_AGE, old);
             } while (hit.p && !hit.alive());
-            free_all(old);
             if (hit.p) {
                 out = hit;
                 return hipSuccess;
@@ -279,7 +276,9 @@ class DevCache {
         if (e == hipSuccess) out.id = DevBlock::id_of(out.p);
         return e;
     }
-    // A block no work uses any more: the device is waited for first.
+    // A block no work uses any more: the device is waited for first.  What has grown old is freed
+    // here, where that waits for nothing, and not by a request: freeing waits for all work on the
+    // device, and a plan may be set up while others run.
     void put(DevBlock b) {
         const int dev = b.dev;
         int cur = dev;
@@ -287,12 +286,17 @@ class DevCache {
         if (cur != dev) (void)hipSetDevice(dev);
         const bool idle = hipDeviceSynchronize() == hipSuccess;
         std::vector<DevBlock> old;
-        if (idle && in_range(dev) && b.bytes <= CACHE_BYTES && b.id != 0) {
+        if (in_range(dev)) {
             std::lock_guard<std::mutex> lk(mu);
             auto &v = blks[dev];
-            b.stamp = clock[dev];
-            v.push_back(b);
-            held_[dev] += b.bytes;
+            if (idle && b.bytes <= CACHE_BYTES && b.id != 0) {
+                b.stamp = clock[dev];
+                v.push_back(b);
+                held_[dev] += b.bytes;
+            } else {
+                old.push_back(b);
+            }
+            expire(dev, CACHE_AGE, old);
             while (held_[dev] > CACHE_BYTES) { // the longest unused block goes first
                 size_t o = 0;
                 for (size_t i = 1; i < v.size(); i++)

@@ -153,8 +153,28 @@ static void budget() {
     blfid_state_destroy(st);
 }
 
+// Setting up plans never frees memory (which waits for all work on the device): blocks that 256
+// requests have passed over go with the next released plan.
+static void age() {
+    blfid_plan_destroy(plan(6, 64, 512, BLFID_FP64, 400));
+    blfid_plan *big = plan(6, 64, 512, BLFID_FP64, 400);
+    REQUIRE(blfid_plan_run(big, 1, nullptr) == BLFID_OK);
+    blfid_plan_destroy(big);
+    double kept = 0, now = 0;
+    REQUIRE(blfid_memory_kept(&kept) == BLFID_OK && kept > 0);
+    const long freed = fake::n_free, waits = fake::n_sync;
+    std::vector<blfid_plan *> ps;
+    for (int i = 0; i < 120; i++) ps.push_back(plan(2, 16, 64, BLFID_FP64, 10)); // three requests each
+    REQUIRE(fake::n_free == freed && fake::n_sync == waits);
+    blfid_plan_destroy(ps.back());
+    ps.pop_back();
+    REQUIRE(fake::n_free > freed);
+    REQUIRE(blfid_memory_kept(&now) == BLFID_OK && now < kept / 10);
+    for (auto *p : ps) blfid_plan_destroy(p);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}};
     std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();

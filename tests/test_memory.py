@@ -7,7 +7,7 @@ import subprocess
 import pytest
 
 CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
-CHECKS = ["workspace", "release", "reset", "budget"]
+CHECKS = ["workspace", "release", "reset", "budget", "age"]
 
 
 @pytest.fixture(scope="module")
