@@ -165,7 +165,7 @@ void crystal_tensor(double pxx, double pyy, double pzz, double a, double b, doub
 // be handed to any thread and stream.
 constexpr size_t CACHE_BYTES = (size_t)4 << 30;
 constexpr unsigned long CACHE_AGE = 256;
-constexpr int CACHE_DEVICES = 64;
+constexpr int CACHE_DEVICES = 64, CACHE_BLOCKS = 512;
 
 // One device allocation.  `id` is the runtime's own number of it, unique in the process: a block
 // whose address no longer has that number went with a hipDeviceReset, and the address may be
@@ -187,39 +187,43 @@ struct DevBlock {
 };
 
 class DevCache {
+    // plain arrays: releasing a block happens in destructors and must not throw
+    struct Kept {
+        DevBlock blk[CACHE_BLOCKS];
+        int n = 0;
+        size_t bytes = 0;
+        unsigned long clock = 0; // requests so far
+    };
     std::mutex mu;
-    std::vector<DevBlock> blks[CACHE_DEVICES];
-    size_t held_[CACHE_DEVICES] = {0};
-    unsigned long clock[CACHE_DEVICES] = {0};
+    Kept dev_[CACHE_DEVICES];
 
     static bool in_range(int dev) { return dev >= 0 && dev < CACHE_DEVICES; }
     // takes block i out of the list
-    DevBlock take(int dev, size_t i) {
-        auto &v = blks[dev];
-        const DevBlock b = v[i];
-        held_[dev] -= b.bytes;
-        v[i] = v.back();
-        v.pop_back();
+    static DevBlock take(Kept &k, int i) {
+        const DevBlock b = k.blk[i];
+        k.bytes -= b.bytes;
+        k.blk[i] = k.blk[--k.n];
         return b;
     }
-    // takes every block older than `age` requests out of the list (the caller frees them)
-    void expire(int dev, unsigned long age, std::vector<DevBlock> &out) {
-        for (size_t i = 0; i < blks[dev].size();) {
-            if (clock[dev] - blks[dev][i].stamp >= age) out.push_back(take(dev, i));
-            else i++;
-        }
+    static void free_block(const DevBlock &b) {
+        if (b.id == 0 || b.alive()) (void)hipFree(b.p);
     }
-    static void free_all(const std::vector<DevBlock> &v) {
-        for (const DevBlock &b : v)
-            if (b.id == 0 || b.alive()) (void)hipFree(b.p);
-    }
-    void free_held(int dev) {
-        std::vector<DevBlock> old;
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            expire(dev, 0, old);
+    // Frees the blocks that `age` requests have passed over, and the longest unused ones of those
+    // left while they hold more than `most` bytes.
+    void trim(int dev, unsigned long age, size_t most) {
+        Kept &k = dev_[dev];
+        for (;;) {
+            DevBlock b;
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                int o = 0;
+                for (int i = 1; i < k.n; i++)
+                    if (k.blk[i].stamp < k.blk[o].stamp) o = i;
+                if (k.n == 0 || (k.clock - k.blk[o].stamp < age && k.bytes <= most)) return;
+                b = take(k, o);
+            }
+            free_block(b);
         }
-        free_all(old);
     }
 
   public:
@@ -229,7 +233,7 @@ class DevCache {
         hipError_t e = hipMalloc(p, bytes);
         if (e == hipErrorOutOfMemory && in_range(dev)) {
             (void)hipGetLastError();
-            free_held(dev);
+            trim(dev, 0, 0);
             e = hipMalloc(p, bytes);
         }
         if (e != hipSuccess) {
@@ -249,18 +253,18 @@ class DevCache {
         const size_t want = std::max(bytes, std::min(limit, (bytes + step - 1) / step * step));
         const size_t most = std::min(limit, want < ((size_t)64 << 20) ? 2 * want : want + want / 8);
         if (in_range(dev)) {
+            Kept &k = dev_[dev];
             DevBlock hit;
             do {
                 std::lock_guard<std::mutex> lk(mu);
-                if (!hit.p) clock[dev]++;
+                if (!hit.p) k.clock++;
                 hit = DevBlock();
-                auto &v = blks[dev];
-                size_t best = v.size();
-                for (size_t i = 0; i < v.size(); i++)
-                    if (v[i].bytes >= bytes && v[i].bytes <= most &&
-                        (best == v.size() || v[i].bytes < v[best].bytes))
+                int best = -1;
+                for (int i = 0; i < k.n; i++)
+                    if (k.blk[i].bytes >= bytes && k.blk[i].bytes <= most &&
+                        (best < 0 || k.blk[i].bytes < k.blk[best].bytes))
                         best = i;
-                if (best < v.size()) hit = take(dev, best);
+                if (best >= 0) hit = take(k, best);
             } while (hit.p && !hit.alive());
             if (hit.p) {
                 out = hit;
@@ -284,36 +288,26 @@ class DevCache {
         int cur = dev;
         (void)hipGetDevice(&cur);
         if (cur != dev) (void)hipSetDevice(dev);
-        const bool idle = hipDeviceSynchronize() == hipSuccess;
-        std::vector<DevBlock> old;
-        if (in_range(dev)) {
+        bool keep = hipDeviceSynchronize() == hipSuccess && in_range(dev) && b.id != 0 && b.bytes <= CACHE_BYTES;
+        if (keep) {
             std::lock_guard<std::mutex> lk(mu);
-            auto &v = blks[dev];
-            if (idle && b.bytes <= CACHE_BYTES && b.id != 0) {
-                b.stamp = clock[dev];
-                v.push_back(b);
-                held_[dev] += b.bytes;
-            } else {
-                old.push_back(b);
+            Kept &k = dev_[dev];
+            keep = k.n < CACHE_BLOCKS;
+            if (keep) {
+                b.stamp = k.clock;
+                k.bytes += b.bytes;
+                k.blk[k.n++] = b;
             }
-            expire(dev, CACHE_AGE, old);
-            while (held_[dev] > CACHE_BYTES) { // the longest unused block goes first
-                size_t o = 0;
-                for (size_t i = 1; i < v.size(); i++)
-                    if (v[i].stamp < v[o].stamp) o = i;
-                old.push_back(take(dev, o));
-            }
-        } else {
-            old.push_back(b);
         }
-        free_all(old);
+        if (!keep) free_block(b);
+        if (in_range(dev)) trim(dev, CACHE_AGE, CACHE_BYTES);
         if (cur != dev) (void)hipSetDevice(cur);
     }
     // Frees everything held for the current device.
     hipError_t release() {
         int dev = -1;
         const hipError_t e = hipGetDevice(&dev);
-        if (e == hipSuccess && in_range(dev)) free_held(dev);
+        if (e == hipSuccess && in_range(dev)) trim(dev, 0, 0);
         return e;
     }
     // Bytes held for the current device: free memory as far as a memory budget is concerned.
@@ -321,7 +315,7 @@ class DevCache {
         int dev = -1;
         if (hipGetDevice(&dev) != hipSuccess || !in_range(dev)) return 0;
         std::lock_guard<std::mutex> lk(mu);
-        return held_[dev];
+        return dev_[dev].bytes;
     }
 };
 // never destroyed: objects released while the process ends must not outlive it

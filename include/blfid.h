@@ -276,11 +276,11 @@ blfid_status blfid_plan_set_workspace(blfid_plan *plan, blfid_workspace *ws);
 /* Device memory kept between plans.  The blocks that destroyed plans and states give up stay with
  * the library for the next ones, at most 4 GiB per device: allocating and freeing took most of a
  * one-call FID.  A kept block that 256 later requests have passed over is freed by the next plan or
- * state destroyed, and all of them
- * before an allocation of this library is reported as BLFID_ERR_NOMEM.  Other allocators of the
- * process and other processes on the device cannot make it give them back: a program that is done
- * with its plans, or is about to measure or take the device's free memory, calls
- * blfid_memory_release.  Both calls concern the current device and may be made from any thread. */
+ * state destroyed, and all of them before an allocation of this library is reported as
+ * BLFID_ERR_NOMEM.  Other allocators of the process and other processes on the device cannot make
+ * it give them back: a program that is done with its plans, or is about to measure or take the
+ * device's free memory, calls blfid_memory_release.  Both calls concern the current device and may
+ * be made from any thread. */
 blfid_status blfid_memory_kept(double *bytes);
 blfid_status blfid_memory_release(void);
 

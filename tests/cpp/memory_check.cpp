@@ -7,6 +7,16 @@
 #include <functional>
 
 static int fails = 0;
+
+// host allocations fail while this is set
+static bool no_host_memory = false;
+void *operator new(size_t n) {
+    void *p = no_host_memory ? nullptr : std::malloc(n);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 #define REQUIRE(c)                                                                               \
     do {                                                                                         \
         if (!(c)) {                                                                              \
@@ -173,8 +183,19 @@ static void age() {
     for (auto *p : ps) blfid_plan_destroy(p);
 }
 
+// Releasing plans takes no host memory (a destructor that threw would end the process).
+static void host_memory() {
+    blfid_plan *p = plan(4, 32, 128, BLFID_FP64, 50);
+    REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+    no_host_memory = true;
+    blfid_plan_destroy(p);
+    const blfid_status st = blfid_memory_release();
+    no_host_memory = false;
+    REQUIRE(st == BLFID_OK && fake::used == 0);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}};
     std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
