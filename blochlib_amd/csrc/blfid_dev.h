@@ -109,10 +109,6 @@ inline long tuned_cap(const DevPlan *P, int fam, int M) {
 #define CORR_PPT 8
 #define CORR_SEG_CHUNKS 64
 #define CORR_SEG_MIN 8
-__device__ __host__ inline int corr_seg_chunks(int nchunk) {
-    const int c = (nchunk + CORR_SEG_MIN - 1) / CORR_SEG_MIN;
-    return c < 4 ? 4 : c > CORR_SEG_CHUNKS ? CORR_SEG_CHUNKS : c;
-}
 // log2 of the transform length of the FFT variant, or 0 where the direct sum is taken.  A power of
 // two from 16 to 512 is transformed at its own length; any other n from CORR_PAD_MIN to 256 is
 // zero-padded to the power of two L >= 2 n, whose cyclic correlation holds the linear one, folded
@@ -128,24 +124,40 @@ __host__ __device__ inline int corr_fft_ln(int n) {
     return ln;
 }
 __host__ __device__ inline bool corr_use_fft(int n) { return corr_fft_ln(n) > 0; }
-// elements per chunk: the FFT variant fills CORR_SPAN points
-__device__ __host__ inline int corr_chunk(int n) {
-    const int ln = corr_fft_ln(n);
-    if (ln > 0) return CORR_SPAN >> ln;
+// elements per chunk of the direct sum
+__device__ __host__ inline int corr_direct_chunk(int n) {
     int npg = (n + CORR_PPT - 1) / CORR_PPT;
     int a = CORR_SPAN / n, b = 256 / npg;
     int ch = a < b ? a : b;
     return ch < 1 ? 1 : ch;
 }
-__device__ __host__ inline int corr_range_segments(int nchunk) {
+// elements per chunk: the FFT variant fills CORR_SPAN points
+__device__ __host__ inline int corr_chunk(int n) {
+    const int ln = corr_fft_ln(n);
+    return ln > 0 ? CORR_SPAN >> ln : corr_direct_chunk(n);
+}
+// Chunks per segment: about CORR_SEG_MIN segments (a few crystallites fill the device), of up to
+// CORR_SEG_CHUNKS chunks.  A crystallite's partial sums of npts points take CORR_PART_BYTES at
+// most (FIDs beyond 30000 points) as long as a segment then stays within CORR_SEG_CHUNKS chunks of
+// the direct sum's elements: longer segments would hold a batch to fewer, longer tasks, and a
+// million-point FID took eight times the storage of its results per crystallite.
+#define CORR_PART_BYTES (4 << 20)
+__device__ __host__ inline int corr_seg_chunks(int n, int npts, int nchunk) {
+    int c = (nchunk + CORR_SEG_MIN - 1) / CORR_SEG_MIN;
+    c = c < 4 ? 4 : c > CORR_SEG_CHUNKS ? CORR_SEG_CHUNKS : c;
+    const int most = CORR_SEG_CHUNKS * corr_direct_chunk(n) / corr_chunk(n);
+    while (c < most && (double)((nchunk + c - 1) / c) * npts * 16.0 > CORR_PART_BYTES) c = c < most / 2 ? 2 * c : most;
+    return c;
+}
+__device__ __host__ inline int corr_range_segments(int n, int npts, int nchunk) {
     if (nchunk <= 0) return 0;
-    const int spc = corr_seg_chunks(nchunk);
+    const int spc = corr_seg_chunks(n, npts, nchunk);
     return (nchunk + spc - 1) / spc;
 }
 // FID partial sums of a correlation: the segments of the autocorrelation chunks [0, A) and of
 // the general chunks [A, nchunk), each range segmented on its own
-__device__ __host__ inline int corr_segments(int n, long Etot, int auto_chunks = 0) {
+__device__ __host__ inline int corr_segments(int n, int npts, long Ecorr, int auto_chunks = 0) {
     const int CH = corr_chunk(n);
-    const int nchunk = (int)((Etot + CH - 1) / CH);
-    return corr_range_segments(auto_chunks) + corr_range_segments(nchunk - auto_chunks);
+    const int nchunk = (int)((Ecorr + CH - 1) / CH);
+    return corr_range_segments(n, npts, auto_chunks) + corr_range_segments(n, npts, nchunk - auto_chunks);
 }

@@ -531,6 +531,7 @@ struct blfid_plan {
     // generation and working storage of the slices so far
     int sl_next = -1, sl_norm = 1;
     long sl_Kb = 0;
+    int sl_cuts = 0;
     unsigned long sl_gen = 0;
     char *sl_base = nullptr;
     ~blfid_plan() {
@@ -1449,7 +1450,7 @@ blfid_status blfid_plan_set_operators(blfid_plan *pl, const double *rho_d, const
         pl->corr_auto = !pl->rt_from_q ? 0 : !pl->rt_rev ? nchunk : (int)(first_rev / CH);
     }
     if (pl->spinning && !pl->ptop)
-        pl->nparts = nc > 0 ? corr_segments(pl->n, nc, corr_use_fft(pl->n) ? pl->corr_auto : 0) : 1;
+        pl->nparts = nc > 0 ? corr_segments(pl->n, pl->npts, nc, corr_use_fft(pl->n) ? pl->corr_auto : 0) : 1;
     else
         pl->nparts = std::max<int>(1, (int)pl->pairs.size());
     Tables t;
@@ -2015,7 +2016,7 @@ static blfid_status run_upto(blfid_plan *pl, int normalize, hipStream_t st, int 
             avail = 0.4 * (double)(fre + pl->own_ws.n + dev_cache().held());
         }
     }
-    const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
+    const long Kb = blfid_layout::fit_batch(sh, psh, pl->K, avail);
     if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
     size_t off[blfid_layout::R_COUNT];
     const size_t need = blfid_layout::layout_bytes(sh, Kb, off);
@@ -2297,7 +2298,7 @@ blfid_status blfid_plan_graph_capture(blfid_plan *pl, int normalize) {
         HIPCHK(hipMemGetInfo(&fre, &tot));
         avail = 0.4 * (double)(fre + pl->own_ws.n + dev_cache().held());
     }
-    const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
+    const long Kb = blfid_layout::fit_batch(sh, psh, pl->K, avail);
     if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
     size_t off[blfid_layout::R_COUNT];
     const size_t need = blfid_layout::layout_bytes(sh, Kb, off);
@@ -2367,7 +2368,7 @@ blfid_status blfid_plan_run_slice(blfid_plan *pl, int c_begin, int c_end, int no
             HIPCHK(hipMemGetInfo(&fre, &tot));
             avail = 0.4 * (double)(fre + pl->own_ws.n + dev_cache().held());
         }
-        const long Kb = blfid_layout::choose_batch(sh, pl->K, avail);
+        const long Kb = blfid_layout::fit_batch(sh, psh, pl->K, avail, &pl->sl_cuts);
         if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
         HIPCHK(pl->own_ws.alloc(blfid_layout::layout_bytes(sh, Kb), (size_t)avail));
         HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
@@ -2381,6 +2382,7 @@ blfid_status blfid_plan_run_slice(blfid_plan *pl, int c_begin, int c_end, int no
     }
     blfid_layout::Shape sh, psh;
     full_shape(pl, sh, psh);
+    for (int c = 0; c < pl->sl_cuts; c++) (void)blfid_layout::fewer_slots(sh, psh);
     size_t off[blfid_layout::R_COUNT];
     (void)blfid_layout::layout_bytes(sh, pl->sl_Kb, off);
     pl->last_stream = st;
@@ -2457,7 +2459,7 @@ blfid_status blfid_plan_run_noalloc(blfid_plan *pl, int normalize, double *fid_o
     if (s != BLFID_OK) return s;
     blfid_layout::Shape sh, psh;
     noalloc_shape(pl, sh, psh);
-    const long Kb = blfid_layout::choose_batch(sh, pl->K, (double)BLFID_NOALLOC_SCRATCH_BYTES);
+    const long Kb = blfid_layout::fit_batch(sh, psh, pl->K, (double)BLFID_NOALLOC_SCRATCH_BYTES);
     if (Kb < 1)
         return fail(BLFID_ERR_NOMEM,
                     "one crystallite of this plan needs " +

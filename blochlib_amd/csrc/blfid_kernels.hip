@@ -3743,7 +3743,7 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
     // only (not on the batch), so a crystallite's FID is summed in the same grouping whatever
     // the batch size.  The segment's FID partial sums (t = tid + 256 m) stay in registers and
     // are stored once at the segment's end (hold), or accumulated in part[] per chunk.
-    const int spc = corr_seg_chunks(nchunk);
+    const int spc = corr_seg_chunks(n, P.npts, nchunk);
     const int nsg = (nchunk + spc - 1) / spc;
     const long ntask = (long)Kb * nsg;
     // FFT variant: with J = ceil(npts / n) periods, z_e^t = z_e^p (z_e^n)^j for t = p + n j, so
@@ -4908,7 +4908,7 @@ static void launch_corr_t(bool autoc, const DevPlan *P, int Kb, const void *Qt, 
                           const double *thetas, double *part, int lo, int hi, int seg_base,
                           hipStream_t st) {
     typedef typename CX<R>::T CT;
-    const long ntask = (long)Kb * corr_range_segments(hi - lo);
+    const long ntask = (long)Kb * corr_range_segments(P->n, P->npts, hi - lo);
     const long cap = tuned_cap(P, 5, 2);
     const int grid = (int)(ntask < cap ? ntask : cap);
     if (grid <= 0) return;
@@ -4957,7 +4957,7 @@ extern "C" int blfid_dev_launch_corr(int prec, const DevPlan *P, int Kb, const v
     const int CH = corr_chunk(P->n);
     const int nchunk = (int)((P->Ecorr + CH - 1) / CH);
     const int A = corr_use_fft(P->n) ? min(max(P->corr_auto_chunks, 0), nchunk) : 0;
-    const int segA = corr_range_segments(A);
+    const int segA = corr_range_segments(P->n, P->npts, A);
     // four points per thread up to 1024 FID points, eight above (variants 0 and 1: variant 1
     // runs the complex64 four-point kernels at two waves per SIMD); variant 2: eight throughout
     for (int pass = 0; pass < 2; pass++) {

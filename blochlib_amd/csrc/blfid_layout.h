@@ -129,4 +129,28 @@ inline long choose_batch(const Shape &s, long K, double avail) {
     return lo;
 }
 
+// Halves the scratch-slot counts of the layout and of its preparation `ps`; false when all are one.
+inline bool fewer_slots(Shape &s, Shape &ps) {
+    bool any = false;
+    for (int *q : {&s.exp_slots, &s.qr_slots, &s.eig_slots, &ps.exp_slots, &ps.qr_slots, &ps.eig_slots})
+        if (*q > 1) {
+            *q /= 2;
+            any = true;
+        }
+    return any;
+}
+
+// The batch for `avail` bytes; where one crystallite does not fit beside the full scratch-slot
+// counts, these are halved `cuts` times until it does (fewer workgroups in flight, the same
+// results), so that only a crystallite's own storage decides whether a plan can run.
+inline long fit_batch(Shape &s, Shape &ps, long K, double avail, int *cuts = nullptr) {
+    for (int c = 0;; c++) {
+        const long Kb = choose_batch(s, K, avail);
+        if (Kb >= 1 || !fewer_slots(s, ps)) {
+            if (cuts) *cuts = c;
+            return Kb;
+        }
+    }
+}
+
 } // namespace blfid_layout

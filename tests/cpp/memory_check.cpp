@@ -194,8 +194,66 @@ static void host_memory() {
     REQUIRE(st == BLFID_OK && fake::used == 0);
 }
 
+// Working storage of one crystallite as earlier versions of the library laid it out, from the plan's
+// own tables: full scratch-slot counts whatever the powder, eigen-solver slots of the block's matrix
+// alone, FID parts of 64 correlation chunks.  `part` > 0: the slot regions cut to that many bytes.
+static size_t former_need(const blfid_plan *p, double part = 0) {
+    blfid_layout::Shape s = shape_of(p);
+    const size_t L = s.Lsum, bm2 = (size_t)s.bmax * s.bmax, cs = s.prec ? 8 : 16, rs = s.prec ? 4 : 8;
+    auto slots = [&](double total, double per, int lo, int hi) {
+        const double c = std::max<double>(lo, std::min<double>(hi, std::floor(total / per)));
+        return (size_t)(part > 0 ? std::max(1.0, std::min(c, std::floor(part / per))) : c);
+    };
+    const bool p2 = (s.n & (s.n - 1)) == 0 && s.n >= 16 && s.n <= 512;
+    const int ch = p2 ? CORR_SPAN / s.n : std::max(1, std::min(CORR_SPAN / s.n, 256 / ((s.n + 7) / 8)));
+    const size_t nchunk = (p->Etot + ch - 1) / ch, parts = (nchunk + 63) / 64;
+    const size_t sz[] = {s.n * L * cs, s.n * L * cs, s.n * (size_t)s.Estr * cs,
+                         s.rt_from_q ? 0 : s.n * (size_t)s.Estr * cs,
+                         slots(2.5e9, 9.0 * bm2 * 8.0, 64, 16384) * 9 * bm2 * rs, s.prec ? L * cs : 0, L * 16,
+                         s.N * (size_t)8, slots(2.5e9, 3.0 * bm2 * 16.0, 64, 16384) * 3 * bm2 * 16,
+                         parts * 2 * s.npts * 8,
+                         s.eig_slots ? slots(1.0e9, bm2 * 16.0, 64, 2048) * bm2 * 16 : 0,
+                         blfid_layout::ngroups(s.K) * 4 * (size_t)s.npts * 8};
+    size_t o = 0;
+    for (size_t x : sz) o += blfid_layout::align256(x);
+    return o;
+}
+// What fitted a memory budget, a workspace or the static scratch before still does.
+static void accepted() {
+    fake::limit = (size_t)256 << 30;
+    const struct { int S, n, npts; blfid_precision prec; int K; bool general; } cases[] = {
+        {5, 64, 512, BLFID_C64, 2000, false},     {6, 128, 2048, BLFID_C64, 1000, true},
+        {8, 128, 2048, BLFID_C64, 500, true},     {9, 32, 256, BLFID_C64, 1000, false},
+        {9, 32, 256, BLFID_FP64, 1000, true},     {10, 16, 64, BLFID_C64, 500, false},
+        {6, 64, 300000, BLFID_C64, 200, true},    {6, 45, 2000000, BLFID_FP64, 100, true},
+        {7, 100, 1000000, BLFID_C64, 300, false},
+    };
+    for (auto &c : cases) {
+        blfid_plan *p = plan(c.S, c.n, c.npts, c.prec, c.K, c.general);
+        const double need = (double)former_need(p);
+        REQUIRE(blfid_plan_set_memory_budget(p, need) == BLFID_OK);
+        REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+        REQUIRE((double)p->own_ws.blk.bytes <= need);
+        p->own_ws.release();
+        for (int k = 0; k < 3; k++) REQUIRE(blfid_plan_run_slice(p, k * c.K / 3, (k + 1) * c.K / 3, 1, nullptr) == BLFID_OK);
+        REQUIRE((double)p->own_ws.blk.bytes <= need);
+        p->own_ws.release();
+        REQUIRE(blfid_plan_graph_capture(p, 1) == BLFID_OK);
+        blfid_workspace *w = nullptr;
+        REQUIRE(blfid_workspace_create(need, &w) == BLFID_OK);
+        REQUIRE(blfid_plan_set_workspace(p, w) == BLFID_OK);
+        REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+        REQUIRE(blfid_plan_set_workspace(p, nullptr) == BLFID_OK);
+        blfid_workspace_destroy(w);
+        double out = 0;
+        if (former_need(p, BLFID_NOALLOC_SCRATCH_BYTES / 8.0) <= BLFID_NOALLOC_SCRATCH_BYTES)
+            REQUIRE(blfid_plan_run_noalloc(p, 1, &out, nullptr) == BLFID_OK);
+        blfid_plan_destroy(p);
+    }
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}};
     std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
