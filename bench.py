@@ -56,22 +56,34 @@ METRIC = "crystallite-steps/s + FIDs/s at ≤1e-5 rel L2 vs FP64 oracle; p50/p99
 COUNTER_SUMMARY = os.path.join(ROOT, "profiles", "config2_batched_{prec}_hbm_counters.txt")
 
 
-def corr_flops_per_elem(n: int, P: int, autoc: bool = False) -> float:
-    """Executed flops of k_corr per correlation element and crystallite (as the engine counts
-    them): for n a power of two from 16 to 512 three mixed-radix FFTs (radix-8 passes of a
-    56-flop DFT and 7 twiddle products per butterfly, the last pass of radix 2, 4 or 8 without
-    twiddles) and the scaled product, else the direct sum; plus twiddle staging and the FID
-    sums.  autoc: the autocorrelation variant (R = conj(Q)) with two transforms, a |q|^2 / n
-    product (4 flops per point) and the staging of Q alone (9 n)."""
+def corr_transform_length(n: int) -> int:
+    """Points of the transforms k_corr correlates n steps with (corr_fft_ln in blfid_dev.h): n
+    itself for a power of two from 16 to 512, the power of two from 2 n up that zero-padded ones
+    take for any other n from 9 to 256, or 0 where it takes the direct sum."""
+    if n & (n - 1) == 0:
+        return n if 16 <= n <= 512 else 0
+    return 1 << (2 * n - 1).bit_length() if 9 <= n <= 256 else 0
+
+
+def corr_flops_per_elem(n: int, P: int, autoc: bool = False, length: int | None = None) -> float:
+    """Flops of k_corr per correlation element and crystallite with transforms of `length` points
+    (corr_transform_length(n) is what the engine executes and counts; without it, unpadded
+    transforms for n a power of two from 16 to 512 and else the direct sum): three mixed-radix
+    FFTs (radix-8 passes of a 56-flop DFT and 7 twiddle products per butterfly, the last pass of
+    radix 2, 4 or 8 without twiddles) and the scaled product, or the direct sum (length 0); plus
+    twiddle staging and the FID sums.  autoc: the autocorrelation variant (R = conj(Q)) with two
+    transforms, a |q|^2 / n product (4 flops per point) and the staging of Q alone (9 n)."""
+    if length is None:
+        length = n if 16 <= n <= 512 and (n & (n - 1)) == 0 else 0
     c = 8.0 * n * n
     stage = 18.0 * n
-    if 16 <= n <= 512 and (n & (n - 1)) == 0:
-        ln = int(n).bit_length() - 1
+    if length:
+        ln = int(length).bit_length() - 1
         npass = (ln + 2) // 3
         rl = 1 << (ln - 3 * (npass - 1))
         dft = {2: 4.0, 4: 16.0, 8: 56.0}[rl]
         t = 2.0 if autoc else 3.0
-        c = t * (npass - 1) * (n / 8.0) * 98.0 + t * (n / rl) * dft + (4.0 if autoc else 8.0) * n
+        c = t * (npass - 1) * (length / 8.0) * 98.0 + t * (length / rl) * dft + (4.0 if autoc else 8.0) * length
         if autoc:
             stage = 9.0 * n
     return c + stage + 14.0 * P
@@ -673,7 +685,8 @@ def main():
     if dom == "k_corr":
         n, P = wls[0].steps, wls[0].npts
         d = fams[dom]
-        ratio = (14.0 * n * n + 14.0 * P) / corr_flops_per_elem(n, P, corr_is_autocorrelation(wls))
+        ratio = (14.0 * n * n + 14.0 * P) / corr_flops_per_elem(
+            n, P, corr_is_autocorrelation(wls), corr_transform_length(n))
         roof["canonical_flops_per_launch"] = ratio * d["flops"] / d["launches"]
         roof["canonical_tflops"] = ratio * d["flops"] / (d["ms"] * 1e-3) / 1e12
         roof["canonical_note"] = (
