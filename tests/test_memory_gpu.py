@@ -1,6 +1,7 @@
 """Device memory kept from closed plans: counted, given back on request, and free as far as a
 server's default budget is concerned."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -17,6 +18,15 @@ def free_bytes():
     f, t = ctypes.c_size_t(), ctypes.c_size_t()
     assert L.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
     return f.value
+
+
+def comes_free(want):
+    """The driver gives freed memory back in the background: whether `want` bytes become free."""
+    for _ in range(100):
+        if free_bytes() >= want:
+            return True
+        time.sleep(0.05)
+    return False
 
 
 def one_call():
@@ -42,5 +52,5 @@ def test_release_and_server_budget():
     assert kept > 64 << 20
     engine.release_memory()
     assert engine.memory_kept() == 0
-    assert free_bytes() >= before + kept - (2 << 20)
+    assert comes_free(before + kept - (2 << 20))
     assert np.array_equal(one_call(), ref)
