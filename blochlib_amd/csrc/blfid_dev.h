@@ -88,6 +88,7 @@ struct DevPlan {
     int tn_corr;           // k_corr variant: 0 four FID points per thread up to 1024 points
                            // (eight above) at the default occupancy, 1 the same at two waves
                            // per SIMD (no register spill), 2 eight points per thread
+    int eig_sweeps;        // sweeps of k_eigb_* over the whole device (0: EIGB_SWEEPS)
     int tn_qr;             // k_qr form per complex64 tile class: bit M-1 set takes the other form
                            // (per-step for classes 1-2, step-walking for 3-4; class 1 by k_bq1)
 };

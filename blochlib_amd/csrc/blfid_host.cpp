@@ -539,6 +539,7 @@ struct blfid_plan {
     int sl_next = -1, sl_norm = 1;
     long sl_Kb = 0;
     int sl_cuts = 0;
+    int eig_sweeps = 0; // blfid_plan_set_eig_sweeps
     unsigned long sl_gen = 0;
     char *sl_base = nullptr;
     ~blfid_plan() {
@@ -974,6 +975,7 @@ static void refresh_devplan(blfid_plan *pl) {
     for (int f = 0; f < 9; f++) d.tn_cap[f] = pl->tn[6 + f];
     d.tn_corr = pl->tn[5];
     d.tn_qr = pl->tn[15];
+    d.eig_sweeps = pl->eig_sweeps;
 }
 
 // ------------------------------------------------------------------------------ C ABI
@@ -2525,6 +2527,14 @@ blfid_status blfid_plan_set_workspace(blfid_plan *pl, blfid_workspace *w) {
     pl->gen++; // a recorded graph no longer matches the plan
     pl->ws = w;
     if (w) pl->own_ws.release();
+    return BLFID_OK;
+}
+
+blfid_status blfid_plan_set_eig_sweeps(blfid_plan *pl, int sweeps) {
+    if (!pl) return fail(BLFID_ERR_INVALID, "plan is NULL");
+    if (sweeps < 0 || sweeps > 12) return fail(BLFID_ERR_INVALID, "sweeps outside 0..12");
+    pl->gen++; // a recorded graph no longer matches the plan
+    pl->eig_sweeps = sweeps;
     return BLFID_OK;
 }
 

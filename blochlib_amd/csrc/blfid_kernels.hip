@@ -2555,11 +2555,13 @@ __global__ void __launch_bounds__(NT, MB == 16 ? 5 : MB <= 48 ? 4 : 1) k_eig(Dev
 //                transposes the left one), and W_.q <- W_.q V_q likewise
 // Sweeps repeat until no rotation of a sweep exceeds sqrt(tol_rot) (as in k_eig): the flag of a
 // sweep is read by the kernels of the next, which leave a finished task alone.  EIGB_SWEEPS
-// sweeps are launched (six to eight are used); k_eigb_tail then finishes a task that needs more,
-// in one workgroup, and reads off the phases.  A round moves M and W once.
+// sweeps are launched; k_eigb_tail then finishes a task that needs more with the same rounds in one
+// workgroup, and reads off the phases.  A round moves M and W once.
 // Bound by HBM / MALL traffic and the rotations' latency.  One workgroup per block held the device to
 // as many CUs as there were blocks, each round limited by one CU's L2 path: 64 crystallites of
-// 10 spins (blocks up to 252 states) 198 -> 82 ms.
+// 10 spins (blocks up to 252 states) 198 -> 79 ms.  Most blocks end after eight to eleven sweeps, and
+// a launch that finds its task finished costs little: 10 spins 78.9 ms at 12 sweeps, 81.3 at 10, 89.1
+// at 9, 104 at 8, 123 at 6; 9 spins FP64 x 8 crystallites 5.01, 4.89, 4.84, 5.52, 6.85 ms.
 #define BJ_NB 8
 #define BJ_NS (2 * BJ_NB)
 #define BJ_MAXPAIR 16 /* b <= 16 BJ_MAXPAIR */
@@ -2592,22 +2594,24 @@ __global__ void __launch_bounds__(256) k_eigb_init(DevPlan P, int t0, const int 
     }
     if (blockIdx.x == 0 && threadIdx.x < 2 * EIGB_SWEEPS + BJ_MAXPAIR) eigb_flags(Ms, gslot)[threadIdx.x] = 0;
 }
+// LDS of a wave's rotations
+struct EigbLds {
+    cd S[BJ_NS * (BJ_NS + 1)], V[BJ_NS * (BJ_NS + 1)], rs[BJ_NB];
+    double rc[BJ_NB];
+};
+// One wave: the joint-Jacobi sweep of pair pi in round `round`, its rotation to the slot's V and its
+// "rotated" flag; returns whether a rotation was large.
 template <typename R>
-__global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
-                                                 int sweep, int round, cd *__restrict__ gscr, size_t gslot) {
+__device__ __forceinline__ bool eigb_rot(int b, int round, int pi, cd *Ms, size_t gslot, EigbLds &L) {
     constexpr int NB = BJ_NB, NS = BJ_NS, LS = NS + 1;
     constexpr double tol_stop = __is_same(R, double) ? 3.1622776601683795e-8 : 1e-5;
     constexpr double tol_off = __is_same(R, double) ? 1e-17 : 1e-12;
-    __shared__ cd Sp[NS * LS], Vp[NS * LS], rs[NB];
-    __shared__ double rc[NB];
-    const int task = t0 + blockIdx.y, pi = blockIdx.x, lane = threadIdx.x;
-    const int b = P.blk_dim[grp[task % ngrp]];
-    if (pi >= eigb_nbk(b) / 2 || round >= eigb_nbk(b) - 1) return;
-    cd *Ms = gscr + gslot * blockIdx.y;
-    int *fl = eigb_flags(Ms, gslot);
-    if (sweep > 0 && !fl[sweep - 1]) return;
+    cd *Sp = L.S, *Vp = L.V, *rs = L.rs;
+    double *rc = L.rc;
+    const int lane = threadIdx.x & 63;
     cd *V = Ms + gslot - EIGB_EXTRA + pi * NS * NS;
     const int gl = eigb_index(b, round, pi, lane & 15);
+    auto sync = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); };
 #pragma unroll
     for (int u = 0; u < 4; u++) {
         const int i = lane & 15, j = (lane >> 4) + 4 * u;
@@ -2615,7 +2619,7 @@ __global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *_
         Sp[i + j * LS] = gl >= 0 && gj >= 0 ? Ms[gl + (size_t)gj * b] : cmk(0, 0);
         Vp[i + j * LS] = cmk(i == j ? 1.0 : 0.0, 0.0);
     }
-    __syncthreads();
+    sync();
     bool any = false, large = false;
     for (int sr = 0; sr < NS - 1; sr++) {
         // circle method: position 0 fixed, the others turn; rotation k pairs positions k and NS-1-k
@@ -2634,7 +2638,7 @@ __global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *_
             rc[lane] = cth;
             rs[lane] = sth;
         }
-        __syncthreads();
+        sync();
         // S <- R^H S R on the 2 x 2 block of rotations (ki, kj); V <- V R, two entries pairs a lane
         {
             const int ki = lane & 7, kj = lane >> 3;
@@ -2663,7 +2667,7 @@ __global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *_
                 Vp[row + q2 * LS] = csub(cscale(wq, cj), cmul(cconj(sj), wp));
             }
         }
-        __syncthreads();
+        sync();
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -2671,30 +2675,26 @@ __global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *_
         V[i + j * NS] = Vp[i + j * LS];
     }
     const bool a2 = __any(any), l2 = __any(large);
-    if (lane == 0) {
-        fl[EIGB_SWEEPS + pi] = a2;
-        if (l2) atomicOr(&fl[sweep], 1);
-    }
+    if (lane == 0) eigb_flags(Ms, gslot)[EIGB_SWEEPS + pi] = a2;
+    return l2;
 }
-// grid: x: 16 x 16 tiles of M, then of W; y: task.  Tile t = p + npr q.
-__global__ void __launch_bounds__(64) k_eigb_upd(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
-                                                 int sweep, int round, cd *__restrict__ bufW,
-                                                 cd *__restrict__ gscr, size_t gslot) {
+// One wave: 16 x 16 tile t of round `round`, those of M (t = p + npr q) and then those of W.
+__device__ __forceinline__ int eigb_tiles(int b) {
+    const int npr = eigb_nbk(b) / 2;
+    return npr * npr + (b + 15) / 16 * npr;
+}
+__device__ __forceinline__ void eigb_upd(int b, int round, int tile, cd *Ms, size_t gslot, cd *W) {
     constexpr int NS = BJ_NS;
-    const int task = t0 + blockIdx.y, c = task / ngrp, blk = grp[task % ngrp], b = P.blk_dim[blk];
     const int npr = eigb_nbk(b) / 2, nrt = (b + 15) / 16;
-    if (round >= 2 * npr - 1 || (int)blockIdx.x >= npr * npr + nrt * npr) return;
-    cd *Ms = gscr + gslot * blockIdx.y;
     const int *fl = eigb_flags(Ms, gslot);
-    if (sweep > 0 && !fl[sweep - 1]) return;
-    const bool isW = (int)blockIdx.x >= npr * npr;
-    const int t = isW ? blockIdx.x - npr * npr : blockIdx.x;
+    const bool isW = tile >= npr * npr;
+    const int t = isW ? tile - npr * npr : tile;
     const int p = isW ? t % nrt : t % npr, q = isW ? t / nrt : t / npr;
     const bool rq = fl[EIGB_SWEEPS + q], rp = !isW && fl[EIGB_SWEEPS + p];
     if (!rq && !rp) return;
-    const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
     const cd *Vb = Ms + gslot - EIGB_EXTRA;
-    cd *X = isW ? bufW + (size_t)c * P.Lsum + P.blk_uoff[blk] : Ms;
+    cd *X = isW ? W : Ms;
     // the tile as left operand (row r, column 4 v + g) and V_q as right operand (row 4 v + g,
     // column r)
     const int gr = isW ? (16 * p + r < b ? 16 * p + r : -1) : eigb_index(b, round, p, r);
@@ -2741,161 +2741,62 @@ __global__ void __launch_bounds__(64) k_eigb_upd(DevPlan P, int t0, const int *_
         if (orow >= 0 && oc >= 0) X[orow + (size_t)oc * b] = cmk(sr[v], si[v]);
     }
 }
-// Sweeps beyond EIGB_SWEEPS of the tasks whose last flag is still set, one workgroup per task (up
-// to 40 sweeps in all), then every task's phases and its storage-precision W.
+// grid: x: pair; y: task
 template <typename R>
-__global__ void __launch_bounds__(512) k_eigb_tail(DevPlan P, int t0, int nt, const int *__restrict__ grp,
-                                                   int ngrp, int mode, cd *__restrict__ bufW,
-                                                 typename CX<R>::T *__restrict__ bufWr,
-                                                 double *__restrict__ outv, cd *__restrict__ gscr,
-                                                 size_t gslot) {
+__global__ void __launch_bounds__(64) k_eigb_rot(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
+                                                 int sweep, int round, cd *__restrict__ gscr, size_t gslot) {
+    __shared__ EigbLds L;
+    const int task = t0 + blockIdx.y, pi = blockIdx.x;
+    const int b = P.blk_dim[grp[task % ngrp]];
+    if (pi >= eigb_nbk(b) / 2 || round >= eigb_nbk(b) - 1) return;
+    cd *Ms = gscr + gslot * blockIdx.y;
+    int *fl = eigb_flags(Ms, gslot);
+    if (sweep > 0 && !fl[sweep - 1]) return;
+    if (eigb_rot<R>(b, round, pi, Ms, gslot, L) && threadIdx.x == 0) atomicOr(&fl[sweep], 1);
+}
+// grid: x: tile; y: task
+__global__ void __launch_bounds__(64) k_eigb_upd(DevPlan P, int t0, const int *__restrict__ grp, int ngrp,
+                                                 int sweep, int round, cd *__restrict__ bufW,
+                                                 cd *__restrict__ gscr, size_t gslot) {
+    const int task = t0 + blockIdx.y, c = task / ngrp, blk = grp[task % ngrp], b = P.blk_dim[blk];
+    if (round >= eigb_nbk(b) - 1 || (int)blockIdx.x >= eigb_tiles(b)) return;
+    cd *Ms = gscr + gslot * blockIdx.y;
+    if (sweep > 0 && !eigb_flags(Ms, gslot)[sweep - 1]) return;
+    eigb_upd(b, round, blockIdx.x, Ms, gslot, bufW + (size_t)c * P.Lsum + P.blk_uoff[blk]);
+}
+// Sweeps beyond the launched ones of the tasks whose last flag is still set, the same rounds by the
+// waves of one workgroup per task (up to 40 sweeps in all), then every task's phases and its
+// storage-precision W.
+#define EIGB_TAIL_W 8
+template <typename R>
+__global__ void __launch_bounds__(64 * EIGB_TAIL_W) k_eigb_tail(DevPlan P, int t0, int nt, const int *__restrict__ grp,
+                                                                int ngrp, int mode, int sweeps, cd *__restrict__ bufW,
+                                                                typename CX<R>::T *__restrict__ bufWr,
+                                                                double *__restrict__ outv, cd *__restrict__ gscr,
+                                                                size_t gslot) {
     typedef typename CX<R>::T CT;
-    constexpr int NT = 512, NB = BJ_NB, NS = BJ_NS, LS = NS + 1;
-    constexpr int RW = NB * NB + NB * NS; // rotation work items per pair and sub-round
-    constexpr double tol_stop = __is_same(R, double) ? 3.1622776601683795e-8 : 1e-5;
-    constexpr double tol_off = __is_same(R, double) ? 1e-17 : 1e-12;
-    __shared__ cd sS[BJ_MAXPAIR * NS * LS];
-    __shared__ cd sV[BJ_MAXPAIR * NS * NS];
-    __shared__ double rc[BJ_MAXPAIR * NB];
-    __shared__ cd rs[BJ_MAXPAIR * NB];
-    __shared__ int rp[BJ_MAXPAIR * NB], rq[BJ_MAXPAIR * NB];
-    __shared__ int s_gi[BJ_MAXPAIR * NS]; // global index of each pair's local index, -1 absent
-    __shared__ int s_rot[BJ_MAXPAIR];
+    constexpr int NW = EIGB_TAIL_W, NT = 64 * NW;
+    __shared__ EigbLds L[NW];
     __shared__ int s_any;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, w = tid >> 6;
     for (int ti = blockIdx.x; ti < nt; ti += gridDim.x) {
         const int task = t0 + ti, g = task % ngrp, c = task / ngrp;
         cd *Ms = gscr + gslot * ti;
         const int blk = grp[g], b = P.blk_dim[blk];
-        const bool done = !eigb_flags(Ms, gslot)[EIGB_SWEEPS - 1];
         cd *W = bufW + (size_t)c * P.Lsum + P.blk_uoff[blk];
-        const int nbk = 2 * ((b + NS - 1) / NS); // even number of column blocks
-        const int npr = nbk / 2;                 // pairs per round, <= BJ_MAXPAIR
-        __syncthreads();
-        for (int sweep = EIGB_SWEEPS; sweep < 40 && !done; sweep++) {
+        bool go = eigb_flags(Ms, gslot)[sweeps - 1] != 0;
+        for (int sweep = sweeps; sweep < 40 && go; sweep++) {
             if (tid == 0) s_any = 0;
-            for (int round = 0; round < nbk - 1; round++) {
-                for (int x = tid; x < npr * NS; x += NT) {
-                    const int pi = x / NS, l = x % NS;
-                    const int pa = pi, pb = nbk - 1 - pi;
-                    const int ia = pa == 0 ? 0 : ((pa - 1 + round) % (nbk - 1)) + 1;
-                    const int ib = pb == 0 ? 0 : ((pb - 1 + round) % (nbk - 1)) + 1;
-                    const int Pb = min(ia, ib), Qb = max(ia, ib);
-                    const int gi = l < NB ? Pb * NB + l : Qb * NB + (l - NB);
-                    s_gi[x] = gi < b ? gi : -1;
-                }
-                if (tid < BJ_MAXPAIR) s_rot[tid] = 0;
+            __syncthreads();
+            for (int round = 0; round < eigb_nbk(b) - 1; round++) {
+                for (int pi = w; pi < eigb_nbk(b) / 2; pi += NW)
+                    if (eigb_rot<R>(b, round, pi, Ms, gslot, L[w]) && (tid & 63) == 0) s_any = 1;
                 __syncthreads();
-                for (int x = tid; x < npr * NS * NS; x += NT) {
-                    const int pi = x / (NS * NS), e = x % (NS * NS), i = e % NS, j = e / NS;
-                    const int gi = s_gi[pi * NS + i], gj = s_gi[pi * NS + j];
-                    sS[pi * NS * LS + i + j * LS] =
-                        (gi >= 0 && gj >= 0) ? Ms[gi + (size_t)gj * b] : cmk(0, 0);
-                    sV[pi * NS * NS + e] = cmk(i == j ? 1.0 : 0.0, 0.0);
-                }
-                __syncthreads();
-                // one joint-Jacobi sweep of every pair's submatrix (circle method over NS)
-                for (int sr = 0; sr < NS - 1; sr++) {
-                    for (int x = tid; x < npr * NB; x += NT) {
-                        const int pi = x / NB, k = x % NB;
-                        const int pa = k, pb = NS - 1 - k;
-                        const int ia = pa == 0 ? 0 : ((pa - 1 + sr) % (NS - 1)) + 1;
-                        const int ib = pb == 0 ? 0 : ((pb - 1 + sr) % (NS - 1)) + 1;
-                        const int p = min(ia, ib), q = max(ia, ib);
-                        const cd *Sp = sS + pi * NS * LS;
-                        double cth = 1.0;
-                        cd sth = cmk(0, 0);
-                        bool big = false;
-                        if (s_gi[pi * NS + p] >= 0 && s_gi[pi * NS + q] >= 0 &&
-                            jj_rotation(Sp[p + p * LS], Sp[q + q * LS], Sp[p + q * LS],
-                                        Sp[q + p * LS], tol_off, tol_stop, cth, sth, big)) {
-                            s_rot[pi] = 1;
-                            if (big) s_any = 1;
-                        }
-                        rc[x] = cth;
-                        rs[x] = sth;
-                        rp[x] = p;
-                        rq[x] = q;
-                    }
-                    __syncthreads();
-                    // S <- R^H S R on every 2 x 2 block of rotation pairs; V <- V R
-                    for (int x = tid; x < npr * RW; x += NT) {
-                        const int pi = x / RW, e = x % RW;
-                        if (e < NB * NB) {
-                            cd *Sp = sS + pi * NS * LS;
-                            const int ki = pi * NB + e % NB, kj = pi * NB + e / NB;
-                            const int p = rp[ki], q = rq[ki], p2 = rp[kj], q2 = rq[kj];
-                            const double ci = rc[ki], cj = rc[kj];
-                            const cd si = rs[ki], sj = rs[kj];
-                            const cd a = Sp[p + p2 * LS], bb2 = Sp[p + q2 * LS];
-                            const cd c2 = Sp[q + p2 * LS], d = Sp[q + q2 * LS];
-                            const cd a1 = cadd(cscale(a, ci), cmul(cconj(si), c2));
-                            const cd c1 = csub(cscale(c2, ci), cmul(si, a));
-                            const cd b1 = cadd(cscale(bb2, ci), cmul(cconj(si), d));
-                            const cd d1 = csub(cscale(d, ci), cmul(si, bb2));
-                            Sp[p + p2 * LS] = cadd(cscale(a1, cj), cmul(sj, b1));
-                            Sp[p + q2 * LS] = csub(cscale(b1, cj), cmul(cconj(sj), a1));
-                            Sp[q + p2 * LS] = cadd(cscale(c1, cj), cmul(sj, d1));
-                            Sp[q + q2 * LS] = csub(cscale(d1, cj), cmul(cconj(sj), c1));
-                        } else {
-                            cd *Vp = sV + pi * NS * NS;
-                            const int f = e - NB * NB, row = f % NS, k = pi * NB + f / NS;
-                            const int p = rp[k], q = rq[k];
-                            const double cth = rc[k];
-                            const cd sth = rs[k];
-                            const cd wp = Vp[row + p * NS], wq = Vp[row + q * NS];
-                            Vp[row + p * NS] = cadd(cscale(wp, cth), cmul(sth, wq));
-                            Vp[row + q * NS] = csub(cscale(wq, cth), cmul(cconj(sth), wp));
-                        }
-                    }
-                    __syncthreads();
-                }
-                // rows of every rotated pair: M(idx, col) <- V^H M(idx, col)
-                for (int x = tid; x < npr * b; x += NT) {
-                    const int pi = x / b, col = x % b;
-                    if (!s_rot[pi]) continue;
-                    const int *gi = s_gi + pi * NS;
-                    const cd *Vp = sV + pi * NS * NS;
-                    cd m[NS];
-#pragma unroll
-                    for (int l = 0; l < NS; l++)
-                        m[l] = gi[l] >= 0 ? Ms[gi[l] + (size_t)col * b] : cmk(0, 0);
-#pragma unroll
-                    for (int i = 0; i < NS; i++) {
-                        if (gi[i] < 0) continue;
-                        cd acc = cmk(0, 0);
-#pragma unroll
-                        for (int l = 0; l < NS; l++) cfma(acc, cconj(Vp[l + i * NS]), m[l]);
-                        Ms[gi[i] + (size_t)col * b] = acc;
-                    }
-                }
-                __syncthreads();
-                // columns of every rotated pair: M(row, idx) <- M(row, idx) V, W likewise
-                for (int x = tid; x < 2 * npr * b; x += NT) {
-                    const int which = x / (npr * b), y = x % (npr * b), pi = y / b, row = y % b;
-                    if (!s_rot[pi]) continue;
-                    const int *gi = s_gi + pi * NS;
-                    const cd *Vp = sV + pi * NS * NS;
-                    cd *X = which ? W : Ms;
-                    cd m[NS];
-#pragma unroll
-                    for (int l = 0; l < NS; l++)
-                        m[l] = gi[l] >= 0 ? X[row + (size_t)gi[l] * b] : cmk(0, 0);
-#pragma unroll
-                    for (int j = 0; j < NS; j++) {
-                        if (gi[j] < 0) continue;
-                        cd acc = cmk(0, 0);
-#pragma unroll
-                        for (int l = 0; l < NS; l++) cfma(acc, m[l], Vp[l + j * NS]);
-                        X[row + (size_t)gi[j] * b] = acc;
-                    }
-                }
+                for (int t = w; t < eigb_tiles(b); t += NW) eigb_upd(b, round, t, Ms, gslot, W);
                 __syncthreads();
             }
-            // every thread reads the flag before the next sweep's reset by thread 0
-            const int any = s_any;
-            __syncthreads();
-            if (!any) break;
+            go = s_any != 0;
+            __syncthreads(); // read by every thread before the next sweep clears it
         }
         double *o = outv + (size_t)c * P.N + P.blk_soff[blk];
         for (int r = tid; r < b; r += NT) {
@@ -2906,7 +2807,6 @@ __global__ void __launch_bounds__(512) k_eigb_tail(DevPlan P, int t0, int nt, co
             CT *Wr = bufWr + (size_t)c * P.Lsum + P.blk_uoff[blk];
             for (int e = tid; e < b * b; e += NT) Wr[e] = CX<R>::from(W[e]);
         }
-        __syncthreads();
     }
 }
 
@@ -4733,16 +4633,17 @@ static void launch_eigb(const DevPlan *P, int Kb, const int *grp, int ngrp, cons
                         size_t src_stride, int mode, cd *bufW, void *bufWr, double *outv, cd *gscr,
                         size_t gslot, int nslots, int bmax, hipStream_t st) {
     typedef typename CX<R>::T CT;
+    const int sweeps = P->eig_sweeps < 1 || P->eig_sweeps > EIGB_SWEEPS ? EIGB_SWEEPS : P->eig_sweeps;
     const int ntask = Kb * ngrp, npr = eigb_nbk(bmax) / 2, nrt = (bmax + 15) / 16;
     for (int t0 = 0; t0 < ntask; t0 += nslots) {
         const int nt = ntask - t0 < nslots ? ntask - t0 : nslots;
         k_eigb_init<R><<<dim3(16, nt), 256, 0, st>>>(*P, t0, grp, ngrp, (const CT *)src, src_stride, bufW, gscr, gslot);
-        for (int sweep = 0; sweep < EIGB_SWEEPS; sweep++)
+        for (int sweep = 0; sweep < sweeps; sweep++)
             for (int round = 0; round < 2 * npr - 1; round++) {
                 k_eigb_rot<R><<<dim3(npr, nt), 64, 0, st>>>(*P, t0, grp, ngrp, sweep, round, gscr, gslot);
                 k_eigb_upd<<<dim3(npr * npr + nrt * npr, nt), 64, 0, st>>>(*P, t0, grp, ngrp, sweep, round, bufW, gscr, gslot);
             }
-        k_eigb_tail<R><<<nt, 512, 0, st>>>(*P, t0, nt, grp, ngrp, mode, bufW, (CT *)bufWr, outv, gscr, gslot);
+        k_eigb_tail<R><<<nt, 64 * EIGB_TAIL_W, 0, st>>>(*P, t0, nt, grp, ngrp, mode, sweeps, bufW, (CT *)bufWr, outv, gscr, gslot);
     }
 }
 

@@ -103,6 +103,7 @@ def lib():
         L.blfid_plan_set_workspace.argtypes = [vp, vp]
         L.blfid_memory_kept.argtypes = [_d]
         L.blfid_plan_set_profiling.argtypes = [vp, ctypes.c_int]
+        L.blfid_plan_set_eig_sweeps.argtypes = [vp, ctypes.c_int]
         L.blfid_plan_phase_times.argtypes = [vp, _d, _i, _d]
         L.blfid_plan_phase_bytes.argtypes = [vp, _d]
         L.blfid_state_create.argtypes = [ctypes.c_int, ctypes.c_int, _d, _d, _d, _d,
@@ -348,6 +349,10 @@ class Plan:
     KERNELS = ("k_exp", "k_dyson", "k_eig", "k_bmul", "k_qr", "k_corr", "k_reduce",
                "k_static_fid", "k_expdyson")
     NSLOT = 72  # BLFID_NSLOT
+
+    def set_eig_sweeps(self, sweeps: int):
+        """Eigen-solver sweeps launched over the whole device (blocks above 80 states), 0: default."""
+        _check(lib().blfid_plan_set_eig_sweeps(self.h, int(sweeps)))
 
     def set_profiling(self, on: bool = True):
         _check(lib().blfid_plan_set_profiling(self.h, int(bool(on))))

@@ -308,6 +308,11 @@ blfid_status blfid_plan_phase_times(blfid_plan *plan, double *ms, int *launches,
  * powder sum).  Beside counter-measured traffic it shows re-reads and spills. */
 blfid_status blfid_plan_phase_bytes(blfid_plan *plan, double *bytes);
 
+/* Sweeps of the eigen-solver that a run launches over the whole device for blocks above 80 states,
+ * 1 to 12 (0: the default, 12).  Blocks that need more finish inside one workgroup each with the
+ * same rotations in the same order: results agree to rounding. */
+blfid_status blfid_plan_set_eig_sweeps(blfid_plan *plan, int sweeps);
+
 /* Launch autotuner (no counterpart in the reference, whose CPU loops have no launch shape).
  * A tuning is BLFID_TUNE_LEN ints:
  *   [0..4]  propagator method of tile class M = 1..5 (blocks of 16(M-1)+1 .. 16M states, class 5
