@@ -113,9 +113,18 @@ inline long tuned_cap(const DevPlan *P, int fam, int M) {
 // log2 of the transform length of the FFT variant, or 0 where the direct sum is taken.  A power of
 // two from 16 to 512 is transformed at its own length; any other n from CORR_PAD_MIN to 256 is
 // zero-padded to the power of two L >= 2 n, whose cyclic correlation holds the linear one, folded
-// back to period n (two or three transforms of at most 4 n points against 8 n^2 flops: figures at
-// k_corr).  Smaller n stay direct (the padded chunks would hold mostly zeros), larger n would need
-// transforms beyond 512 points.
+// back to period n (two or three transforms of at most 4 n points against 8 n^2 flops).  Direct sum
+// and padded transforms, k_corr in us, 1154 crystallites (4 spins FP64, 512 points | 6 spins FP64
+// and complex64, 1000 points):
+//   n    5: 105 133 | 1350 1539, 1252 1274      n  65: 217 180 | 2820 1869, 2574 1705
+//   n    8: 110 109 | 1375 1402, 1289 1276      n 100: 333 194 | 3796 2032, 3250 1932
+//   n    9: 109  57 | 1687 1005, 1555  844      n 127: 448 200 | 5429 1970, 4566 1871
+//   n   31: 130  62 | 1952  655, 1841  592      n 129: 469 542 | 5544 5603, 4575 3250
+//   n   33: 162 101 | 1693 1149, 1569 1038      n 160: 923 566 | 7868 5700, 6247 3273
+//   n   45: 184 104 | 1861 1144, 1730 1032      n 255: 1251 624 | 14801 6140, 11111 3563
+// so the direct sum is kept below 9, where the padded chunks would hold mostly zeros, and above 256,
+// which would need transforms beyond 512 points; just above 128 the two are even.  Both are as far from
+// extended-precision FIDs.
 #define CORR_PAD_MIN 9
 __host__ __device__ inline int corr_fft_ln(int n) {
     const bool p2 = (n & (n - 1)) == 0;

@@ -861,9 +861,8 @@ template <> struct ExpTol<double> { static constexpr double tol = 1e-17, rmax = 
 template <> struct ExpTol<float> { static constexpr double tol = 2e-8, rmax = 2.0; };
 
 // The 16 x 16 complex64 variant is held to four waves per SIMD (128 registers, no spills; three
-// without the bound).  The FP64 49-64-state variant (like k_dyson's and k_qr's) is held to three
-// workgroups per CU: 168 registers instead of 234 with 17 spilled, still 16% faster than two
-// (k_dyson 14%, no spills; k_qr 21%, 6 spilled).
+// without the bound), the blocks above 80 states to two workgroups per CU.  FP64 blocks of at most
+// 80 states take k_expdyson_d.
 template <int M, typename R>
 __global__ void __launch_bounds__(NThr<M>::v, (M == 1 && sizeof(R) == 4) ? 4 : M == 5 ? 2 : 1) k_exp(DevPlan P, int Kb, int c0,
                                                     const int *__restrict__ grp, int ngrp,
@@ -1130,37 +1129,30 @@ __device__ __forceinline__ void chain_mfma(int b, int n, const cf *__restrict__ 
 // U *= X is U = X U in propogation.cc:273, 288).  Product k goes to slot k % akeep of the
 // crystallite's akeep slots: all of them for gamma-COMPUTE, two alternating ones when only
 // the period propagator A_n is needed.
-template <int M, typename R, bool SPLIT = false>
-__global__ void __launch_bounds__(NThr<M>::v, (M == 3 && sizeof(R) == 4) ? 3 : (M == 4 && sizeof(R) == 4) ? 2 : (M == 4 && sizeof(R) == 8) ? 3 : 1) k_dyson(DevPlan P, int Kb, const int *__restrict__ grp,
-                                                      int ngrp,
-                                                      const typename CX<R>::T *__restrict__ bufU,
-                                                      typename CX<R>::T *__restrict__ bufA) {
+// complex64 blocks of at most 80 states in the tuned two-kernel form, and every BF16x3 block (FP64
+// chains are k_expdyson_d's, larger blocks k_dyson_big's).
+template <int M, bool SPLIT>
+__global__ void __launch_bounds__(NThr<M>::v, M == 3 ? 3 : M == 4 ? 2 : 1) k_dyson(DevPlan P, int Kb, const int *__restrict__ grp,
+                                                      int ngrp, const cf *__restrict__ bufU,
+                                                      cf *__restrict__ bufA) {
     constexpr int NT = NThr<M>::v;
-    typedef typename CX<R>::T CT;
-    constexpr bool CHAIN = std::is_same<R, float>::value && !SPLIT;
-    constexpr int CHB = 4 * 16 * M * (16 * M + LDS_PAD) * 4, GB = CGemm<M, NT, R, SPLIT>::BYTES;
-    __shared__ __align__(16) char smem[CHAIN && CHB > GB ? CHB : GB];
+    constexpr int CHB = 4 * 16 * M * (16 * M + LDS_PAD) * 4, GB = CGemm<M, NT, float, SPLIT>::BYTES;
+    __shared__ __align__(16) char smem[!SPLIT && CHB > GB ? CHB : GB];
     const long ntask = (long)Kb * ngrp;
     for (long task = blockIdx.x; task < ntask; task += gridDim.x) {
         const int g = (int)(task % ngrp), c = (int)(task / ngrp);
         const int blk = grp[g], b = P.blk_dim[blk];
-        const size_t base = (size_t)c * P.n * P.Lsum + P.blk_uoff[blk];
-        const size_t abase = (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
-        const CT *U0 = bufU + base;
-        CT *A0 = bufA + abase;
-        if (CHAIN) {
-            if constexpr (CHAIN)
-                chain_mfma<M, NT, true>(b, P.n, U0, P.Lsum, nullptr, A0, P.Lsum, P.akeep,
-                                        (float *)smem);
-        } else if constexpr (!CHAIN) {
+        const cf *U0 = bufU + (size_t)c * P.n * P.Lsum + P.blk_uoff[blk];
+        cf *A0 = bufA + (size_t)c * P.akeep * P.Lsum + P.blk_uoff[blk];
+        if constexpr (!SPLIT) {
+            chain_mfma<M, NT, true>(b, P.n, U0, P.Lsum, nullptr, A0, P.Lsum, P.akeep, (float *)smem);
+        } else {
             for (int e = threadIdx.x; e < b * b; e += NT) A0[e] = U0[e];
             __syncthreads();
-            for (int k = 1; k < P.n; k++) {
-                const CT *Uk = bufU + base + (size_t)k * P.Lsum;
-                const CT *Ap = bufA + abase + (size_t)((k - 1) % P.akeep) * P.Lsum;
-                CT *Ak = bufA + abase + (size_t)(k % P.akeep) * P.Lsum;
-                CGemm<M, NT, R, SPLIT>::run(b, b, b, Uk, b, false, Ap, b, Ak, b, smem);
-            }
+            for (int k = 1; k < P.n; k++)
+                CGemm<M, NT, float, true>::run(b, b, b, U0 + (size_t)k * P.Lsum, b, false,
+                                               A0 + (size_t)((k - 1) % P.akeep) * P.Lsum, b,
+                                               A0 + (size_t)(k % P.akeep) * P.Lsum, b, smem);
         }
     }
 }
@@ -3382,7 +3374,8 @@ __global__ void __launch_bounds__(64, sizeof(R) == 4 ? 4 : 2) k_bq1(DevPlan P, i
 // each thread walking a run of k with one sincos and complex multiplies.  Thread (el, pg)
 // then computes F_p(el) for p in [8 pg, 8 pg + 8):
 //   F_p(e) = sum_i Rt_i(e) Qt_{(i+p)%n}(e)
-// For n a power of two (16 <= n <= 2 CORR_TW) the correlation is formed with FFTs instead:
+// For n a power of two (16 <= n <= 2 CORR_TW), and zero-padded for any other n from 9 to CORR_TW
+// (corr_fft_ln), the correlation is formed with FFTs instead:
 //   F = IDFT( Rtilde . DFT(Qt) ),  Rtilde_k = sum_i Rt_i e^{+2 pi i ik/n},
 // as in-place mixed-radix passes in LDS (radix 8, the last pass radix 2, 4 or 8): staging and
 // the twiddles fuse into the first forward pass, the last forward pass, the product and the first
@@ -3392,7 +3385,7 @@ __global__ void __launch_bounds__(64, sizeof(R) == 4 ? 4 : 2) k_bq1(DevPlan P, i
 // stored as the segment's partial FID part[c][sg][t] (accumulated chunk by chunk by the thread
 // owning t when the FID is too long to hold).  No atomics: each (crystallite, segment, point) has
 // one writer, and k_reduce adds the segments in order, so the FID does not depend on scheduling.
-// CH = min(CORR_SPAN / n, 256 / ceil(n/8)) is computed identically on the host (blfid_dev.h).
+// CH (corr_chunk) and the segments (corr_seg_chunks) are computed identically on the host.
 // Q rows are Estr elements apart (Etot padded to 16 elements).  The elements are those of the
 // plan's list (Ecorr of them: corr_pos in the Q row, corr_r / corr_s their states), which leaves
 // out what is zero by structure: a block of several packed components has eigenvectors of one
@@ -3592,8 +3585,7 @@ template <int LN, int NPT, bool PAD> struct CorrTiles {
 // NPT FID points per thread are held over a segment (npts <= 256 NPT).  LN > 0 selects the FFT
 // variant with transforms of 2^LN points (CorrFft<LN>): n = 2^LN, or (PAD) any n <= 2^(LN-1), the
 // sequences zero-padded and the linear correlation folded to period n afterwards.  LN = 0 is the
-// direct sum for any n.  PAD against the direct sum (6 spins, 1154 crystallites, n = 100, 1000
-// points, complex64): 10.6 -> 4.7 ms.  The complex64 FFT variant
+// direct sum for any n (PAD against it: figures at corr_fft_ln).  The complex64 FFT variant
 // with four points is held to three waves per SIMD (168 registers: at four it spilled, and its
 // sixteen loads per chunk then waited on the spill reloads); the others are bound by LDS or
 // registers at two.  OCC > 0 replaces that bound (a variant the launch autotuner may choose).
@@ -3718,7 +3710,7 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                     const double ph = ok ? (th_r - th_s) / (double)n : 0.0;
                     if (j == 0) {
                         sphi[el] = ph;
-                        sstep[el] = cexpi(256.0 * ph);
+                        if (!hold) sstep[el] = cexpi(256.0 * ph);
                     }
                     // Q: okf masks a padded element; R = conj(Q) + reverse Q (rosym, reverse
                     // masked by rvf when the element has none) or the stored R
@@ -3912,7 +3904,7 @@ __global__ void __launch_bounds__(256, OCC > 0 ? OCC : (LN > 0 && sizeof(R) == 4
                 __syncthreads();
             }
             if (FFT && hold) {
-                // every element of the chunk: those past Etot are zero in G
+                // every element of the chunk: those past Ecorr are zero in G
                 for (int g0 = 0; g0 < CH; g0 += GE) {
                     if (g0 > 0) { // the next elements' table
                         __syncthreads();
@@ -4573,21 +4565,6 @@ extern "C" int blfid_dev_launch_expdyson_d(int M, const DevPlan *P, int Kb, int 
     return (int)hipGetLastError();
 }
 
-template <typename R>
-static void launch_dyson(int M, const DevPlan *P, int Kb, const int *grp, int ngrp, int grid,
-                         const void *bufU, void *bufA, hipStream_t st) {
-    typedef typename CX<R>::T CT;
-    const CT *U = (const CT *)bufU;
-    CT *A = (CT *)bufA;
-    switch (M) {
-    case 1: LAUNCH_SPLIT(k_dyson, 1, R, grid, 64, st, *P, Kb, grp, ngrp, U, A); break;
-    case 2: LAUNCH_SPLIT(k_dyson, 2, R, grid, 256, st, *P, Kb, grp, ngrp, U, A); break;
-    case 3: LAUNCH_SPLIT(k_dyson, 3, R, grid, 256, st, *P, Kb, grp, ngrp, U, A); break;
-    case 4: LAUNCH_SPLIT(k_dyson, 4, R, grid, 256, st, *P, Kb, grp, ngrp, U, A); break;
-    default: LAUNCH_SPLIT(k_dyson, 5, R, grid, 256, st, *P, Kb, grp, ngrp, U, A); break;
-    }
-}
-
 // The first nbig blocks of grp have more than DEV_LDS_BLOCK states (at most bmax): wave tiles, but
 // in the BF16x3 form.  FP64 chains of smaller blocks are k_expdyson_d's.
 extern "C" int blfid_dev_launch_dyson(int prec, int M, const DevPlan *P, int Kb, const int *grp,
@@ -4606,7 +4583,21 @@ extern "C" int blfid_dev_launch_dyson(int prec, int M, const DevPlan *P, int Kb,
     }
     const long ntask = (long)Kb * ngrp;
     const int grid = (int)(ntask < cap ? ntask : cap);
-    if (grid > 0 && prec) launch_dyson<float>(M, P, Kb, grp, ngrp, grid, bufU, bufA, st);
+    if (grid <= 0 || !prec) return (int)hipGetLastError();
+#define DYSON_LAUNCH(M_)                                                                         \
+    do {                                                                                         \
+        const cf *U = (const cf *)bufU;                                                          \
+        if (P->bf16x3) k_dyson<M_, true><<<grid, NThr<M_>::v, 0, st>>>(*P, Kb, grp, ngrp, U, (cf *)bufA); \
+        else k_dyson<M_, false><<<grid, NThr<M_>::v, 0, st>>>(*P, Kb, grp, ngrp, U, (cf *)bufA); \
+    } while (0)
+    switch (M) {
+    case 1: DYSON_LAUNCH(1); break;
+    case 2: DYSON_LAUNCH(2); break;
+    case 3: DYSON_LAUNCH(3); break;
+    case 4: DYSON_LAUNCH(4); break;
+    default: DYSON_LAUNCH(5); break;
+    }
+#undef DYSON_LAUNCH
     return (int)hipGetLastError();
 }
 
