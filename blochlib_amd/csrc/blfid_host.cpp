@@ -673,30 +673,39 @@ static blfid_status build_tables(blfid_plan *pl) {
             pl->ff_term.insert(pl->ff_term.end(), lists[q].begin(), lists[q].end());
             pl->ff_off[q + 1] = (int)pl->ff_term.size();
         }
-        // The same Hamiltonian as quadratic forms in v = R_P^T u for the fused kernel: with
-        // w = (vx^2, vy^2, vz^2, 2 vx vy, 2 vx vz, 2 vy vz) every term's zz_t = C_t . w, so the
-        // diagonal of basis state a is xd_cst[a] . (1, w) and the flip-flop coefficient of the
-        // ordered pair (i, j) is xd_fpr[i S + j] . (1, w) (entry 0 holds the constant part).
+        // The same Hamiltonian as quadratic forms in v = R_P^T u for the fused kernels (of spinning
+        // and pulse plans): with w = (vx^2, vy^2, vz^2, 2 vx vy, 2 vx vz, 2 vy vz) every term's
+        // zz_t = C_t . w, so the diagonal of basis state a is xd_cst[a] . (1, w) and the flip-flop
+        // coefficient of the ordered pair (i, j) is xd_fpr[i S + j] . (1, w) (entry 0 holds the
+        // constant part).  A term's sign in state a is the parity of a on its spins' bits, so the
+        // diagonals are the Walsh-Hadamard transform of the terms put at those bits: N log N sums.
         const int nt = (int)(pl->terms.size() / DEV_TERM_STRIDE);
-        pl->xd_cst.assign((size_t)N * 7, 0.0);
-        std::vector<ext> up(tens.size()); // each term with its spins up: other states change its sign
-        std::vector<int> flips(nt);       // bits of its spins
-        for (int t = 0; t < nt; t++) {
-            const double *c = &pl->terms[DEV_TERM_STRIDE * t];
-            const int i = (int)c[8], j = (int)c[9];
-            flips[t] = 1 << (S - 1 - i) | (j >= 0 ? 1 << (S - 1 - j) : 0);
-            for (int q = 0; q < 6; q++) up[6 * t + q] = (j >= 0 ? 0.25 : 0.5) * c[6] * tens[6 * t + q];
-        }
-        for (int a = 0; a < N; a++) {
-            ext o[7] = {dconst[a]};
+        const bool fused = pl->spinning || pl->ptop;
+        pl->xd_cst.assign(fused ? (size_t)N * 7 : 0, 0.0);
+        if (fused) {
+            std::vector<ext> f((size_t)N * 6, 0);
             for (int t = 0; t < nt; t++) {
-                const ext sign = 1 - 2 * __builtin_parity(a & flips[t]), *c = &up[6 * t];
-                for (int q = 0; q < 6; q++) o[1 + q] += sign * c[q];
+                const double *c = &pl->terms[DEV_TERM_STRIDE * t];
+                const int i = (int)c[8], j = (int)c[9];
+                ext *o = &f[6 * (size_t)(1 << (S - 1 - i) | (j >= 0 ? 1 << (S - 1 - j) : 0))];
+                for (int q = 0; q < 6; q++) o[q] += (j >= 0 ? 0.25 : 0.5) * c[6] * tens[6 * t + q];
             }
-            std::copy(o, o + 7, &pl->xd_cst[(size_t)a * 7]);
+            for (int h = 1; h < N; h *= 2)
+                for (int a = 0; a < N; a++)
+                    if (!(a & h))
+                        for (int q = 0; q < 6; q++) {
+                            ext &x = f[6 * (size_t)a + q], &y = f[6 * (size_t)(a + h) + q];
+                            const ext u = x, v = y;
+                            x = u + v;
+                            y = u - v;
+                        }
+            for (int a = 0; a < N; a++) {
+                pl->xd_cst[(size_t)a * 7] = (double)dconst[a];
+                std::copy(&f[6 * (size_t)a], &f[6 * (size_t)a] + 6, &pl->xd_cst[(size_t)a * 7 + 1]);
+            }
         }
-        pl->xd_fpr.assign((size_t)S * S * 7, 0.0);
-        for (size_t q = 0; q < lists.size(); q++) {
+        pl->xd_fpr.assign(fused ? (size_t)S * S * 7 : 0, 0.0);
+        for (size_t q = 0; q < lists.size() && fused; q++) {
             ext o[7] = {ffconst[q]};
             for (int t : lists[q])
                 for (int k = 0; k < 6; k++) o[1 + k] += pl->terms[DEV_TERM_STRIDE * t + 7] * tens[6 * t + k];
