@@ -362,6 +362,68 @@ template <typename T> struct DevTab {
     T *p = nullptr;
 };
 
+// Synchronous copies that do not wait for other streams' work.  A copy of up to 16 KiB is a kernel on
+// the null stream's hardware queue, one of four that all streams of a process share, and waits there
+// for everything a stream on the same queue has been given; a larger one from or to pageable memory
+// waits there whenever the runtime's 4 MiB of staging have been used up.  In a server of four streams
+// the set-up of a plan took up to 0.8 s that way.  Copies of more than 16 KiB between pinned memory and
+// the device never wait (9 us, where one of 16 KiB pageable takes 14 us), so these go through a
+// pinned buffer in pieces of COPY_LEAST to COPY_PIECE bytes: short ones copy COPY_LEAST bytes (the
+// device block must hold as many).  One buffer per process, a quarter MiB, made on first use.
+constexpr size_t COPY_LEAST = 16640, COPY_PIECE = (size_t)256 << 10;
+class CopyStage {
+    std::mutex mu;
+    char *pin = nullptr;
+    unsigned long long id = 0;
+
+    bool ready() {
+        if (pin && id && DevBlock::id_of(pin) != id) pin = nullptr; // went with a hipDeviceReset
+        if (!pin) {
+            if (hipHostMalloc((void **)&pin, COPY_PIECE, hipHostMallocPortable) != hipSuccess) {
+                (void)hipGetLastError();
+                pin = nullptr;
+            } else {
+                id = DevBlock::id_of(pin);
+            }
+        }
+        return pin != nullptr;
+    }
+    static size_t piece(size_t left) {
+        return left <= COPY_PIECE ? left : left < COPY_PIECE + COPY_LEAST ? left / 2 : COPY_PIECE;
+    }
+
+  public:
+    hipError_t to_device(void *dst, const void *src, size_t bytes) {
+        std::lock_guard<std::mutex> lk(mu);
+        if (!ready()) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+        hipError_t e = hipSuccess;
+        for (size_t o = 0; o < bytes && e == hipSuccess;) {
+            const size_t n = piece(bytes - o);
+            std::memcpy(pin, (const char *)src + o, n);
+            e = hipMemcpy((char *)dst + o, pin, std::max(n, COPY_LEAST), hipMemcpyHostToDevice);
+            o += n;
+        }
+        return e;
+    }
+    hipError_t to_host(void *dst, const void *src, size_t bytes) {
+        std::lock_guard<std::mutex> lk(mu);
+        if (!ready()) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+        hipError_t e = hipSuccess;
+        for (size_t o = 0; o < bytes && e == hipSuccess;) {
+            const size_t n = piece(bytes - o);
+            e = hipMemcpy(pin, (const char *)src + o, std::max(n, COPY_LEAST), hipMemcpyDeviceToHost);
+            if (e == hipSuccess) std::memcpy((char *)dst + o, pin, n);
+            o += n;
+        }
+        return e;
+    }
+};
+// never destroyed, as the block cache
+CopyStage &copy_stage() {
+    static CopyStage *c = new CopyStage();
+    return *c;
+}
+
 // Host tables gathered into one device block with one copy; every table starts on 256 bytes.
 class Tables {
     std::vector<char> h;
@@ -376,8 +438,8 @@ class Tables {
         at.push_back({(void **)&t.p, o});
     }
     hipError_t commit(DevBuf<char> &buf) {
-        hipError_t e = buf.alloc(h.size());
-        if (e == hipSuccess) e = hipMemcpy(buf.p, h.data(), h.size(), hipMemcpyHostToDevice);
+        hipError_t e = buf.alloc(std::max(h.size(), COPY_LEAST));
+        if (e == hipSuccess) e = copy_stage().to_device(buf.p, h.data(), h.size());
         for (auto &q : at) *q.first = e == hipSuccess ? buf.p + q.second : nullptr;
         return e;
     }
@@ -511,7 +573,7 @@ struct blfid_plan {
     double2 *bufW = nullptr;
     double *thetas = nullptr, *part = nullptr, *grp = nullptr;
     double2 *scrEig = nullptr;
-    DevBuf<double> fid_out;
+    DevBuf<double> fid_out; // at least COPY_LEAST bytes
     DevBuf<double> d_expflops; // propagator flop counters while profiling
     double budget = 0;
     int Kb = 0;
@@ -2041,7 +2103,7 @@ static blfid_status run_upto(blfid_plan *pl, int normalize, hipStream_t st, int 
         HIPCHK(pl->own_ws.alloc(need, (size_t)avail));
         base = pl->own_ws.p;
     }
-    HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
+    HIPCHK(pl->fid_out.alloc(std::max<size_t>((size_t)2 * pl->npts, COPY_LEAST / sizeof(double))));
     blfid_status rs = enqueue_range(pl, sh, base, off, Kb, normalize, pl->fid_out.p, st, 0,
                                     c_end, true, true);
     pl->ran = rs == BLFID_OK && c_end == pl->K;
@@ -2113,8 +2175,8 @@ static blfid_status state_fill(blfid_state *st, const double *rho, int all, hipS
             HIPCHK(hipMemcpyAsync(st->rho.p, rho, (size_t)st->K * NN * sizeof(double2),
                                   hipMemcpyHostToDevice, s));
     } else {
-        HIPCHK(st->rho0.alloc(NN));
-        HIPCHK(hipMemcpy(st->rho0.p, rho, NN * sizeof(double2), hipMemcpyHostToDevice));
+        HIPCHK(st->rho0.alloc(std::max(NN, COPY_LEAST / sizeof(double2))));
+        HIPCHK(copy_stage().to_device(st->rho0.p, rho, NN * sizeof(double2)));
         LAUNCHCHK(blfid_dev_launch_state_fill(st->K, st->N, st->rho0.p, st->rho.p, s));
     }
     HIPCHK(hipStreamSynchronize(s));
@@ -2133,8 +2195,8 @@ blfid_status blfid_state_project(blfid_state *st, const double *op, void *stream
     if (!(nrm > 0.0)) return fail(BLFID_ERR_INVALID, "the cycler operator is zero");
     hipStream_t s = (hipStream_t)stream;
     HIPCHK(hipStreamSynchronize(s)); // the staging buffer may still feed earlier work
-    HIPCHK(st->rho0.alloc(NN));
-    HIPCHK(hipMemcpy(st->rho0.p, op, NN * sizeof(double2), hipMemcpyHostToDevice));
+    HIPCHK(st->rho0.alloc(std::max(NN, COPY_LEAST / sizeof(double2))));
+    HIPCHK(copy_stage().to_device(st->rho0.p, op, NN * sizeof(double2)));
     LAUNCHCHK(blfid_dev_launch_state_project(st->K, st->N, st->rho0.p, 1.0 / nrm, st->rho.p, s));
     HIPCHK(hipStreamSynchronize(s));
     return BLFID_OK;
@@ -2314,7 +2376,7 @@ blfid_status blfid_plan_graph_capture(blfid_plan *pl, int normalize) {
     size_t off[blfid_layout::R_COUNT];
     const size_t need = blfid_layout::layout_bytes(sh, Kb, off);
     HIPCHK(pl->own_ws.alloc(need, (size_t)avail));
-    HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
+    HIPCHK(pl->fid_out.alloc(std::max<size_t>((size_t)2 * pl->npts, COPY_LEAST / sizeof(double))));
     if (pl->gexec) (void)hipGraphExecDestroy(pl->gexec);
     if (pl->graph) (void)hipGraphDestroy(pl->graph);
     pl->gexec = nullptr;
@@ -2382,7 +2444,7 @@ blfid_status blfid_plan_run_slice(blfid_plan *pl, int c_begin, int c_end, int no
         const long Kb = blfid_layout::fit_batch(sh, psh, pl->K, avail, &pl->sl_cuts);
         if (Kb < 1) return fail(BLFID_ERR_NOMEM, "one crystallite does not fit the memory budget");
         HIPCHK(pl->own_ws.alloc(blfid_layout::layout_bytes(sh, Kb), (size_t)avail));
-        HIPCHK(pl->fid_out.alloc((size_t)2 * pl->npts));
+        HIPCHK(pl->fid_out.alloc(std::max<size_t>((size_t)2 * pl->npts, COPY_LEAST / sizeof(double))));
         pl->sl_Kb = Kb;
         pl->sl_gen = pl->gen;
         pl->sl_norm = normalize;
@@ -2786,7 +2848,7 @@ blfid_status blfid_plan_fetch(blfid_plan *pl, double *out) {
     if (!pl || !out) return fail(BLFID_ERR_INVALID, "NULL argument");
     if (!pl->ran) return fail(BLFID_ERR_INVALID, "plan has not been run");
     HIPCHK(hipStreamSynchronize(pl->last_stream));
-    HIPCHK(hipMemcpy(out, pl->fid_out.p, sizeof(double) * 2 * pl->npts, hipMemcpyDeviceToHost));
+    HIPCHK(copy_stage().to_host(out, pl->fid_out.p, sizeof(double) * 2 * pl->npts));
     return BLFID_OK;
 }
 

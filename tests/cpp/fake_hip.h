@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 
@@ -22,6 +23,7 @@ static std::map<size_t, Range> mem; // by address
 static size_t limit = (size_t)64 << 30, used = 0;
 static unsigned long long next_id = 1;
 static long n_malloc = 0, n_free = 0, n_sync = 0;
+static size_t copy_min = SIZE_MAX, copy_max = 0; // sizes of the synchronous copies
 static hipError_t last = hipSuccess;
 
 static hipError_t err(hipError_t e) {
@@ -60,12 +62,18 @@ static void reset() {
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) { return fake::alloc(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = std::malloc(n); return *p ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipFree(void *p) { return p ? fake::release(p) : hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *, size_t n, hipMemcpyKind k) {
+    fake::copy_min = n < fake::copy_min ? n : fake::copy_min;
+    fake::copy_max = n > fake::copy_max ? n : fake::copy_max;
     if (k == hipMemcpyDeviceToHost) std::memset(d, 0, n);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *, size_t n, hipMemcpyKind k, hipStream_t) {
+    if (k == hipMemcpyDeviceToHost) std::memset(d, 0, n);
+    return hipSuccess;
+}
 hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) {
     *f = fake::limit - fake::used;

@@ -252,8 +252,26 @@ static void accepted() {
     }
 }
 
+// Hand-overs and fetches copy in pieces of more than 16 KiB that fit the pinned buffer, whatever the
+// size of the plan's tables and of its FID.
+static void copies() {
+    fake::limit = (size_t)256 << 30;
+    for (int S : {1, 3, 10})
+        for (int npts : {1, 64, 1039, 1040, 1041, 5000, 400000}) {
+            blfid_plan *p = plan(S, 16, npts, BLFID_FP64, S == 3 ? 200000 : 7, true);
+            REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+            std::vector<double> fid(2 * npts + 1, 1.5);
+            REQUIRE(blfid_plan_fetch(p, fid.data()) == BLFID_OK);
+            REQUIRE(fid[2 * npts] == 1.5 && fid[2 * npts - 1] == 0.0); // the whole FID and no more
+            REQUIRE(p->fid_out.blk.bytes >= std::max((size_t)16 * npts, COPY_LEAST));
+            blfid_plan_destroy(p);
+            if (S == 10 && npts > 1) break;
+        }
+    REQUIRE(fake::copy_min > 16 * 1024 && fake::copy_max <= COPY_PIECE);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}, {"copies", copies}};
     std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
