@@ -101,9 +101,10 @@ def corr_is_autocorrelation(wls) -> bool:
     return True
 
 
-# What each kernel family issues on MI355X, per precision: "mfma" where its products run on the
-# matrix cores (complex64 Dyson chain, B = A W and Q products), "valu" where they run on the
-# vector ALUs (the propagator's real Taylor GEMMs, the FFT correlation, every FP64 product).
+# What each kernel family of the complex64 form issues on MI355X: "mfma" where its products run on
+# the matrix cores, "valu" where they run on the vector ALUs (the propagator's real products up to 80
+# states outside the fused chain, the FFT correlation, the eigen-solver).  The FP64 form's products
+# run on FP64 matrix cores, whose published rate equals the vector rate: it is rated as "valu".
 ISSUES = {"k_exp": "valu", "k_dyson": "mfma", "k_expdyson": "mfma", "k_bmul": "mfma", "k_qr": "mfma",
           "k_corr": "valu", "k_eig": "valu", "k_reduce": "valu", "k_static_fid": "valu"}
 

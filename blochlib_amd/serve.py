@@ -213,8 +213,9 @@ class FIDServer:
 
     def slice_size(self, p: engine.Plan, K: int) -> int:
         """Crystallites per slice: about slice_flops of the plan's work, but enough that the
-        per-(crystallite, block) launches (the eigen-solver's, one workgroup each) still have
-        fill_tasks workgroups, at least min_slice, at most the whole powder."""
+        launches of one workgroup per crystallite and block (the propagator chains and, up to 80
+        states, the eigen-solver) still have fill_tasks workgroups, at least min_slice, at most the
+        whole powder.  On the 48-request mix: makespan 32.7 s at 1024, 34.1 at 512, 34.9 at 64."""
         st = p.stats()
         per = max(st["flops_per_cs"] * max(p.steps, 1), 1.0)
         fill = -(-self.fill_tasks // max(int(st["blocks"]), 1))
