@@ -1687,7 +1687,8 @@ static double pair_elems(const blfid_plan *pl, const std::vector<int> &g) {
     return s;
 }
 
-static blfid_layout::Shape shape_of(const blfid_plan *pl) {
+// any_powder: with the scratch slots of an arbitrarily large powder
+static blfid_layout::Shape shape_of(const blfid_plan *pl, bool any_powder = false) {
     blfid_layout::Shape s;
     s.prec = pl->prec;
     s.kind = pl->ptop ? 2 : (pl->spinning ? 0 : 1);
@@ -1705,7 +1706,7 @@ static blfid_layout::Shape shape_of(const blfid_plan *pl) {
     s.Estr = pl->Estr;
     s.K = pl->K;
     s.rho_elems = (pl->prep || pl->state) ? pl->Etot : 0;
-    if (pl->K > 0) {
+    if (pl->K > 0 && !any_powder) {
         // no more scratch slots than the largest launch has tasks (a few crystallites: the
         // slots were most of the plan's storage)
         auto tasks = [&](const std::map<int, std::vector<int>> &g) {
@@ -1732,8 +1733,9 @@ static blfid_layout::Shape prep_shape_of(const blfid_plan *pp) {
 }
 
 // The plan's layout with its preparation's (ps, referenced by s.prep) when it has one.
-static void full_shape(const blfid_plan *pl, blfid_layout::Shape &s, blfid_layout::Shape &ps) {
-    s = shape_of(pl);
+static void full_shape(const blfid_plan *pl, blfid_layout::Shape &s, blfid_layout::Shape &ps,
+                       bool any_powder = false) {
+    s = shape_of(pl, any_powder);
     if (pl->prep) {
         ps = prep_shape_of(pl->prep);
         s.prep = &ps;
@@ -1781,7 +1783,7 @@ blfid_status blfid_plan_stats(const blfid_plan *pl, double *out) {
     out[3] = (double)pl->bmax;
     out[4] = bytes_per_crystallite(pl);
     blfid_layout::Shape sh, ps;
-    full_shape(pl, sh, ps);
+    full_shape(pl, sh, ps, true); // a budget made from it holds for the plan's next powder too
     out[5] = (double)blfid_layout::layout_bytes(sh, 0);
     return BLFID_OK;
 }

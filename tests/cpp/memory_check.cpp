@@ -270,8 +270,28 @@ static void copies() {
     REQUIRE(fake::copy_min > 16 * 1024 && fake::copy_max <= COPY_PIECE);
 }
 
+// The fixed storage that blfid_plan_stats names is that of any powder: a budget made from it for a
+// batch of crystallites holds the batch after the plan is given a larger powder.
+static void footprint() {
+    fake::limit = (size_t)256 << 30;
+    for (auto prec : {BLFID_FP64, BLFID_C64})
+        for (int S : {5, 8, 9}) {
+            blfid_plan *p = plan(S, 32, 256, prec, 10);
+            double st[6];
+            REQUIRE(blfid_plan_stats(p, st) == BLFID_OK);
+            const double budget = st[5] + 64 * st[4];
+            const size_t group = blfid_layout::ngroups(3000) * 4 * 256 * 8 / (size_t)st[4] + 1;
+            std::vector<double> a(3000, 0.3);
+            REQUIRE(blfid_plan_set_powder(p, a.data(), a.data(), a.data(), a.data(), 3000) == BLFID_OK);
+            REQUIRE(blfid_plan_set_memory_budget(p, budget) == BLFID_OK);
+            REQUIRE(blfid_plan_run(p, 1, nullptr) == BLFID_OK);
+            REQUIRE(p->Kb + (int)group >= 64);
+            blfid_plan_destroy(p);
+        }
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}, {"copies", copies}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}, {"copies", copies}, {"footprint", footprint}};
     std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();
