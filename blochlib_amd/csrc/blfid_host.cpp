@@ -1147,6 +1147,10 @@ blfid_status blfid_plan_create(const blfid_system *sys, double wr_hz, double rot
             delete pl;
             return fail(BLFID_ERR_INVALID, "sw/wr rounds to zero steps per rotor period");
         }
+        if (n > CORR_SPAN) { // the correlation holds a period of one element on chip
+            delete pl;
+            return fail(BLFID_ERR_UNSUPPORTED, "more than " + std::to_string(CORR_SPAN) + " steps per rotor period (sw/wr)");
+        }
         pl->n = n;
         pl->sw_adj = (double)(n * wr_hz);
         double tmin = t0, tmax = t0 + 1.0 / wr_hz;

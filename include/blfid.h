@@ -74,7 +74,8 @@ typedef struct blfid_plan blfid_plan;
 
 /* Plan for one spin system and one acquisition: replaces constructing
  * oneFID(sys, npts, sw, wr, rotor_deg, t0) (oneFID.h:103-108) + compute(sys, wr, sw, t0, t0+1/wr)
- * (compute.h:213-235).  wr == 0 or rotor_deg == 0 selects the static FID (oneFID.h:216). */
+ * (compute.h:213-235).  wr == 0 or rotor_deg == 0 selects the static FID (oneFID.h:216).  A spinning
+ * plan has at most 2048 steps per rotor period (sw/wr); more are BLFID_ERR_UNSUPPORTED. */
 blfid_status blfid_plan_create(const blfid_system *sys, double wr_hz, double rotor_deg,
                                double sw_hz, int npts, double t0, blfid_precision prec,
                                blfid_plan **out);

@@ -290,8 +290,25 @@ static void footprint() {
         }
 }
 
+// Steps per period beyond what the correlation kernel holds on chip are refused, the most it holds
+// are not.
+static void steps() {
+    Sys sy(2);
+    blfid_plan *p = nullptr;
+    for (int n : {2049, 3000, 100000}) {
+        REQUIRE(blfid_plan_create(&sy.s, 10.0, 54.7356, 10.0 * n, 64, 0.0, BLFID_FP64, &p) == BLFID_ERR_UNSUPPORTED && !p);
+        REQUIRE(corr_chunk(n) * (long)n > CORR_SPAN);
+    }
+    for (int n = 1; n <= 2048; n++) {
+        REQUIRE(corr_use_fft(n) || corr_chunk(n) * n <= CORR_SPAN);
+        REQUIRE(corr_use_fft(n) || corr_chunk(n) * ((n + CORR_PPT - 1) / CORR_PPT) <= 256);
+    }
+    REQUIRE(blfid_plan_create(&sy.s, 10.0, 54.7356, 10.0 * 2048, 64, 0.0, BLFID_FP64, &p) == BLFID_OK);
+    blfid_plan_destroy(p);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}, {"copies", copies}, {"footprint", footprint}};
+    const std::map<std::string, std::function<void()>> checks = {{"workspace", workspace}, {"release", release}, {"reset", reset}, {"budget", budget}, {"age", age}, {"host_memory", host_memory}, {"accepted", accepted}, {"copies", copies}, {"footprint", footprint}, {"steps", steps}};
     std::setvbuf(stdout, nullptr, _IONBF, 0);
     if (argc != 2 || !checks.count(argv[1])) return 2;
     checks.at(argv[1])();

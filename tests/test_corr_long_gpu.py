@@ -22,3 +22,15 @@ def test_long_fid(n, npts):
     c, _ = O.powder_fid(sy, WR, workloads.MAGIC_DEG, n * WR, npts, pw, rho, det)
     g, _ = engine.powder_fid(sy, WR, workloads.MAGIC_DEG, n * WR, npts, pw, rho, det)
     assert np.linalg.norm(g - c) < 1e-10 * np.linalg.norm(c)
+
+
+# step counts whose periods are only just held on chip, one element at a time
+@pytest.mark.parametrize("n,npts", [(513, 700), (1024, 2100), (1025, 1500), (2047, 2500), (2048, 900)])
+def test_many_steps(n, npts):
+    sy = workloads.small_cluster(3, 33)
+    pw = zcw(1154).subset(np.array([100, 801]))
+    rho, det = sy.op("Iy_0+0.5*Iz_1"), sy.op("Ip")
+    print(f"[corr] n={n} npts={npts}", flush=True)
+    c, _ = O.powder_fid(sy, 100.0, workloads.MAGIC_DEG, n * 100.0, npts, pw, rho, det)
+    g, _ = engine.powder_fid(sy, 100.0, workloads.MAGIC_DEG, n * 100.0, npts, pw, rho, det)
+    assert np.linalg.norm(g - c) < 1e-10 * np.linalg.norm(c)

@@ -7,7 +7,7 @@ import subprocess
 import pytest
 
 CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
-CHECKS = ["workspace", "release", "reset", "budget", "age", "host_memory", "accepted", "copies", "footprint"]
+CHECKS = ["workspace", "release", "reset", "budget", "age", "host_memory", "accepted", "copies", "footprint", "steps"]
 
 
 @pytest.fixture(scope="module")
